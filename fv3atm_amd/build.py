@@ -28,6 +28,7 @@ HIP_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17", "-Wall", "-
 HIP_SOURCES = {
     "tp_plain.hip": ["-ffp-contract=off"],
     "mapz_plain.hip": ["-ffp-contract=off"],
+    "mapz_fields.hip": ["-ffp-contract=off"],
     "capi.hip": ["-ffp-contract=off"],
     "fused.hip": ["-ffp-contract=off"],
     "fused32.hip": ["-ffp-contract=fast"],  # compiled once per part (FUSED32_NPART)

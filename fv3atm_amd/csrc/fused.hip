@@ -7,6 +7,7 @@
 #include "fused.h"
 #include "fused_kernel.h"
 #include "mapz_fast.h"
+#include "mapz_fields.h"
 
 namespace fv3 {
 
@@ -56,6 +57,11 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   // the host-array entry points run the transport alone (c.transport_only)
   const bool remap_phase = !c.transport_only;
   const bool fast_remap = remap_phase && std::is_same<T, float>::value && c.remap_mode != 1 && npz >= 8;
+  // the FP64 remap of the column tables (mapz_fields.hip), out of place too
+  const bool fields = remap_phase && std::is_same<T, double>::value && npz <= FIELDS_MAX_KM;
+  std::vector<int> kt(nq, kord_tr);
+  if (fields && remap_orders_check(npz, nq, kt.data(), pt != nullptr, kord_tm)) return 1;
+  const bool oop = fast_remap || fields;
   // the per-column remap synchronises the host with the stream, so only the
   // column-shared FP32 remap can be captured
   if (c.graph_safe && !fast_remap)
@@ -100,10 +106,11 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     if (cap < 1) return set_error("nsplit < 1 from a non-finite Courant number");
     c.last_nsplit = h;
   }
-  // The FP32 form remaps out of place: the last transport pass of every
+  // The remap runs out of place: the last transport pass of every
   // level lands in q_tmp (the caller's q_out serves as the alternate pass
   // buffer), and the remap writes q_out.
   T *q_tmp = nullptr, *pt_src = nullptr;
+  char *tab = nullptr;  // the column tables
   std::vector<RemapCols> cols(nt);  // column data of every tile
   if (fast_remap) {
     if (remap_fast_check(npz, (long long)ni * nj, d.s2, kord_tr, kord_tm, pt != nullptr)) return 1;
@@ -112,6 +119,12 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     q_tmp = (T *)sc;
     pt_src = pt ? (T *)(sc + b_q) : nullptr;
     for (int t = 0; t < nt; t++) cols[t] = remap_cols_carve(sc + b_q + b_pt + b_col * t, npz, (long long)ni * nj);
+  } else if (fields) {
+    char *sc = (char *)ctx_scratch(c, b_q + b_pt + coltab_bytes<T>(npz, (long long)ni * nj * nt));
+    if (!sc) return 1;
+    q_tmp = (T *)sc;
+    pt_src = pt ? (T *)(sc + b_q) : nullptr;
+    tab = sc + b_q + b_pt;
   } else if (cap > 1) {
     q_tmp = (T *)ctx_scratch(c, sizeof(T) * qsize);
     if (!q_tmp) return 1;
@@ -162,8 +175,8 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   }
   a.nsplit = nspl;
   a.q_in = q_in;
-  a.q_out = fast_remap ? q_tmp : q_out;
-  a.q_tmp = fast_remap ? q_out : q_tmp;
+  a.q_out = oop ? q_tmp : q_out;
+  a.q_tmp = oop ? q_out : q_tmp;
   a.cx = cx; a.cy = cy; a.mfx = mfx; a.mfy = mfy; a.dp1 = dp1;
   const GridDev<T> &g = grid_of<T>(c);
   a.area = g.area; a.rarea = g.rarea; a.dxa = g.dxa; a.dya = g.dya; a.dx = g.dx; a.dy = g.dy;
@@ -290,8 +303,25 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
       }
     }
   }
-  if (!fast_remap && remap_phase) {
-    std::vector<int> kt(nq, kord_tr);
+  if (fields) {
+    FieldsArgs<T> fa{};
+    fa.tab = coltab_carve<T>(tab, npz, (long long)ni * nj * nt);
+    ColSource cs{};
+    cs.ptop = ptop;
+    cs.ak = ak;
+    cs.bk = bk;
+    cs.delp = cs.delp_out = delp_out;
+    if (fields_prep<T>(c, fa.tab, cs, ni, nj, false)) return 1;
+    fa.set[fa.nset++] = tracer_set<T>(c, q_tmp, q_out, nq);
+    for (int iq = 0; iq <= nq; iq++) fa.kord[iq] = (signed char)std::min(iq < nq ? kord_tr : kord_tm, 17);
+    if (pt) {
+      FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(T) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, s));
+      FieldSet<T> &x = fa.set[fa.nset++] = cell_set<T>(c, pt_src, pt, 1);
+      x.use_qmin = true;
+      x.qmin = (T)t_min;
+    }
+    if (fields_run<T>(c, fa, ni, nj)) return 1;
+  } else if (!fast_remap && remap_phase) {
     if (remap_tracers_plain<T>(c, npz, nq, ak, bk, ptop, delp_out, q_out, pt, kt.data(), kord_tm,
                                t_min, 0))
       return 1;
@@ -301,6 +331,7 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     c.last_passes = cap;
     c.ev_valid = true;
   }
+  if (fields) FV3_HIP(hipStreamSynchronize(s));  // FP64 steps return when they are done
   if (nsplit_cap > 0 && !c.graph_safe) {
     int hf = 0;
     FV3_HIP(hipMemcpyAsync(&hf, flag, sizeof(int), hipMemcpyDeviceToHost, s));

@@ -9,10 +9,9 @@
 // (ccpp/data/CCPP_typedefs.F90:434-504, kmp by the rule at :1714-1718), and
 // a total-energy fix-up with compensated FP64 global sums.
 //
-// Every column goes through the plain column kernel (mapz_column.h: one
-// thread per column, upstream evaluation order), so the FP64 form matches a
-// CPU FP64 evaluation; fields the kernel does not address in place are
-// gathered into [level][column] buffers and scattered back.
+// Every column is remapped in upstream evaluation order (mapz_fields.hip: one
+// thread per column and field over shared column tables), so the FP64 form
+// matches a CPU FP64 evaluation.
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -20,6 +19,7 @@
 #include "../../include/fv3atm_amd.h"
 #include "fv3_internal.h"
 #include "mapz_column.h"
+#include "mapz_fields.h"
 
 namespace fv3 {
 
@@ -114,9 +114,10 @@ __global__ void k_gather(T *field, T *buf, int dir, int km, int wi, long long nc
     *f = buf[idx];
 }
 
-// delz <-> -delz/delp (before: dp is the Lagrangian delp; after: dp2 from pe2)
+// delz <-> -delz/delp (delp: the Lagrangian thickness before the remap, the
+// Eulerian one after it)
 template <typename T>
-__global__ void k_delz(Geo g, int t, int dir, T *dz, const double *delp, const double *pe2) {
+__global__ void k_delz(Geo g, int t, int dir, T *dz, const double *delp) {
   const long long nc = (long long)g.ni * g.nj;
   const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= nc * g.km) return;
@@ -124,10 +125,8 @@ __global__ void k_delz(Geo g, int t, int dir, T *dz, const double *delp, const d
   const int k = (int)(idx / nc) + 1;
   const int i = g.is + (int)(col % g.ni), j = g.js + (int)(col / g.ni);
   T *p = dz + t * g.spz + idx;
-  if (dir == 0)
-    *p = -*p / T(delp[((long long)t * g.km + (k - 1)) * g.s2 + (long long)(j - g.jsd) * g.nid + (i - g.isd)]);
-  else
-    *p = -*p * T(pe2[(long long)k * nc + col] - pe2[(long long)(k - 1) * nc + col]);
+  const T dp = T(delp[((long long)t * g.km + (k - 1)) * g.s2 + (long long)(j - g.jsd) * g.nid + (i - g.isd)]);
+  *p = dir == 0 ? -*p / dp : -*p * dp;
 }
 
 // column total energy sum_k (cp pt pkz + (ua^2 + va^2)/2) dp; dp from delp
@@ -334,8 +333,9 @@ int l2e_full(Ctx &c, const fv3_l2e_args &a) {
     off += (b + 255) & ~(size_t)255;
     return o;
   };
-  const size_t o_pe1 = take(sizeof(double) * (km + 1) * ncmax), o_pe2 = take(sizeof(double) * (km + 1) * ncmax);
-  const size_t o_buf = take(sizeof(T) * km * ncmax), o_ws = take(sizeof(T) * ncmax);
+  const long long ncol = km > FIELDS_MAX_KM ? ncmax : 0;  // of the one-thread-per-column form
+  const size_t o_pe1 = take(sizeof(double) * (km + 1) * ncol), o_pe2 = take(sizeof(double) * (km + 1) * ncol);
+  const size_t o_buf = take(sizeof(T) * km * ncol), o_ws = take(sizeof(T) * ncol);
   const size_t o_e = take(sizeof(double) * 3 * ncell), o_part = take(sizeof(KS) * KS_GRID * 3);
   const size_t o_sum = take(sizeof(double) * 4);
   char *base = (char *)l2e_arena(c, off);
@@ -355,65 +355,121 @@ int l2e_full(Ctx &c, const fv3_l2e_args &a) {
   }
   FV3_HIP(hipGetLastError());
 
-  // one field of tile t over the columns of a kind through the column kernel
-  auto remap_kind = [&](int t, int kind, T *field, long long lev, int ld, int di, int dj, int iv, int kord,
-                        const T *qs) -> int {
-    const int wi = kind == 2 ? g.ni + 1 : g.ni, wj = kind == 1 ? g.nj + 1 : g.nj;
-    const long long nc = (long long)wi * wj;
-    hipLaunchKernelGGL(k_col_pressures, grid1(nc), dim3(256), 0, s, g, t, kind, a.ptop, a.ak, a.bk, a.pe, a.ps,
-                       pe1, pe2, nc);
-    hipLaunchKernelGGL(k_gather<T>, grid1(nc * km), dim3(256), 0, s, field, buf, 0, km, wi, nc, lev, ld, di, dj);
-    FV3_HIP(hipGetLastError());
-    RemapArgs<T> r{};
-    r.mode = 1;
-    r.km = km;
-    r.kn = km;
-    r.ncol = nc;
-    r.pe1_in = pe1;
-    r.pe2_in = pe2;
-    r.q1_in = buf;
-    r.q2_out = buf;
-    r.qs_in = qs;
-    r.q1_stride = nc;
-    r.q2_stride = nc;
-    r.iv = iv;
-    r.kord1 = kord;
-    r.variant = 0;
-    if (remap_launch<T>(c, r)) return 1;
-    hipLaunchKernelGGL(k_gather<T>, grid1(nc * km), dim3(256), 0, s, field, buf, 1, km, wi, nc, lev, ld, di, dj);
-    FV3_HIP(hipGetLastError());
-    return 0;
-  };
-  for (int t = 0; t < nt; t++) {
-    // u (isd:ied, jsd:jed+1): columns is:ie x js:je+1
-    if (remap_kind(t, 1, u + (long long)t * km * g.su, g.su, g.nid, g.is - g.isd, g.js - g.jsd, -1, a.kord_mt,
-                   nullptr))
-      return 1;
-    // v (isd:ied+1, jsd:jed): columns is:ie+1 x js:je
-    if (remap_kind(t, 2, v + (long long)t * km * g.sv, g.sv, g.nid + 1, g.is - g.isd, g.js - g.jsd, -1,
-                   a.kord_mt, nullptr))
-      return 1;
+  if (km <= FIELDS_MAX_KM) {
+    if (remap_orders_check(km, a.nq, a.kord_tr, true, a.kord_tm)) return 1;
+    // u, v, w: the field copied to scratch, its columns' tables, the remap back
+    auto remap_one = [&](int kind, int ni, int nj, FieldSet<T> x, T *field, size_t n, int kord) -> int {
+      const size_t b_tab = coltab_bytes<T>(km, (long long)ni * nj * nt);
+      char *ws = (char *)ctx_scratch(c, b_tab + sizeof(T) * n);
+      if (!ws) return 1;
+      T *copy = (T *)(ws + b_tab);
+      FV3_HIP(hipMemcpyAsync(copy, field, sizeof(T) * n, hipMemcpyDeviceToDevice, s));
+      FieldsArgs<T> f{};
+      f.tab = coltab_carve<T>(ws, km, (long long)ni * nj * nt);
+      ColSource cs{};
+      cs.kind = kind;
+      cs.ptop = a.ptop;
+      cs.ak = a.ak;
+      cs.bk = a.bk;
+      cs.delp = a.delp;
+      cs.pe = a.pe;
+      cs.ps = a.ps;
+      if (fields_prep<T>(c, f.tab, cs, ni, nj, x.iv == -2)) return 1;
+      x.src = copy + (x.src - field);
+      f.nset = 1;
+      f.set[0] = x;
+      f.kord[0] = (signed char)std::min(kord, 17);
+      return fields_run<T>(c, f, ni, nj);
+    };
+    const long long o0 = (long long)(g.js - g.jsd) * g.nid + (g.is - g.isd);
+    FieldSet<T> x = cell_set<T>(c, u, u, -1);  // u (isd:ied, jsd:jed+1): columns is:ie x js:je+1
+    x.lev = g.su;
+    x.tstride = x.ststride = g.su * km;
+    if (remap_one(1, g.ni, g.nj + 1, x, u, (size_t)(g.su * km * nt), a.kord_mt)) return 1;
+    x = cell_set<T>(c, v, v, -1);  // v (isd:ied+1, jsd:jed): columns is:ie+1 x js:je
+    x.src = x.dst = v + o0 + (g.js - g.jsd);
+    x.ld = g.nid + 1;
+    x.lev = g.sv;
+    x.tstride = x.ststride = g.sv * km;
+    if (remap_one(2, g.ni + 1, g.nj, x, v, (size_t)(g.sv * km * nt), a.kord_mt)) return 1;
     if (!a.hydrostatic) {
-      // w: cell columns with the surface value ws as the bottom boundary
-      FV3_HIP(hipMemcpyAsync(wsb, (const T *)a.ws + (long long)t * g.ni * g.nj, sizeof(T) * g.ni * g.nj,
-                             hipMemcpyDeviceToDevice, s));
-      if (remap_kind(t, 0, w + (long long)t * km * g.s2, g.s2, g.nid, g.is - g.isd, g.js - g.jsd, -2, a.kord_wz,
-                     wsb))
-        return 1;
-      // delz as -delz/delp over the cell columns (delz is (is:ie, js:je, km))
-      hipLaunchKernelGGL(k_delz<T>, grid1((long long)g.ni * g.nj * km), dim3(256), 0, s, g, t, 0, dz, a.delp, pe2);
-      if (remap_kind(t, 0, dz + t * g.spz, (long long)g.ni * g.nj, g.ni, 0, 0, 1, a.kord_wz, nullptr)) return 1;
-      hipLaunchKernelGGL(k_delz<T>, grid1((long long)g.ni * g.nj * km), dim3(256), 0, s, g, t, 1, dz, a.delp, pe2);
-      FV3_HIP(hipGetLastError());
+      x = cell_set<T>(c, w, w, -2);  // w: the surface value ws as the bottom boundary
+      x.qs = (const T *)a.ws;
+      if (remap_one(0, g.ni, g.nj, x, w, (size_t)(g.s2 * km * nt), a.kord_wz)) return 1;
+      // delz goes as -delz/delp
+      for (int t = 0; t < nt; t++)
+        hipLaunchKernelGGL(k_delz<T>, grid1((long long)g.ni * g.nj * km), dim3(256), 0, s, g, t, 0, dz, a.delp);
     }
-  }
-  // tracers, pt, delp <- dp2
-  {
-    std::vector<int> kt(std::max(1, a.nq), 0);
-    for (int iq = 0; iq < a.nq; iq++) kt[iq] = a.kord_tr[iq];
-    if (remap_tracers_plain<T>(c, km, a.nq, a.ak, a.bk, a.ptop, a.delp, q, pt, kt.data(), a.kord_tm, a.t_min,
-                               a.fill))
+    if (remap_cells_inplace<T>(c, km, a.nq, a.ak, a.bk, a.ptop, a.delp, q, pt, a.hydrostatic ? nullptr : dz,
+                               a.kord_tr, a.kord_tm, a.kord_wz, a.t_min, a.fill))
       return 1;
+    if (!a.hydrostatic)
+      for (int t = 0; t < nt; t++)
+        hipLaunchKernelGGL(k_delz<T>, grid1((long long)g.ni * g.nj * km), dim3(256), 0, s, g, t, 1, dz, a.delp);
+    FV3_HIP(hipGetLastError());
+  } else {  // longer columns: one thread per column
+    // one field of tile t over the columns of a kind through the column kernel
+    auto remap_kind = [&](int t, int kind, T *field, long long lev, int ld, int di, int dj, int iv, int kord,
+                          const T *qs) -> int {
+      const int wi = kind == 2 ? g.ni + 1 : g.ni, wj = kind == 1 ? g.nj + 1 : g.nj;
+      const long long nc = (long long)wi * wj;
+      hipLaunchKernelGGL(k_col_pressures, grid1(nc), dim3(256), 0, s, g, t, kind, a.ptop, a.ak, a.bk, a.pe, a.ps,
+                         pe1, pe2, nc);
+      hipLaunchKernelGGL(k_gather<T>, grid1(nc * km), dim3(256), 0, s, field, buf, 0, km, wi, nc, lev, ld, di, dj);
+      FV3_HIP(hipGetLastError());
+      RemapArgs<T> r{};
+      r.mode = 1;
+      r.km = km;
+      r.kn = km;
+      r.ncol = nc;
+      r.pe1_in = pe1;
+      r.pe2_in = pe2;
+      r.q1_in = buf;
+      r.q2_out = buf;
+      r.qs_in = qs;
+      r.q1_stride = nc;
+      r.q2_stride = nc;
+      r.iv = iv;
+      r.kord1 = kord;
+      r.variant = 0;
+      if (remap_launch<T>(c, r)) return 1;
+      hipLaunchKernelGGL(k_gather<T>, grid1(nc * km), dim3(256), 0, s, field, buf, 1, km, wi, nc, lev, ld, di, dj);
+      FV3_HIP(hipGetLastError());
+      return 0;
+    };
+    for (int t = 0; t < nt; t++) {
+      // u (isd:ied, jsd:jed+1): columns is:ie x js:je+1
+      if (remap_kind(t, 1, u + (long long)t * km * g.su, g.su, g.nid, g.is - g.isd, g.js - g.jsd, -1, a.kord_mt,
+                     nullptr))
+        return 1;
+      // v (isd:ied+1, jsd:jed): columns is:ie+1 x js:je
+      if (remap_kind(t, 2, v + (long long)t * km * g.sv, g.sv, g.nid + 1, g.is - g.isd, g.js - g.jsd, -1,
+                     a.kord_mt, nullptr))
+        return 1;
+      if (!a.hydrostatic) {
+        // w: cell columns with the surface value ws as the bottom boundary
+        FV3_HIP(hipMemcpyAsync(wsb, (const T *)a.ws + (long long)t * g.ni * g.nj, sizeof(T) * g.ni * g.nj,
+                               hipMemcpyDeviceToDevice, s));
+        if (remap_kind(t, 0, w + (long long)t * km * g.s2, g.s2, g.nid, g.is - g.isd, g.js - g.jsd, -2, a.kord_wz,
+                       wsb))
+          return 1;
+        // delz as -delz/delp over the cell columns (delz is (is:ie, js:je, km))
+        hipLaunchKernelGGL(k_delz<T>, grid1((long long)g.ni * g.nj * km), dim3(256), 0, s, g, t, 0, dz, a.delp);
+        if (remap_kind(t, 0, dz + t * g.spz, (long long)g.ni * g.nj, g.ni, 0, 0, 1, a.kord_wz, nullptr)) return 1;
+      }
+    }
+    // tracers, pt, delp <- dp2
+    {
+      std::vector<int> kt(std::max(1, a.nq), 0);
+      for (int iq = 0; iq < a.nq; iq++) kt[iq] = a.kord_tr[iq];
+      if (remap_tracers_plain<T>(c, km, a.nq, a.ak, a.bk, a.ptop, a.delp, q, pt, kt.data(), a.kord_tm, a.t_min,
+                                 a.fill))
+        return 1;
+    }
+    if (!a.hydrostatic)
+      for (int t = 0; t < nt; t++)
+        hipLaunchKernelGGL(k_delz<T>, grid1((long long)g.ni * g.nj * km), dim3(256), 0, s, g, t, 1, dz, a.delp);
+    FV3_HIP(hipGetLastError());
   }
   const double rrg = -a.rdgas / a.grav;
   for (int t = 0; t < nt; t++)

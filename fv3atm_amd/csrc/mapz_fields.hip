@@ -1,0 +1,669 @@
+// mapz_fields.hip -- vertical remap (upstream fv_mapz.F90: cs_profile /
+// scalar_profile, cs_limiters, and the layer integrals of map1_ppm, map1_q2,
+// map_scalar and mapn_tracer) in upstream evaluation order, for the FP64
+// forms, the full Lagrangian_to_Eulerian and the tangent-linear step.
+//
+// What depends on a column's pressures alone -- the elimination factors of
+// the interface solve, the source layers and fractions of every target
+// interface -- is the same for every field of the column: k_fields_prep
+// computes it once per column into [level][column] tables, and k_fields runs
+// one thread per (column, field).  The solve, the limiters and the layer
+// sums of a column are sequential in upstream's order, so that FP64 results
+// equal a CPU FP64 evaluation bit for bit.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <mutex>
+
+#include "fv3_internal.h"
+#include "mapz_fields.h"
+
+namespace fv3 {
+
+namespace {
+
+// ---- a / b from y = 1/b (rounded): two residual corrections of a*y.  The
+// first leaves q within one unit in the last place, so that the second is
+// a/b correctly rounded (Markstein, IBM J. Res. Dev. 34, 1990): the value of
+// the division it replaces, in five instructions.
+template <typename R>
+__device__ __forceinline__ R quot(R a, R b, R y) {
+  R q = a * y;
+  q = fma(fma(-b, q, a), y, q);
+  return fma(fma(-b, q, a), y, q);
+}
+__device__ __forceinline__ D1 quot(const D1 &a, double b, double y) {
+  D1 r(quot(a.v, b, y));
+  r.d[0] = a.d[0] * y;
+  return r;
+}
+
+constexpr int PREP_COLS = 64;
+
+struct PrepGeo {
+  int km, ni, nj, ncb, is, js, isd, jsd, nid, cni;  // cni: cells along i (the pe array's rows are cni + 2)
+  long long ncol, ncols, s2, spe;
+};
+
+// One workgroup per 64 columns: every level's thickness is loaded at once and
+// the interfaces are kept in LDS, so that the two serial chains that follow --
+// the elimination (wave 0) and the search of the target interfaces (wave 1) --
+// wait for no memory.  (A thread per column with a load in each step of both
+// chains took 1.3 us per level.)
+template <typename R>
+__global__ void __launch_bounds__(128) k_fields_prep(const PrepGeo g, const ColSource s, const ColTab<R> tab,
+                                                     const bool iv2) {
+  extern __shared__ double pe1_lds[];  // [km + 1][PREP_COLS]
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = (int)blockIdx.x / g.ncb, cb = (int)blockIdx.x % g.ncb;
+  const int km = g.km;
+  const long long c0 = (long long)cb * PREP_COLS + lane;
+  const bool act = c0 < g.ncol;
+  const long long lc = act ? c0 : g.ncol - 1;  // lanes past the last column repeat it and store nothing
+  const int ii = (int)(lc % g.ni), jj = (int)(lc / g.ni);
+  const int i = g.is + ii, j = g.js + jj;
+  const long long cell = (long long)(j - g.jsd) * g.nid + (i - g.isd);
+  const long long col = tile * g.ncol + lc, nc = g.ncols;
+  double *P = pe1_lds + lane;
+  auto PE1 = [&](int k) -> double & { return P[(k - 1) * PREP_COLS]; };
+  double psl = 0.0;  // kinds 1, 2: the sum of the two cells' surface pressures
+  if (s.kind == 0) {
+    const double *dl = s.delp + (long long)tile * km * g.s2 + cell;
+    for (int k = wave; k < km; k += 2) P[(k + 1) * PREP_COLS] = dl[(long long)k * g.s2];
+    __syncthreads();
+    if (wave == 0) {
+      double p = s.ptop;
+      PE1(1) = p;
+      for (int k = 1; k <= km; k++) PE1(k + 1) = p = p + PE1(k + 1);
+    }
+  } else {
+    const double *pe = s.pe + tile * g.spe, *ps = s.ps + tile * g.s2;
+    const int w = g.cni + 2;
+    auto at = [&](int a, int k, int b) {
+      return pe[((long long)(b - (g.js - 1)) * (km + 1) + (k - 1)) * w + (a - (g.is - 1))];
+    };
+    const int di = s.kind == 2 ? 1 : 0, dj = 1 - di;
+    for (int k = 1 + wave; k <= km + 1; k += 2) PE1(k) = 0.5 * (at(i - di, k, j - dj) + at(i, k, j));
+    psl = ps[cell - (di ? 1 : g.nid)] + ps[cell];
+  }
+  __syncthreads();
+  if (wave == 0) {
+    // the interface solve's factors
+    R gp = R(0), d4 = R(0);
+    auto put = [&](int k, R d, R bt, R gg) {
+      if (act) tab.el[(long long)(k - 1) * nc + col] = Elim<R>{d, bt, R(1) / bt, gg};
+    };
+    double dprev = PE1(2) - PE1(1);
+    if (act) tab.d1[col] = dprev;
+    R bot0 = R(0), bot1 = R(0), bot2 = R(1);
+    if (iv2) {
+      gp = R(0.5);  // G(2)
+      put(1, R(0), R(1), gp);
+      for (int k = 2; k <= km; k++) {
+        const double dk = PE1(k + 1) - PE1(k);
+        if (act) tab.d1[(long long)(k - 1) * nc + col] = dk;
+        const R grat = R(dprev / dk);
+        const R bet = R(2) + grat + grat - gp;
+        gp = grat / bet;  // G(k+1)
+        put(k, R(1), bet, k < km ? gp : R(0));
+        if (k == km) bot0 = grat;
+        dprev = dk;
+      }
+    } else {
+      const double d2 = PE1(3) - PE1(2);
+      const R grat = R(d2 / dprev);
+      const R bet = grat * (grat + R(0.5));
+      gp = (R(1) + grat * (grat + R(1.5))) / bet;
+      put(1, (grat + grat) * (grat + R(1)), bet, gp);
+      for (int k = 2; k <= km; k++) {
+        const double dk = PE1(k + 1) - PE1(k);
+        if (act) tab.d1[(long long)(k - 1) * nc + col] = dk;
+        d4 = R(dprev / dk);
+        const R bt = R(2) + d4 + d4 - gp;
+        gp = d4 / bt;
+        put(k, d4, bt, gp);
+        dprev = dk;
+      }
+      const R a_bot = R(1) + d4 * (d4 + R(1.5));
+      bot0 = R(2) * d4 * (d4 + R(1));
+      bot1 = a_bot;
+      bot2 = d4 * (d4 + R(0.5)) - a_bot * gp;
+    }
+    if (act) {
+      tab.bot[col] = bot0;
+      tab.bot[nc + col] = bot1;
+      tab.bot[2 * nc + col] = bot2;
+    }
+    return;
+  }
+  // the target layers: upstream's search from the last layer found
+  const double pbot = PE1(km + 1);
+  auto PE2 = [&](int k) -> double {
+    if (s.kind == 0) return k == 1 ? s.ptop : (k == km + 1 ? pbot : s.ak[k - 1] + s.bk[k - 1] * pbot);
+    return s.ak[k - 1] + 0.5 * s.bk[k - 1] * psl;
+  };
+  double *dout = s.delp_out ? s.delp_out + (long long)tile * km * g.s2 + cell : nullptr;
+  int k0 = 1;
+  double pa = PE2(1);
+  for (int k = 1; k <= km; k++) {
+    const double pb = PE2(k + 1);
+    int lt = 0, lb = km + 1;
+    bool one = false;
+    double pl = 0.0, pr = 0.0, dt = 0.0, db = 0.0;
+    for (int l = k0; l <= km; l++) {
+      const double a = PE1(l), b = PE1(l + 1);
+      if (pa >= a && pa <= b) {
+        lt = l;
+        pl = (pa - a) / (b - a);
+        if (pb <= b) {
+          one = true;
+          pr = (pb - a) / (b - a);
+          k0 = lb = l;
+          break;
+        }
+        dt = b - pa;
+        for (int m = l + 1; m <= km; m++)
+          if (!(pb > PE1(m + 1))) {
+            db = pb - PE1(m);
+            pr = db / (PE1(m + 1) - PE1(m));
+            k0 = lb = m;
+            break;
+          }
+        break;
+      }
+    }
+    const double den = pb - pa;
+    if (act) {
+      const long long o = (long long)(k - 1) * nc + col;
+      tab.r0[o] = make_double2(pl, pr);
+      tab.r1[o] = make_double2(dt, db);
+      tab.r2[o] = make_double2(den, 1.0 / den);
+      tab.rc[o] = lt | lb << 12 | (one ? 1 << 24 : 0);
+      if (dout) dout[(long long)(k - 1) * g.s2] = den;
+    }
+    pa = pb;
+  }
+}
+
+// ---- the field kernel
+constexpr int FD_B = 8;      // levels per regenerated block
+constexpr int FD_WAVES = 4;  // fields per workgroup (one per wave)
+
+struct TargetRec {
+  double2 r0, r1, r2;
+  int rc;
+};
+
+// One wave: 64 columns of one field.  Three passes over the levels:
+//   down  the elimination; the entry value of every FD_B-level block to LDS;
+//   up    each block's eliminated values again from its entry value, then
+//         the back substitution; the block's exit value replaces the entry
+//         value in LDS;
+//   down  the eliminated values once more (their chain is carried), the block's
+//         interface values by back substitution from its exit value, into LDS,
+//         then level by level the interface limits, extremum flags, cell
+//         limiters and layer integrals over a window of six cell means.
+// Only the block ends and one block are kept (18 KB of LDS per wave in FP64
+// at 127 levels: two waves per SIMD); the field's second and third reads come
+// from cache.  The divisions by the field-independent pivots use their stored
+// reciprocals (quot).  Bound by VALU issue at two waves per SIMD.  Measured
+// against one thread per column looping over its fields with every work array
+// in HBM (at C96 144 waves on 1024 SIMDs): C384 L127 9 tracers + pt FP64 18.7
+// -> 4.9 ms plus 0.76 ms of tables, C96 L64 4 tracers + pt 1.79 -> 0.19 + 0.06
+// ms; the FP32 full remap of C192 L127 (13 fields) 12.4 -> 1.9 + 1.0 ms.
+template <typename T>
+__global__ void __launch_bounds__(64 * FD_WAVES, 2) k_fields(const FieldsArgs<T> a) {
+  using R = typename RealOf<T>::type;
+  extern __shared__ __align__(16) char fd_lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // blocks are dealt round-robin to the 8 XCDs: renumber so that the field
+  // groups of one column block run on one XCD, one after another
+  const unsigned bid = blockIdx.x, nx = 8, q8 = a.nwg / nx, r8 = a.nwg % nx;
+  const unsigned xcd = bid % nx, idx = bid / nx;
+  const unsigned logical = xcd < r8 ? xcd * (q8 + 1) + idx : r8 * (q8 + 1) + (xcd - r8) * q8 + idx;
+  const int cblk = (int)(logical / a.nfg), fg = (int)(logical % a.nfg);
+  const int f = fg * FD_WAVES + wave;
+  if (f >= a.nf) return;  // whole wave; no barriers below
+  int si = 0, fi = f;
+  while (si + 1 < a.nset && fi >= a.set[si].count) fi -= a.set[si++].count;
+  const FieldSet<T> &S = a.set[si];
+  const int iv = S.iv, kord = a.kord[f], akord = kord < 0 ? -kord : kord;
+  const bool use_qmin = S.use_qmin, mapn = S.mapn;
+  const R qmin = S.qmin;
+  const int tile = cblk / a.ncb, cb = cblk % a.ncb;
+  const long long c0 = (long long)cb * 64 + lane;
+  const bool act = c0 < a.ncol;
+  const long long lc = act ? c0 : a.ncol - 1;
+  const long long nc = a.ncols, col = tile * a.ncol + lc;
+  const int km = a.km, nb = (km + FD_B - 1) / FD_B;
+  const unsigned cell = (unsigned)((lc / a.ni) * S.ld + lc % a.ni);
+  const long long fbase = fi * S.fstride + tile * S.tstride, sbase = fi * S.sfstride + tile * S.ststride;
+  const R *src = S.src + sbase, *src_t = nullptr;
+  if constexpr (sizeof(T) != sizeof(R)) src_t = S.src_t + sbase;
+  const long long lev = S.lev;
+  const unsigned cbyte = cell * (unsigned)sizeof(R);
+  auto ld = [&](int k) -> T {  // scalar level base, lane byte offset
+    const R v = *reinterpret_cast<const R *>(reinterpret_cast<const char *>(src + (k - 1) * lev) + cbyte);
+    if constexpr (sizeof(T) == sizeof(R)) {
+      return v;
+    } else {
+      T r(v);
+      r.d[0] = *reinterpret_cast<const R *>(reinterpret_cast<const char *>(src_t + (k - 1) * lev) + cbyte);
+      return r;
+    }
+  };
+  const Elim<R> *el = a.tab.el + col;
+  auto lde = [&](int k) -> Elim<R> { return el[(long long)(k - 1) * nc]; };
+  T *lds = reinterpret_cast<T *>(fd_lds) + (size_t)wave * (nb + 2 * FD_B + 4) * 64 + lane;
+  auto CP = [&](int b) -> T & { return lds[b * 64]; };
+  auto BQ = [&](int j) -> T & { return lds[(nb + j) * 64]; };
+  auto BA = [&](int j) -> T & { return lds[(nb + FD_B + 2 + j) * 64]; };
+  const bool iv2 = iv == -2;
+  const T qs = iv2 ? T(S.qs[tile * a.ncol + lc]) : T(R(0));
+  const R bot0 = a.tab.bot[col], bot1 = a.tab.bot[nc + col], bot2 = a.tab.bot[2 * nc + col];
+
+  struct Blk {
+    T av[FD_B + 1];  // a(k0-1 .. k0+B-1)
+    Elim<R> e[FD_B];
+  };
+  auto fetch = [&](int b, Blk &x) {
+    const int k0 = b * FD_B + 1;
+#pragma unroll
+    for (int j = 0; j <= FD_B; j++) x.av[j] = ld(min(max(k0 - 1 + j, 1), km));
+#pragma unroll
+    for (int j = 0; j < FD_B; j++) x.e[j] = lde(min(k0 + j, km));
+  };
+  // the eliminated values of block b from the one above it
+  auto eliminate = [&](int b, const Blk &x, T q, T (&qv)[FD_B], const T &a2nd) {
+    const int k0 = b * FD_B + 1;
+#pragma unroll
+    for (int j = 0; j < FD_B; j++) {
+      const int k = k0 + j;
+      if (k <= km) {
+        if (k == 1) {
+          q = iv2 ? R(1.5) * x.av[1] : quot(x.e[0].d4 * x.av[1] + a2nd, x.e[0].bt, x.e[0].y);
+        } else {
+          T n = R(3) * (x.av[j] + x.e[j].d4 * x.av[j + 1]);
+          if (iv2 && k == km) n = n - bot0 * qs;
+          q = quot(n - q, x.e[j].bt, x.e[j].y);
+        }
+      }
+      qv[j] = q;
+    }
+    return q;
+  };
+  const T a2nd = ld(2);
+
+  // ---- down: elimination
+  T q = T(R(0));
+  {
+    Blk cur, nxt;
+    fetch(0, cur);
+    for (int b = 0; b < nb; b++) {
+      if (b + 1 < nb) fetch(b + 1, nxt);
+      CP(b) = q;
+      T qv[FD_B];
+      q = eliminate(b, cur, q, qv, a2nd);
+      cur = nxt;
+    }
+  }
+  const T qbot = iv2 ? qs : T((bot0 * ld(km) + ld(km - 1) - bot1 * q) / bot2);
+
+  // ---- up: the value below every block
+  {
+    Blk cur, nxt;
+    fetch(nb - 1, cur);
+    q = qbot;
+    for (int b = nb - 1; b >= 0; b--) {
+      if (b > 0) fetch(b - 1, nxt);
+      const T entry = CP(b);
+      CP(b) = q;
+      if (b > 0) {
+        T qv[FD_B];
+        eliminate(b, cur, entry, qv, a2nd);
+#pragma unroll
+        for (int j = FD_B - 1; j >= 0; j--)
+          if (b * FD_B + 1 + j <= km) q = qv[j] - cur.e[j].g * q;
+      }
+      cur = nxt;
+    }
+  }
+
+  // ---- down: limits, cells, layer integrals
+  const bool lim = akord <= 16;
+  const T zero = T(R(0));
+  T A_4 = zero, A_3 = zero, A_2 = zero, A_1 = zero, A_0 = zero, A_p = ld(1);  // a(p-4 .. p+1)
+  T L_2 = zero, L_1 = zero, L_0 = zero;                                      // limited Q(p-2 .. p)
+  int E_3 = 0, E_2 = 0, E_1 = 0;                                             // flags of cells p-3 .. p-1
+  // the open target: its records (and the next target's, in flight), partial sum
+  int kt = 1;
+  bool open = false;
+  const double2 *p0 = a.tab.r0 + col, *p1 = a.tab.r1 + col, *p2 = a.tab.r2 + col;
+  const int *pc = a.tab.rc + col;
+  auto rec = [&](int k) -> TargetRec {
+    const long long o = (long long)(min(k, km) - 1) * nc;
+    return TargetRec{p0[o], p1[o], p2[o], pc[o]};
+  };
+  TargetRec tr = rec(1), tn = rec(2);
+  char *dlane = reinterpret_cast<char *>(S.dst + fbase) + cbyte;
+  char *dlane_t = nullptr;
+  if constexpr (sizeof(T) != sizeof(R)) dlane_t = reinterpret_cast<char *>(S.dst_t + fbase) + cbyte;
+  const long long levb = lev * (long long)sizeof(R);
+  using SumT = typename std::conditional<sizeof(T) == sizeof(R), double, D1>::type;  // sums in FP64
+  SumT acc(0.0);
+  auto wide = [](const T &v) -> SumT { return (SumT)v; };
+  auto emit = [&](const T &v) {
+    if (act) {
+      if constexpr (sizeof(T) == sizeof(R)) {
+        *reinterpret_cast<R *>(dlane) = v;
+      } else {
+        *reinterpret_cast<R *>(dlane) = v.v;
+        *reinterpret_cast<R *>(dlane_t) = v.d[0];
+      }
+    }
+    dlane += levb;
+    if constexpr (sizeof(T) != sizeof(R)) dlane_t += levb;
+    kt++;
+    tr = tn;
+    tn = rec(kt + 1);
+  };
+  auto narrow = [](const SumT &v) -> T {
+    if constexpr (sizeof(T) == sizeof(R)) return T(v);
+    else return v;
+  };
+  const double *d1p = a.tab.d1 + col;
+  double d1n = d1p[0];  // thickness of the next cell
+
+  T chain = zero;  // the eliminated value above the block
+  Blk cur, nxt;
+  fetch(0, cur);
+  for (int b = 0; b < nb; b++) {
+    const int k0 = b * FD_B + 1;
+    {
+      T qv[FD_B];
+      chain = eliminate(b, cur, chain, qv, a2nd);
+      q = CP(b);
+#pragma unroll
+      for (int j = FD_B - 1; j >= 0; j--)
+        if (k0 + j <= km) {
+          q = qv[j] - cur.e[j].g * q;
+          BQ(j) = q;
+        }
+    }
+    const bool last = b + 1 == nb;
+    if (!last) fetch(b + 1, nxt);
+#pragma unroll
+    for (int j = 0; j + 1 < FD_B; j++) BA(j) = cur.av[j + 2];  // a(k0+1 ..)
+    if (!last) BA(FD_B - 1) = nxt.av[1];
+    if (last) BQ(km + 1 - k0) = qbot;
+    const int pend = last ? km + 2 : k0 + FD_B - 1;
+    for (int p = k0; p <= pend; p++) {
+      A_4 = A_3;
+      A_3 = A_2;
+      A_2 = A_1;
+      A_1 = A_0;
+      A_0 = A_p;
+      if (p < km) A_p = BA(p - k0);
+      L_2 = L_1;
+      L_1 = L_0;
+      if (p <= km + 1) L_0 = BQ(p - k0);
+      // interface p lies between cells p-1 (A_1) and p (A_0)
+      if (lim && p >= 2 && p <= km) {
+        const T lo = mn2(A_1, A_0), hi = mx2(A_1, A_0);
+        if (p == 2 || p == km) {
+          L_0 = mx2(mn2(L_0, hi), lo);
+        } else {
+          const T glo = A_1 - A_2, ghi = A_p - A_0;
+          const T dn = mn2(L_0, hi);
+          T v;
+          if (glo * ghi > zero) {
+            v = mx2(dn, lo);
+          } else if (glo > zero) {
+            v = mx2(L_0, lo);
+          } else {
+            v = iv == 0 ? mx2(zero, dn) : dn;
+          }
+          L_0 = v;
+        }
+      }
+      E_3 = E_2;
+      E_2 = E_1;
+      // flags of cell p-1: 1 extm, 2 ext5, 4 ext6
+      if (lim && p >= 2 && p <= km + 1) {
+        const int e = p - 1;
+        const bool em = e == 1 || e == km ? (L_1 - A_1) * (L_0 - A_1) > zero
+                                          : (A_1 - A_2) * (A_0 - A_1) < zero;
+        E_1 = em ? 1 : 0;
+        if (akord > 9) {
+          const T x0 = R(2) * A_1 - (L_1 + L_0), x1 = fabs(L_1 - L_0);
+          E_1 |= (fabs(x0) > x1 ? 2 : 0) | (fabs(R(3) * x0) > x1 ? 4 : 0);
+        }
+      }
+      const int c = p - 2;
+      if (c < 1) continue;
+      // ---- cell c = p-2: a(c) is A_2, its interface values L_2, L_1
+      T a1 = A_2, a2 = L_2, a3 = L_1, a4;
+      if (!lim) {
+        a4 = R(3) * (R(2) * a1 - (a2 + a3));
+      } else if (c == 1 || c == 2 || c >= km - 1) {
+        if (c == 1) {
+          if (iv == 0) {
+            a2 = mx2(zero, a2);
+          } else if (iv == -1) {
+            if (a2 * a1 <= zero) a2 = zero;
+          }
+        } else if (c == km) {
+          if (iv == 0) {
+            a3 = mx2(zero, a3);
+          } else if (iv == -1) {
+            if (a3 * a1 <= zero) a3 = zero;
+          }
+        }
+        a4 = R(3) * (R(2) * a1 - (a2 + a3));
+        cs_lim1(a1, a2, a3, a4, (E_2 & 1) != 0, c == 1 || c == km ? 1 : 2);
+      } else {
+        const T gk = A_2 - A_3, gk1 = A_1 - A_2, gk2 = A_0 - A_1, gkm1 = A_3 - A_4;
+        const bool low = use_qmin && a1 < T(qmin);
+        if (akord < 9) {
+          huynh2(a1, a2, a3, gk, gk1, gk2, gkm1);
+          a4 = R(3) * (R(2) * a1 - (a2 + a3));
+        } else if (akord == 9) {
+          if ((E_2 & 1) && ((E_3 & 1) || (E_1 & 1) || low)) {
+            a2 = a1;
+            a3 = a1;
+            a4 = zero;
+          } else {
+            a4 = R(6) * a1 - R(3) * (a2 + a3);
+            if (fabs(a4) > fabs(a2 - a3)) {
+              huynh2(a1, a2, a3, gk, gk1, gk2, gkm1);
+              a4 = R(6) * a1 - R(3) * (a2 + a3);
+            }
+          }
+        } else {
+          if (E_2 & 2) {
+            if ((E_3 & 2) || (E_1 & 2) || low) {
+              a2 = a1;
+              a3 = a1;
+            } else if ((E_3 & 4) || (E_1 & 4)) {
+              huynh2(a1, a2, a3, gk, gk1, gk2, gkm1);
+            }
+          } else if (E_2 & 4) {
+            if ((E_3 & 2) || (E_1 & 2)) huynh2(a1, a2, a3, gk, gk1, gk2, gkm1);
+          }
+          a4 = R(3) * (R(2) * a1 - (a2 + a3));
+        }
+        if (iv == 0) cs_lim1(a1, a2, a3, a4, (E_2 & 1) != 0, 0);
+      }
+      // ---- the target layers that end, lie or begin in source layer c
+      const double d1c = d1n;
+      d1n = d1p[(long long)(min(c + 1, km) - 1) * nc];
+      const double r3 = 1.0 / 3.0, r23 = 2.0 / 3.0;
+      while (kt <= km) {
+        const int lt = tr.rc & 0xfff, lb = (tr.rc >> 12) & 0xfff;
+        if (open) {
+          if (lb != c) {
+            acc = acc + d1c * wide(A_2);
+            break;
+          }
+          const double esl = tr.r0.y;
+          acc = acc + tr.r1.y * wide(a2 + R(0.5 * esl) * (a3 - a2 + a4 * R(1.0 - r23 * esl)));
+          emit(narrow(quot(acc, tr.r2.x, tr.r2.y)));
+          open = false;
+        } else if (lt == 0) {
+          emit(narrow(SumT(0.0 / tr.r2.x)));
+        } else if (lt > c) {
+          break;
+        } else {
+          const double pl = tr.r0.x;
+          if (tr.rc >> 24) {
+            const double pr = tr.r0.y, z = pr * (pr + pl) + pl * pl;
+            const T tail = mapn ? T(a4 * R(r3 * z)) : T(a4 * R(r3) * R(z));
+            emit(a2 + (a4 + a3 - a2) * R(0.5 * (pr + pl)) - tail);
+          } else {
+            acc = tr.r1.x * wide(a2 + (a4 + a3 - a2) * R(0.5 * (1.0 + pl)) - a4 * R(r3 * (1.0 + pl * (1.0 + pl))));
+            open = true;
+            break;
+          }
+        }
+      }
+    }
+    cur = nxt;
+  }
+  // a target that ends below the source, and those no layer holds
+  while (kt <= km) {
+    emit(narrow(open ? quot(acc, tr.r2.x, tr.r2.y) : SumT(0.0 / tr.r2.x)));
+    open = false;
+  }
+}
+
+template <typename T>
+size_t fields_lds(int km) {
+  const int nb = (km + FD_B - 1) / FD_B;
+  return sizeof(T) * FD_WAVES * (size_t)(nb + 2 * FD_B + 4) * 64;
+}
+
+size_t prep_lds(int km) { return sizeof(double) * (size_t)(km + 1) * PREP_COLS; }
+
+}  // namespace
+
+template <typename R>
+size_t coltab_bytes(int km, long long ncols) {
+  auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t n = (size_t)km * ncols;
+  return al(sizeof(Elim<R>) * n) + al(sizeof(double) * n) + 3 * al(sizeof(double2) * n) + al(sizeof(int) * n) +
+         al(sizeof(R) * 3 * (size_t)ncols);
+}
+
+template <typename R>
+ColTab<R> coltab_carve(void *base, int km, long long ncols) {
+  ColTab<R> t{};
+  char *p = (char *)base;
+  auto take = [&](size_t b) {
+    char *r = p;
+    p += (b + 255) & ~(size_t)255;
+    return r;
+  };
+  const size_t n = (size_t)km * ncols;
+  t.el = (Elim<R> *)take(sizeof(Elim<R>) * n);
+  t.d1 = (double *)take(sizeof(double) * n);
+  t.r0 = (double2 *)take(sizeof(double2) * n);
+  t.r1 = (double2 *)take(sizeof(double2) * n);
+  t.r2 = (double2 *)take(sizeof(double2) * n);
+  t.rc = (int *)take(sizeof(int) * n);
+  t.bot = (R *)take(sizeof(R) * 3 * (size_t)ncols);
+  return t;
+}
+
+// More than 64 KB of dynamic LDS per workgroup must be allowed per kernel.
+int fields_setup() {
+  static std::once_flag once;
+  static hipError_t err = hipSuccess;
+  std::call_once(once, [] {
+    auto allow = [](const void *fn, size_t b) {
+      if (err == hipSuccess) err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
+    };
+    allow(reinterpret_cast<const void *>(&k_fields_prep<float>), prep_lds(FIELDS_MAX_KM));
+    allow(reinterpret_cast<const void *>(&k_fields_prep<double>), prep_lds(FIELDS_MAX_KM));
+    allow(reinterpret_cast<const void *>(&k_fields<float>), fields_lds<float>(FIELDS_MAX_KM));
+    allow(reinterpret_cast<const void *>(&k_fields<double>), fields_lds<double>(FIELDS_MAX_KM));
+  });
+  FV3_HIP(err);
+  return 0;
+}
+
+template <typename R>
+int fields_prep(Ctx &c, const ColTab<R> &tab, const ColSource &src, int ni, int nj, bool iv2) {
+  const Dims &d = c.d;
+  if (c.npz > FIELDS_MAX_KM) return set_error("column tables support km <= %d (got %d)", FIELDS_MAX_KM, c.npz);
+  if (fields_setup()) return 1;
+  PrepGeo g{};
+  g.km = c.npz; g.ni = ni; g.nj = nj; g.is = d.is; g.js = d.js; g.isd = d.isd; g.jsd = d.jsd; g.nid = d.nid;
+  g.cni = d.ie - d.is + 1;
+  g.ncol = (long long)ni * nj;
+  g.ncols = g.ncol * c.ntiles;
+  g.s2 = d.s2;
+  g.spe = (long long)(g.cni + 2) * (g.km + 1) * (d.je - d.js + 3);
+  g.ncb = (int)((g.ncol + PREP_COLS - 1) / PREP_COLS);
+  hipLaunchKernelGGL(k_fields_prep<R>, dim3((unsigned)g.ncb * (unsigned)c.ntiles), dim3(128), prep_lds(g.km), c.stream,
+                     g, src, tab, iv2);
+  FV3_HIP(hipGetLastError());
+  return 0;
+}
+
+template <typename T>
+int fields_run(Ctx &c, FieldsArgs<T> &a, int ni, int nj) {
+  a.km = c.npz;
+  a.ni = ni;
+  a.ncol = (long long)ni * nj;
+  a.ncols = a.ncol * c.ntiles;
+  a.ncb = (int)((a.ncol + 63) / 64);
+  a.nf = 0;
+  for (int s = 0; s < a.nset; s++) a.nf += a.set[s].count;
+  if (a.nf == 0) return 0;
+  a.nfg = (a.nf + FD_WAVES - 1) / FD_WAVES;
+  const long long nwg = (long long)a.ncb * c.ntiles * a.nfg;
+  if (nwg > 0x7fffffffLL) return set_error("remap grid too large");
+  a.nwg = (unsigned)nwg;
+  hipLaunchKernelGGL(k_fields<T>, dim3(a.nwg), dim3(64 * FD_WAVES), fields_lds<T>(a.km), c.stream, a);
+  FV3_HIP(hipGetLastError());
+  return 0;
+}
+
+template <typename T>
+FieldSet<T> cell_set(const Ctx &c, const T *src, T *dst, int iv) {
+  const Dims &d = c.d;
+  const long long o0 = (long long)(d.js - d.jsd) * d.nid + (d.is - d.isd);
+  FieldSet<T> f{};
+  f.src = src + o0;
+  f.dst = dst + o0;
+  f.lev = d.s2;
+  f.ld = d.nid;
+  f.fstride = f.tstride = f.sfstride = f.ststride = d.s2 * c.npz;
+  f.count = 1;
+  f.iv = iv;
+  return f;
+}
+
+template <typename T>
+FieldSet<T> tracer_set(const Ctx &c, const T *src, T *dst, int nq) {
+  FieldSet<T> f = cell_set(c, src, dst, 0);
+  f.tstride = f.ststride = f.fstride * nq;
+  f.count = nq;
+  f.use_qmin = true;
+  f.mapn = nq > 5;  // mapn_tracer, else map1_q2
+  return f;
+}
+
+#define FV3_FIELDS(T)                                                                                            \
+  template size_t coltab_bytes<T>(int, long long);                                                               \
+  template ColTab<T> coltab_carve<T>(void *, int, long long);                                                    \
+  template int fields_prep<T>(Ctx &, const ColTab<T> &, const ColSource &, int, int, bool);                      \
+  template int fields_run<T>(Ctx &, FieldsArgs<T> &, int, int);                                                  \
+  template FieldSet<T> cell_set<T>(const Ctx &, const T *, T *, int);                                            \
+  template FieldSet<T> tracer_set<T>(const Ctx &, const T *, T *, int);
+FV3_FIELDS(double)
+FV3_FIELDS(float)
+#undef FV3_FIELDS
+
+}  // namespace fv3

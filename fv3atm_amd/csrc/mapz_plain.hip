@@ -10,6 +10,7 @@
 
 #include "fv3_internal.h"
 #include "mapz_column.h"
+#include "mapz_fields.h"
 
 namespace fv3 {
 
@@ -62,17 +63,118 @@ int remap_launch(Ctx &c, RemapArgs<T> &a) {
   return 0;
 }
 
+// fillz over the columns of one tracer (D2: the target thickness, the first
+// of each pair of r2)
 template <typename T>
-int remap_tracers_plain(Ctx &c, int km, int nq, const double *ak, const double *bk, double ptop,
-                        double *delp, T *q, T *pt, const int *kord_tr, int kord_tm, double t_min,
-                        int fill) {
+__global__ void __launch_bounds__(64) k_fillz(T *q, const double2 *r2, T *dm, int km, int ni, int ld, long long lev,
+                                              long long nc, long long ncol, long long col0) {
+  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= ncol) return;
+  const long long cell = (c / ni) * ld + c % ni;
+  double *d2 = const_cast<double *>(reinterpret_cast<const double *>(r2 + col0 + c));
+  fillz_col<T>(CV<T>{q + cell, lev}, CV<double>{d2, 2 * nc}, CV<T>{dm + c, ncol}, km);
+}
+
+// The remap in place of the cell columns: the sources of the fields are
+// copied to scratch, at most about 512 MB of tracers at a time; pt and delz go
+// with the first of them.
+template <typename T>
+int remap_cells_inplace(Ctx &c, int km, int nq, const double *ak, const double *bk, double ptop, double *delp, T *q,
+                        T *pt, T *dz, const int *kord_tr, int kord_tm, int kord_dz, double t_min, int fill) {
+  const Dims &d = c.d;
+  hipStream_t s = c.stream;
+  const int ni = d.ie - d.is + 1, nj = d.je - d.js + 1, nt = c.ntiles;
+  const long long ncol = (long long)ni * nj, ncols = ncol * nt, fld = d.s2 * km;
+  const size_t b_field = sizeof(T) * (size_t)fld * nt, b_dz = sizeof(T) * (size_t)(ncols * km);
+  const int part = (int)std::max<size_t>(1, std::min<size_t>(std::max(nq, 1), ((size_t)512 << 20) / b_field));
+  size_t off = 0;
+  auto take = [&](size_t b) {
+    const size_t o = off;
+    off += (b + 255) & ~(size_t)255;
+    return o;
+  };
+  const size_t o_tab = take(coltab_bytes<T>(km, ncols)), o_dm = take(fill ? sizeof(T) * (size_t)(km + 1) * ncol : 0);
+  const size_t o_q = take(nq > 0 ? b_field * part : 0), o_pt = take(pt ? b_field : 0), o_dz = take(dz ? b_dz : 0);
+  char *ws = (char *)ctx_scratch(c, off);
+  if (!ws) return 1;
+  T *dm = (T *)(ws + o_dm), *cq = (T *)(ws + o_q), *cpt = (T *)(ws + o_pt), *cdz = (T *)(ws + o_dz);
+  const ColTab<T> tab = coltab_carve<T>(ws + o_tab, km, ncols);
+  ColSource src{};
+  src.ptop = ptop;
+  src.ak = ak;
+  src.bk = bk;
+  src.delp = src.delp_out = delp;
+  if (fields_prep<T>(c, tab, src, ni, nj, false)) return 1;
+  if (pt) FV3_HIP(hipMemcpyAsync(cpt, pt, b_field, hipMemcpyDeviceToDevice, s));
+  if (dz) FV3_HIP(hipMemcpyAsync(cdz, dz, b_dz, hipMemcpyDeviceToDevice, s));
+  for (int q0 = 0; q0 == 0 || q0 < nq; q0 += part) {
+    FieldsArgs<T> a{};
+    a.tab = tab;
+    int f = 0;
+    const int cnt = std::min(part, nq - q0);
+    if (cnt > 0) {
+      for (int t = 0; t < nt; t++)
+        FV3_HIP(hipMemcpyAsync(cq + t * fld * cnt, q + (t * (long long)nq + q0) * fld, sizeof(T) * fld * cnt,
+                               hipMemcpyDeviceToDevice, s));
+      FieldSet<T> &x = a.set[a.nset++] = tracer_set<T>(c, cq, q + q0 * fld, nq);
+      x.count = cnt;
+      x.ststride = fld * cnt;
+      for (; f < cnt; f++) a.kord[f] = (signed char)std::min(kord_tr[q0 + f], 17);
+    }
+    if (pt && q0 == 0) {
+      FieldSet<T> &x = a.set[a.nset++] = cell_set<T>(c, cpt, pt, 1);
+      x.use_qmin = true;
+      x.qmin = (T)t_min;
+      a.kord[f++] = (signed char)std::min(kord_tm, 17);
+    }
+    if (dz && q0 == 0) {
+      FieldSet<T> &x = a.set[a.nset++];
+      x.src = cdz;
+      x.dst = dz;
+      x.lev = ncol;
+      x.ld = ni;
+      x.tstride = x.ststride = ncol * km;
+      x.count = 1;
+      x.iv = 1;
+      a.kord[f++] = (signed char)std::min(kord_dz, 17);
+    }
+    if (fields_run<T>(c, a, ni, nj)) return 1;
+  }
+  if (fill) {
+    const long long o0 = (long long)(d.js - d.jsd) * d.nid + (d.is - d.isd);
+    for (int t = 0; t < nt; t++)
+      for (int iq = 0; iq < nq; iq++)
+        hipLaunchKernelGGL(k_fillz<T>, dim3((unsigned)((ncol + 63) / 64)), dim3(64), 0, s,
+                           q + (t * (long long)nq + iq) * fld + o0, tab.r2, dm, km, ni, d.nid, d.s2, ncols, ncol,
+                           t * ncol);
+    FV3_HIP(hipGetLastError());
+  }
+  return 0;
+}
+
+int remap_orders_check(int km, int nq, const int *kord_tr, bool with_pt, int kord_tm) {
   if (km < 4) return set_error("remap needs km >= 4 (got %d)", km);
   for (int iq = 0; iq < nq; iq++)
     if (!(kord_tr[iq] > 7 && (kord_tr[iq] <= 10 || kord_tr[iq] > 16)))
       return set_error("kord_tr(%d)=%d: implemented orders are 8, 9, 10 and > 16", iq + 1, kord_tr[iq]);
-  if (pt && !(kord_tm > 7 && (kord_tm <= 10 || kord_tm > 16)))
+  if (with_pt && !(kord_tm > 7 && (kord_tm <= 10 || kord_tm > 16)))
     return set_error("kord_tm=%d: implemented orders are 8, 9, 10 and > 16", kord_tm);
   if (nq > REMAP_MAX_NQ) return set_error("nq=%d exceeds %d", nq, REMAP_MAX_NQ);
+  return 0;
+}
+
+template <typename T>
+int remap_tracers_plain(Ctx &c, int km, int nq, const double *ak, const double *bk, double ptop,
+                        double *delp, T *q, T *pt, const int *kord_tr, int kord_tm, double t_min,
+                        int fill) {
+  if (remap_orders_check(km, nq, kord_tr, pt != nullptr, kord_tm)) return 1;
+  if (km <= FIELDS_MAX_KM) {
+    if (remap_cells_inplace<T>(c, km, nq, ak, bk, ptop, delp, q, pt, (T *)nullptr, kord_tr, kord_tm, 0, t_min, fill))
+      return 1;
+    FV3_HIP(hipStreamSynchronize(c.stream));
+    return 0;
+  }
+  // longer columns: one thread per column
   const Dims &d = c.d;
   RemapArgs<T> a{};
   a.mode = 0;
@@ -107,6 +209,10 @@ template int remap_tracers_plain<double>(Ctx &, int, int, const double *, const 
                                          double *, double *, double *, const int *, int, double, int);
 template int remap_tracers_plain<float>(Ctx &, int, int, const double *, const double *, double,
                                         double *, float *, float *, const int *, int, double, int);
+template int remap_cells_inplace<double>(Ctx &, int, int, const double *, const double *, double, double *, double *,
+                                         double *, double *, const int *, int, int, double, int);
+template int remap_cells_inplace<float>(Ctx &, int, int, const double *, const double *, double, double *, float *,
+                                        float *, float *, const int *, int, int, double, int);
 template int remap_launch<double>(Ctx &, RemapArgs<double> &);
 template int remap_launch<float>(Ctx &, RemapArgs<float> &);
 
