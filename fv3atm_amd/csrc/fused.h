@@ -16,10 +16,11 @@ int launch_fused_f32(const FusedArgs<float> &a, int cfg, const KindStreams &s);
 // tracers per round (waves x tracers per wave) of the lean kind of cfg
 int fused32_round(int cfg);
 
-// per-level sub-cycle counts on the device (cmax, nsplit; no scaling)
+// per-level sub-cycle counts on the device (cmax, nsplit; no scaling); with
+// xfx, yfx (layouts of cx, cy) the same pass writes the area fluxes
 template <typename T>
 int device_nsplit(Ctx &c, const T *cx, const T *cy, bool per_level, int q_split, double *cmax,
-                  int *nsplit, T *frac);
+                  int *nsplit, T *frac, T *xfx = nullptr, T *yfx = nullptr);
 
 // Device scratch handed to a step by its caller instead of the context's
 // arenas (the no-allocation entry point); base == nullptr: the context's.

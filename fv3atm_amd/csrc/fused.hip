@@ -17,13 +17,13 @@ static void go64(const FusedArgs<double> &a, const KindStreams &s) {
   int n[7];
   fused_grid_split(a, n);
   auto grid = [&](int c) { return dim3((unsigned)c, (unsigned)a.npz, (unsigned)a.ntiles); };
-  if (n[0] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 0, 1>), grid(n[0]), b, 0, s.k[0], a);
-  if (n[1] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 1, 1>), grid(n[1]), b, 0, s.k[1], a);
-  if (n[2] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 2, 1>), grid(n[2]), b, 0, s.k[2], a);
-  if (n[3] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 3, 1>), grid(n[3]), b, 0, s.k[2], a);
-  if (n[4] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 4, 1>), grid(n[4]), b, 0, s.k[3], a);
-  if (n[5] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 5, 1>), grid(n[5]), b, 0, s.k[2], a);
-  if (n[6] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 6, 1>), grid(n[6]), b, 0, s.k[3], a);
+  if (n[0] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 0, 2>), grid(n[0]), b, 0, s.k[0], a);
+  if (n[1] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 1, 2>), grid(n[1]), b, 0, s.k[1], a);
+  if (n[2] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 2, 2>), grid(n[2]), b, 0, s.k[2], a);
+  if (n[3] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 3, 2>), grid(n[3]), b, 0, s.k[2], a);
+  if (n[4] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 4, 2>), grid(n[4]), b, 0, s.k[3], a);
+  if (n[5] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 5, 2>), grid(n[5]), b, 0, s.k[2], a);
+  if (n[6] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 6, 2>), grid(n[6]), b, 0, s.k[3], a);
 }
 
 int launch_fused_f64(const FusedArgs<double> &a, const KindStreams &s) {
@@ -95,7 +95,21 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   double *cmax = (double *)(base + o_cmax);
   T *frac = (T *)(base + o_frac);
   int *nspl = (int *)(base + o_ns), *flag = c.graph_safe ? c.step_flag : (int *)(base + o_flag);
-  if (device_nsplit<T>(c, cx, cy, c.step_per_level, c.step_per_level ? 0 : c.step_q_split, cmax, nspl, frac))
+  // FP64: the scratch (area fluxes first, which the sub-cycle counts' pass over
+  // the Courant numbers also computes) is sized before the counts are known
+  T *xfx = nullptr, *yfx = nullptr, *q_tmp64 = nullptr;
+  const size_t b_xf = (sizeof(T) * d.sx * npz * nt + 255) & ~(size_t)255;
+  const size_t b_yf = (sizeof(T) * d.sy * npz * nt + 255) & ~(size_t)255;
+  char *sc64 = nullptr;
+  if constexpr (std::is_same<T, double>::value) {
+    sc64 = (char *)ctx_scratch(c, b_xf + b_yf + b_q + (fields ? b_pt + coltab_bytes<T>(npz, (long long)ni * nj * nt) : 0));
+    if (!sc64) return 1;
+    xfx = (T *)sc64;
+    yfx = (T *)(sc64 + b_xf);
+    sc64 += b_xf + b_yf;
+    q_tmp64 = (T *)sc64;
+  }
+  if (device_nsplit<T>(c, cx, cy, c.step_per_level, c.step_per_level ? 0 : c.step_q_split, cmax, nspl, frac, xfx, yfx))
     return 1;
   int cap = nsplit_cap;
   if (cap <= 0) {
@@ -119,12 +133,10 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     q_tmp = (T *)sc;
     pt_src = pt ? (T *)(sc + b_q) : nullptr;
     for (int t = 0; t < nt; t++) cols[t] = remap_cols_carve(sc + b_q + b_pt + b_col * t, npz, (long long)ni * nj);
-  } else if (fields) {
-    char *sc = (char *)ctx_scratch(c, b_q + b_pt + coltab_bytes<T>(npz, (long long)ni * nj * nt));
-    if (!sc) return 1;
-    q_tmp = (T *)sc;
-    pt_src = pt ? (T *)(sc + b_q) : nullptr;
-    tab = sc + b_q + b_pt;
+  } else if (sc64) {
+    q_tmp = q_tmp64;
+    pt_src = pt ? (T *)(sc64 + b_q) : nullptr;
+    tab = sc64 + b_q + b_pt;
   } else if (cap > 1) {
     q_tmp = (T *)ctx_scratch(c, sizeof(T) * qsize);
     if (!q_tmp) return 1;
@@ -177,6 +189,7 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   a.q_in = q_in;
   a.q_out = oop ? q_tmp : q_out;
   a.q_tmp = oop ? q_out : q_tmp;
+  a.xfx = xfx; a.yfx = yfx;
   a.cx = cx; a.cy = cy; a.mfx = mfx; a.mfy = mfy; a.dp1 = dp1;
   const GridDev<T> &g = grid_of<T>(c);
   a.area = g.area; a.rarea = g.rarea; a.dxa = g.dxa; a.dya = g.dya; a.dx = g.dx; a.dy = g.dy;

@@ -19,9 +19,8 @@ template <typename T>
 struct StripCtx {
   int i, ic, j0, h, nix, niy, lo_q, lo_fx, lo_mx;  // lane column; block rows; lane offsets in the row layouts
   bool col_out, lane_in, edge_strip, edge_rows, corner_wg, scale;
-  bool gen_src;  // q sources by the general (halo, six-tile, corner) rules
   T frac;
-  const T *cxk, *cyk, *mfxk, *mfyk;
+  const T *cxk, *cyk, *mfxk, *mfyk, *xfxk, *yfxk;
   const double *dp1k;
   long long tg, tdx, tdy, tgf;  // this tile's offsets in the metric arrays (s2, dx, dy, gfac)
   EdgeCoef ec;                  // FP32 edge strips: the lane's cube-edge coefficients
@@ -31,37 +30,34 @@ struct StripCtx {
 template <typename T>
 struct TrState {
   YPipe<T> py, pj;
-  T fx2_r[6];
   T fy2_prev, Fy_prev;
   const T *qin, *qhalo;
   const T *qsrc0;  // pass input of tile 1 at this tracer and level (six-tile halos)
   T *qout;
-  __amdgpu_buffer_rsrc_t qout_r;  // FP32: qout as a buffer (scalar row offset, lane offset)
-  __amdgpu_buffer_rsrc_t qin_r;   // FP32: qin likewise
+  __amdgpu_buffer_rsrc_t qout_r;  // qout as a buffer (scalar row offset, lane offset)
+  __amdgpu_buffer_rsrc_t qin_r;   // qin likewise
 };
 
 // level data carried between rows
 template <typename T>
 struct LvState {
-  T area_r[6], cx_r[6];
   T yfx_prev, mfy_prev;
 };
 
-// Everything row_step reads from HBM for one input row, fetched one row ahead
-// so that the loads of row t+1 are in flight while row t computes.  Upwind
-// metric candidates for both signs of the Courant number are fetched, so no
-// address depends on a loaded value.
+// Everything row_step reads for one input row, from the LDS ring.  The area
+// fluxes: FP32 the upwind factors for both signs of the Courant number, FP64
+// the fluxes themselves (k_area_flux, in upstream's product order).
 template <typename T, int NT>
 struct RowIn {
   T area, cyu, cxu, mfy, mfx, rarea;
-  T ya, yb, yc, yd, ye;  // FP32: gyp gym; FP64: dya(j-1) sg3(j-1) dya(j) sg1(j) dx
-  T xa, xb, xc, xd, xe;  // FP32: gxp gxm; FP64: dxa(i-1) sg2(i-1) dxa(i) sg0(i) dy
+  T ya, yb;  // FP32: gyp gym; FP64: the area flux through the y-face
+  T xa, xb;  // FP32: gxp gxm; FP64: through the x-face
   double dp1;
-  T area_m, cxm_u;  // FP32: area and cx of row r-3, from the LDS ring
+  T area_m, cxm_u;  // area and cx of row r-3
   T qy[NT], qx[NT];
-  T qw[NT][4];      // FP32: the y-sweep sources of rows r-1 .. r-4, from the LDS ring
-  T fx2m[NT];       // FP32: the inner x-flux of row r-3 (kept in the ring by this wave)
-  float *fx2w[NT];  // FP32: where this row's inner x-flux goes
+  T qw[NT][4];  // the y-sweep sources of rows r-1 .. r-4
+  T fx2m[NT];   // the inner x-flux of row r-3 (kept in the ring by this wave)
+  T *fx2w[NT];  // where this row's inner x-flux goes
 };
 
 // q sources per input row of a kind: the strips with corner cells read the
@@ -154,60 +150,6 @@ __device__ __forceinline__ void q_src(const FusedArgs<T> &a, const StripCtx<T> &
   }
 }
 
-template <typename T, int NT>
-__device__ __forceinline__ void row_fetch(const FusedArgs<T> &a, const StripCtx<T> &sc,
-                                          const TrState<T> (&st)[NT], const bool (&act)[NT], int t,
-                                          RowIn<T, NT> &in) {
-  constexpr bool fp64 = sizeof(T) == 8;
-  const RowIdx<T> x = row_idx(a, sc, t);
-  const int nid = a.nid;
-  // wave-uniform row bases, indexed by the lane's 32-bit column offset
-  in.area = (a.area + sc.tg + x.orow)[sc.lo_q];
-  in.cyu = (sc.cyk + (long long)(x.fc - a.js) * nid)[sc.lo_q];
-  const long long frow = (long long)(x.fc - a.jsd) * nid;
-  const long long gxrow = (long long)(x.rc - a.jsd) * (nid + 1) + (a.is - a.isd);
-  const long long urow = x.orow + (a.is - a.isd);
-  if constexpr (fp64) {
-    in.ya = (a.dya + sc.tg + frow - nid)[sc.lo_q];
-    in.yb = (a.sin_sg + 9 * sc.tg + 3 * a.ms2 + frow - nid)[sc.lo_q];
-    in.yc = (a.dya + sc.tg + frow)[sc.lo_q];
-    in.yd = (a.sin_sg + 9 * sc.tg + 1 * a.ms2 + frow)[sc.lo_q];
-    in.ye = (a.dx + sc.tdx + frow)[sc.lo_q];
-    in.xa = (a.dxa + sc.tg + urow - 1)[sc.lo_fx];
-    in.xb = (a.sin_sg + 9 * sc.tg + 2 * a.ms2 + urow - 1)[sc.lo_fx];
-    in.xc = (a.dxa + sc.tg + urow)[sc.lo_fx];
-    in.xd = (a.sin_sg + 9 * sc.tg + 0 * a.ms2 + urow)[sc.lo_fx];
-    in.xe = (a.dy + sc.tdy + gxrow)[sc.lo_fx];
-  } else {
-    in.ya = (a.gyp + sc.tgf + frow)[sc.lo_q];
-    in.yb = (a.gym + sc.tgf + frow)[sc.lo_q];
-    in.xa = (a.gxp + sc.tgf + gxrow)[sc.lo_fx];
-    in.xb = (a.gxm + sc.tgf + gxrow)[sc.lo_fx];
-  }
-  in.cxu = (sc.cxk + (long long)(x.rc - a.jsd) * sc.nix)[sc.lo_fx];
-  in.mfy = (sc.mfyk + (long long)(x.fc - a.js) * sc.niy)[sc.lo_mx];
-  in.mfx = (sc.mfxk + (long long)(x.mc - a.js) * sc.nix)[sc.lo_fx];
-  in.rarea = T(0);
-  in.dp1 = 0.0;
-  if (x.out_row) {
-    in.rarea = (a.rarea + sc.tg + x.corow)[sc.lo_q];
-    in.dp1 = (sc.dp1k + x.corow)[sc.lo_q];
-  }
-#pragma unroll
-  for (int n = 0; n < NT; n++) {
-    if (!act[n]) continue;
-    const T *py, *px;
-    if (sc.gen_src)
-      q_src<T, 2>(a, sc, st[n], x, py, px);
-    else
-      q_src<T, 0>(a, sc, st[n], x, py, px);
-    const T qy = *py;
-    const T qx = sc.gen_src ? *px : qy;
-    in.qy[n] = qy;
-    in.qx[n] = qx;
-  }
-}
-
 // One input row r = j0 - 3 + t of the streaming pass; U = t mod 6.  HO: the
 // advection order when fixed at compile time (0: taken from the arguments).
 // TW = t for the block's first six input rows, 6 after them.  Those rows
@@ -220,7 +162,6 @@ __device__ __forceinline__ void row_step(const FusedArgs<T> &a, const StripCtx<T
                                          LvState<T> &lv, TrState<T> (&st)[NT], const bool (&act)[NT],
                                          int t, const RowIn<T, NT> &in) {
   constexpr bool fp64 = sizeof(T) == 8;
-  constexpr int M3 = (U + 3) % 6;  // slot of row r-3
   const int nid = a.nid;
   const RowIdx<T> x = row_idx(a, sc, t);
   const int r = x.r;
@@ -229,42 +170,37 @@ __device__ __forceinline__ void row_step(const FusedArgs<T> &a, const StripCtx<T
 
   // ---- level data of this row (shared by the NT tracers)
   const T area_r = in.area;
-  if constexpr (fp64) lv.area_r[U] = area_r;
   const T cyu = in.cyu;
   // x * (1/nsplit) with 1/1 = 1 exactly: unconditional scaling rounds the same
   const T cys = TW >= 5 ? cyu * sc.frac : T(0);
   T yfx = T(0);
   if constexpr (TW >= 5) {
-    const bool pos = cyu > T(0);
     if constexpr (fp64)
-      yfx = pos ? cyu * in.ya * in.ye * in.yb : cyu * in.yc * in.ye * in.yd;
+      yfx = in.ya;
     else
-      yfx = cyu * (pos ? in.ya : in.yb);
+      yfx = cyu * (cyu > T(0) ? in.ya : in.yb);
     yfx = yfx * sc.frac;
   }
   const T cxr_u = in.cxu;
-  if constexpr (fp64) lv.cx_r[U] = cxr_u;
   const T cxr = cxr_u * sc.frac;
   T xfx;
   {
-    const bool pos = cxr_u > T(0);
     if constexpr (fp64)
-      xfx = pos ? cxr_u * in.xa * in.xe * in.xb : cxr_u * in.xc * in.xe * in.xd;
+      xfx = in.xa;
     else
-      xfx = cxr_u * (pos ? in.xa : in.xb);
+      xfx = cxr_u * (cxr_u > T(0) ? in.xa : in.xb);
     xfx = xfx * sc.frac;
   }
   const T xfxp = from_right(xfx);
   const T rax = area_r + xfx - xfxp;
-  const T area_m = fp64 ? lv.area_r[M3] : in.area_m;
+  const T area_m = in.area_m;
   T rrax = T(0), rray = T(0), ray = T(1);
   if constexpr (TW >= 6) ray = area_m + lv.yfx_prev - yfx;
   if constexpr (!fp64) {
     rrax = __builtin_amdgcn_rcpf(rax);
     if constexpr (TW >= 6) rray = __builtin_amdgcn_rcpf(ray);
   }
-  const T cxm_u = fp64 ? lv.cx_r[M3] : in.cxm_u;  // cx of row m (row r-3, loaded 3 steps ago)
-  const T cxm = TW >= 6 ? cxm_u * sc.frac : T(0);
+  const T cxm = TW >= 6 ? in.cxm_u * sc.frac : T(0);  // cx of row r-3
   const T mfys = TW >= 5 ? in.mfy * sc.frac : T(0);
   const T mfxs = TW >= 6 ? in.mfx * sc.frac : T(0);
   const T mfxp = TW >= 6 ? from_right(mfxs) : T(0);
@@ -290,10 +226,9 @@ __device__ __forceinline__ void row_step(const FusedArgs<T> &a, const StripCtx<T
     dd4 = dya_at(r);
   }
   // output row: thickness and area factors shared by the tracers
-  // (FP32 reads rarea and dp1 of every row from the ring and computes them
-  // without a branch; only output rows store)
-  T rarea = T(0), d1 = T(0), rdp2 = T(0), dp2 = T(0);
-  if (TW >= 6 && (!fp64 || x.out_row)) {
+  // (of every row, without a branch; only output rows store)
+  T rarea = T(0), d1 = T(0), rdp2 = T(0), dp2 = T(1);
+  if constexpr (TW >= 6) {
     rarea = in.rarea;
     const T ddiv = ((mfxs - mfxp) + (lv.mfy_prev - mfys)) * rarea;
     T xd = (T)in.dp1;
@@ -306,14 +241,13 @@ __device__ __forceinline__ void row_step(const FusedArgs<T> &a, const StripCtx<T
   // ---- the tracers
 #pragma unroll
   for (int n = 0; n < NT; n++) {
-    // FP32: an inactive tracer of an active wave computes on tracer 0's rows
-    // (what its ring slots hold) and stores nothing, so no branch per tracer
-    if (fp64 && !act[n]) continue;
+    // an inactive tracer of an active wave computes on tracer 0's rows (what
+    // its ring slots hold) and stores nothing, so no branch per tracer
     TrState<T> &s = st[n];
     const T qy = in.qy[n], qx = in.qx[n];
     // inner y-sweep at face r-2 and q_i of row r-3
-    const T fy2 = ypipe_step<T, U, TW, !fp64>(s.py, qy, in.qw[n], cys, ord_in, role_y, dd0, dd1, dd2, dd3, dd4);
-    const T qm = fp64 ? s.py.w[M3] : in.qw[n][2];
+    const T fy2 = ypipe_step<T, U, TW, true>(s.py, qy, in.qw[n], cys, ord_in, role_y, dd0, dd1, dd2, dd3, dd4);
+    const T qm = in.qw[n][2];
     // outer x-sweep of row r-3, inner x-sweep of row r, q_j of row r
     T fx = T(0);
     if constexpr (TW >= 6) {
@@ -325,10 +259,7 @@ __device__ __forceinline__ void row_step(const FusedArgs<T> &a, const StripCtx<T
       fx = xsweep<SIDE>(q_i, cxm, sc.i, a.is, a.ie, a.npx, a.edge, sc.edge_strip, hord, dxa_m, sc.ec);
     }
     const T fx2 = xsweep<SIDE>(qx, cxr, sc.i, a.is, a.ie, a.npx, a.edge, sc.edge_strip, ord_in, dxa_r, sc.ec);
-    if constexpr (fp64)
-      s.fx2_r[U] = fx2;
-    else
-      in.fx2w[n][0] = fx2;
+    in.fx2w[n][0] = fx2;
     const T fx2p = from_right(fx2);
     T q_j;
     if constexpr (fp64)
@@ -344,12 +275,15 @@ __device__ __forceinline__ void row_step(const FusedArgs<T> &a, const StripCtx<T
       s.Fy_prev = Fy;
       continue;
     }
-    const T Fx = T(0.5) * (fx + (fp64 ? s.fx2_r[M3] : in.fx2m[n])) * mfxs;
+    const T Fx = T(0.5) * (fx + in.fx2m[n]) * mfxs;
     const T Fxp = from_right(Fx);
     if (act[n] && x.out_row && sc.col_out) {
+      // the row as the scalar offset, the lane's column as the vector offset
       if constexpr (fp64) {
-        (s.qout + x.corow)[sc.lo_q] = (qm * d1 + (Fx - Fxp + s.Fy_prev - Fy) * rarea) / dp2;
-      } else {  // the row as the scalar offset, the lane's column as the vector offset
+        typedef unsigned u2 __attribute__((ext_vector_type(2)));
+        const double v = (qm * d1 + (Fx - Fxp + s.Fy_prev - Fy) * rarea) / dp2;
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), s.qout_r, sc.lo_q * 8, (int)x.corow * 8, 0);
+      } else {
         const float v = (qm * d1 + (Fx - Fxp + s.Fy_prev - Fy) * rarea) * rdp2;
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), s.qout_r, sc.lo_q * 4,
                                               (int)x.corow * 4, 0);
@@ -361,29 +295,46 @@ __device__ __forceinline__ void row_step(const FusedArgs<T> &a, const StripCtx<T
   lv.mfy_prev = mfys;
 }
 
-// ---- LDS row ring of the FP32 kernels.  Rows are loaded straight into LDS
-// with global_load_lds_dword, or buffer_load_dword ... lds where the row
-// address is a scalar offset (the data in flight holds no VGPRs), so the
-// loads of a row can be issued LR_AHEAD rows ahead.  The waves of a
-// workgroup split the LR_NL level arrays of a row between them (they stream
-// the same strip and level) and each loads its own tracers' rows.  The ring
-// also keeps the four rows behind the one computed: the stencil's values of
-// rows r-1 .. r-4 (y-sweep sources, area and cx of row r-3) are read back
-// from LDS instead of being carried in registers, and each wave keeps its
-// inner x-fluxes there for the three rows until they are averaged: fewer
-// VGPRs, more waves per CU.
+// ---- LDS row ring.  Rows are loaded straight into LDS with
+// global_load_lds_dword, or buffer_load_dword ... lds where the row address is
+// a scalar offset (the data in flight holds no VGPRs), so the loads of a row
+// can be issued LR_AHEAD rows ahead.  A row of 64 doubles is two planes of 64
+// dwords (low and high halves): each lane's address is its own, whatever its
+// column's source, and ds_read2_b32 returns both halves.  The waves of a
+// workgroup split the level arrays of a row between them (they stream the
+// same strip and level) and each loads its own tracers' rows.  The ring also
+// keeps the four rows behind the one computed: the stencil's values of rows
+// r-1 .. r-4 (y-sweep sources, area and cx of row r-3) are read back from LDS
+// instead of being carried in registers, and each wave keeps its inner
+// x-fluxes there for the three rows until they are averaged: fewer VGPRs,
+// more waves per CU.
+//
+// FP64 (W = 4, one tracer per wave): 61 KB of LDS, two workgroups per CU.  (A
+// shorter ring for the level arrays, three workgroups, ran the same: 5.2
+// against 5.0 ms; 5 to 8 waves per workgroup 3.3-3.6 against 3.5 ms at 7
+// tracers, 2.2-2.4 against 1.9 at 4: the vector pipe is the bound.)  The form it replaced held its windows in
+// registers (326 of them: one wave per SIMD) and fetched one row ahead into
+// registers, so that every row waited for HBM: C384 L127 9 tracers, two
+// passes: 10.0 -> 5.0 ms.
 constexpr int LR_DEPTH = 8;  // slots: rows t-4 .. t+3 at row t
 constexpr int LR_AHEAD = 3;  // rows issued ahead of the row computed
-constexpr int LR_NL = 12;  // area cyu cxu mfy mfx rarea gyp gym gxp gxm dp1.lo dp1.hi
 
-template <int W, int NT, int QN>
+// level planes: FP32 area cyu cxu mfy mfx rarea gyp gym gxp gxm dp1.lo dp1.hi;
+// FP64 area cxu cyu mfy mfx rarea yfx xfx dp1, two planes each
+template <typename T>
+constexpr int lr_nl() { return sizeof(T) == 4 ? 12 : 18; }
+template <typename T>
+constexpr int lr_p() { return sizeof(T) / 4; }
+
+template <typename T, int W, int NT, int QN>
 struct LdsRing {
   // per slot: the level arrays and q sources loaded by the DMA
-  float v[LR_DEPTH][LR_NL + W * NT * QN][FT_LANES];
+  float v[LR_DEPTH][lr_nl<T>() + W * NT * QN * lr_p<T>()][FT_LANES];
   // each wave's inner x-fluxes of rows t-3 .. t (written and read by the wave itself)
-  float fx2[4][W * NT][FT_LANES];
+  T fx2[4][W * NT][FT_LANES];
+  __device__ __forceinline__ float (*lev(int t, int j))[FT_LANES] { return v[t & (LR_DEPTH - 1)] + j; }
+  __device__ __forceinline__ float (*q(int t, int j))[FT_LANES] { return v[t & (LR_DEPTH - 1)] + lr_nl<T>() + j; }
 };
-
 __device__ __forceinline__ void lds_dma(const float *src, float *dst_row) {
   __builtin_amdgcn_global_load_lds((const void *)src, (__attribute__((address_space(3))) void *)dst_row, 4, 0, 0);
 }
@@ -396,171 +347,227 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
   __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4));
 }
 
-// issue the loads of input row t into ring slot t mod LR_DEPTH
-template <int W, int NT, int EK>
-__device__ __forceinline__ void ring_issue(const FusedArgs<float> &a, const StripCtx<float> &sc,
-                                           const TrState<float> (&st)[NT],
-                                           LdsRing<W, NT, ek_qn(EK)> &ring, int wave, int t) {
-  constexpr int QN = ek_qn(EK);
-  const RowIdx<float> x = row_idx(a, sc, t);
+// The level planes of a row by their source: the array's address of a row
+// (indices clamped to the domain by the caller), the row's length and the
+// lane's offset in it, in dwords; kind 0 cell columns, 1 x-faces, 2 y-face
+// columns.
+struct PlaneSrc {
+  const float *p;
+  int step, loff;
+};
+// r, f, m: the rows of the cell (input row), the y-face and the output cell
+template <typename T>
+__device__ __forceinline__ PlaneSrc plane_src(const FusedArgs<T> &a, const StripCtx<T> &sc, int j, long long r,
+                                              long long f, long long m) {
   const int nid = a.nid;
-  float(*slot)[FT_LANES] = ring.v[t & (LR_DEPTH - 1)];
-  const long long frow = (long long)(x.fc - a.jsd) * nid;
-  const long long gxrow = (long long)(x.rc - a.jsd) * (nid + 1) + (a.is - a.isd);
-  // uniform row base (scalar) + the lane's column offset in that array's
-  // row layout (cell, x-face, y-face column; dp1 as two 32-bit halves)
-  for (int j = wave; j < LR_NL; j += W) {
-    const float *base;
-    int kind;
+  PlaneSrc s{(const float *)a.area, nid, sc.lo_q};
+  if constexpr (sizeof(T) == 4) {
     switch (j) {
-      case 0: base = a.area + sc.tg + x.orow; kind = 0; break;
-      case 1: base = sc.cyk + (long long)(x.fc - a.js) * nid; kind = 0; break;
-      case 2: base = sc.cxk + (long long)(x.rc - a.jsd) * sc.nix; kind = 1; break;
-      case 3: base = sc.mfyk + (long long)(x.fc - a.js) * sc.niy; kind = 2; break;
-      case 4: base = sc.mfxk + (long long)(x.mc - a.js) * sc.nix; kind = 1; break;
-      case 5: base = a.rarea + sc.tg + x.corow; kind = 0; break;
-      case 6: base = a.gyp + sc.tgf + frow; kind = 0; break;
-      case 7: base = a.gym + sc.tgf + frow; kind = 0; break;
-      case 8: base = a.gxp + sc.tgf + gxrow; kind = 1; break;
-      case 9: base = a.gxm + sc.tgf + gxrow; kind = 1; break;
-      case 10: base = (const float *)(sc.dp1k + x.corow); kind = 3; break;
-      default: base = (const float *)(sc.dp1k + x.corow) + 1; kind = 3; break;
+      case 0: s.p = a.area + sc.tg + (r - a.jsd) * nid; break;
+      case 1: s.p = sc.cyk + (f - a.js) * nid; break;
+      case 2: s.p = sc.cxk + (r - a.jsd) * sc.nix; s.step = sc.nix; s.loff = sc.lo_fx; break;
+      case 3: s.p = sc.mfyk + (f - a.js) * sc.niy; s.step = sc.niy; s.loff = sc.lo_mx; break;
+      case 4: s.p = sc.mfxk + (m - a.js) * sc.nix; s.step = sc.nix; s.loff = sc.lo_fx; break;
+      case 5: s.p = a.rarea + sc.tg + (m - a.jsd) * nid; break;
+      case 6: s.p = a.gyp + sc.tgf + (f - a.jsd) * nid; break;
+      case 7: s.p = a.gym + sc.tgf + (f - a.jsd) * nid; break;
+      case 8: s.p = a.gxp + sc.tgf + (r - a.jsd) * (nid + 1) + (a.is - a.isd); s.step = nid + 1; s.loff = sc.lo_fx; break;
+      case 9: s.p = a.gxm + sc.tgf + (r - a.jsd) * (nid + 1) + (a.is - a.isd); s.step = nid + 1; s.loff = sc.lo_fx; break;
+      case 10: s.p = (const float *)(sc.dp1k + (m - a.jsd) * nid); s.step = 2 * nid; s.loff = 2 * sc.lo_q; break;
+      case 11: s.p = (const float *)(sc.dp1k + (m - a.jsd) * nid) + 1; s.step = 2 * nid; s.loff = 2 * sc.lo_q; break;
+      default: break;  // past the last plane: not issued
     }
-    const int off = kind == 0 ? sc.lo_q : (kind == 1 ? sc.lo_fx : (kind == 2 ? sc.lo_mx : 2 * sc.lo_q));
-    lds_dma(base + off, slot[j]);
+  } else {
+    const double *p = a.area;
+    int step = nid, loff = sc.lo_q;
+    switch (j >> 1) {
+      case 0: p = a.area + sc.tg + (r - a.jsd) * nid; break;
+      case 1: p = sc.cxk + (r - a.jsd) * sc.nix; step = sc.nix; loff = sc.lo_fx; break;
+      case 2: p = sc.cyk + (f - a.js) * nid; break;
+      case 3: p = sc.mfyk + (f - a.js) * sc.niy; step = sc.niy; loff = sc.lo_mx; break;
+      case 4: p = sc.mfxk + (m - a.js) * sc.nix; step = sc.nix; loff = sc.lo_fx; break;
+      case 5: p = a.rarea + sc.tg + (m - a.jsd) * nid; break;
+      case 6: p = sc.yfxk + (f - a.js) * nid; break;
+      case 7: p = sc.xfxk + (r - a.jsd) * sc.nix; step = sc.nix; loff = sc.lo_fx; break;
+      case 8: p = sc.dp1k + (m - a.jsd) * nid; break;
+      default: break;
+    }
+    s.p = (const float *)p + (j & 1);
+    s.step = 2 * step;
+    s.loff = 2 * loff;
   }
+  return s;
+}
+
+// the q sources of input row x of this wave's tracers, each lane's own address
+template <typename T, int W, int NT, int EK>
+__device__ __forceinline__ void issue_q(const FusedArgs<T> &a, const StripCtx<T> &sc, const TrState<T> (&st)[NT],
+                                        const RowIdx<T> &x, LdsRing<T, W, NT, ek_qn(EK)> &ring, int wave, int t) {
+  constexpr int QN = ek_qn(EK), P = lr_p<T>();
   // inactive tracers load tracer 0: every wave issues the same count
 #pragma unroll
   for (int n = 0; n < NT; n++) {
-    const float *py, *px;
-    q_src<float, EK>(a, sc, st[n], x, py, px);
-    lds_dma(py, slot[LR_NL + (wave * NT + n) * QN]);
-    if (QN == 2) lds_dma(px, slot[LR_NL + (wave * NT + n) * QN + 1]);
+    const T *py, *px;
+    q_src<T, EK>(a, sc, st[n], x, py, px);
+    float(*d)[FT_LANES] = ring.q(t, (wave * NT + n) * QN * P);
+#pragma unroll
+    for (int h = 0; h < P; h++) {
+      lds_dma((const float *)py + h, d[h]);
+      if (QN == 2) lds_dma((const float *)px + h, d[P + h]);
+    }
   }
+}
+
+// issue the loads of input row t into ring slot t mod LR_DEPTH
+template <typename T, int W, int NT, int EK>
+__device__ __forceinline__ void ring_issue(const FusedArgs<T> &a, const StripCtx<T> &sc, const TrState<T> (&st)[NT],
+                                           LdsRing<T, W, NT, ek_qn(EK)> &ring, int wave, int t) {
+  const RowIdx<T> x = row_idx(a, sc, t);
+  if constexpr (sizeof(T) == 8) {
+    for (int j = wave; j < lr_nl<T>(); j += W) {
+      const PlaneSrc s = plane_src(a, sc, j, x.rc, x.fc, x.mc);
+      lds_dma(s.p + s.loff, *ring.lev(t, j));
+    }
+  } else {
+    // (the same addresses as plane_src's, from the row offsets at hand: fewer scalar registers)
+    const int nid = a.nid;
+    const long long frow = (long long)(x.fc - a.jsd) * nid;
+    const long long gxrow = (long long)(x.rc - a.jsd) * (nid + 1) + (a.is - a.isd);
+    for (int j = wave; j < lr_nl<T>(); j += W) {
+      const float *base;
+      int kind;
+      switch (j) {
+        case 0: base = a.area + sc.tg + x.orow; kind = 0; break;
+        case 1: base = sc.cyk + (long long)(x.fc - a.js) * nid; kind = 0; break;
+        case 2: base = sc.cxk + (long long)(x.rc - a.jsd) * sc.nix; kind = 1; break;
+        case 3: base = sc.mfyk + (long long)(x.fc - a.js) * sc.niy; kind = 2; break;
+        case 4: base = sc.mfxk + (long long)(x.mc - a.js) * sc.nix; kind = 1; break;
+        case 5: base = a.rarea + sc.tg + x.corow; kind = 0; break;
+        case 6: base = a.gyp + sc.tgf + frow; kind = 0; break;
+        case 7: base = a.gym + sc.tgf + frow; kind = 0; break;
+        case 8: base = a.gxp + sc.tgf + gxrow; kind = 1; break;
+        case 9: base = a.gxm + sc.tgf + gxrow; kind = 1; break;
+        case 10: base = (const float *)(sc.dp1k + x.corow); kind = 3; break;
+        default: base = (const float *)(sc.dp1k + x.corow) + 1; kind = 3; break;
+      }
+      const int off = kind == 0 ? sc.lo_q : (kind == 1 ? sc.lo_fx : (kind == 2 ? sc.lo_mx : 2 * sc.lo_q));
+      lds_dma(base + off, *ring.lev(t, j));
+    }
+  }
+  issue_q<T, W, NT, EK>(a, sc, st, x, ring, wave, t);
 }
 
 // Lean blocks never clamp a row (every input row and every stencil row lies
 // inside the compute domain), so each level array's row address is affine in
-// the row: the wave's share of the level arrays is set up once per round as
-// (row-0 address, elements per row, lane offset) and each row costs one
-// multiply-add per array.  (The edge kinds, short of scalar registers, keep
+// the row: the wave's share of the level planes is set up once per round as
+// (row-0 address, dwords per row, lane offset) and each row costs one
+// multiply-add per plane.  (The edge kinds, short of scalar registers, keep
 // the per-row address expressions.)
-template <int W>
+template <typename T, int W>
 struct LeanRows {
-  static constexpr int M = (LR_NL + W - 1) / W;
-  const float *p[M];
+  static constexpr int M = (lr_nl<T>() + W - 1) / W;
   int step[M], loff[M];
-  __amdgpu_buffer_rsrc_t r[M];  // p[m] as a buffer: row t at scalar offset 4 t step, lane at 4 loff
+  __amdgpu_buffer_rsrc_t r[M];  // row t at scalar offset 4 t step, lane at 4 loff
 };
 
-template <int W>
-__device__ __forceinline__ LeanRows<W> lean_rows(const FusedArgs<float> &a, const StripCtx<float> &sc,
-                                                 int wave) {
-  LeanRows<W> lr;
-  const int nid = a.nid;
+template <typename T, int W>
+__device__ __forceinline__ LeanRows<T, W> lean_rows(const FusedArgs<T> &a, const StripCtx<T> &sc, int wave) {
+  LeanRows<T, W> lr;
   const long long r0 = sc.j0 - NG;  // input row of t = 0
 #pragma unroll
-  for (int m = 0; m < LeanRows<W>::M; m++) {
-    const int j = wave + m * W;
-    const float *p = a.area;
-    int step = nid, loff = sc.lo_q;
-    switch (j) {
-      case 0: p = a.area + sc.tg + (r0 - a.jsd) * nid; break;
-      case 1: p = sc.cyk + (r0 - 2 - a.js) * nid; break;
-      case 2: p = sc.cxk + (r0 - a.jsd) * sc.nix; step = sc.nix; loff = sc.lo_fx; break;
-      case 3: p = sc.mfyk + (r0 - 2 - a.js) * sc.niy; step = sc.niy; loff = sc.lo_mx; break;
-      case 4: p = sc.mfxk + (r0 - 3 - a.js) * sc.nix; step = sc.nix; loff = sc.lo_fx; break;
-      case 5: p = a.rarea + sc.tg + (r0 - 3 - a.jsd) * nid; break;
-      case 6: p = a.gyp + sc.tgf + (r0 - 2 - a.jsd) * nid; break;
-      case 7: p = a.gym + sc.tgf + (r0 - 2 - a.jsd) * nid; break;
-      case 8: p = a.gxp + sc.tgf + (r0 - a.jsd) * (nid + 1) + (a.is - a.isd); step = nid + 1; loff = sc.lo_fx; break;
-      case 9: p = a.gxm + sc.tgf + (r0 - a.jsd) * (nid + 1) + (a.is - a.isd); step = nid + 1; loff = sc.lo_fx; break;
-      case 10: p = (const float *)(sc.dp1k + (r0 - 3 - a.jsd) * nid); step = 2 * nid; loff = 2 * sc.lo_q; break;
-      case 11: p = (const float *)(sc.dp1k + (r0 - 3 - a.jsd) * nid) + 1; step = 2 * nid; loff = 2 * sc.lo_q; break;
-      default: break;  // past the last array: not issued
-    }
-    lr.p[m] = p;
-    lr.step[m] = step;
-    lr.loff[m] = loff;
-    lr.r[m] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), (short)0, 0x7fffffff, 0x00020000);
+  for (int m = 0; m < LeanRows<T, W>::M; m++) {
+    const PlaneSrc s = plane_src(a, sc, wave + m * W, r0, r0 - 2, r0 - 3);
+    lr.step[m] = s.step;
+    lr.loff[m] = s.loff;
+    lr.r[m] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(s.p), (short)0, 0x7fffffff, 0x00020000);
   }
   return lr;
 }
 
-template <int W, int NT>
-__device__ __forceinline__ void ring_issue_lean(const FusedArgs<float> &a, const StripCtx<float> &sc,
-                                                const TrState<float> (&st)[NT], const LeanRows<W> &lr,
-                                                LdsRing<W, NT, 1> &ring, int wave, int t) {
-  float(*slot)[FT_LANES] = ring.v[t & (LR_DEPTH - 1)];
+template <typename T, int W, int NT, int QN>
+__device__ __forceinline__ void issue_planes(const LeanRows<T, W> &lr, LdsRing<T, W, NT, QN> &ring, int wave, int t) {
 #pragma unroll
-  for (int m = 0; m < LeanRows<W>::M; m++)
-    if (wave + m * W < LR_NL)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(lr.r[m], (__attribute__((address_space(3))) void *)slot[wave + m * W], 4,
+  for (int m = 0; m < LeanRows<T, W>::M; m++)
+    if (wave + m * W < lr_nl<T>())
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(lr.r[m], (__attribute__((address_space(3))) void *)*ring.lev(t, wave + m * W), 4,
                                                lr.loff[m] * 4, t * lr.step[m] * 4, 0, 0);
-  const int orow = (sc.j0 - NG + t - a.jsd) * a.nid;
-#pragma unroll
-  for (int n = 0; n < NT; n++)  // inactive tracers load tracer 0: every wave issues the same count
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(st[n].qin_r, (__attribute__((address_space(3))) void *)slot[LR_NL + wave * NT + n],
-                                             4, sc.lo_q * 4, orow * 4, 0, 0);
 }
 
-template <int W, int NT, int EK>
-__device__ __forceinline__ void ring_issue_mixed(const FusedArgs<float> &a, const StripCtx<float> &sc,
-                                                 const TrState<float> (&st)[NT], const LeanRows<W> &lr,
-                                                 LdsRing<W, NT, ek_qn(EK)> &ring, int wave, int t) {
-  constexpr int QN = ek_qn(EK);
-  float(*slot)[FT_LANES] = ring.v[t & (LR_DEPTH - 1)];
+template <typename T, int W, int NT>
+__device__ __forceinline__ void ring_issue_lean(const FusedArgs<T> &a, const StripCtx<T> &sc,
+                                                const TrState<T> (&st)[NT], const LeanRows<T, W> &lr,
+                                                LdsRing<T, W, NT, 1> &ring, int wave, int t) {
+  constexpr int P = lr_p<T>();
+  issue_planes(lr, ring, wave, t);
+  const int orow = (sc.j0 - NG + t - a.jsd) * a.nid * (int)sizeof(T);
 #pragma unroll
-  for (int m = 0; m < LeanRows<W>::M; m++)
-    if (wave + m * W < LR_NL)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(lr.r[m], (__attribute__((address_space(3))) void *)slot[wave + m * W], 4,
-                                               lr.loff[m] * 4, t * lr.step[m] * 4, 0, 0);
-  const RowIdx<float> x = row_idx(a, sc, t);
+  for (int n = 0; n < NT; n++)  // inactive tracers load tracer 0: every wave issues the same count
 #pragma unroll
-  for (int n = 0; n < NT; n++) {
-    const float *py, *px;
-    q_src<float, EK>(a, sc, st[n], x, py, px);
-    lds_dma(py, slot[LR_NL + (wave * NT + n) * QN]);
-    if (QN == 2) lds_dma(px, slot[LR_NL + (wave * NT + n) * QN + 1]);
+    for (int h = 0; h < P; h++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          st[n].qin_r, (__attribute__((address_space(3))) void *)*ring.q(t, (wave * NT + n) * P + h), 4,
+          sc.lo_q * (int)sizeof(T), orow + 4 * h, 0, 0);
+}
+
+template <typename T, int W, int NT, int EK>
+__device__ __forceinline__ void ring_issue_mixed(const FusedArgs<T> &a, const StripCtx<T> &sc,
+                                                 const TrState<T> (&st)[NT], const LeanRows<T, W> &lr,
+                                                 LdsRing<T, W, NT, ek_qn(EK)> &ring, int wave, int t) {
+  issue_planes(lr, ring, wave, t);
+  issue_q<T, W, NT, EK>(a, sc, st, row_idx(a, sc, t), ring, wave, t);
+}
+
+// the lane's value of array row a (plane index in units of T's planes from base)
+template <typename T>
+__device__ __forceinline__ T plane_get(float (*rows)[FT_LANES], int lane) {
+  if constexpr (sizeof(T) == 4) {
+    return rows[0][lane];
+  } else {
+    const unsigned long long lo = __float_as_uint(rows[0][lane]), hi = __float_as_uint(rows[1][lane]);
+    return __longlong_as_double((long long)(lo | (hi << 32)));
   }
 }
 
-template <int W, int NT, int QN>
-__device__ __forceinline__ void ring_read(LdsRing<W, NT, QN> &ring, int wave, int lane, int t,
-                                          RowIn<float, NT> &in) {
-  const float(*slot)[FT_LANES] = ring.v[t & (LR_DEPTH - 1)];
-  const float(*slot_m)[FT_LANES] = ring.v[(t - 3) & (LR_DEPTH - 1)];
-  in.area_m = slot_m[0][lane];
-  in.cxm_u = slot_m[2][lane];
-  in.area = slot[0][lane];
-  in.cyu = slot[1][lane];
-  in.cxu = slot[2][lane];
-  in.mfy = slot[3][lane];
-  in.mfx = slot[4][lane];
-  in.rarea = slot[5][lane];
-  in.ya = slot[6][lane];
-  in.yb = slot[7][lane];
-  in.xa = slot[8][lane];
-  in.xb = slot[9][lane];
-  const unsigned long long lo = __float_as_uint(slot[10][lane]), hi = __float_as_uint(slot[11][lane]);
-  in.dp1 = __longlong_as_double((long long)(lo | (hi << 32)));
+template <typename T, int W, int NT, int QN>
+__device__ __forceinline__ void ring_read(LdsRing<T, W, NT, QN> &ring, int wave, int lane, int t, RowIn<T, NT> &in) {
+  constexpr int P = lr_p<T>(), CX = sizeof(T) == 8 ? 1 : 2, CY = 3 - CX;  // cx, cy among the level arrays
+  auto lev = [&](int arr) { return plane_get<T>(ring.lev(t, arr * P), lane); };
+  in.area_m = plane_get<T>(ring.lev(t - 3, 0), lane);
+  in.cxm_u = plane_get<T>(ring.lev(t - 3, CX * P), lane);
+  in.area = lev(0);
+  in.cyu = lev(CY);
+  in.cxu = lev(CX);
+  in.mfy = lev(3);
+  in.mfx = lev(4);
+  in.rarea = lev(5);
+  in.ya = lev(6);
+  if constexpr (sizeof(T) == 4) {
+    in.yb = lev(7);
+    in.xa = lev(8);
+    in.xb = lev(9);
+    in.dp1 = plane_get<double>(ring.lev(t, 10), lane);
+  } else {
+    in.xa = lev(7);
+    in.dp1 = lev(8);
+  }
 #pragma unroll
   for (int n = 0; n < NT; n++) {
+    const int b = (wave * NT + n) * QN * P;
 #pragma unroll
-    for (int d = 1; d <= 4; d++) in.qw[n][d - 1] = ring.v[(t - d) & (LR_DEPTH - 1)][LR_NL + (wave * NT + n) * QN][lane];
+    for (int d = 1; d <= 4; d++) in.qw[n][d - 1] = plane_get<T>(ring.q(t - d, b), lane);
     in.fx2m[n] = ring.fx2[(t - 3) & 3][wave * NT + n][lane];
     in.fx2w[n] = &ring.fx2[t & 3][wave * NT + n][lane];
-    in.qy[n] = slot[LR_NL + (wave * NT + n) * QN][lane];
-    in.qx[n] = QN == 2 ? slot[LR_NL + (wave * NT + n) * QN + 1][lane] : in.qy[n];
+    in.qy[n] = plane_get<T>(ring.q(t, b), lane);
+    in.qx[n] = QN == 2 ? plane_get<T>(ring.q(t, b + P), lane) : in.qy[n];
   }
 }
 
 // wait until this wave's loads of row t are in LDS (loads complete in issue
 // order; ahead = rows issued after t; every wave issues at least NMIN loads
 // per row), then until every wave's are (barrier)
-template <int W, int NT, int QN>
+template <typename T, int W, int NT, int QN>
 __device__ __forceinline__ void ring_wait(int ahead) {
-  constexpr int NMIN = LR_NL / W + NT * QN;
+  constexpr int NMIN = lr_nl<T>() / W + NT * QN * lr_p<T>();
   static_assert((LR_AHEAD - 1) * NMIN < 64, "vmcnt range");
   if (ahead >= 2)
     wait_vm_lgkm0<2 * NMIN>();
@@ -640,7 +647,6 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
   sc.edge_strip = EK >= 2 && a.edge && (i0 - NG <= 2 || i0 - NG + FT_LANES - 1 >= a.npx - 2);
   if constexpr (sizeof(T) == 4) sc.ec = edge_coef_of(sc.edge_strip ? edge_role(sc.i, a.is, a.ie, a.npx, a.edge) : 0);
   sc.edge_rows = EK != 0 && EK <= 4;
-  sc.gen_src = EK != 0;
   sc.corner_wg = a.corners != 0u && (strip == 0 || strip == a.nstrip - 1) &&
                  (EK == 2 ? (vb == 0 || vb == a.nvblk - 1) : (EK == 3 || EK == 4));
   sc.scale = nspl > 1;
@@ -658,6 +664,10 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
   sc.cyk = a.cy + tile * a.tcy + (long long)k * a.sy;
   sc.mfxk = a.mfx + tile * a.tmx + (long long)k * a.smx;
   sc.mfyk = a.mfy + tile * a.tmy + (long long)k * a.smy;
+  if constexpr (sizeof(T) == 8) {
+    sc.xfxk = a.xfx + tile * a.tcx + (long long)k * a.sx;
+    sc.yfxk = a.yfx + tile * a.tcy + (long long)k * a.sy;
+  }
   sc.dp1k = a.dp1 + tile * a.tdp + (long long)k * a.s2;
   const T *in;
   T *out;
@@ -678,36 +688,34 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
       st[n].qin = in + toff + qoff;
       st[n].qhalo = a.q_in + toff + qoff;
       st[n].qout = out + toff + qoff;
-      if constexpr (sizeof(T) == 4) {
-        st[n].qout_r = __builtin_amdgcn_make_buffer_rsrc(st[n].qout, (short)0, 0x7fffffff, 0x00020000);
-        st[n].qin_r = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(st[n].qin), (short)0, 0x7fffffff, 0x00020000);
-      }
+      st[n].qout_r = __builtin_amdgcn_make_buffer_rsrc(st[n].qout, (short)0, 0x7fffffff, 0x00020000);
+      st[n].qin_r = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(st[n].qin), (short)0, 0x7fffffff, 0x00020000);
       st[n].fy2_prev = st[n].Fy_prev = T(0);
     }
     LvState<T> lv;
     lv.yfx_prev = lv.mfy_prev = T(0);
     const bool any = act[0];
-    if constexpr (sizeof(T) == 4) {
+    {
       constexpr int QN = ek_qn(EK);
       static_assert(LR_AHEAD == 3 && LR_DEPTH >= LR_AHEAD + 5, "ring_wait covers up to two rows ahead; rows t-4..t+3 kept");
-      __shared__ LdsRing<W, NT, QN> ring;
+      __shared__ LdsRing<T, W, NT, QN> ring;
       // the previous round's last reads of every slot are done before the
       // prologue overwrites them
-      if (rd > 0) ring_wait<W, NT, QN>(0);
-      const LeanRows<W> lr = lean_rows<W>(a, sc, wave);
+      if (rd > 0) ring_wait<T, W, NT, QN>(0);
+      const LeanRows<T, W> lr = lean_rows<T, W>(a, sc, wave);
       auto issue = [&](int t) {
         if constexpr (EK == 0) {
-          ring_issue_lean<W, NT>(a, sc, st, lr, ring, wave, t);
+          ring_issue_lean<T, W, NT>(a, sc, st, lr, ring, wave, t);
         } else if constexpr (EK >= 5) {  // lean rows: no row index clamps
-          ring_issue_mixed<W, NT, EK>(a, sc, st, lr, ring, wave, t);
+          ring_issue_mixed<T, W, NT, EK>(a, sc, st, lr, ring, wave, t);
         } else {
           // rows whose row indices do not clamp take the affine addresses
           // for the level arrays; the q sources keep their per-lane rules
           const int r = sc.j0 - NG + t;
           if (r >= a.js + NG && r <= a.je)
-            ring_issue_mixed<W, NT, EK>(a, sc, st, lr, ring, wave, t);
+            ring_issue_mixed<T, W, NT, EK>(a, sc, st, lr, ring, wave, t);
           else
-            ring_issue<W, NT, EK>(a, sc, st, ring, wave, t);
+            ring_issue<T, W, NT, EK>(a, sc, st, ring, wave, t);
         }
       };
       // The lean kinds (0, and 5 / 6 in the edge strips, whose blocks are H
@@ -722,10 +730,10 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
 #define FV3_RROW(U, TW)                                                              \
   if (PAD || t0 + U < nrow) {                                                        \
     const int t = t0 + U;                                                            \
-    ring_wait<W, NT, QN>(min(LR_AHEAD - 1, nrow - 1 - t));                           \
+    ring_wait<T, W, NT, QN>(min(LR_AHEAD - 1, nrow - 1 - t));                           \
     if (t + LR_AHEAD < nrow) issue(t + LR_AHEAD);                                    \
     RowIn<T, NT> in;                                                                 \
-    ring_read<W, NT, QN>(ring, wave, lane, t, in);                                   \
+    ring_read<T, W, NT, QN>(ring, wave, lane, t, in);                                   \
     row_step<T, NT, U, HO, ek_side(EK), TW>(a, sc, lv, st, act, t, in);              \
   }
       if (any) {
@@ -741,28 +749,11 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
         }
       } else {  // no tracer of this wave in this round: its loads and barriers only
         for (int t = 0; t < nrun; t++) {
-          ring_wait<W, NT, QN>(min(LR_AHEAD - 1, nrow - 1 - t));
+          ring_wait<T, W, NT, QN>(min(LR_AHEAD - 1, nrow - 1 - t));
           if (t + LR_AHEAD < nrow) issue(t + LR_AHEAD);
         }
       }
 #undef FV3_RROW
-      continue;
-    }
-    // rows are fetched one ahead; the bare s_barrier keeps the waves of the
-    // workgroup (same level data, L1 reuse) in step without waiting for the
-    // loads in flight -- the waves share no memory
-    // double buffer by row parity (6 rows per unrolled step: parity is U's)
-    RowIn<T, NT> buf[2];
-    if (any) row_fetch<T, NT>(a, sc, st, act, 0, buf[0]);
-    for (int t0 = 0; t0 < nrow; t0 += 6) {
-#define FV3_ROW(U)                                                                   \
-  if (any && t0 + U < nrow) {                                                        \
-    if (t0 + U + 1 < nrow) row_fetch<T, NT>(a, sc, st, act, t0 + U + 1, buf[(U + 1) & 1]); \
-    row_step<T, NT, U, HO, ek_side(EK)>(a, sc, lv, st, act, t0 + U, buf[U & 1]); \
-  }                                                                                  \
-  if (W > 1) __builtin_amdgcn_s_barrier();
-      FV3_ROW(0) FV3_ROW(1) FV3_ROW(2) FV3_ROW(3) FV3_ROW(4) FV3_ROW(5)
-#undef FV3_ROW
     }
   }
 }

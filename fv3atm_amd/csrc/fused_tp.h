@@ -59,6 +59,7 @@ struct FusedArgs {
   T *q_out, *q_tmp;
   const T *cx, *cy, *mfx, *mfy;
   const double *dp1;
+  const T *xfx, *yfx;  // FP64 form: area fluxes in the layouts of cx, cy (unscaled)
   // metrics (one tile)
   const T *area, *rarea, *dxa, *dya, *dx, *dy, *sin_sg;
   const T *gxp, *gxm, *gyp, *gym;  // FP32 form: combined upwind area-flux factors

@@ -97,6 +97,57 @@ __global__ void __launch_bounds__(256) k_cmax(const T *cx, const T *cy, const do
   if (threadIdx.x == 0) atomic_max_nonneg(&cmax[k], red[0]);
 }
 
+// k_cmax with the area fluxes of every face in the same pass (each Courant
+// number is read once): cx dxa dy sin_sg with the upwind metric, in that
+// order.  A block takes 64 columns and AF_ROWS rows of a level; a thread's
+// point (i, j) has the x-face and the y-face at its lower sides.
+constexpr int AF_ROWS = 32;
+template <typename T>
+__global__ void __launch_bounds__(256) k_area_flux(const T *cx, const T *cy, const GridDev<T> g, const double *sin_sg64,
+                                                   Dims d, int npz, T *xfx, T *yfx, double *cmax) {
+  const int z = blockIdx.z, tile = z / npz, k = z % npz;
+  const T *sg = g.sin_sg + (long long)tile * 9 * g.s2, *dxa = g.dxa + tile * g.s2, *dya = g.dya + tile * g.s2;
+  const T *dx = g.dx + tile * g.sdx, *dy = g.dy + tile * g.sdy;
+  const double *s5 = sin_sg64 + (long long)tile * 9 * g.s2 + 4 * g.s2;
+  const bool top = (k + 1) < npz / 6;
+  const int i = d.isd + (int)(blockIdx.x * 64 + (threadIdx.x & 63));
+  double m = 0.0;
+  for (int r = threadIdx.x >> 6; r < AF_ROWS; r += 4) {
+    const int j = d.jsd + (int)blockIdx.y * AF_ROWS + r;
+    if (j > d.jed || i > d.ied) continue;
+    const long long cell = (long long)(j - d.jsd) * d.nid + (i - d.isd);
+    T cv = T(0), cw = T(0);
+    if (i >= d.is && i <= d.ie + 1) {
+      const long long o = (long long)z * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is);
+      cv = cx[o];
+      const T dyv = dy[(long long)(j - d.jsd) * (d.nid + 1) + (i - d.isd)];
+      xfx[o] = cv > T(0) ? cv * dxa[cell - 1] * dyv * sg[2 * g.s2 + cell - 1] : cv * dxa[cell] * dyv * sg[cell];
+    }
+    if (j >= d.js && j <= d.je + 1) {
+      const long long o = (long long)z * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd);
+      cw = cy[o];
+      const T dxv = dx[cell];
+      yfx[o] = cw > T(0) ? cw * dya[cell - d.nid] * dxv * sg[3 * g.s2 + cell - d.nid]
+                         : cw * dya[cell] * dxv * sg[1 * g.s2 + cell];
+    }
+    if (i >= d.is && i <= d.ie && j >= d.js && j <= d.je) {
+      const double ax = fabs((double)cv), ay = fabs((double)cw);
+      if (top)
+        m = mx3(m, ax, ay);
+      else
+        m = mx2(m, mx2(ax, ay) + 1.0 - s5[cell]);
+    }
+  }
+  __shared__ double red[256];
+  red[threadIdx.x] = m;
+  __syncthreads();
+  for (int s = 128; s > 0; s >>= 1) {
+    if ((int)threadIdx.x < s) red[threadIdx.x] = mx2(red[threadIdx.x], red[threadIdx.x + s]);
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) atomic_max_nonneg(&cmax[k], red[0]);
+}
+
 // nsplit(k) and 1/nsplit from cmax (tracer_2d_1L per level, tracer_2d global)
 template <typename T>
 __global__ void k_nsplit(const double *cmax, int npz, int per_level, int q_split, int *nsplit,
@@ -128,22 +179,30 @@ __global__ void k_zero(T *p, int n) {
 
 template <typename T>
 int device_nsplit(Ctx &c, const T *cx, const T *cy, bool per_level, int q_split, double *cmax,
-                  int *nsplit, T *frac) {
+                  int *nsplit, T *frac, T *xfx, T *yfx) {
   const Dims d = c.d;
   const int npz = c.npz, nt = c.ntiles;
   hipLaunchKernelGGL(k_zero<double>, dim3(1), dim3(256), 0, c.stream, cmax, npz);
   FV3_HIP(hipGetLastError());
   dim3 b(256), gr((unsigned)std::min(64, (d.ie - d.is + 1) * (d.je - d.js + 1) / 256 + 1), 1,
                   (unsigned)(npz * nt));
-  hipLaunchKernelGGL(k_cmax<T>, gr, b, 0, c.stream, cx, cy, c.grid64.sin_sg, d, npz, c.grid64.s2, cmax);
+  if (xfx) {
+    const dim3 ga((unsigned)((d.nid + 63) / 64), (unsigned)((d.njd + AF_ROWS - 1) / AF_ROWS), (unsigned)(npz * nt));
+    hipLaunchKernelGGL(k_area_flux<T>, ga, b, 0, c.stream, cx, cy, grid_of<T>(c), c.grid64.sin_sg, d, npz, xfx, yfx,
+                       cmax);
+  } else {
+    hipLaunchKernelGGL(k_cmax<T>, gr, b, 0, c.stream, cx, cy, c.grid64.sin_sg, d, npz, c.grid64.s2, cmax);
+  }
   FV3_HIP(hipGetLastError());
   hipLaunchKernelGGL(k_nsplit<T>, dim3(1), dim3(1), 0, c.stream, cmax, npz, per_level ? 1 : 0,
                      q_split, nsplit, frac);
   FV3_HIP(hipGetLastError());
   return 0;
 }
-template int device_nsplit<double>(Ctx &, const double *, const double *, bool, int, double *, int *, double *);
-template int device_nsplit<float>(Ctx &, const float *, const float *, bool, int, double *, int *, float *);
+template int device_nsplit<double>(Ctx &, const double *, const double *, bool, int, double *, int *, double *,
+                                   double *, double *);
+template int device_nsplit<float>(Ctx &, const float *, const float *, bool, int, double *, int *, float *, float *,
+                                  float *);
 
 template <typename T>
 static size_t align_up(size_t b) {
