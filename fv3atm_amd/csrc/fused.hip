@@ -16,14 +16,14 @@ static void go64(const FusedArgs<double> &a, const KindStreams &s) {
   const dim3 b(FT_LANES * 4);
   int n[7];
   fused_grid_split(a, n);
-  auto grid = [&](int c) { return dim3((unsigned)c, (unsigned)a.npz, (unsigned)a.ntiles); };
-  if (n[0] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 0, 2>), grid(n[0]), b, 0, s.k[0], a);
-  if (n[1] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 1, 2>), grid(n[1]), b, 0, s.k[1], a);
-  if (n[2] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 2, 2>), grid(n[2]), b, 0, s.k[2], a);
-  if (n[3] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 3, 2>), grid(n[3]), b, 0, s.k[2], a);
-  if (n[4] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 4, 2>), grid(n[4]), b, 0, s.k[3], a);
-  if (n[5] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 5, 2>), grid(n[5]), b, 0, s.k[2], a);
-  if (n[6] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 6, 2>), grid(n[6]), b, 0, s.k[3], a);
+  auto grid = [&](int k) { return dim3(fused_grid_x(a, n[k], 4), (unsigned)a.npz, (unsigned)a.ntiles); };
+  if (n[0] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 0, 2>), grid(0), b, 0, s.k[0], a);
+  if (n[1] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 1, 2>), grid(1), b, 0, s.k[1], a);
+  if (n[2] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 2, 2>), grid(2), b, 0, s.k[2], a);
+  if (n[3] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 3, 2>), grid(3), b, 0, s.k[2], a);
+  if (n[4] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 4, 2>), grid(4), b, 0, s.k[3], a);
+  if (n[5] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 5, 2>), grid(5), b, 0, s.k[2], a);
+  if (n[6] > 0) hipLaunchKernelGGL((k_fused_tp<double, 4, 1, HO, 6, 2>), grid(6), b, 0, s.k[3], a);
 }
 
 int launch_fused_f64(const FusedArgs<double> &a, const KindStreams &s) {
@@ -156,9 +156,7 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   a.tmx = d.smx * npz;
   a.tmy = d.smy * npz;
   a.tdp = d.s2 * npz;
-  a.H = std::min(nj, c.fused_h > 0 ? c.fused_h : 60);
   a.nstrip = (ni + FT_BX - 1) / FT_BX;
-  a.nvblk = (nj + a.H - 1) / a.H;
   // interior strips: every lane's column i0-3..i0+60 lies in the compute
   // domain and, on a cube face, 3 or more cells inside the tile; their lean
   // rows lt..lb keep every input row j0-3..j0+H+2 in the domain and every
@@ -179,7 +177,15 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     int s0 = -1, s1 = -2;
     for (int st = 0; st < a.nstrip; st++)
       if (strip_ok(st)) { if (s0 < 0) s0 = st; s1 = st; }
-    if (s0 >= 0 && a.lb >= a.lt) {
+    const bool inner = s0 >= 0 && a.lb >= a.lt;
+    const int rows = inner ? a.lb - a.lt + 1 : nj;
+    // (resident workgroups of four waves: three per CU in FP32, two in FP64)
+    const long long units = (long long)a.nstrip * npz * nt * ((nq + 3) / 4);
+    a.H = c.fused_h > 0 ? c.fused_h
+                        : fused_block_rows(rows, units, sizeof(T) == 4 ? 768 : 512, inner ? 2.5 : 2.0 * NG);
+    a.H = std::min(nj, a.H);
+    a.nvblk = (nj + a.H - 1) / a.H;
+    if (inner) {
       a.s_lo = s0;
       a.s_hi = s1;
       a.nmid = (a.lb - a.lt + a.H) / a.H;

@@ -598,39 +598,28 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
   // whole block: this level is done, or needs more passes than are launched
   // (reported by the caller's nsplit check; nothing is written for it)
   if (a.it > nspl || nspl > a.cap) return;
-  int strip, vb, j0, h;
+  constexpr int per_round = W * NT;
+  const int rounds = (a.nq + per_round - 1) / per_round;
+  int strip, vb, j0, h, rd = 0;
   {
     const int ns = a.s_hi >= a.s_lo ? a.s_hi - a.s_lo + 1 : 0;
-    const int bx = (int)blockIdx.x;
-    if constexpr (EK == 0) {  // interior strips, lean rows
-      strip = a.s_lo + bx % ns;
-      vb = bx / ns;
-      j0 = a.lt + vb * a.H;
-      h = min(a.H, a.lb + 1 - j0);
-    } else if constexpr (EK == 1) {  // interior strips, the rows above and below the lean rows
-      strip = a.s_lo + bx % ns;
-      vb = bx / ns;
-      j0 = vb == 0 ? a.js : a.lb + 1;
-      h = vb == 0 ? a.lt - a.js : a.je - a.lb;
-    } else if constexpr (EK == 2) {  // every strip (no interior strip exists)
-      strip = bx % a.nstrip;
-      vb = bx / a.nstrip;
+    // strips of this kind, left of (3, 5) or right of (4, 6) the interior ones (0, 1); 2: all
+    const int nside = EK <= 1 ? ns : (EK == 2 ? a.nstrip : (EK == 3 || EK == 5 ? a.s_lo : a.nstrip - 1 - a.s_hi));
+    const int s0 = EK <= 1 ? a.s_lo : (EK == 4 || EK == 6 ? a.s_hi + 1 : 0);
+    int bx = (int)blockIdx.x;
+    if (rounds > 1) fused_block_round(bx, (int)gridDim.x / rounds, rounds, bx, rd);
+    strip = s0 + bx % nside;
+    vb = bx / nside;
+    if constexpr (EK == 2) {  // every strip (no interior strip exists), whole height
       j0 = a.js + vb * a.H;
       h = min(a.H, a.je + 1 - j0);
-    } else {
-      // 3 / 5: strips left of the interior strips; 4 / 6: right of them
-      const int nside = EK == 3 || EK == 5 ? a.s_lo : a.nstrip - 1 - a.s_hi;
-      strip = (EK == 3 || EK == 5 ? 0 : a.s_hi + 1) + bx % nside;
-      vb = bx / nside;
-      if constexpr (EK <= 4) {  // the top and bottom blocks
-        j0 = vb == 0 ? a.js : a.lb + 1;
-        h = vb == 0 ? a.lt - a.js : a.je - a.lb;
-      } else {  // the lean rows
-        j0 = a.lt + vb * a.H;
-        h = min(a.H, a.lb + 1 - j0);
-      }
+    } else if constexpr (EK == 0 || EK >= 5) {  // lean rows
+      j0 = a.lt + vb * a.H;
+      h = min(a.H, a.lb + 1 - j0);
+    } else {  // the rows above and below the lean rows
+      j0 = vb == 0 ? a.js : a.lb + 1;
+      h = vb == 0 ? a.lt - a.js : a.je - a.lb;
     }
-    (void)ns;
   }
   const int i0 = a.is + strip * FT_BX;
   StripCtx<T> sc;
@@ -672,90 +661,81 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
   const T *in;
   T *out;
   pass_buffers(a, nspl, in, out);
-  const int per_round = W * NT;
-  const int rounds = (a.nq + per_round - 1) / per_round;
   const int nrow = sc.h + 2 * NG;
-  for (int rd = 0; rd < rounds; rd++) {
-    TrState<T> st[NT];
-    bool act[NT];
+  TrState<T> st[NT];
+  bool act[NT];
 #pragma unroll
-    for (int n = 0; n < NT; n++) {
-      const int iq = rd * per_round + wave * NT + n;
-      act[n] = iq < a.nq;
-      const long long qoff = (long long)(act[n] ? iq : 0) * a.npz * a.s2 + (long long)k * a.s2;
-      const long long toff = (long long)blockIdx.z * a.tq;
-      st[n].qsrc0 = in + qoff;
-      st[n].qin = in + toff + qoff;
-      st[n].qhalo = a.q_in + toff + qoff;
-      st[n].qout = out + toff + qoff;
-      st[n].qout_r = __builtin_amdgcn_make_buffer_rsrc(st[n].qout, (short)0, 0x7fffffff, 0x00020000);
-      st[n].qin_r = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(st[n].qin), (short)0, 0x7fffffff, 0x00020000);
-      st[n].fy2_prev = st[n].Fy_prev = T(0);
-    }
-    LvState<T> lv;
-    lv.yfx_prev = lv.mfy_prev = T(0);
-    const bool any = act[0];
-    {
-      constexpr int QN = ek_qn(EK);
-      static_assert(LR_AHEAD == 3 && LR_DEPTH >= LR_AHEAD + 5, "ring_wait covers up to two rows ahead; rows t-4..t+3 kept");
-      __shared__ LdsRing<T, W, NT, QN> ring;
-      // the previous round's last reads of every slot are done before the
-      // prologue overwrites them
-      if (rd > 0) ring_wait<T, W, NT, QN>(0);
-      const LeanRows<T, W> lr = lean_rows<T, W>(a, sc, wave);
-      auto issue = [&](int t) {
-        if constexpr (EK == 0) {
-          ring_issue_lean<T, W, NT>(a, sc, st, lr, ring, wave, t);
-        } else if constexpr (EK >= 5) {  // lean rows: no row index clamps
-          ring_issue_mixed<T, W, NT, EK>(a, sc, st, lr, ring, wave, t);
-        } else {
-          // rows whose row indices do not clamp take the affine addresses
-          // for the level arrays; the q sources keep their per-lane rules
-          const int r = sc.j0 - NG + t;
-          if (r >= a.js + NG && r <= a.je)
-            ring_issue_mixed<T, W, NT, EK>(a, sc, st, lr, ring, wave, t);
-          else
-            ring_issue<T, W, NT, EK>(a, sc, st, ring, wave, t);
-        }
-      };
-      // The lean kinds (0, and 5 / 6 in the edge strips, whose blocks are H
-      // rows) run whole groups of six rows: the rows past the block read ring
-      // slots that were not reloaded (in-bounds LDS) and store nothing
-      // (x.out_row is false there), and the loop carries no per-row guard.
-      // Every wave of the workgroup steps through the same rows, so the
-      // barriers in ring_wait pair up.
-      constexpr bool PAD = EK == 0 || EK >= 5;
-      const int nrun = PAD ? (nrow + 5) / 6 * 6 : nrow;
-      for (int t = 0; t < LR_AHEAD && t < nrow; t++) issue(t);
-#define FV3_RROW(U, TW)                                                              \
-  if (PAD || t0 + U < nrow) {                                                        \
-    const int t = t0 + U;                                                            \
-    ring_wait<T, W, NT, QN>(min(LR_AHEAD - 1, nrow - 1 - t));                           \
-    if (t + LR_AHEAD < nrow) issue(t + LR_AHEAD);                                    \
-    RowIn<T, NT> in;                                                                 \
-    ring_read<T, W, NT, QN>(ring, wave, lane, t, in);                                   \
-    row_step<T, NT, U, HO, ek_side(EK), TW>(a, sc, lv, st, act, t, in);              \
+  for (int n = 0; n < NT; n++) {
+    const int iq = rd * per_round + wave * NT + n;
+    act[n] = iq < a.nq;
+    const long long qoff = (long long)(act[n] ? iq : 0) * a.npz * a.s2 + (long long)k * a.s2;
+    const long long toff = (long long)blockIdx.z * a.tq;
+    st[n].qsrc0 = in + qoff;
+    st[n].qin = in + toff + qoff;
+    st[n].qhalo = a.q_in + toff + qoff;
+    st[n].qout = out + toff + qoff;
+    st[n].qout_r = __builtin_amdgcn_make_buffer_rsrc(st[n].qout, (short)0, 0x7fffffff, 0x00020000);
+    st[n].qin_r = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(st[n].qin), (short)0, 0x7fffffff, 0x00020000);
+    st[n].fy2_prev = st[n].Fy_prev = T(0);
   }
-      if (any) {
-        // the lean kind runs the block's first six input rows (the y-pipes'
-        // warm-up) as their own unrolled group; the edge kinds would need
-        // more VGPRs with it (kinds 5 and 6: 142 against 95)
-        if constexpr (EK == 0) {
-          constexpr int t0 = 0;
-          FV3_RROW(0, 0) FV3_RROW(1, 1) FV3_RROW(2, 2) FV3_RROW(3, 3) FV3_RROW(4, 4) FV3_RROW(5, 5)
-        }
-        for (int t0 = EK == 0 ? 6 : 0; t0 < nrun; t0 += 6) {
-          FV3_RROW(0, 6) FV3_RROW(1, 6) FV3_RROW(2, 6) FV3_RROW(3, 6) FV3_RROW(4, 6) FV3_RROW(5, 6)
-        }
-      } else {  // no tracer of this wave in this round: its loads and barriers only
-        for (int t = 0; t < nrun; t++) {
-          ring_wait<T, W, NT, QN>(min(LR_AHEAD - 1, nrow - 1 - t));
-          if (t + LR_AHEAD < nrow) issue(t + LR_AHEAD);
-        }
-      }
+  LvState<T> lv;
+  lv.yfx_prev = lv.mfy_prev = T(0);
+  const bool any = act[0];
+  constexpr int QN = ek_qn(EK);
+  static_assert(LR_AHEAD == 3 && LR_DEPTH >= LR_AHEAD + 5, "ring_wait covers up to two rows ahead; rows t-4..t+3 kept");
+  __shared__ LdsRing<T, W, NT, QN> ring;
+  const LeanRows<T, W> lr = lean_rows<T, W>(a, sc, wave);
+  auto issue = [&](int t) {
+    if constexpr (EK == 0) {
+      ring_issue_lean<T, W, NT>(a, sc, st, lr, ring, wave, t);
+    } else if constexpr (EK >= 5) {  // lean rows: no row index clamps
+      ring_issue_mixed<T, W, NT, EK>(a, sc, st, lr, ring, wave, t);
+    } else {
+      // rows whose row indices do not clamp take the affine addresses
+      // for the level arrays; the q sources keep their per-lane rules
+      const int r = sc.j0 - NG + t;
+      if (r >= a.js + NG && r <= a.je)
+        ring_issue_mixed<T, W, NT, EK>(a, sc, st, lr, ring, wave, t);
+      else
+        ring_issue<T, W, NT, EK>(a, sc, st, ring, wave, t);
+    }
+  };
+  // The lean kinds (0, and 5 / 6 in the edge strips, whose blocks are H
+  // rows) run whole groups of six rows: the rows past the block read ring
+  // slots that were not reloaded (in-bounds LDS) and store nothing
+  // (x.out_row is false there), and the loop carries no per-row guard.
+  // Every wave of the workgroup steps through the same rows, so the
+  // barriers in ring_wait pair up.
+  constexpr bool PAD = EK == 0 || EK >= 5;
+  const int nrun = PAD ? (nrow + 5) / 6 * 6 : nrow;
+  for (int t = 0; t < LR_AHEAD && t < nrow; t++) issue(t);
+#define FV3_RROW(U, TW)                                                 \
+  if (PAD || t0 + U < nrow) {                                           \
+    const int t = t0 + U;                                               \
+    ring_wait<T, W, NT, QN>(min(LR_AHEAD - 1, nrow - 1 - t));           \
+    if (t + LR_AHEAD < nrow) issue(t + LR_AHEAD);                       \
+    RowIn<T, NT> in;                                                    \
+    ring_read<T, W, NT, QN>(ring, wave, lane, t, in);                   \
+    row_step<T, NT, U, HO, ek_side(EK), TW>(a, sc, lv, st, act, t, in); \
+  }
+  if (any) {
+    // the lean kind runs the block's first six input rows (the y-pipes'
+    // warm-up) as their own unrolled group; the edge kinds would need
+    // more VGPRs with it (kinds 5 and 6: 142 against 95)
+    if constexpr (EK == 0) {
+      constexpr int t0 = 0;
+      FV3_RROW(0, 0) FV3_RROW(1, 1) FV3_RROW(2, 2) FV3_RROW(3, 3) FV3_RROW(4, 4) FV3_RROW(5, 5)
+    }
+    for (int t0 = EK == 0 ? 6 : 0; t0 < nrun; t0 += 6) {
+      FV3_RROW(0, 6) FV3_RROW(1, 6) FV3_RROW(2, 6) FV3_RROW(3, 6) FV3_RROW(4, 6) FV3_RROW(5, 6)
+    }
+  } else {  // no tracer of this wave in this round: its loads and barriers only
+    for (int t = 0; t < nrun; t++) {
+      ring_wait<T, W, NT, QN>(min(LR_AHEAD - 1, nrow - 1 - t));
+      if (t + LR_AHEAD < nrow) issue(t + LR_AHEAD);
+    }
+  }
 #undef FV3_RROW
-    }
-  }
 }
 
 }  // namespace fv3

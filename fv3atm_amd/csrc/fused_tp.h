@@ -24,6 +24,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <type_traits>
 
 #include "fv3_device.h"
@@ -82,6 +83,58 @@ inline void fused_grid_split(const FusedArgs<T> &a, int (&n)[7]) {
   n[4] = nr * 2;  // right of them: top and bottom blocks
   n[5] = nl * a.nmid;  // left strips, lean rows
   n[6] = nr * a.nmid;  // right strips, lean rows
+}
+
+// Workgroups along x of a kind with n blocks: one for each round of per_round
+// tracers.  (A workgroup that ran its block's rounds one after another left
+// long chains at the end of a pass: C768 L127 30 tracers 31.2 against 29.6 ms
+// a step, a C203 L75 11-tracer tile 1.67 against 1.12 ms.)
+template <typename T>
+inline unsigned fused_grid_x(const FusedArgs<T> &a, int n, int per_round) {
+  return (unsigned)n * (unsigned)((a.nq + per_round - 1) / per_round);
+}
+
+// Rows per block when the caller sets none: `rows` rows in b blocks of H (a
+// multiple of 6, the row loop's unrolling), b minimising the modelled time of a
+// pass, (H + warm) rows -- warm: what a block's first rows cost beyond its own --
+// times the turns that `units` workgroups per block take on `slots` resident
+// ones (a fraction of a last turn costs a whole one when there are few).  At
+// most 60 rows (C768: 36 20.0, 48 19.5, 60 19.3 ms of transport; longer blocks
+// leave fewer to balance) and at least 12 (C48 L32, one tracer: 48 rows 132 us
+// of transport, 24 97, 12 81, 9 86, 6 93).  A C192 face's 181 lean rows go as
+// 4 x 48 rather than 3 x 60 + 1 (5.26 against 5.65 ms a step).
+inline int fused_block_rows(int rows, long long units, int slots, double warm) {
+  int best = 12;
+  double t_best = 1e300;
+  for (int b = 1; b <= rows; b++) {
+    const int h = ((rows + b - 1) / b + 5) / 6 * 6;
+    if (h > 60) continue;
+    if (h < 12) break;
+    const double x = (double)units * ((rows + h - 1) / h) / slots;
+    const double t = (h + warm) * (x < 4.0 ? ceil(x) : x + 1.0);
+    if (t < t_best) {
+      t_best = t;
+      best = h;
+    }
+  }
+  return best;
+}
+
+// Block and round of workgroup x (nb blocks): eight blocks at a time, rounds
+// outermost among them, so that the rounds of a block have numbers equal
+// modulo 8 and run on one XCD, close together (they read the same level rows
+// through its L2).
+__host__ __device__ __forceinline__ void fused_block_round(int x, int nb, int rounds, int &b, int &r) {
+  const int full = nb & ~7, per = 8 * rounds;
+  if (x < full * rounds) {
+    const int in = x % per;
+    b = x / per * 8 + (in & 7);
+    r = in >> 3;
+  } else {
+    const int in = x - full * rounds, m = nb - full;
+    b = full + in % m;
+    r = in / m;
+  }
 }
 
 // ---- cross-lane shifts: value of lane l-1 / l+1 (DPP wave_shr:1 / wave_shl:1)

@@ -168,7 +168,7 @@ int fv3_ctx_set_timing(fv3_ctx *ctx, int on);
  * the fused transport launch shape, waves per workgroup x tracers per wave
  * (0..14; the default is 12: 8 waves x 2 tracers for the interior kernel, 4 x 1
  * at three workgroups per CU for the edge kernels); rows the interior rows per
- * block (0 = 60);
+ * block (0 = chosen by the tile's size, at most 60);
  * remap the vertical remap kernel: 0 (default) = column-shared, a column's
  * levels spread over 16 or 32 lanes of a wave (npz <= 127; larger npz take
  * kernel 2), 1 = one thread per column, 2 = column-shared, one thread per
