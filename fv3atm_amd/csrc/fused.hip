@@ -125,14 +125,14 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   // buffer), and the remap writes q_out.
   T *q_tmp = nullptr, *pt_src = nullptr;
   char *tab = nullptr;  // the column tables
-  std::vector<RemapCols> cols(nt);  // column data of every tile
+  RemapCols cols{};  // column data of the first tile
   if (fast_remap) {
     if (remap_fast_check(npz, (long long)ni * nj, d.s2, kord_tr, kord_tm, pt != nullptr)) return 1;
     char *sc = ext ? arena.base + head : (char *)ctx_scratch(c, b_q + b_pt + b_col * nt);
     if (!sc) return 1;
     q_tmp = (T *)sc;
     pt_src = pt ? (T *)(sc + b_q) : nullptr;
-    for (int t = 0; t < nt; t++) cols[t] = remap_cols_carve(sc + b_q + b_pt + b_col * t, npz, (long long)ni * nj);
+    cols = remap_cols_carve(sc + b_q + b_pt, npz, (long long)ni * nj);
   } else if (sc64) {
     q_tmp = q_tmp64;
     pt_src = pt ? (T *)(sc64 + b_q) : nullptr;
@@ -220,11 +220,7 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   auto remap_prep = [&]() -> int {
     FV3_HIP(hipMemcpyAsync(delp_out, dp1, sizeof(double) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, sp));
     if (pt) FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(T) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, sp));
-    for (int t = 0; t < nt; t++)
-      if (remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1 + t * d.s2 * npz, delp_out + t * d.s2 * npz,
-                              cols[t], sp))
-        return 1;
-    return 0;
+    return remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1, delp_out, cols, b_col, sp);
   };
   if (early) {
     FV3_HIP(hipEventRecord(c.fork_ev, s));
@@ -254,7 +250,7 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   const int nfork = !conc ? 0 : (pipe ? 2 : 3);
   const T *const pass_in = a.q_in;
   T *const pass_out = a.q_out, *const pass_tmp = a.q_tmp;
-  const long long tq = a.tq, tl = d.s2 * npz;
+  const long long tq = a.tq;
   for (int q0 = 0; q0 < nq; q0 += cq) {
     const int nqc = std::min(cq, nq - q0);
     const long long qoff = (long long)q0 * npz * d.s2;
@@ -284,11 +280,9 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
         FV3_HIP(hipEventRecord(c.chunk_ev, s));
         FV3_HIP(hipStreamWaitEvent(sp, c.chunk_ev, 0));
         const bool last = q0 + nqc >= nq;
-        for (int t = 0; t < nt; t++)
-          if (remap_fast_fields_f32(c, npz, nqc, q_tmp + t * tq + qoff, q_out + t * tq + qoff,
-                                    last && pt_src ? pt_src + t * tl : nullptr, last && pt ? pt + t * tl : nullptr,
-                                    kord_tr, kord_tm, t_min, cols[t], sp))
-            return 1;
+        if (remap_fast_fields_f32(c, npz, nqc, q_tmp + qoff, q_out + qoff, last ? pt_src : nullptr,
+                                  last ? pt : nullptr, kord_tr, kord_tm, t_min, cols, b_col, tq, sp))
+          return 1;
       }
     }
   }
@@ -315,11 +309,8 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   if (timing && !pipe) FV3_HIP(hipEventRecord(c.ev[2], s));
   if constexpr (std::is_same<T, float>::value) {
     if (fast_remap && !pipe) {
-      for (int t = 0; t < nt; t++) {
-        if (remap_fast_fields_f32(c, npz, nq, q_tmp + t * tq, q_out + t * tq, pt_src ? pt_src + t * tl : nullptr,
-                                  pt ? pt + t * tl : nullptr, kord_tr, kord_tm, t_min, cols[t], s))
-          return 1;
-      }
+      if (remap_fast_fields_f32(c, npz, nq, q_tmp, q_out, pt_src, pt, kord_tr, kord_tm, t_min, cols, b_col, tq, s))
+        return 1;
     }
   }
   if (fields) {
@@ -375,14 +366,9 @@ int remap_only_f32(Ctx &c, int nq, const float *q_src, float *q_dst, float *pt, 
   const long long tq = d.s2 * npz * nq, tl = d.s2 * npz;
   FV3_HIP(hipMemcpyAsync(delp_out, dp1, sizeof(double) * tl * nt, hipMemcpyDeviceToDevice, s));
   if (pt) FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(float) * tl * nt, hipMemcpyDeviceToDevice, s));
-  for (int t = 0; t < nt; t++) {
-    const RemapCols cols = remap_cols_carve(sc + b_pt + b_col * t, npz, (long long)ni * nj);
-    if (remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1 + t * tl, delp_out + t * tl, cols, s)) return 1;
-    if (remap_fast_fields_f32(c, npz, nq, q_src + t * tq, q_dst + t * tq, pt_src ? pt_src + t * tl : nullptr,
-                              pt ? pt + t * tl : nullptr, kord_tr, kord_tm, t_min, cols, s))
-      return 1;
-  }
-  return 0;
+  const RemapCols cols = remap_cols_carve(sc + b_pt, npz, (long long)ni * nj);
+  if (remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1, delp_out, cols, b_col, s)) return 1;
+  return remap_fast_fields_f32(c, npz, nq, q_src, q_dst, pt_src, pt, kord_tr, kord_tm, t_min, cols, b_col, tq, s);
 }
 
 int fused_step(Ctx &c, bool fp32, int nq, const void *q_in, void *q_out, void *pt,

@@ -23,10 +23,12 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "fv3_internal.h"
 #include "mapz_column.h"
 #include "mapz_fast.h"
+#include "mapz_prep.h"
 
 namespace fv3 {
 
@@ -42,89 +44,130 @@ struct PrepArgs {
   double ptop;
   const double *dp1, *ak, *bk;
   double *delp_out;
-  RemapCols cols;
+  RemapCols cols;      // of the first tile
+  long long tdp, tcol; // tile strides: levels (elements), column data (bytes)
 };
 
-// One thread per interior column.
-__global__ void __launch_bounds__(256) k_remap_prep(const PrepArgs a) {
-  const long long col = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (col >= a.ncol) return;
-  const int ii = (int)(col % a.ni), jj = (int)(col / a.ni);
+__device__ __forceinline__ RemapCols tile_cols(RemapCols c, long long bytes) {
+  auto mv = [&](auto *&p) { p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(reinterpret_cast<char *>(p) + bytes); };
+  mv(c.d4); mv(c.rbt); mv(c.gg); mv(c.dp1); mv(c.bot); mv(c.lk); mv(c.cut);
+  return c;
+}
+
+// One workgroup per 64 interior columns of a tile (blockIdx.y): interfaces in
+// LDS, wave 0 the elimination's chain, the other waves the target layers,
+// each on its own (mapz_prep.h).  A column whose interfaces are out of order
+// takes its target layers in sequence on one lane.  One thread per column with
+// a load in each step of both chains took 330 us a C192 L127 tile beside the
+// transport, one launch per tile; six tiles in one launch take 1.2 ms there.
+__global__ void __launch_bounds__(64 * PREP_WAVES) k_remap_prep(const PrepArgs a) {
+  extern __shared__ double pe1_lds[];  // [km + 1][columns]
+  __shared__ int bad[64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long long tile = blockIdx.y;
+  const int pc = prep_cols(a.km);
+  const long long c0 = (long long)blockIdx.x * pc + (lane & (pc - 1));
+  const bool act = lane < pc && c0 < a.ncol;
+  const long long col = min(c0, a.ncol - 1);  // lanes past the last column repeat it and store nothing
+  const int ii = (int)((unsigned)col % (unsigned)a.ni), jj = (int)((unsigned)col / (unsigned)a.ni);
   const long long cell = (long long)(jj + a.js - a.jsd) * a.nid + (ii + a.is - a.isd);
-  const double *dl = a.dp1 + cell;
   const long long s2 = a.s2, nc = a.ncol;
   const int km = a.km;
-  const RemapCols &o = a.cols;
+  const RemapCols o = tile_cols(a.cols, tile * a.tcol);
+  const ColPe P{pe1_lds + (lane & (pc - 1)), pc};
+  if (wave == 0) bad[lane] = 0;
   // Lagrangian interfaces by running sums from ptop, thicknesses as their
   // differences (the Lagrangian_to_Eulerian pe1 / dp1 of the upstream)
-  double p_k = a.ptop;             // PE1(1)
-  double p_k1 = p_k + dl[0];       // PE1(2)
-  double d_prev = p_k1 - p_k;      // D1(1)
-  const double p_k2 = p_k1 + dl[s2];
-  const double grat = (p_k2 - p_k1) / d_prev;
-  const double bet = grat * (grat + 0.5);
-  double g = (1.0 + grat * (grat + 1.5)) / bet;
-  o.d4[col] = (float)((grat + grat) * (grat + 1.0));
-  o.rbt[col] = (float)(1.0 / bet);
-  o.gg[col] = (float)g;
-  o.dp1[col] = (float)d_prev;
-  double d4 = 0.0;
-  p_k = p_k1;
-  for (int k = 2; k <= km; k++) {
-    const double p_n = p_k + dl[(long long)(k - 1) * s2];
-    const double dk = p_n - p_k;
-    d4 = d_prev / dk;
-    const double bt = 2.0 + d4 + d4 - g;
-    g = d4 / bt;
-    const long long o_k = (long long)(k - 1) * nc + col;
-    o.d4[o_k] = (float)d4;
-    o.rbt[o_k] = (float)(1.0 / bt);
-    o.gg[o_k] = (float)g;
-    o.dp1[o_k] = (float)dk;
-    d_prev = dk;
-    p_k = p_n;
-  }
-  const double ps = p_k;  // PE1(km+1)
-  const double a_bot = 1.0 + d4 * (d4 + 1.5);
-  o.bot[col] = (float)(2.0 * d4 * (d4 + 1.0));
-  o.bot[nc + col] = (float)a_bot;
-  o.bot[2 * nc + col] = (float)(1.0 / (d4 * (d4 + 0.5) - a_bot * g));
-
-  // Eulerian interfaces, target thickness, and the containing source layer
-  // of every target interface (the first layer l with pe2 <= PE1(l+1), the
-  // choice the upstream search makes when an interface falls on a source
-  // interface)
+  stage_interfaces(P, km, a.ptop, a.dp1 + tile * a.tdp + cell, s2, wave);
+  __syncthreads();
+  const double ps = P(km + 1);
   auto pe2_of = [&](int k) -> double {
     if (k == 1) return a.ptop;
     if (k == km + 1) return ps;
     return a.ak[k - 1] + a.bk[k - 1] * ps;
   };
-  int l = 1;
-  double lo = a.ptop, hi = a.ptop + dl[0];  // PE1(l), PE1(l+1)
-  double pe2_k = a.ptop;
-  float s_prev = 0.f, wtop_prev = 0.f, rdp2_prev = 0.f;
-  int l_prev = 1;
-  for (int k = 1; k <= km + 1; k++) {
-    const double p = pe2_k;
-    while (l < km && p > hi) {
-      l++;
-      lo = hi;
-      hi = lo + dl[(long long)(l - 1) * s2];
+  {
+    bool b = false;
+    for (int k = 1 + wave; k <= km; k += PREP_WAVES) b = b || !(P(k + 1) > P(k)) || !(pe2_of(k + 1) >= pe2_of(k));
+    if (b) bad[lane] = 1;
+  }
+  __syncthreads();
+  if (wave == 0) {
+    double d_prev = P(2) - P(1);
+    const double grat = (P(3) - P(2)) / d_prev;
+    const double bet = grat * (grat + 0.5);
+    double g = (1.0 + grat * (grat + 1.5)) / bet;
+    if (act) {
+      o.d4[col] = (float)((grat + grat) * (grat + 1.0));
+      o.rbt[col] = (float)(1.0 / bet);
+      o.gg[col] = (float)g;
+      o.dp1[col] = (float)d_prev;
     }
-    if (k >= 2) {  // close target k-1: its bottom piece lies in layer l
-      const long long o_t = (long long)(k - 2) * nc + col;
-      o.cut[o_t] = make_float4(s_prev, wtop_prev, (float)(p - lo), rdp2_prev);
-      o.lk[o_t] = l_prev;
+    double d4 = 0.0;
+    for (int k4 = 2; k4 <= km; k4 += 4) {
+      double dk[4], rat[4];
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        const int k = min(k4 + m, km);
+        dk[m] = P(k + 1) - P(k);
+        rat[m] = (m == 0 ? d_prev : dk[m - 1]) / dk[m];
+      }
+#pragma unroll
+      for (int m = 0; m < 4; m++) {
+        const int k = k4 + m;
+        if (k > km) break;
+        d4 = rat[m];
+        const double bt = 2.0 + d4 + d4 - g;
+        g = d4 / bt;
+        if (act) {
+          const long long o_k = (long long)(k - 1) * nc + col;
+          o.d4[o_k] = (float)d4;
+          o.rbt[o_k] = (float)(1.0 / bt);
+          o.gg[o_k] = (float)g;
+          o.dp1[o_k] = (float)dk[m];
+        }
+      }
+      d_prev = dk[3];
     }
-    if (k <= km) {
-      const double p_next = pe2_of(k + 1);
-      const double dp2 = p_next - p;
-      a.delp_out[(long long)(k - 1) * s2 + cell] = dp2;
-      s_prev = (float)((p - lo) / (hi - lo));
-      wtop_prev = (float)(hi - p);
-      rdp2_prev = (float)(1.0 / dp2);
-      l_prev = l;
-      pe2_k = p_next;
+    if (act) {
+      const double a_bot = 1.0 + d4 * (d4 + 1.5);
+      o.bot[col] = (float)(2.0 * d4 * (d4 + 1.0));
+      o.bot[nc + col] = (float)a_bot;
+      o.bot[2 * nc + col] = (float)(1.0 / (d4 * (d4 + 0.5) - a_bot * g));
+    }
+    return;
+  }
+  // Eulerian interfaces, target thickness, and the containing source layer
+  // of every target interface (the first layer l with pe2 <= PE1(l+1), the
+  // choice the upstream search makes when an interface falls on a source
+  // interface)
+  double *dout = a.delp_out + tile * a.tdp + cell;
+  auto put = [&](int k, double p, double p_next, int l, int lb) {
+    const double dp2 = p_next - p, lo = P(l), hi = P(l + 1);
+    if (!act) return;
+    const long long o_t = (long long)(k - 1) * nc + col;
+    o.cut[o_t] = make_float4((float)((p - lo) / (hi - lo)), (float)(hi - p), (float)(p_next - P(lb)), (float)(1.0 / dp2));
+    o.lk[o_t] = l;
+    dout[(long long)(k - 1) * s2] = dp2;
+  };
+  if (!bad[lane]) {
+    for (int k = wave; k <= km; k += PREP_WAVES - 1) {
+      const double pa = pe2_of(k), pb = pe2_of(k + 1);
+      put(k, pa, pb, P.layer_of(pa, k, km), P.layer_of(pb, k, km));
+    }
+  } else if (wave == 1) {
+    int l = 1;
+    double pa = a.ptop;
+    auto walk = [&](double p) {
+      while (l < km && p > P(l + 1)) l++;
+    };
+    walk(pa);
+    for (int k = 1; k <= km; k++) {
+      const double pb = pe2_of(k + 1);
+      const int lt = l;
+      walk(pb);
+      put(k, pa, pb, lt, l);
+      pa = pb;
     }
   }
 }
@@ -518,9 +561,10 @@ struct RowsArgs {
   unsigned nwg;
   long long ncol, s2;
   float t_min;
-  const float *q_src, *pt_src;
+  const float *q_src, *pt_src;  // of the first tile
   float *q_dst, *pt_dst;
   RemapCols cols;
+  long long tq, tpt, tcol;  // tile strides: tracers, one field (elements), column data (bytes)
 };
 
 // Cross-lane moves.  Each result is pinned by an empty volatile asm where it
@@ -642,7 +686,11 @@ __global__ void __launch_bounds__(64 * RW_WAVES, 4) k_remap_rows(const RowsArgs 
   float *const s_tiles = reinterpret_cast<float *>(rw_lds + WGC * RC::row);
   auto tile_in = [&](int f) { return s_tiles + (f & 1) * 2 * WGC * ST::row; };
   auto tile_out = [&](int f) { return s_tiles + ((f & 1) * 2 + 1) * WGC * ST::row; };
-  auto field_dst = [&](int f) { return f >= a.nq ? a.pt_dst : a.q_dst + (long long)f * a.km * a.s2; };
+  const long long tile = blockIdx.y;
+  const float *const q_src = a.q_src + tile * a.tq, *const pt_src = a.pt_src + tile * a.tpt;
+  float *const q_dst = a.q_dst + tile * a.tq, *const pt_dst = a.pt_dst + tile * a.tpt;
+  const RemapCols cols = tile_cols(a.cols, tile * a.tcol);
+  auto field_dst = [&](int f) { return f >= a.nq ? pt_dst : q_dst + (long long)f * a.km * a.s2; };
   const int tid = threadIdx.x, lane = tid & 63, cw = lane / L;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // blocks are dealt round-robin to the 8 XCDs: renumber so that neighbouring
@@ -687,9 +735,9 @@ __global__ void __launch_bounds__(64 * RW_WAVES, 4) k_remap_rows(const RowsArgs 
   float d4[M], rbt[M], gg[M], dp1[M], st[M], wt[M], wb[M], rd[M];
   int ltc[M];
   {
-    const Rsrc r_d4 = make_rsrc(a.cols.d4, cbytes), r_rbt = make_rsrc(a.cols.rbt, cbytes);
-    const Rsrc r_gg = make_rsrc(a.cols.gg, cbytes), r_dp1 = make_rsrc(a.cols.dp1, cbytes);
-    const Rsrc r_lk = make_rsrc(a.cols.lk, cbytes), r_cut = make_rsrc(a.cols.cut, 4u * cbytes);
+    const Rsrc r_d4 = make_rsrc(cols.d4, cbytes), r_rbt = make_rsrc(cols.rbt, cbytes);
+    const Rsrc r_gg = make_rsrc(cols.gg, cbytes), r_dp1 = make_rsrc(cols.dp1, cbytes);
+    const Rsrc r_lk = make_rsrc(cols.lk, cbytes), r_cut = make_rsrc(cols.cut, 4u * cbytes);
     const unsigned vc = (unsigned)k0c * lvl + (unsigned)col * 4u;
 #pragma unroll
     for (int i = 0; i < M; i++) {
@@ -710,7 +758,7 @@ __global__ void __launch_bounds__(64 * RW_WAVES, 4) k_remap_rows(const RowsArgs 
       }
     }
   }
-  const float bot0 = a.cols.bot[col], bot1 = a.cols.bot[nc + col], bot2 = a.cols.bot[2 * nc + col];
+  const float bot0 = cols.bot[col], bot1 = cols.bot[nc + col], bot2 = cols.bot[2 * nc + col];
   // the source layer and fraction of the bottom interface of the lane's last
   // target (the last lane's last target is padding: km+1 <= L M)
   // (the moves run for every lane before the selection: the last lane's value
@@ -744,7 +792,7 @@ __global__ void __launch_bounds__(64 * RW_WAVES, 4) k_remap_rows(const RowsArgs 
 
   float qn[M];  // the thread's staged elements of the next field
   {
-    const Rsrc r0 = make_rsrc(a.nq > 0 ? a.q_src : a.pt_src, fbytes);
+    const Rsrc r0 = make_rsrc(a.nq > 0 ? q_src : pt_src, fbytes);
 #pragma unroll
     for (int j = 0; j < M; j++) qn[j] = ldf(r0, vtc + (unsigned)j * kstep, 0);
   }
@@ -772,7 +820,7 @@ __global__ void __launch_bounds__(64 * RW_WAVES, 4) k_remap_rows(const RowsArgs 
     }
     if (f + 1 < a.nf) {  // next field's elements, in flight while this one is computed
       const int fn = f + 1;
-      const float *src = fn >= a.nq ? a.pt_src : a.q_src + (long long)fn * km * a.s2;
+      const float *src = fn >= a.nq ? pt_src : q_src + (long long)fn * km * a.s2;
 #pragma unroll
       for (int j = 0; j < M; j++) qn[j] = ldf(make_rsrc(src, fbytes), vtc + (unsigned)j * kstep, 0);
     }
@@ -987,6 +1035,7 @@ RemapCols remap_cols_carve(void *base, int km, long long ncol) {
 // the field kernel addresses a tile's column data (d4 .. lk, and cut) and one
 // field's levels with 32-bit byte offsets
 static int check_sizes(int km, long long ncol, long long s2) {
+  if (km > PREP_MAX_KM) return set_error("fast remap supports km <= %d (got %d)", PREP_MAX_KM, km);
   auto al = [](long long b) { return (b + 255) & ~255LL; };
   const long long span = 4 * al(4LL * km * ncol) + al(12LL * ncol) + 4LL * km * ncol;
   if (span >= (1LL << 31) || 16LL * km * ncol >= (1LL << 31) || 4LL * km * s2 >= (1LL << 31))
@@ -1012,7 +1061,7 @@ static int check_orders(int km, int kord_tr, int kord_tm, bool with_pt) {
 }
 
 int remap_fast_prep_f32(Ctx &c, int km, const double *ak, const double *bk, double ptop,
-                        const double *dp1, double *delp_out, const RemapCols &cols, hipStream_t s) {
+                        const double *dp1, double *delp_out, const RemapCols &cols, size_t cols_stride, hipStream_t s) {
   const Dims &d = c.d;
   if (km < 8) return set_error("fast remap needs km >= 8 (got %d)", km);
   const int ni = d.ie - d.is + 1, nj = d.je - d.js + 1;
@@ -1020,8 +1069,10 @@ int remap_fast_prep_f32(Ctx &c, int km, const double *ak, const double *bk, doub
   PrepArgs pa{};
   pa.km = km; pa.ni = ni; pa.is = d.is; pa.js = d.js; pa.isd = d.isd; pa.jsd = d.jsd; pa.nid = d.nid;
   pa.ncol = ncol; pa.s2 = d.s2; pa.ptop = ptop; pa.dp1 = dp1; pa.ak = ak; pa.bk = bk;
-  pa.delp_out = delp_out; pa.cols = cols;
-  hipLaunchKernelGGL(k_remap_prep, dim3((unsigned)((ncol + 255) / 256)), dim3(256), 0, s, pa);
+  pa.delp_out = delp_out; pa.cols = cols; pa.tdp = d.s2 * km; pa.tcol = (long long)cols_stride;
+  if (remap_rows_setup()) return 1;
+  hipLaunchKernelGGL(k_remap_prep, dim3((unsigned)((ncol + prep_cols(km) - 1) / prep_cols(km)), (unsigned)c.ntiles),
+                     dim3(64 * PREP_WAVES), prep_lds(km), s, pa);
   FV3_HIP(hipGetLastError());
   return 0;
 }
@@ -1038,42 +1089,30 @@ int remap_rows_setup() {
     const size_t lds[3] = {rows_lds_bytes<2, 16>(), rows_lds_bytes<4, 16>(), rows_lds_bytes<4, 32>()};
     for (int v = 0; v < 3 && err == hipSuccess; v++)
       err = hipFuncSetAttribute(fn[v], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds[v]);
+    if (err == hipSuccess)
+      err = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_remap_prep),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)prep_lds(PREP_MAX_KM));
   });
   FV3_HIP(err);
   return 0;
 }
 
 int remap_fast_fields_f32(Ctx &c, int km, int nq, const float *q_src, float *q_dst, const float *pt_src,
-                          float *pt_dst, int kord_tr, int kord_tm, double t_min, const RemapCols &cols,
-                          hipStream_t s) {
+                          float *pt_dst, int kord_tr, int kord_tm, double t_min, const RemapCols &cols0,
+                          size_t cols_stride, long long tq, hipStream_t s) {
   const Dims &d = c.d;
   if (check_orders(km, kord_tr, kord_tm, pt_src != nullptr)) return 1;
   const int ni = d.ie - d.is + 1, nj = d.je - d.js + 1;
   const long long ncol = (long long)ni * nj;
-  FieldArgs fa{};
-  fa.km = km; fa.nb = (km + RF_B - 1) / RF_B; fa.ni = ni; fa.is = d.is; fa.js = d.js;
-  fa.isd = d.isd; fa.jsd = d.jsd; fa.nid = d.nid; fa.nq = nq; fa.nf = nq + (pt_src ? 1 : 0);
-  fa.nfg = (fa.nf + RF_WAVES - 1) / RF_WAVES; fa.kord_tr = kord_tr; fa.kord_tm = kord_tm;
-  fa.ncol = ncol; fa.s2 = d.s2; fa.t_min = (float)t_min;
-  fa.q_src = q_src; fa.pt_src = pt_src; fa.q_dst = q_dst; fa.pt_dst = pt_dst; fa.cols = cols;
-  {
-    if (check_sizes(km, ncol, d.s2)) return 1;
-    const char *b = (const char *)cols.d4;
-    const long long cut = (long long)sizeof(float4) * km * ncol, span = (const char *)cols.lk - b + 4LL * km * ncol;
-    fa.o_rbt = (unsigned)((const char *)cols.rbt - b);
-    fa.o_gg = (unsigned)((const char *)cols.gg - b);
-    fa.o_dp1 = (unsigned)((const char *)cols.dp1 - b);
-    fa.o_bot = (unsigned)((const char *)cols.bot - b);
-    fa.o_lk = (unsigned)((const char *)cols.lk - b);
-    fa.b_cols = (unsigned)span;
-    fa.b_cut = (unsigned)cut;
-  }
+  const int nf = nq + (pt_src ? 1 : 0);
+  if (check_sizes(km, ncol, d.s2)) return 1;
   if (c.remap_mode == 0 && km + 1 <= 128 && rows_fits(km, ncol, d.s2)) {
     RowsArgs ra{};
     ra.km = km; ra.ni = ni; ra.is = d.is; ra.js = d.js; ra.isd = d.isd; ra.jsd = d.jsd; ra.nid = d.nid;
-    ra.nq = nq; ra.nf = fa.nf; ra.kord_tr = kord_tr; ra.kord_tm = kord_tm;
+    ra.nq = nq; ra.nf = nf; ra.kord_tr = kord_tr; ra.kord_tm = kord_tm;
     ra.ncol = ncol; ra.s2 = d.s2; ra.t_min = (float)t_min;
-    ra.q_src = q_src; ra.pt_src = pt_src; ra.q_dst = q_dst; ra.pt_dst = pt_dst; ra.cols = cols;
+    ra.q_src = q_src; ra.pt_src = pt_src; ra.q_dst = q_dst; ra.pt_dst = pt_dst; ra.cols = cols0;
+    ra.tq = tq; ra.tpt = d.s2 * km; ra.tcol = (long long)cols_stride;
     // levels per lane x lanes per column: 2 x 16, 4 x 16 or 4 x 32
     const int M = km + 1 <= 32 ? 2 : 4, L = km + 1 <= 64 ? 16 : 32;
     const long long per_wg = (long long)RW_WAVES * (64 / L);
@@ -1083,22 +1122,43 @@ int remap_fast_fields_f32(Ctx &c, int km, int nq, const float *q_src, float *q_d
     const size_t lds = M == 2 ? rows_lds_bytes<2, 16>() : L == 16 ? rows_lds_bytes<4, 16>() : rows_lds_bytes<4, 32>();
     if (remap_rows_setup()) return 1;
     if (M == 2)
-      hipLaunchKernelGGL((k_remap_rows<2, 16>), dim3((unsigned)nwg), dim3(64 * RW_WAVES), lds, s, ra);
+      hipLaunchKernelGGL((k_remap_rows<2, 16>), dim3((unsigned)nwg, (unsigned)c.ntiles), dim3(64 * RW_WAVES), lds, s, ra);
     else if (L == 16)
-      hipLaunchKernelGGL((k_remap_rows<4, 16>), dim3((unsigned)nwg), dim3(64 * RW_WAVES), lds, s, ra);
+      hipLaunchKernelGGL((k_remap_rows<4, 16>), dim3((unsigned)nwg, (unsigned)c.ntiles), dim3(64 * RW_WAVES), lds, s, ra);
     else
-      hipLaunchKernelGGL((k_remap_rows<4, 32>), dim3((unsigned)nwg), dim3(64 * RW_WAVES), lds, s, ra);
+      hipLaunchKernelGGL((k_remap_rows<4, 32>), dim3((unsigned)nwg, (unsigned)c.ntiles), dim3(64 * RW_WAVES), lds, s, ra);
     FV3_HIP(hipGetLastError());
     return 0;
   }
-  const long long ncb = (ncol + RF_COLS - 1) / RF_COLS;
-  const long long nwg = ncb * fa.nfg;
-  if (nwg > 0x7fffffffLL) return set_error("remap grid too large");
-  fa.nwg = (unsigned)nwg;
-  const size_t lds = sizeof(float) * fa.nb * RF_COLS * RF_WAVES;
-  if (lds > 64 * 1024) return set_error("fast remap supports km <= %d (got %d)", 64 * RF_B - 1, km);
-  hipLaunchKernelGGL((k_remap_fields<RF_B>), dim3((unsigned)nwg), dim3(RF_COLS * RF_WAVES), lds, s, fa);
-  FV3_HIP(hipGetLastError());
+  const long long tl = d.s2 * km;
+  for (int t = 0; t < c.ntiles; t++) {
+    const RemapCols cols = remap_cols_carve((char *)cols0.d4 + t * cols_stride, km, ncol);
+    FieldArgs fa{};
+    fa.km = km; fa.nb = (km + RF_B - 1) / RF_B; fa.ni = ni; fa.is = d.is; fa.js = d.js;
+    fa.isd = d.isd; fa.jsd = d.jsd; fa.nid = d.nid; fa.nq = nq; fa.nf = nq + (pt_src ? 1 : 0);
+    fa.nfg = (fa.nf + RF_WAVES - 1) / RF_WAVES; fa.kord_tr = kord_tr; fa.kord_tm = kord_tm;
+    fa.ncol = ncol; fa.s2 = d.s2; fa.t_min = (float)t_min;
+    fa.q_src = q_src + t * tq; fa.pt_src = pt_src ? pt_src + t * tl : nullptr;
+    fa.q_dst = q_dst + t * tq; fa.pt_dst = pt_dst ? pt_dst + t * tl : nullptr; fa.cols = cols;
+    {
+      const char *b = (const char *)cols.d4;
+      const long long cut = (long long)sizeof(float4) * km * ncol, span = (const char *)cols.lk - b + 4LL * km * ncol;
+      fa.o_rbt = (unsigned)((const char *)cols.rbt - b);
+      fa.o_gg = (unsigned)((const char *)cols.gg - b);
+      fa.o_dp1 = (unsigned)((const char *)cols.dp1 - b);
+      fa.o_bot = (unsigned)((const char *)cols.bot - b);
+      fa.o_lk = (unsigned)((const char *)cols.lk - b);
+      fa.b_cols = (unsigned)span;
+      fa.b_cut = (unsigned)cut;
+    }
+    const long long ncb = (ncol + RF_COLS - 1) / RF_COLS;
+    const long long nwg = ncb * fa.nfg;
+    if (nwg > 0x7fffffffLL) return set_error("remap grid too large");
+    fa.nwg = (unsigned)nwg;
+    const size_t lds = sizeof(float) * fa.nb * RF_COLS * RF_WAVES;
+      hipLaunchKernelGGL((k_remap_fields<RF_B>), dim3((unsigned)nwg), dim3(RF_COLS * RF_WAVES), lds, s, fa);
+    FV3_HIP(hipGetLastError());
+  }
   return 0;
 }
 
