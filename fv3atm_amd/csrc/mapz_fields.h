@@ -58,6 +58,8 @@ ColTab<R> coltab_carve(void *base, int km, long long ncols);
 
 // Largest km the kernels take (the column's interfaces are staged in LDS).
 constexpr int FIELDS_MAX_KM = 255;
+// ... and for (value, tangent) pairs, whose block ends are twice as large
+constexpr int FIELDS_MAX_KM_TL = 160;
 
 // What the tables are made from: cell columns of delp (kind 0: pe1 = ptop +
 // running sum, pe2 = ak + bk ps; delp_out, when given, receives the target

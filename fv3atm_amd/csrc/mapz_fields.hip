@@ -235,7 +235,7 @@ struct TargetRec {
 // -> 4.9 ms plus 0.76 ms of tables, C96 L64 4 tracers + pt 1.79 -> 0.19 + 0.06
 // ms; the FP32 full remap of C192 L127 (13 fields) 12.4 -> 1.9 + 1.0 ms.
 template <typename T>
-__global__ void __launch_bounds__(64 * FD_WAVES, 2) k_fields(const FieldsArgs<T> a) {
+__global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields(const FieldsArgs<T> a) {
   using R = typename RealOf<T>::type;
   extern __shared__ __align__(16) char fd_lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -608,6 +608,7 @@ int fields_setup() {
     allow(reinterpret_cast<const void *>(&k_fields_prep<double>), prep_lds(FIELDS_MAX_KM));
     allow(reinterpret_cast<const void *>(&k_fields<float>), fields_lds<float>(FIELDS_MAX_KM));
     allow(reinterpret_cast<const void *>(&k_fields<double>), fields_lds<double>(FIELDS_MAX_KM));
+    allow(reinterpret_cast<const void *>(&k_fields<D1>), std::min<size_t>(fields_lds<D1>(FIELDS_MAX_KM), 160 * 1024));
   });
   FV3_HIP(err);
   return 0;
@@ -643,6 +644,7 @@ int fields_run(Ctx &c, FieldsArgs<T> &a, int ni, int nj) {
   a.nf = 0;
   for (int s = 0; s < a.nset; s++) a.nf += a.set[s].count;
   if (a.nf == 0) return 0;
+  if (fields_lds<T>(a.km) > 160 * 1024) return set_error("remap of %d levels does not fit in LDS", a.km);
   a.nfg = (a.nf + FD_WAVES - 1) / FD_WAVES;
   const long long nwg = (long long)a.ncb * c.ntiles * a.nfg;
   if (nwg > 0x7fffffffLL) return set_error("remap grid too large");
@@ -686,6 +688,7 @@ FieldSet<T> tracer_set(const Ctx &c, const T *src, T *dst, int nq) {
   template FieldSet<T> tracer_set<T>(const Ctx &, const T *, T *, int);
 FV3_FIELDS(double)
 FV3_FIELDS(float)
+template int fields_run<D1>(Ctx &, FieldsArgs<D1> &, int, int);
 #undef FV3_FIELDS
 
 }  // namespace fv3

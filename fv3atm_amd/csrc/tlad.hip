@@ -25,6 +25,7 @@
 #include "fused.h"
 #include "fv3_internal.h"
 #include "mapz_column.h"
+#include "mapz_fields.h"
 
 namespace fv3 {
 
@@ -76,6 +77,8 @@ struct Fld<D1> {
 
 // (isd:ied, jsd:jed) working field along a row / column, with the
 // copy_corners substitution of the given direction in the corner blocks
+// (corners 0 for a line that meets none: the test on every access was most of
+// the inner x-sweep's time)
 template <typename S>
 struct FieldLine {
   const double *v, *t;
@@ -144,8 +147,9 @@ struct SubTemps {
 // ---- forward stages of one sub-cycle over the active slabs of a chunk.
 // slab p -> field slab z = zs[p] (iq*npz + k); work field (wv, wt) updated
 // in place on the interior.
-template <typename S>
-int subcycle_forward(hipStream_t s, const Geo &G, const LevelData &L, const int *zs, int np,
+// HO: the advection order of all four sweeps when it is one compile-time value (0: as given).
+template <typename S, int HO>
+int subcycle_forward_o(hipStream_t s, const Geo &G, const LevelData &L, const int *zs, int np,
                      double *wv, double *wt, const SubTemps<S> &T, const double *dpa,
                      const double *dpb, int ord_in, int ord_ou, bool update) {
   const Dims d = G.d;
@@ -157,10 +161,10 @@ int subcycle_forward(hipStream_t s, const Geo &G, const LevelData &L, const int 
   if (box(s, [=] __device__(int i, int j, int p) {
         const int z = zs[p], k = z % npz;
         FieldLine<S> qa{wv + (long long)z * d.s2, wt ? wt + (long long)z * d.s2 : nullptr, i, false,
-                        d.isd, d.jsd, d.nid, d.npx, d.npy, 2, corners};
+                        d.isd, d.jsd, d.nid, d.npx, d.npy, 2, i < 1 || i >= d.npx ? corners : 0u};
         MLine da{dya + (i - d.isd), d.jsd, d.nid};
         const S cv = S(L.cy[(long long)k * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)]);
-        T.fy2[(long long)p * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)] = ppm_flux<S>(qa, da, j, cv, gy, ord_in);
+        T.fy2[(long long)p * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)] = ppm_flux<S>(qa, da, j, cv, gy, HO ? HO : ord_in);
       }, d.isd, d.ied, d.js, d.je + 1, np))
     return -1;
   // q_i over (isd:ied, js:je)
@@ -182,17 +186,17 @@ int subcycle_forward(hipStream_t s, const Geo &G, const LevelData &L, const int 
         Line<S> qa{T.qi + (long long)p * d.sry + (long long)(j - d.js) * d.nid, d.isd, 1};
         MLine da{dxa + (long long)(j - d.jsd) * d.nid, d.isd, 1};
         const S cv = S(L.cx[(long long)k * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)]);
-        T.fx[(long long)p * d.smx + (long long)(j - d.js) * d.nix + (i - d.is)] = ppm_flux<S>(qa, da, i, cv, gx, ord_ou);
+        T.fx[(long long)p * d.smx + (long long)(j - d.js) * d.nix + (i - d.is)] = ppm_flux<S>(qa, da, i, cv, gx, HO ? HO : ord_ou);
       }, d.is, d.ie + 1, d.js, d.je, np))
     return -1;
   // fx2 = xppm(q with dir-1 corners, ord_in) over (is:ie+1, jsd:jed)
   if (box(s, [=] __device__(int i, int j, int p) {
         const int z = zs[p], k = z % npz;
         FieldLine<S> qa{wv + (long long)z * d.s2, wt ? wt + (long long)z * d.s2 : nullptr, j, true,
-                        d.isd, d.jsd, d.nid, d.npx, d.npy, 1, corners};
+                        d.isd, d.jsd, d.nid, d.npx, d.npy, 1, j < 1 || j >= d.npy ? corners : 0u};
         MLine da{dxa + (long long)(j - d.jsd) * d.nid, d.isd, 1};
         const S cv = S(L.cx[(long long)k * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)]);
-        T.fx2[(long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)] = ppm_flux<S>(qa, da, i, cv, gx, ord_in);
+        T.fx2[(long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)] = ppm_flux<S>(qa, da, i, cv, gx, HO ? HO : ord_in);
       }, d.is, d.ie + 1, d.jsd, d.jed, np))
     return -1;
   // q_j over (is:ie, jsd:jed)
@@ -214,7 +218,7 @@ int subcycle_forward(hipStream_t s, const Geo &G, const LevelData &L, const int 
         Line<S> qa{T.qj + (long long)p * d.srx + (i - d.is), d.jsd, d.niy};
         MLine da{dya + (i - d.isd), d.jsd, d.nid};
         const S cv = S(L.cy[(long long)k * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)]);
-        T.fy[(long long)p * d.smy + (long long)(j - d.js) * d.niy + (i - d.is)] = ppm_flux<S>(qa, da, j, cv, gy, ord_ou);
+        T.fy[(long long)p * d.smy + (long long)(j - d.js) * d.niy + (i - d.is)] = ppm_flux<S>(qa, da, j, cv, gy, HO ? HO : ord_ou);
       }, d.is, d.ie, d.js, d.je + 1, np))
     return -1;
   if (!update) return 0;
@@ -256,10 +260,11 @@ int subcycle_forward(hipStream_t s, const Geo &G, const LevelData &L, const int 
 // Local Jacobians (6 weights per face) of the four sweeps of one sub-cycle,
 // from the primal temporaries.
 struct SweepW {
-  double *fy2, *fx, *fx2, *fy;  // 6 per face, face layouts of sy, smx, sx, smy
+  double *fy2, *fx, *fx2, *fy;  // six planes of np slabs, face layouts of sy, smx, sx, smy
 };
 
-int sweep_weights(hipStream_t s, const Geo &G, const LevelData &L, const int *zs, int np,
+template <int HO>
+int sweep_weights_o(hipStream_t s, const Geo &G, const LevelData &L, const int *zs, int np,
                   const double *wv, const SubTemps<double> &T, const SweepW &W, int ord_in,
                   int ord_ou) {
   const Dims d = G.d;
@@ -267,16 +272,17 @@ int sweep_weights(hipStream_t s, const Geo &G, const LevelData &L, const int *zs
   const LineGeom gx{d.is, d.ie, d.npx, d.edge}, gy{d.js, d.je, d.npy, d.edge};
   const unsigned corners = d.bounded ? 0u : d.corners;
   const double *dxa = G.dxa, *dya = G.dya;
-  auto put = [] __device__(double *w, long long face, const D6 &f) {
-    for (int n = 0; n < 6; n++) w[face * 6 + n] = f.d[n];
+  auto put = [] __device__(double *w, long long face, long long plane, const D6 &f) {
+    for (int n = 0; n < 6; n++) w[n * plane + face] = f.d[n];
   };
   if (box(s, [=] __device__(int i, int j, int p) {
         const int z = zs[p], k = z % npz;
-        FieldLine<double> base{wv + (long long)z * d.s2, nullptr, i, false, d.isd, d.jsd, d.nid, d.npx, d.npy, 2, corners};
+        FieldLine<double> base{wv + (long long)z * d.s2, nullptr, i, false, d.isd, d.jsd, d.nid, d.npx, d.npy, 2, i < 1 || i >= d.npx ? corners : 0u};
         Seed6<FieldLine<double>> qa{base, j};
         MLine da{dya + (i - d.isd), d.jsd, d.nid};
         const D6 cv(L.cy[(long long)k * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)]);
-        put(W.fy2, (long long)p * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd), ppm_flux<D6>(qa, da, j, cv, gy, ord_in));
+        put(W.fy2, (long long)p * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd), (long long)np * d.sy,
+            ppm_flux<D6>(qa, da, j, cv, gy, HO ? HO : ord_in));
       }, d.isd, d.ied, d.js, d.je + 1, np))
     return -1;
   if (box(s, [=] __device__(int i, int j, int p) {
@@ -285,16 +291,18 @@ int sweep_weights(hipStream_t s, const Geo &G, const LevelData &L, const int *zs
         Seed6<Line<double>> qa{base, i};
         MLine da{dxa + (long long)(j - d.jsd) * d.nid, d.isd, 1};
         const D6 cv(L.cx[(long long)k * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)]);
-        put(W.fx, (long long)p * d.smx + (long long)(j - d.js) * d.nix + (i - d.is), ppm_flux<D6>(qa, da, i, cv, gx, ord_ou));
+        put(W.fx, (long long)p * d.smx + (long long)(j - d.js) * d.nix + (i - d.is), (long long)np * d.smx,
+            ppm_flux<D6>(qa, da, i, cv, gx, HO ? HO : ord_ou));
       }, d.is, d.ie + 1, d.js, d.je, np))
     return -1;
   if (box(s, [=] __device__(int i, int j, int p) {
         const int z = zs[p], k = z % npz;
-        FieldLine<double> base{wv + (long long)z * d.s2, nullptr, j, true, d.isd, d.jsd, d.nid, d.npx, d.npy, 1, corners};
+        FieldLine<double> base{wv + (long long)z * d.s2, nullptr, j, true, d.isd, d.jsd, d.nid, d.npx, d.npy, 1, j < 1 || j >= d.npy ? corners : 0u};
         Seed6<FieldLine<double>> qa{base, i};
         MLine da{dxa + (long long)(j - d.jsd) * d.nid, d.isd, 1};
         const D6 cv(L.cx[(long long)k * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)]);
-        put(W.fx2, (long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is), ppm_flux<D6>(qa, da, i, cv, gx, ord_in));
+        put(W.fx2, (long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is), (long long)np * d.sx,
+            ppm_flux<D6>(qa, da, i, cv, gx, HO ? HO : ord_in));
       }, d.is, d.ie + 1, d.jsd, d.jed, np))
     return -1;
   if (box(s, [=] __device__(int i, int j, int p) {
@@ -303,10 +311,24 @@ int sweep_weights(hipStream_t s, const Geo &G, const LevelData &L, const int *zs
         Seed6<Line<double>> qa{base, j};
         MLine da{dya + (i - d.isd), d.jsd, d.nid};
         const D6 cv(L.cy[(long long)k * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)]);
-        put(W.fy, (long long)p * d.smy + (long long)(j - d.js) * d.niy + (i - d.is), ppm_flux<D6>(qa, da, j, cv, gy, ord_ou));
+        put(W.fy, (long long)p * d.smy + (long long)(j - d.js) * d.niy + (i - d.is), (long long)np * d.smy,
+            ppm_flux<D6>(qa, da, j, cv, gy, HO ? HO : ord_ou));
       }, d.is, d.ie, d.js, d.je + 1, np))
     return -1;
   return 0;
+}
+
+template <typename S>
+int subcycle_forward(hipStream_t s, const Geo &G, const LevelData &L, const int *zs, int np, double *wv, double *wt,
+                     const SubTemps<S> &T, const double *dpa, const double *dpb, int ord_in, int ord_ou, bool update) {
+  return ord_in == 8 && ord_ou == 8
+             ? subcycle_forward_o<S, 8>(s, G, L, zs, np, wv, wt, T, dpa, dpb, ord_in, ord_ou, update)
+             : subcycle_forward_o<S, 0>(s, G, L, zs, np, wv, wt, T, dpa, dpb, ord_in, ord_ou, update);
+}
+int sweep_weights(hipStream_t s, const Geo &G, const LevelData &L, const int *zs, int np, const double *wv,
+                  const SubTemps<double> &T, const SweepW &W, int ord_in, int ord_ou) {
+  return ord_in == 8 && ord_ou == 8 ? sweep_weights_o<8>(s, G, L, zs, np, wv, T, W, ord_in, ord_ou)
+                                    : sweep_weights_o<0>(s, G, L, zs, np, wv, T, W, ord_in, ord_ou);
 }
 
 // Adjoint temporaries of one slab
@@ -408,7 +430,7 @@ int subcycle_adjoint(hipStream_t s, const Geo &G, const LevelData &L, const int 
         for (int f = m - 2; f <= m + 3; f++) {
           if (f < d.js || f > d.je + 1) continue;
           const long long face = (long long)p * d.smy + (long long)(f - d.js) * d.niy + (i - d.is);
-          acc += W.fy[face * 6 + (m - f + 3)] * A.fy[face];
+          acc += W.fy[(m - f + 3) * ((long long)np * d.smy) + face] * A.fy[face];
         }
         A.qj[(long long)p * d.srx + (long long)(m - d.jsd) * d.niy + (i - d.is)] = acc;
       }, d.is, d.ie, d.jsd, d.jed, np))
@@ -442,7 +464,7 @@ int subcycle_adjoint(hipStream_t s, const Geo &G, const LevelData &L, const int 
         for (int f = m - 2; f <= m + 3; f++) {
           if (f < d.is || f > d.ie + 1) continue;
           const long long face = (long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (f - d.is);
-          acc += W.fx2[face * 6 + (m - f + 3)] * A.fx2[face];
+          acc += W.fx2[(m - f + 3) * ((long long)np * d.sx) + face] * A.fx2[face];
         }
         int si, sj;
         if (full && corners && corner_src(m, j, d.npx, d.npy, 1, corners, si, sj)) {
@@ -459,7 +481,7 @@ int subcycle_adjoint(hipStream_t s, const Geo &G, const LevelData &L, const int 
         for (int f = m - 2; f <= m + 3; f++) {
           if (f < d.is || f > d.ie + 1) continue;
           const long long face = (long long)p * d.smx + (long long)(j - d.js) * d.nix + (f - d.is);
-          acc += W.fx[face * 6 + (m - f + 3)] * A.fx[face];
+          acc += W.fx[(m - f + 3) * ((long long)np * d.smx) + face] * A.fx[face];
         }
         A.qi[(long long)p * d.sry + (long long)(j - d.js) * d.nid + (m - d.isd)] = acc;
       }, d.isd, d.ied, d.js, d.je, np))
@@ -491,7 +513,7 @@ int subcycle_adjoint(hipStream_t s, const Geo &G, const LevelData &L, const int 
         for (int f = m - 2; f <= m + 3; f++) {
           if (f < d.js || f > d.je + 1) continue;
           const long long face = (long long)p * d.sy + (long long)(f - d.js) * d.nid + (i - d.isd);
-          acc += W.fy2[face * 6 + (m - f + 3)] * A.fy2[face];
+          acc += W.fy2[(m - f + 3) * ((long long)np * d.sy) + face] * A.fy2[face];
         }
         const long long o = (long long)(m - d.jsd) * d.nid + (i - d.isd);
         if (!full) {
@@ -764,11 +786,21 @@ struct RemapAD {
   const double *gbar;  // adjoint of the remapped tracers
   double *abar;        // adjoint of the remap input (out)
   // scratch [level][column]
-  double *pe1, *pe2, *d1, *d2, *a4, *qi, *gam, *dm, *qraw, *bar;  // bar: 4 x km adjoints of a1..a4
+  double *pe1, *pe2, *d1, *d2, *a4, *qi, *gam, *qraw, *bar;  // bar: 4 x km adjoints of a1..a4
   uint8_t *flags;
+  int iq0;           // first tracer of the launch
+  long long stride;  // bytes between the scratch of two tracers
 };
 
-__global__ void __launch_bounds__(64) k_remap_ad(const RemapAD a) {
+// one thread per (column, tracer)
+__global__ void __launch_bounds__(64) k_remap_ad(const RemapAD a0) {
+  RemapAD a = a0;
+  {
+    const long long o = blockIdx.y * a0.stride;
+    auto mv = [&](double *&p) { p = reinterpret_cast<double *>(reinterpret_cast<char *>(p) + o); };
+    mv(a.pe1); mv(a.pe2); mv(a.d1); mv(a.d2); mv(a.a4); mv(a.qi); mv(a.gam); mv(a.qraw); mv(a.bar);
+    a.flags += o;
+  }
   const long long col = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (col >= a.ncol) return;
   const long long nc = a.ncol;
@@ -785,7 +817,8 @@ __global__ void __launch_bounds__(64) k_remap_ad(const RemapAD a) {
   CV<uint8_t> E1{a.flags + col, 3 * nc}, E5{a.flags + nc + col, 3 * nc}, E6{a.flags + 2 * nc + col, 3 * nc};
   const bool mapn = a.nq > 5;
   const double r3 = 1.0 / 3.0, r23 = 2.0 / 3.0;
-  for (int iq = 0; iq < a.nq; iq++) {
+  {
+    const int iq = a.iq0 + (int)blockIdx.y;
     const long long base = (long long)iq * km * a.s2 + cell;
     for (int k = 1; k <= km; k++) A1(k) = a.qv[base + (long long)(k - 1) * a.s2];
     // primal profile (for the extremum flags)
@@ -1157,9 +1190,11 @@ int step_tl(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
   const size_t per_slab = sizeof(D1) * (d.sy + d.sry + d.smx + d.sx + d.srx + d.smy);
   const int chunk = (int)std::max<long long>(1, std::min<long long>(std::min(nslab, 65535), (2ll << 30) / (long long)per_slab));
   const long long ncol = (long long)(d.ie - d.is + 1) * (d.je - d.js + 1);
-  const size_t remap_b = kord_tr ? sizeof(double) * ncol * (4 * (npz + 1)) + sizeof(D1) * ncol * (7 * (npz + 1)) +
-                                       3 * ncol * (npz + 1) + 4096
-                                 : 0;
+  const size_t remap_b = !kord_tr ? 0
+                         : npz <= FIELDS_MAX_KM_TL
+                             ? coltab_bytes<double>(npz, ncol * nt) + 256
+                             : sizeof(double) * ncol * (4 * (npz + 1)) + sizeof(D1) * ncol * (7 * (npz + 1)) +
+                                   3 * ncol * (npz + 1) + 4096;
   const size_t bytes = tlad_prep_bytes(d, npz, nb) * nt + 2 * sizeof(double) * qsize + sizeof(int) * nslab +
                        per_slab * chunk + remap_b + 8192 * nt;
   char *base = (char *)ctx_scratch(c, bytes);
@@ -1219,6 +1254,39 @@ int step_tl(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
     FV3_HIP(hipStreamSynchronize(s));
     return 0;
   }
+  if (npz <= FIELDS_MAX_KM_TL) {
+    // every tracer's value and tangent over shared column tables (mapz_fields.hip)
+    const int ni = d.ie - d.is + 1, nj = d.je - d.js + 1;
+    const long long o0 = (long long)(d.js - d.jsd) * d.nid + (d.is - d.isd);
+    FieldsArgs<D1> f{};
+    f.tab = coltab_carve<double>(take(coltab_bytes<double>(npz, ncol * nt)), npz, ncol * nt);
+    if ((size_t)(cur - base) > bytes) return set_error("tangent-linear scratch layout overflow");
+    ColSource cs{};
+    cs.ptop = ptop;
+    cs.ak = ak;
+    cs.bk = bk;
+    cs.delp = dp1;
+    cs.delp_out = delp_out;
+    if (fields_prep<double>(c, f.tab, cs, ni, nj, false)) return 1;
+    for (int q1st = 0; q1st < nq; q1st += REMAP_MAX_NQ) {  // the sub-cycled tracers, REMAP_MAX_NQ at a time
+      const long long oq = (long long)q1st * npz * d.s2 + o0;
+      f.nset = 1;
+      FieldSet<D1> &x = f.set[0];
+      x = FieldSet<D1>{};
+      x.src = wv + oq; x.src_t = wt + oq; x.dst = q1 + oq; x.dst_t = dq1 + oq;
+      x.fstride = x.sfstride = d.s2 * npz;
+      x.tstride = x.ststride = qt;
+      x.lev = d.s2;
+      x.ld = d.nid;
+      x.count = std::min(REMAP_MAX_NQ, nq - q1st);
+      x.use_qmin = true;
+      x.mapn = nq > 5;
+      for (int iq = 0; iq < x.count; iq++) f.kord[iq] = (signed char)std::min(kord_tr, 17);
+      if (fields_run<D1>(c, f, ni, nj)) return 1;
+    }
+    FV3_HIP(hipStreamSynchronize(s));
+    return 0;
+  }
   RemapTL r{};
   r.km = npz; r.nq = nq; r.ni = d.ie - d.is + 1; r.is = d.is; r.js = d.js; r.isd = d.isd; r.jsd = d.jsd;
   r.nid = d.nid; r.kord = kord_tr; r.ncol = ncol; r.s2 = d.s2; r.ak = ak; r.bk = bk; r.ptop = ptop;
@@ -1265,7 +1333,10 @@ int step_ad(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
                           sizeof(double) * 6 * faces_n +
                           sizeof(double) * (d.s2 + d.smx + d.smy + d.smx + d.sx + d.smy + d.sy + d.srx + d.sry + 36);
   const int chunk = (int)std::max<long long>(1, std::min<long long>(std::min(nslab, 65535), (2ll << 30) / (long long)per_slab));
-  const size_t remap_b = kord_tr ? sizeof(double) * ncol * (npz + 1) * 16 + 3 * ncol * (npz + 1) + 4096 : 0;
+  // the remap's scratch per tracer, for as many at a time as fit in 2 GB
+  const size_t remap_1 = (sizeof(double) * ncol * (npz + 2) * 16 + 3 * ncol * (npz + 1) + 4096 + 255) & ~(size_t)255;
+  const int nq_r = (int)std::max<size_t>(1, std::min<size_t>(std::min(nq, 65535), ((size_t)2 << 30) / remap_1));
+  const size_t remap_b = kord_tr ? remap_1 * nq_r : 0;
   // checkpoints: the state entering every sub-cycle, plus the transported state
   const size_t bytes = tlad_prep_bytes(d, npz, nb) * nt + sizeof(double) * qsize * (nb + 2) + sizeof(int) * nslab +
                        per_slab * chunk + remap_b + 8192 * nt;
@@ -1347,15 +1418,18 @@ int step_ad(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
     r.a4 = (double *)take(sizeof(double) * ncol * 4 * npz);
     r.qi = (double *)take(sizeof(double) * ncol * (npz + 1));
     r.gam = (double *)take(sizeof(double) * ncol * (npz + 2));
-    r.dm = nullptr;
     r.qraw = (double *)take(sizeof(double) * ncol * (npz + 1));
     r.bar = (double *)take(sizeof(double) * ncol * 4 * npz);
     r.flags = (uint8_t *)take(3 * ncol * npz);
-    if ((size_t)(cur - base) > bytes) return set_error("adjoint scratch layout overflow");
+    r.stride = (long long)remap_1;
+    if ((size_t)(cur - (char *)r.pe1) > remap_1 || (size_t)((char *)r.pe1 + remap_b - base) > bytes)
+      return set_error("adjoint scratch layout overflow");
     for (int t = 0; t < nt; t++) {
       r.dp1 = dp1 + (long long)t * d.s2 * npz;
       r.qv = qT + t * qt; r.gbar = qbar1 + t * qt; r.abar = qbar + t * qt;
-      hipLaunchKernelGGL(k_remap_ad, dim3((unsigned)((ncol + 63) / 64)), dim3(64), 0, s, r);
+      for (r.iq0 = 0; r.iq0 < nq; r.iq0 += nq_r)
+        hipLaunchKernelGGL(k_remap_ad, dim3((unsigned)((ncol + 63) / 64), (unsigned)std::min(nq_r, nq - r.iq0)),
+                           dim3(64), 0, s, r);
       FV3_HIP(hipGetLastError());
     }
   } else {
