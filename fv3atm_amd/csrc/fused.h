@@ -22,6 +22,15 @@ template <typename T>
 int device_nsplit(Ctx &c, const T *cx, const T *cy, bool per_level, int q_split, double *cmax,
                   int *nsplit, T *frac, T *xfx = nullptr, T *yfx = nullptr);
 
+// the area fluxes alone, FP64 (unscaled, every tile)
+int area_fluxes(Ctx &c, const double *cx, const double *cy, double *xfx, double *yfx);
+// One FP64 transport pass from q_in (halos included) into the interior of q_out
+// on the levels with nsplit(k) > 0, from the thickness dp (tile stride tdp) at
+// the pass's start; winds unscaled, scaled in flight by 1 / nsplit(k).
+int fused_pass64(Ctx &c, int nq, int hord, const double *q_in, double *q_out, const double *dp, long long tdp,
+                 const double *cx, const double *cy, const double *mfx, const double *mfy, const double *xfx,
+                 const double *yfx, const int *nsplit);
+
 // Device scratch handed to a step by its caller instead of the context's
 // arenas (the no-allocation entry point); base == nullptr: the context's.
 struct StepArena {

@@ -43,6 +43,78 @@ __global__ void k_nsplit_check(const int *nsplit, int npz, int cap, int *flag) {
   }
 }
 
+// The geometry, metrics and strides of a pass over nq tracers of every tile.
+template <typename T>
+static FusedArgs<T> fused_geometry(const Ctx &c, int nq, int hord) {
+  const Dims &d = c.d;
+  const int npz = c.npz, nt = c.ntiles, ni = d.ie - d.is + 1, nj = d.je - d.js + 1;
+  FusedArgs<T> a{};
+  a.is = d.is; a.ie = d.ie; a.js = d.js; a.je = d.je;
+  a.isd = d.isd; a.ied = d.ied; a.jsd = d.jsd; a.jed = d.jed;
+  a.npx = d.npx; a.npy = d.npy; a.nid = d.nid;
+  a.s2 = d.s2; a.sx = d.sx; a.sy = d.sy; a.smx = d.smx; a.smy = d.smy;
+  a.corners = d.bounded ? 0u : d.corners;
+  a.edge = d.edge;
+  a.npz = npz; a.nq = nq; a.hord = hord;
+  a.ntiles = nt;
+  a.tq = d.s2 * npz * nq;
+  a.tcx = d.sx * npz;
+  a.tcy = d.sy * npz;
+  a.tmx = d.smx * npz;
+  a.tmy = d.smy * npz;
+  a.tdp = d.s2 * npz;
+  a.nstrip = (ni + FT_BX - 1) / FT_BX;
+  // interior strips: every lane's column i0-3..i0+60 lies in the compute
+  // domain and, on a cube face, 3 or more cells inside the tile; their lean
+  // rows lt..lb keep every input row j0-3..j0+H+2 in the domain and every
+  // stencil row off the cube-edge rows, so the lean kernel needs no halo,
+  // corner or cube-edge code
+  {
+    const bool edges = d.edge || (!d.bounded && d.corners != 0u);
+    auto strip_ok = [&](int st) {
+      const int i0 = d.is + st * FT_BX;
+      const int lo = i0 - NG, hi = i0 - NG + FT_LANES - 1;
+      return lo >= d.is && hi <= d.ie && (!edges || (lo >= 3 && hi <= d.npx - 3));
+    };
+    // (js + 6: the output row of the first input row, three above the first
+    // lean row, is itself a domain row, so no row index of a lean block clamps)
+    a.lt = std::max(d.js + 2 * NG, edges ? 8 : d.js + 2 * NG);
+    a.lb = std::min(d.je - NG, edges ? d.npy - 4 : d.je - NG);
+    a.s_lo = 1; a.s_hi = 0; a.nmid = 0;
+    int s0 = -1, s1 = -2;
+    for (int st = 0; st < a.nstrip; st++)
+      if (strip_ok(st)) { if (s0 < 0) s0 = st; s1 = st; }
+    const bool inner = s0 >= 0 && a.lb >= a.lt;
+    const int rows = inner ? a.lb - a.lt + 1 : nj;
+    // (resident workgroups of four waves: three per CU in FP32, two in FP64)
+    const long long units = (long long)a.nstrip * npz * nt * ((nq + 3) / 4);
+    a.H = c.fused_h > 0 ? c.fused_h
+                        : fused_block_rows(rows, units, sizeof(T) == 4 ? 768 : 512, inner ? 2.5 : 2.0 * NG);
+    a.H = std::min(nj, a.H);
+    a.nvblk = (nj + a.H - 1) / a.H;
+    if (inner) {
+      a.s_lo = s0;
+      a.s_hi = s1;
+      a.nmid = (a.lb - a.lt + a.H) / a.H;
+    }
+  }
+  const GridDev<T> &g = grid_of<T>(c);
+  a.area = g.area; a.rarea = g.rarea; a.dxa = g.dxa; a.dya = g.dya; a.dx = g.dx; a.dy = g.dy;
+  a.sin_sg = g.sin_sg; a.ms2 = g.s2;
+  a.tgs2 = g.s2;
+  a.tgdx = g.sdx;
+  a.tgdy = g.sdy;
+  if (sizeof(T) == 4) {
+    a.gxp = (const T *)c.gfac32;
+    a.gxm = a.gxp + (long long)(d.nid + 1) * d.njd;
+    a.gyp = a.gxm + (long long)(d.nid + 1) * d.njd;
+    a.gym = a.gyp + (long long)d.nid * (d.njd + 1);
+    a.gex = a.gym + (long long)d.nid * (d.njd + 1);
+    a.tgf = 2 * (long long)(d.nid + 1) * d.njd + 2 * (long long)d.nid * (d.njd + 1) + (long long)d.nid * d.njd;
+  }
+  return a;
+}
+
 template <typename T>
 static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const double *dp1,
                         double *delp_out, const T *cx, const T *cy, const T *mfx, const T *mfy,
@@ -141,76 +213,14 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     q_tmp = (T *)ctx_scratch(c, sizeof(T) * qsize);
     if (!q_tmp) return 1;
   }
-  FusedArgs<T> a{};
-  a.is = d.is; a.ie = d.ie; a.js = d.js; a.je = d.je;
-  a.isd = d.isd; a.ied = d.ied; a.jsd = d.jsd; a.jed = d.jed;
-  a.npx = d.npx; a.npy = d.npy; a.nid = d.nid;
-  a.s2 = d.s2; a.sx = d.sx; a.sy = d.sy; a.smx = d.smx; a.smy = d.smy;
-  a.corners = d.bounded ? 0u : d.corners;
-  a.edge = d.edge;
-  a.npz = npz; a.nq = nq; a.hord = hord; a.cap = cap;
-  a.ntiles = nt;
-  a.tq = d.s2 * npz * nq;
-  a.tcx = d.sx * npz;
-  a.tcy = d.sy * npz;
-  a.tmx = d.smx * npz;
-  a.tmy = d.smy * npz;
-  a.tdp = d.s2 * npz;
-  a.nstrip = (ni + FT_BX - 1) / FT_BX;
-  // interior strips: every lane's column i0-3..i0+60 lies in the compute
-  // domain and, on a cube face, 3 or more cells inside the tile; their lean
-  // rows lt..lb keep every input row j0-3..j0+H+2 in the domain and every
-  // stencil row off the cube-edge rows, so the lean kernel needs no halo,
-  // corner or cube-edge code
-  {
-    const bool edges = d.edge || (!d.bounded && d.corners != 0u);
-    auto strip_ok = [&](int st) {
-      const int i0 = d.is + st * FT_BX;
-      const int lo = i0 - NG, hi = i0 - NG + FT_LANES - 1;
-      return lo >= d.is && hi <= d.ie && (!edges || (lo >= 3 && hi <= d.npx - 3));
-    };
-    // (js + 6: the output row of the first input row, three above the first
-    // lean row, is itself a domain row, so no row index of a lean block clamps)
-    a.lt = std::max(d.js + 2 * NG, edges ? 8 : d.js + 2 * NG);
-    a.lb = std::min(d.je - NG, edges ? d.npy - 4 : d.je - NG);
-    a.s_lo = 1; a.s_hi = 0; a.nmid = 0;
-    int s0 = -1, s1 = -2;
-    for (int st = 0; st < a.nstrip; st++)
-      if (strip_ok(st)) { if (s0 < 0) s0 = st; s1 = st; }
-    const bool inner = s0 >= 0 && a.lb >= a.lt;
-    const int rows = inner ? a.lb - a.lt + 1 : nj;
-    // (resident workgroups of four waves: three per CU in FP32, two in FP64)
-    const long long units = (long long)a.nstrip * npz * nt * ((nq + 3) / 4);
-    a.H = c.fused_h > 0 ? c.fused_h
-                        : fused_block_rows(rows, units, sizeof(T) == 4 ? 768 : 512, inner ? 2.5 : 2.0 * NG);
-    a.H = std::min(nj, a.H);
-    a.nvblk = (nj + a.H - 1) / a.H;
-    if (inner) {
-      a.s_lo = s0;
-      a.s_hi = s1;
-      a.nmid = (a.lb - a.lt + a.H) / a.H;
-    }
-  }
+  FusedArgs<T> a = fused_geometry<T>(c, nq, hord);
+  a.cap = cap;
   a.nsplit = nspl;
   a.q_in = q_in;
   a.q_out = oop ? q_tmp : q_out;
   a.q_tmp = oop ? q_out : q_tmp;
   a.xfx = xfx; a.yfx = yfx;
   a.cx = cx; a.cy = cy; a.mfx = mfx; a.mfy = mfy; a.dp1 = dp1;
-  const GridDev<T> &g = grid_of<T>(c);
-  a.area = g.area; a.rarea = g.rarea; a.dxa = g.dxa; a.dya = g.dya; a.dx = g.dx; a.dy = g.dy;
-  a.sin_sg = g.sin_sg; a.ms2 = g.s2;
-  a.tgs2 = g.s2;
-  a.tgdx = g.sdx;
-  a.tgdy = g.sdy;
-  if (sizeof(T) == 4) {
-    a.gxp = (const T *)c.gfac32;
-    a.gxm = a.gxp + (long long)(d.nid + 1) * d.njd;
-    a.gyp = a.gxm + (long long)(d.nid + 1) * d.njd;
-    a.gym = a.gyp + (long long)d.nid * (d.njd + 1);
-    a.gex = a.gym + (long long)d.nid * (d.njd + 1);
-    a.tgf = 2 * (long long)(d.nid + 1) * d.njd + 2 * (long long)d.nid * (d.njd + 1) + (long long)d.nid * d.njd;
-  }
   const bool timing = c.timing && !c.graph_safe;
   if (timing) FV3_HIP(hipEventRecord(c.ev[0], s));
   // the remap's column prep (thicknesses only) and the copies it needs run on
@@ -348,6 +358,34 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     FV3_HIP(hipStreamSynchronize(s));
     if (hf) return set_error("a level needs more sub-cycles than nsplit_cap=%d", nsplit_cap);
   }
+  return 0;
+}
+
+int fused_pass64(Ctx &c, int nq, int hord, const double *q_in, double *q_out, const double *dp, long long tdp,
+                 const double *cx, const double *cy, const double *mfx, const double *mfy, const double *xfx,
+                 const double *yfx, const int *nsplit) {
+  hipStream_t s = c.stream;
+  FusedArgs<double> a = fused_geometry<double>(c, nq, hord);
+  a.cap = 0x7fffffff;
+  a.it = 1;  // reads q_in and dp as they are; every level lands in q_out
+  a.nsplit = nsplit;
+  a.q_in = q_in;
+  a.q_out = a.q_tmp = q_out;
+  a.dp1 = dp;
+  if (c.ntiles > 1) a.tdp = tdp;
+  a.cx = cx; a.cy = cy; a.mfx = mfx; a.mfy = mfy; a.xfx = xfx; a.yfx = yfx;
+  const bool conc = c.concurrent_kinds && c.aux[0] && c.aux[1] && c.aux[2];
+  const KindStreams ks = conc ? KindStreams{{s, c.aux[0], c.aux[1], c.aux[2]}} : KindStreams{{s, s, s, s}};
+  if (conc) {
+    FV3_HIP(hipEventRecord(c.fork_ev, s));
+    for (int i = 0; i < 3; i++) FV3_HIP(hipStreamWaitEvent(c.aux[i], c.fork_ev, 0));
+  }
+  if (launch_fused_f64(a, ks)) return 1;
+  if (conc)
+    for (int i = 0; i < 3; i++) {
+      FV3_HIP(hipEventRecord(c.join_ev[i], c.aux[i]));
+      FV3_HIP(hipStreamWaitEvent(s, c.join_ev[i], 0));
+    }
   return 0;
 }
 

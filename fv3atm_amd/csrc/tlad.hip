@@ -34,24 +34,57 @@ namespace {
 using D6 = Dual<6>;
 using D7 = Dual<7>;
 
+// f(i, j, z) over a box of points, a wave on 64 columns of one row
 template <typename F>
 __global__ void __launch_bounds__(256) k_box(F f, int i0, int i1, int j0, int j1) {
-  const int ni = i1 - i0 + 1;
-  const long long n = (long long)ni * (j1 - j0 + 1);
-  const int z = blockIdx.z;
-  for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < n;
-       t += (long long)gridDim.x * blockDim.x)
-    f(i0 + (int)(t % ni), j0 + (int)(t / ni), z);
+  const int i = i0 + (int)(blockIdx.x * 64 + threadIdx.x), j = j0 + (int)(blockIdx.y * 4 + threadIdx.y);
+  if (i <= i1 && j <= j1) f(i, j, (int)blockIdx.z);
 }
 
 template <typename F>
 int box(hipStream_t s, F f, int i0, int i1, int j0, int j1, int nz) {
   if (i1 < i0 || j1 < j0 || nz <= 0) return 0;
-  const long long n = (long long)(i1 - i0 + 1) * (j1 - j0 + 1);
-  dim3 g((unsigned)std::min<long long>((n + 255) / 256, 2048), 1, (unsigned)nz);
-  hipLaunchKernelGGL(k_box<F>, g, dim3(256), 0, s, f, i0, i1, j0, j1);
+  const dim3 g((unsigned)((i1 - i0 + 64) / 64), (unsigned)((j1 - j0 + 4) / 4), (unsigned)nz);
+  hipLaunchKernelGGL(k_box<F>, g, dim3(64, 4), 0, s, f, i0, i1, j0, j1);
   FV3_HIP(hipGetLastError());
   return 0;
+}
+
+// The faces lo..hi of a sweep line whose stencils meet no cube-edge rule and no
+// corner cell; the few faces either side take the general form in a launch of
+// their own, with consecutive lanes along the edge.  (In one launch every wave
+// that held an edge face ran the interior and each edge formula in turn, at
+// the registers of the longest: the Jacobians' inner x-sweep of a C192 face
+// took 1.0 ms for 128 slabs.)
+struct InnerFaces {
+  int lo, hi;
+};
+InnerFaces inner_faces(int s, int e, int np, bool rules) {
+  return rules ? InnerFaces{std::max(s, 4), std::min(e + 1, np - 3)} : InnerFaces{s, e + 1};
+}
+struct Inner {
+  static constexpr bool edge = false;
+};
+struct Edge {
+  static constexpr bool edge = true;
+};
+// face(i, j, z, Inner/Edge) over the x-faces is..ie+1 of rows j0..j1
+template <typename F>
+int x_sweep(hipStream_t s, const Dims &d, F face, int j0, int j1, int nz) {
+  const InnerFaces b = inner_faces(d.is, d.ie, d.npx, d.edge || (!d.bounded && d.corners != 0u));
+  const int is = d.is, nl = b.lo - d.is, ne = nl + d.ie + 1 - b.hi, hi = b.hi;
+  if (box(s, [=] __device__(int i, int j, int z) { face(i, j, z, Inner{}); }, b.lo, b.hi, j0, j1, nz)) return -1;
+  return box(s, [=] __device__(int j, int e, int z) { face(e < nl ? is + e : hi + 1 + e - nl, j, z, Edge{}); }, j0, j1,
+             0, ne - 1, nz);
+}
+// face(i, j, z, Inner/Edge) over the y-faces js..je+1 of columns i0..i1
+template <typename F>
+int y_sweep(hipStream_t s, const Dims &d, F face, int i0, int i1, int nz) {
+  const InnerFaces b = inner_faces(d.js, d.je, d.npy, d.edge || (!d.bounded && d.corners != 0u));
+  const int js = d.js, nl = b.lo - d.js, ne = nl + d.je + 1 - b.hi, hi = b.hi;
+  if (box(s, [=] __device__(int i, int j, int z) { face(i, j, z, Inner{}); }, i0, i1, b.lo, b.hi, nz)) return -1;
+  return box(s, [=] __device__(int i, int e, int z) { face(i, e < nl ? js + e : hi + 1 + e - nl, z, Edge{}); }, i0, i1,
+             0, ne - 1, nz);
 }
 
 // ---- scalar load/store over (value, tangent) array pairs
@@ -154,18 +187,18 @@ int subcycle_forward_o(hipStream_t s, const Geo &G, const LevelData &L, const in
                      const double *dpb, int ord_in, int ord_ou, bool update) {
   const Dims d = G.d;
   const int npz = G.npz;
-  const LineGeom gx{d.is, d.ie, d.npx, d.edge}, gy{d.js, d.je, d.npy, d.edge};
   const unsigned corners = d.bounded ? 0u : d.corners;
   const double *area = G.area, *rarea = G.rarea, *dxa = G.dxa, *dya = G.dya;
   // fy2 = yppm(q with dir-2 corners, ord_in) over (isd:ied, js:je+1)
-  if (box(s, [=] __device__(int i, int j, int p) {
+  if (y_sweep(s, d, [=] __device__(int i, int j, int p, auto where) {
         const int z = zs[p], k = z % npz;
+        const LineGeom g{d.js, d.je, d.npy, where.edge && d.edge};
         FieldLine<S> qa{wv + (long long)z * d.s2, wt ? wt + (long long)z * d.s2 : nullptr, i, false,
-                        d.isd, d.jsd, d.nid, d.npx, d.npy, 2, i < 1 || i >= d.npx ? corners : 0u};
+                        d.isd, d.jsd, d.nid, d.npx, d.npy, 2, where.edge && (i < 1 || i >= d.npx) ? corners : 0u};
         MLine da{dya + (i - d.isd), d.jsd, d.nid};
         const S cv = S(L.cy[(long long)k * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)]);
-        T.fy2[(long long)p * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)] = ppm_flux<S>(qa, da, j, cv, gy, HO ? HO : ord_in);
-      }, d.isd, d.ied, d.js, d.je + 1, np))
+        T.fy2[(long long)p * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)] = ppm_flux<S>(qa, da, j, cv, g, HO ? HO : ord_in);
+      }, d.isd, d.ied, np))
     return -1;
   // q_i over (isd:ied, js:je)
   if (box(s, [=] __device__(int i, int j, int p) {
@@ -181,23 +214,25 @@ int subcycle_forward_o(hipStream_t s, const Geo &G, const LevelData &L, const in
       }, d.isd, d.ied, d.js, d.je, np))
     return -1;
   // fx = xppm(q_i, ord_ou) over (is:ie+1, js:je)
-  if (box(s, [=] __device__(int i, int j, int p) {
+  if (x_sweep(s, d, [=] __device__(int i, int j, int p, auto where) {
         const int z = zs[p], k = z % npz;
+        const LineGeom g{d.is, d.ie, d.npx, where.edge && d.edge};
         Line<S> qa{T.qi + (long long)p * d.sry + (long long)(j - d.js) * d.nid, d.isd, 1};
         MLine da{dxa + (long long)(j - d.jsd) * d.nid, d.isd, 1};
         const S cv = S(L.cx[(long long)k * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)]);
-        T.fx[(long long)p * d.smx + (long long)(j - d.js) * d.nix + (i - d.is)] = ppm_flux<S>(qa, da, i, cv, gx, HO ? HO : ord_ou);
-      }, d.is, d.ie + 1, d.js, d.je, np))
+        T.fx[(long long)p * d.smx + (long long)(j - d.js) * d.nix + (i - d.is)] = ppm_flux<S>(qa, da, i, cv, g, HO ? HO : ord_ou);
+      }, d.js, d.je, np))
     return -1;
   // fx2 = xppm(q with dir-1 corners, ord_in) over (is:ie+1, jsd:jed)
-  if (box(s, [=] __device__(int i, int j, int p) {
+  if (x_sweep(s, d, [=] __device__(int i, int j, int p, auto where) {
         const int z = zs[p], k = z % npz;
+        const LineGeom g{d.is, d.ie, d.npx, where.edge && d.edge};
         FieldLine<S> qa{wv + (long long)z * d.s2, wt ? wt + (long long)z * d.s2 : nullptr, j, true,
-                        d.isd, d.jsd, d.nid, d.npx, d.npy, 1, j < 1 || j >= d.npy ? corners : 0u};
+                        d.isd, d.jsd, d.nid, d.npx, d.npy, 1, where.edge && (j < 1 || j >= d.npy) ? corners : 0u};
         MLine da{dxa + (long long)(j - d.jsd) * d.nid, d.isd, 1};
         const S cv = S(L.cx[(long long)k * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)]);
-        T.fx2[(long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)] = ppm_flux<S>(qa, da, i, cv, gx, HO ? HO : ord_in);
-      }, d.is, d.ie + 1, d.jsd, d.jed, np))
+        T.fx2[(long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)] = ppm_flux<S>(qa, da, i, cv, g, HO ? HO : ord_in);
+      }, d.jsd, d.jed, np))
     return -1;
   // q_j over (is:ie, jsd:jed)
   if (box(s, [=] __device__(int i, int j, int p) {
@@ -213,43 +248,35 @@ int subcycle_forward_o(hipStream_t s, const Geo &G, const LevelData &L, const in
       }, d.is, d.ie, d.jsd, d.jed, np))
     return -1;
   // fy = yppm(q_j, ord_ou) over (is:ie, js:je+1)
-  if (box(s, [=] __device__(int i, int j, int p) {
+  if (y_sweep(s, d, [=] __device__(int i, int j, int p, auto where) {
         const int z = zs[p], k = z % npz;
+        const LineGeom g{d.js, d.je, d.npy, where.edge && d.edge};
         Line<S> qa{T.qj + (long long)p * d.srx + (i - d.is), d.jsd, d.niy};
         MLine da{dya + (i - d.isd), d.jsd, d.nid};
         const S cv = S(L.cy[(long long)k * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)]);
-        T.fy[(long long)p * d.smy + (long long)(j - d.js) * d.niy + (i - d.is)] = ppm_flux<S>(qa, da, j, cv, gy, HO ? HO : ord_ou);
-      }, d.is, d.ie, d.js, d.je + 1, np))
+        T.fy[(long long)p * d.smy + (long long)(j - d.js) * d.niy + (i - d.is)] = ppm_flux<S>(qa, da, j, cv, g, HO ? HO : ord_ou);
+      }, d.is, d.ie, np))
     return -1;
   if (!update) return 0;
-  // flux averaging with the mass fluxes
-  if (box(s, [=] __device__(int i, int j, int p) {
-        const int z = zs[p], k = z % npz;
-        if (i <= d.ie + 1 && j <= d.je) {
-          const long long o = (long long)(j - d.js) * d.nix + (i - d.is);
-          S &f = T.fx[(long long)p * d.smx + o];
-          f = S(0.5) * (f + T.fx2[(long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)]) * S(L.mfx[(long long)k * d.smx + o]);
-        }
-        if (i <= d.ie && j <= d.je + 1) {
-          const long long o = (long long)(j - d.js) * d.niy + (i - d.is);
-          S &f = T.fy[(long long)p * d.smy + o];
-          f = S(0.5) * (f + T.fy2[(long long)p * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)]) * S(L.mfy[(long long)k * d.smy + o]);
-        }
-      }, d.is, d.ie + 1, d.js, d.je + 1, np))
-    return -1;
-  // flux-form update of the interior, in place (each cell reads only itself)
+  // flux averaging with the mass fluxes and the flux-form update of the
+  // interior, in place (each cell reads only itself and its faces)
   if (box(s, [=] __device__(int i, int j, int p) {
         const int z = zs[p], k = z % npz;
         const long long o = (long long)(j - d.jsd) * d.nid + (i - d.isd);
-        const S *fxr = T.fx + (long long)p * d.smx + (long long)(j - d.js) * d.nix;
-        const S *fyc = T.fy + (long long)p * d.smy;
+        auto Fx = [&](int ii) -> S {
+          const long long f = (long long)(j - d.js) * d.nix + (ii - d.is);
+          return S(0.5) * (T.fx[(long long)p * d.smx + f] + T.fx2[(long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (ii - d.is)]) *
+                 S(L.mfx[(long long)k * d.smx + f]);
+        };
+        auto Fy = [&](int jj) -> S {
+          const long long f = (long long)(jj - d.js) * d.niy + (i - d.is);
+          return S(0.5) * (T.fy[(long long)p * d.smy + f] + T.fy2[(long long)p * d.sy + (long long)(jj - d.js) * d.nid + (i - d.isd)]) *
+                 S(L.mfy[(long long)k * d.smy + f]);
+        };
         double *v = wv + (long long)z * d.s2;
         double *t = wt ? wt + (long long)z * d.s2 : nullptr;
         const S w = Fld<S>::ld(v, t, o);
-        const S val = (w * S(dpa[(long long)k * d.s2 + o]) +
-                       (fxr[i - d.is] - fxr[i + 1 - d.is] + fyc[(long long)(j - d.js) * d.niy + (i - d.is)] -
-                        fyc[(long long)(j + 1 - d.js) * d.niy + (i - d.is)]) *
-                           S(rarea[o])) /
+        const S val = (w * S(dpa[(long long)k * d.s2 + o]) + (Fx(i) - Fx(i + 1) + Fy(j) - Fy(j + 1)) * S(rarea[o])) /
                       S(dpb[(long long)k * d.s2 + o]);
         Fld<S>::st(v, t, o, val);
       }, d.is, d.ie, d.js, d.je, np))
@@ -269,51 +296,54 @@ int sweep_weights_o(hipStream_t s, const Geo &G, const LevelData &L, const int *
                   int ord_ou) {
   const Dims d = G.d;
   const int npz = G.npz;
-  const LineGeom gx{d.is, d.ie, d.npx, d.edge}, gy{d.js, d.je, d.npy, d.edge};
   const unsigned corners = d.bounded ? 0u : d.corners;
   const double *dxa = G.dxa, *dya = G.dya;
   auto put = [] __device__(double *w, long long face, long long plane, const D6 &f) {
     for (int n = 0; n < 6; n++) w[n * plane + face] = f.d[n];
   };
-  if (box(s, [=] __device__(int i, int j, int p) {
+  if (y_sweep(s, d, [=] __device__(int i, int j, int p, auto where) {
         const int z = zs[p], k = z % npz;
-        FieldLine<double> base{wv + (long long)z * d.s2, nullptr, i, false, d.isd, d.jsd, d.nid, d.npx, d.npy, 2, i < 1 || i >= d.npx ? corners : 0u};
+        const LineGeom g{d.js, d.je, d.npy, where.edge && d.edge};
+        FieldLine<double> base{wv + (long long)z * d.s2, nullptr, i, false, d.isd, d.jsd, d.nid, d.npx, d.npy, 2, where.edge && (i < 1 || i >= d.npx) ? corners : 0u};
         Seed6<FieldLine<double>> qa{base, j};
         MLine da{dya + (i - d.isd), d.jsd, d.nid};
         const D6 cv(L.cy[(long long)k * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)]);
         put(W.fy2, (long long)p * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd), (long long)np * d.sy,
-            ppm_flux<D6>(qa, da, j, cv, gy, HO ? HO : ord_in));
-      }, d.isd, d.ied, d.js, d.je + 1, np))
+            ppm_flux<D6>(qa, da, j, cv, g, HO ? HO : ord_in));
+      }, d.isd, d.ied, np))
     return -1;
-  if (box(s, [=] __device__(int i, int j, int p) {
+  if (x_sweep(s, d, [=] __device__(int i, int j, int p, auto where) {
         const int z = zs[p], k = z % npz;
+        const LineGeom g{d.is, d.ie, d.npx, where.edge && d.edge};
         Line<double> base{T.qi + (long long)p * d.sry + (long long)(j - d.js) * d.nid, d.isd, 1};
         Seed6<Line<double>> qa{base, i};
         MLine da{dxa + (long long)(j - d.jsd) * d.nid, d.isd, 1};
         const D6 cv(L.cx[(long long)k * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)]);
         put(W.fx, (long long)p * d.smx + (long long)(j - d.js) * d.nix + (i - d.is), (long long)np * d.smx,
-            ppm_flux<D6>(qa, da, i, cv, gx, HO ? HO : ord_ou));
-      }, d.is, d.ie + 1, d.js, d.je, np))
+            ppm_flux<D6>(qa, da, i, cv, g, HO ? HO : ord_ou));
+      }, d.js, d.je, np))
     return -1;
-  if (box(s, [=] __device__(int i, int j, int p) {
+  if (x_sweep(s, d, [=] __device__(int i, int j, int p, auto where) {
         const int z = zs[p], k = z % npz;
-        FieldLine<double> base{wv + (long long)z * d.s2, nullptr, j, true, d.isd, d.jsd, d.nid, d.npx, d.npy, 1, j < 1 || j >= d.npy ? corners : 0u};
+        const LineGeom g{d.is, d.ie, d.npx, where.edge && d.edge};
+        FieldLine<double> base{wv + (long long)z * d.s2, nullptr, j, true, d.isd, d.jsd, d.nid, d.npx, d.npy, 1, where.edge && (j < 1 || j >= d.npy) ? corners : 0u};
         Seed6<FieldLine<double>> qa{base, i};
         MLine da{dxa + (long long)(j - d.jsd) * d.nid, d.isd, 1};
         const D6 cv(L.cx[(long long)k * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is)]);
         put(W.fx2, (long long)p * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is), (long long)np * d.sx,
-            ppm_flux<D6>(qa, da, i, cv, gx, HO ? HO : ord_in));
-      }, d.is, d.ie + 1, d.jsd, d.jed, np))
+            ppm_flux<D6>(qa, da, i, cv, g, HO ? HO : ord_in));
+      }, d.jsd, d.jed, np))
     return -1;
-  if (box(s, [=] __device__(int i, int j, int p) {
+  if (y_sweep(s, d, [=] __device__(int i, int j, int p, auto where) {
         const int z = zs[p], k = z % npz;
+        const LineGeom g{d.js, d.je, d.npy, where.edge && d.edge};
         Line<double> base{T.qj + (long long)p * d.srx + (i - d.is), d.jsd, d.niy};
         Seed6<Line<double>> qa{base, j};
         MLine da{dya + (i - d.isd), d.jsd, d.nid};
         const D6 cv(L.cy[(long long)k * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd)]);
         put(W.fy, (long long)p * d.smy + (long long)(j - d.js) * d.niy + (i - d.is), (long long)np * d.smy,
-            ppm_flux<D6>(qa, da, j, cv, gy, HO ? HO : ord_ou));
-      }, d.is, d.ie, d.js, d.je + 1, np))
+            ppm_flux<D6>(qa, da, j, cv, g, HO ? HO : ord_ou));
+      }, d.is, d.ie, np))
     return -1;
   return 0;
 }
@@ -1338,7 +1368,8 @@ int step_ad(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
   const int nq_r = (int)std::max<size_t>(1, std::min<size_t>(std::min(nq, 65535), ((size_t)2 << 30) / remap_1));
   const size_t remap_b = kord_tr ? remap_1 * nq_r : 0;
   // checkpoints: the state entering every sub-cycle, plus the transported state
-  const size_t bytes = tlad_prep_bytes(d, npz, nb) * nt + sizeof(double) * qsize * (nb + 2) + sizeof(int) * nslab +
+  const size_t bytes = tlad_prep_bytes(d, npz, nb) * nt + sizeof(double) * qsize * (nb + 2) +
+                       sizeof(int) * ((size_t)nslab + (size_t)npz * nb) + sizeof(double) * (d.sx + d.sy) * npz * nt +
                        per_slab * chunk + remap_b + 8192 * nt;
   const long long *hu = nullptr, *hd = nullptr;
   const int *hp = nullptr;
@@ -1358,6 +1389,8 @@ int step_ad(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
   double *ck = (double *)take(sizeof(double) * qsize * (nb + 1));  // ck[it-1]: input of sub-cycle it; ck[nmax]: final
   double *qbar = (double *)take(sizeof(double) * qsize);
   int *zs = (int *)take(sizeof(int) * nslab);
+  int *ns_it = (int *)take(sizeof(int) * npz * nb);
+  double *xfx = (double *)take(sizeof(double) * d.sx * npz * nt), *yfx = (double *)take(sizeof(double) * d.sy * npz * nt);
   char *tmp = take(per_slab * chunk);
   const int ord_in = hord == 10 ? 8 : hord, ord_ou = hord;
   // temporaries
@@ -1386,23 +1419,24 @@ int step_ad(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
       for (int k = 0; k < npz; k++)
         if (P0.nsplit[k] >= it) acts[it].push_back(iq * npz + k);
   }
+  // (each sub-cycle by the fused FP64 transport, bit for bit the stages; the
+  // counts of pass it: nsplit(k) where it reaches it, else 0)
+  {
+    std::vector<int> counts((size_t)nb * npz);
+    for (int it = 1; it <= nb; it++)
+      for (int k = 0; k < npz; k++) counts[(size_t)(it - 1) * npz + k] = P0.nsplit[k] >= it ? P0.nsplit[k] : 0;
+    FV3_HIP(hipMemcpyAsync(ns_it, counts.data(), sizeof(int) * counts.size(), hipMemcpyHostToDevice, s));
+    FV3_HIP(hipStreamSynchronize(s));  // counts goes out of scope
+  }
+  if (area_fluxes(c, cx, cy, xfx, yfx)) return 1;
+  const long long tdp = nt > 1 ? P[1].dp_hist - P[0].dp_hist : 0;
   for (int it = 1; it <= nb; it++) {
     double *prev = ck + (long long)(it - 1) * qsize, *next = ck + (long long)it * qsize;
     if (faces && halo_fill<double>(c, prev, qt, nullptr, 0, nslab)) return 1;
     FV3_HIP(hipMemcpyAsync(next, prev, sizeof(double) * qsize, hipMemcpyDeviceToDevice, s));
-    const std::vector<int> &act = acts[it];
-    FV3_HIP(hipMemcpyAsync(zs, act.data(), sizeof(int) * act.size(), hipMemcpyHostToDevice, s));
-    for (int t = 0; t < nt; t++) {
-      const Geo G = geo_of(c, t);
-      const double *dpa = P[t].dp_hist + (long long)(it - 1) * npz * d.s2, *dpb = P[t].dp_hist + (long long)it * npz * d.s2;
-      for (size_t p0 = 0; p0 < act.size(); p0 += chunk) {
-        const int np = (int)std::min<size_t>(chunk, act.size() - p0);
-        if (subcycle_forward<double>(s, G, P[t].L, zs + p0, np, next + t * qt, nullptr, T, dpa, dpb, ord_in, ord_ou,
-                                     true))
-          return 1;
-      }
-    }
-    FV3_HIP(hipStreamSynchronize(s));
+    if (fused_pass64(c, nq, hord, prev, next, P[0].dp_hist + (long long)(it - 1) * npz * d.s2, tdp, cx, cy, mfx, mfy,
+                     xfx, yfx, ns_it + (size_t)(it - 1) * npz))
+      return 1;
   }
   const double *qT = ck + (long long)nb * qsize;
   // ---- remap adjoint: qbar = (d remap / d qT)^T qbar1 on the interior

@@ -138,6 +138,7 @@ __global__ void __launch_bounds__(256) k_area_flux(const T *cx, const T *cy, con
         m = mx2(m, mx2(ax, ay) + 1.0 - s5[cell]);
     }
   }
+  if (!cmax) return;
   __shared__ double red[256];
   red[threadIdx.x] = m;
   __syncthreads();
@@ -178,6 +179,21 @@ __global__ void k_zero(T *p, int n) {
 }
 
 template <typename T>
+static int launch_area_flux(Ctx &c, const T *cx, const T *cy, T *xfx, T *yfx, double *cmax) {
+  const Dims &d = c.d;
+  const dim3 g((unsigned)((d.nid + 63) / 64), (unsigned)((d.njd + AF_ROWS - 1) / AF_ROWS),
+               (unsigned)(c.npz * c.ntiles));
+  hipLaunchKernelGGL(k_area_flux<T>, g, dim3(256), 0, c.stream, cx, cy, grid_of<T>(c), c.grid64.sin_sg, d, c.npz, xfx,
+                     yfx, cmax);
+  FV3_HIP(hipGetLastError());
+  return 0;
+}
+
+int area_fluxes(Ctx &c, const double *cx, const double *cy, double *xfx, double *yfx) {
+  return launch_area_flux<double>(c, cx, cy, xfx, yfx, nullptr);
+}
+
+template <typename T>
 int device_nsplit(Ctx &c, const T *cx, const T *cy, bool per_level, int q_split, double *cmax,
                   int *nsplit, T *frac, T *xfx, T *yfx) {
   const Dims d = c.d;
@@ -187,9 +203,7 @@ int device_nsplit(Ctx &c, const T *cx, const T *cy, bool per_level, int q_split,
   dim3 b(256), gr((unsigned)std::min(64, (d.ie - d.is + 1) * (d.je - d.js + 1) / 256 + 1), 1,
                   (unsigned)(npz * nt));
   if (xfx) {
-    const dim3 ga((unsigned)((d.nid + 63) / 64), (unsigned)((d.njd + AF_ROWS - 1) / AF_ROWS), (unsigned)(npz * nt));
-    hipLaunchKernelGGL(k_area_flux<T>, ga, b, 0, c.stream, cx, cy, grid_of<T>(c), c.grid64.sin_sg, d, npz, xfx, yfx,
-                       cmax);
+    if (launch_area_flux<T>(c, cx, cy, xfx, yfx, cmax)) return 1;
   } else {
     hipLaunchKernelGGL(k_cmax<T>, gr, b, 0, c.stream, cx, cy, c.grid64.sin_sg, d, npz, c.grid64.s2, cmax);
   }
