@@ -51,7 +51,8 @@ __device__ __forceinline__ long long pe_at(const Geo &g, int i, int k, int j) {
 }
 
 // Lagrangian interfaces and ps on the compute domain and its one-cell ring
-__global__ void k_pe_ring(Geo g, int t, double ptop, const double *delp, double *pe, double *ps) {
+__global__ void __launch_bounds__(64) k_pe_ring(Geo g, int t, double ptop, const double *__restrict__ delp,
+                                                double *__restrict__ pe, double *__restrict__ ps) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   const int w = g.ni + 2;
   if (idx >= w * (g.nj + 2)) return;
@@ -60,7 +61,18 @@ __global__ void k_pe_ring(Geo g, int t, double ptop, const double *delp, double 
   double *p = pe + t * g.spe;
   double v = ptop;
   p[pe_at(g, i, 1, j)] = v;
-  for (int k = 1; k <= g.km; k++) {
+  int k = 1;
+  for (; k + 7 <= g.km; k += 8) {  // eight loads in flight
+    double d[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) d[m] = dl[(long long)(k + m - 1) * g.s2];
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      v = v + d[m];
+      p[pe_at(g, i, k + m + 1, j)] = v;
+    }
+  }
+  for (; k <= g.km; k++) {
     v = v + dl[(long long)(k - 1) * g.s2];
     p[pe_at(g, i, k + 1, j)] = v;
   }
@@ -136,6 +148,7 @@ __device__ double column_te(const Geo &g, int t, int i, int j, double cp, const 
   double te = 0.0;
   const long long cell = (long long)(j - g.jsd) * g.nid + (i - g.isd);
   const long long pc = (long long)(j - g.js) * g.ni + (i - g.is);
+#pragma unroll 4
   for (int k = 1; k <= g.km; k++) {
     const T *uk = u + ((long long)t * g.km + (k - 1)) * g.su;
     const T *vk = v + ((long long)t * g.km + (k - 1)) * g.sv;
@@ -160,11 +173,17 @@ __global__ void k_te(Geo g, int t, double cp, const T *u, const T *v, const T *p
   te[(long long)t * g.ni * g.nj + idx] = column_te<T>(g, t, i, j, cp, u, v, pt, pkz, delp);
 }
 
-// Eulerian pe (compute domain), peln, pk, pkz
+// Eulerian pe (compute domain), peln, pk, pkz: one thread per column and
+// PR_LEV levels, each with its layers' upper interfaces (and the next one's,
+// recomputed, for the hydrostatic layer means).  One thread per column was one
+// log and exp after another: C192 L127 150 us.
+constexpr int PR_LEV = 4;
 template <typename T>
-__global__ void k_pressures(Geo g, int t, double ptop, const double *ak, const double *bk, double akap,
-                            double rrg, int hydrostatic, const double *ps, const double *delp, const T *pt,
-                            const T *delz, double *pe, double *peln, double *pk, double *pkz) {
+__global__ void k_pressures(Geo g, int t, double ptop, const double *__restrict__ ak, const double *__restrict__ bk,
+                            double akap, double rrg, int hydrostatic, const double *__restrict__ ps,
+                            const double *__restrict__ delp, const T *__restrict__ pt, const T *__restrict__ delz,
+                            double *__restrict__ pe, double *__restrict__ peln, double *__restrict__ pk,
+                            double *__restrict__ pkz) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= g.ni * g.nj) return;
   const int i = g.is + idx % g.ni, j = g.js + idx / g.ni;
@@ -173,29 +192,35 @@ __global__ void k_pressures(Geo g, int t, double ptop, const double *ak, const d
   const long long nc = (long long)g.ni * g.nj;
   double *pl = peln + t * g.spl + (long long)(j - g.js) * (g.km + 1) * g.ni + (i - g.is);
   double *pkc = pk + t * g.spk + idx;
-  for (int k = 1; k <= g.km + 1; k++) {
+  const int k0 = 1 + (int)blockIdx.y * PR_LEV, k1 = min(k0 + PR_LEV - 1, g.km);
+  double lp_k = 0.0, pk_k = 0.0;  // of interface k
+  for (int k = k0; k <= k1 + 1; k++) {
     const double p = k == 1 ? ptop : (k == g.km + 1 ? psv : ak[k - 1] + bk[k - 1] * psv);
-    pe[t * g.spe + pe_at(g, i, k, j)] = p;
-    const double lp = log(p);
-    pl[(long long)(k - 1) * g.ni] = lp;
-    pkc[(long long)(k - 1) * nc] = exp(akap * lp);
-  }
-  for (int k = 1; k <= g.km; k++) {
-    double *o = pkz + t * g.spz + (long long)(k - 1) * nc + idx;
-    if (hydrostatic) {
-      *o = (pkc[(long long)k * nc] - pkc[(long long)(k - 1) * nc]) /
-           (akap * (pl[(long long)k * g.ni] - pl[(long long)(k - 1) * g.ni]));
-    } else {
-      const double dz = (double)delz[t * g.spz + (long long)(k - 1) * nc + idx];
-      const double ptk = (double)pt[((long long)t * g.km + (k - 1)) * g.s2 + cell];
-      // p = rho R pt p^akap, so p^akap = (rho R pt)^(akap / (1 - akap))
-      const double k1k = akap / (1.0 - akap);
-      *o = exp(k1k * log(rrg * delp[((long long)t * g.km + (k - 1)) * g.s2 + cell] / dz * ptk));
+    const bool own = k <= k1 || k == g.km + 1;
+    if (!own && !hydrostatic) break;
+    const double lp = log(p), pkv = exp(akap * lp);
+    if (own) {
+      pe[t * g.spe + pe_at(g, i, k, j)] = p;
+      pl[(long long)(k - 1) * g.ni] = lp;
+      pkc[(long long)(k - 1) * nc] = pkv;
     }
+    if (hydrostatic && k > k0)
+      pkz[t * g.spz + (long long)(k - 2) * nc + idx] = (pkv - pk_k) / (akap * (lp - lp_k));
+    lp_k = lp;
+    pk_k = pkv;
+  }
+  if (hydrostatic) return;
+  for (int k = k0; k <= k1; k++) {
+    const double dz = (double)delz[t * g.spz + (long long)(k - 1) * nc + idx];
+    const double ptk = (double)pt[((long long)t * g.km + (k - 1)) * g.s2 + cell];
+    // p = rho R pt p^akap, so p^akap = (rho R pt)^(akap / (1 - akap))
+    const double k1k = akap / (1.0 - akap);
+    pkz[t * g.spz + (long long)(k - 1) * nc + idx] =
+        exp(k1k * log(rrg * delp[((long long)t * g.km + (k - 1)) * g.s2 + cell] / dz * ptk));
   }
 }
 
-// Neumaier sums of x[i] * w[i] (w may be NULL) over n values, deterministic:
+// Neumaier sums over n values, deterministic:
 // block partials of fixed strided order, then one block combines them.
 struct KS {
   double s, c;
@@ -212,11 +237,14 @@ __device__ __forceinline__ void kmerge(KS &a, const KS &b) {
 
 constexpr int KS_BLOCK = 256, KS_GRID = 256;
 
-__global__ void __launch_bounds__(KS_BLOCK) k_ksum_part(const double *x, const double *w, long long n, KS *part) {
+// the sums of blockIdx.y = 0, 1, 2: x, x + n, x + 2 n
+__global__ void __launch_bounds__(KS_BLOCK) k_ksum_part(const double *x, long long n, KS *part) {
+  x += blockIdx.y * n;
+  part += blockIdx.y * KS_GRID;
   __shared__ KS sh[KS_BLOCK];
   KS k{0.0, 0.0};
   for (long long i = (long long)blockIdx.x * KS_BLOCK + threadIdx.x; i < n; i += (long long)KS_BLOCK * KS_GRID)
-    kadd(k, w ? x[i] * w[i] : x[i]);
+    kadd(k, x[i]);
   sh[threadIdx.x] = k;
   __syncthreads();
   for (int s = KS_BLOCK / 2; s > 0; s >>= 1) {
@@ -226,11 +254,16 @@ __global__ void __launch_bounds__(KS_BLOCK) k_ksum_part(const double *x, const d
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-__global__ void k_ksum_final(const KS *part, int np, double *out) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
+// one block per sum: the partials to LDS, merged in order by one thread
+__global__ void __launch_bounds__(KS_GRID) k_ksum_final(const KS *part, double *out) {
+  __shared__ KS sh[KS_GRID];
+  sh[threadIdx.x] = part[blockIdx.x * KS_GRID + threadIdx.x];
+  __syncthreads();
+  if (threadIdx.x == 0) {
     KS k{0.0, 0.0};
-    for (int i = 0; i < np; i++) kmerge(k, part[i]);
-    *out = k.s + k.c;
+#pragma unroll 8
+    for (int i = 0; i < KS_GRID; i++) kmerge(k, sh[i]);
+    out[blockIdx.x] = k.s + k.c;
   }
 }
 
@@ -347,10 +380,10 @@ int l2e_full(Ctx &c, const fv3_l2e_args &a) {
   double *sums = (double *)(base + o_sum);
 
   for (int t = 0; t < nt; t++) {
-    hipLaunchKernelGGL(k_pe_ring, grid1((long long)(g.ni + 2) * (g.nj + 2)), dim3(256), 0, s, g, t, a.ptop, a.delp,
-                       a.pe, a.ps);
+    hipLaunchKernelGGL(k_pe_ring, dim3((unsigned)(((long long)(g.ni + 2) * (g.nj + 2) + 63) / 64)), dim3(64), 0, s, g,
+                       t, a.ptop, a.delp, a.pe, a.ps);
     if (energy)
-      hipLaunchKernelGGL(k_te<T>, grid1((long long)g.ni * g.nj), dim3(256), 0, s, g, t, a.cp, u, v, pt, a.pkz,
+      hipLaunchKernelGGL(k_te<T>, dim3((unsigned)(((long long)g.ni * g.nj + 63) / 64)), dim3(64), 0, s, g, t, a.cp, u, v, pt, a.pkz,
                          a.delp, a.te0_2d);
   }
   FV3_HIP(hipGetLastError());
@@ -473,7 +506,8 @@ int l2e_full(Ctx &c, const fv3_l2e_args &a) {
   }
   const double rrg = -a.rdgas / a.grav;
   for (int t = 0; t < nt; t++)
-    hipLaunchKernelGGL(k_pressures<T>, grid1((long long)g.ni * g.nj), dim3(256), 0, s, g, t, a.ptop, a.ak, a.bk,
+    hipLaunchKernelGGL(k_pressures<T>, dim3(grid1((long long)g.ni * g.nj).x, (unsigned)((km + PR_LEV - 1) / PR_LEV)),
+                       dim3(256), 0, s, g, t, a.ptop, a.ak, a.bk,
                        a.akap, rrg, a.hydrostatic, a.ps, a.delp, pt, dz, a.pe, a.peln, a.pk, a.pkz);
   FV3_HIP(hipGetLastError());
   // fast physics: the caller's hook sees the Eulerian state
@@ -506,13 +540,10 @@ int l2e_full(Ctx &c, const fv3_l2e_args &a) {
   // total-energy fix-up: the domain's energy loss back into pt
   if (energy && a.consv > 0.0) {
     for (int t = 0; t < nt; t++)
-      hipLaunchKernelGGL(k_energy_terms<T>, grid1((long long)g.ni * g.nj), dim3(256), 0, s, g, t, a.cp, a.ptop, u,
+      hipLaunchKernelGGL(k_energy_terms<T>, dim3((unsigned)(((long long)g.ni * g.nj + 63) / 64)), dim3(64), 0, s, g, t, a.cp, a.ptop, u,
                          v, pt, a.pkz, a.delp, a.ps, c.grid64.area, a.te0_2d, e0, e1, em);
-    for (int m = 0; m < 3; m++) {
-      hipLaunchKernelGGL(k_ksum_part, dim3(KS_GRID), dim3(KS_BLOCK), 0, s, e0 + m * ncell, (const double *)nullptr,
-                         ncell, part + m * KS_GRID);
-      hipLaunchKernelGGL(k_ksum_final, dim3(1), dim3(1), 0, s, part + m * KS_GRID, KS_GRID, sums + m);
-    }
+    hipLaunchKernelGGL(k_ksum_part, dim3(KS_GRID, 3), dim3(KS_BLOCK), 0, s, e0, ncell, part);
+    hipLaunchKernelGGL(k_ksum_final, dim3(3), dim3(KS_GRID), 0, s, part, sums);
     hipLaunchKernelGGL(k_dtmp, dim3(1), dim3(1), 0, s, sums, a.consv, sums + 3);
     hipLaunchKernelGGL(k_add_dtmp<T>, grid1((long long)g.ni * g.nj * km * nt), dim3(256), 0, s, g, nt, pt, a.pkz,
                        sums + 3);
