@@ -42,6 +42,10 @@ struct alignas(4 * sizeof(R)) Elim {
 //   rc   its source layers: top | bottom << 12 | (both in one layer) << 24
 //        (top 0: no layer holds it; bottom km + 1: it ends below the source)
 //   bot  [3][column] bottom-row factors
+//   win  [column] how many source layers one target layer takes in over the 64
+//        columns of a block together, at most (a block with a column whose
+//        interfaces are out of order: NO_WINDOW)
+constexpr int NO_WINDOW = 1 << 20;
 template <typename R>
 struct ColTab {
   Elim<R> *el;
@@ -49,6 +53,7 @@ struct ColTab {
   double2 *r0, *r1, *r2;
   int *rc;
   R *bot;
+  int *win;
 };
 
 template <typename R>
@@ -96,7 +101,7 @@ constexpr int FIELDS_MAX_SETS = 3;
 template <typename T>
 struct FieldsArgs {
   using R = typename RealOf<T>::type;
-  int km, ni, ncb, nf, nfg, nset;
+  int km, ni, ncb, ntiles, nf, nset;
   unsigned nwg;
   long long ncol, ncols;  // columns per tile, of every tile
   ColTab<R> tab;

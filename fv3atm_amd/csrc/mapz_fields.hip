@@ -58,7 +58,7 @@ template <typename R>
 __global__ void __launch_bounds__(64 * PREP_WAVES) k_fields_prep(const PrepGeo g, const ColSource s,
                                                                  const ColTab<R> tab, const bool iv2) {
   extern __shared__ double pe1_lds[];  // [km + 1][64]
-  __shared__ int bad[64];
+  __shared__ int bad[64], win;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int tile = (int)blockIdx.x / g.ncb, cb = (int)blockIdx.x % g.ncb;
   const int km = g.km;  // at most FIELDS_MAX_KM: 64 columns fit
@@ -70,7 +70,10 @@ __global__ void __launch_bounds__(64 * PREP_WAVES) k_fields_prep(const PrepGeo g
   const long long cell = (long long)(j - g.jsd) * g.nid + (i - g.isd);
   const long long col = tile * g.ncol + lc, nc = g.ncols;
   const ColPe P{pe1_lds + lane, 64};
-  if (wave == 0) bad[lane] = 0;
+  if (wave == 0) {
+    bad[lane] = 0;
+    win = 0;
+  }
   double psl = 0.0;  // kinds 1, 2: the sum of the two cells' surface pressures
   if (s.kind == 0) {
     stage_interfaces(P, km, s.ptop, s.delp + (long long)tile * km * g.s2 + cell, g.s2, wave);
@@ -150,7 +153,6 @@ __global__ void __launch_bounds__(64 * PREP_WAVES) k_fields_prep(const PrepGeo g
       tab.bot[nc + col] = bot1;
       tab.bot[2 * nc + col] = bot2;
     }
-    return;
   }
   // the target layers
   double *dout = s.delp_out ? s.delp_out + (long long)tile * km * g.s2 + cell : nullptr;
@@ -163,7 +165,8 @@ __global__ void __launch_bounds__(64 * PREP_WAVES) k_fields_prep(const PrepGeo g
     tab.rc[o] = lt | lb << 12 | (one ? 1 << 24 : 0);
     if (dout) dout[(long long)(k - 1) * g.s2] = den;
   };
-  if (!bad[lane]) {
+  if (wave > 0 && !bad[lane]) {
+    int w = 0;  // source layers that one target layer of the block's columns takes in, at most
     for (int k = wave; k <= km; k += PREP_WAVES - 1) {
       const double pa = PE2(k), pb = PE2(k + 1);
       const int lt = P.layer_of(pa, k, km), lb = P.layer_of(pb, k, km);
@@ -171,8 +174,16 @@ __global__ void __launch_bounds__(64 * PREP_WAVES) k_fields_prep(const PrepGeo g
       const bool one = lt == lb;
       const double db = pb - c;
       put(k, lt, lb, one, (pa - a) / (b - a), db / (P(lb + 1) - c), one ? 0.0 : b - pa, one ? 0.0 : db, pb - pa);
+      int lo = __builtin_amdgcn_readfirstlane(lt), hi = __builtin_amdgcn_readfirstlane(lb);
+      for (unsigned long long m; (m = __ballot(lt < lo)) != 0;) lo = __builtin_amdgcn_readlane(lt, __builtin_ctzll(m));
+      for (unsigned long long m; (m = __ballot(lb > hi)) != 0;) hi = __builtin_amdgcn_readlane(lb, __builtin_ctzll(m));
+      w = max(w, hi - lo + 1);
     }
-  } else if (wave == 1) {  // upstream's search
+    atomicMax(&win, w);
+  } else if (wave > 0) {
+    atomicMax(&win, NO_WINDOW);
+  }
+  if (wave == 1 && bad[lane]) {  // upstream's search
     int k0 = 1;
     double pa = PE2(1);
     for (int k = 1; k <= km; k++) {
@@ -206,11 +217,23 @@ __global__ void __launch_bounds__(64 * PREP_WAVES) k_fields_prep(const PrepGeo g
       pa = pb;
     }
   }
+  __syncthreads();
+  if (wave == 0 && act) tab.win[col] = win;
 }
 
 // ---- the field kernel
 constexpr int FD_B = 8;      // levels per regenerated block
 constexpr int FD_WAVES = 4;  // fields per workgroup (one per wave)
+// source cells kept in LDS for the targets (fewer for (value, tangent) pairs,
+// whose cells are twice as large)
+template <typename T>
+constexpr int FD_RING = sizeof(T) > 8 ? 4 : 5;
+// LDS rows of 64 values per wave: block ends, a block's interface values, and
+// three coefficients per kept cell
+template <typename T>
+__host__ __device__ constexpr int fd_rows(int nb) {
+  return nb + FD_B + 3 * FD_RING<T>;
+}
 
 struct TargetRec {
   double2 r0, r1, r2;
@@ -226,28 +249,39 @@ struct TargetRec {
 //         interface values by back substitution from its exit value, into LDS,
 //         then level by level the interface limits, extremum flags, cell
 //         limiters and layer integrals over a window of six cell means.
-// Only the block ends and one block are kept (18 KB of LDS per wave in FP64
-// at 127 levels: two waves per SIMD); the field's second and third reads come
-// from cache.  The divisions by the field-independent pivots use their stored
-// reciprocals (quot).  Bound by VALU issue at two waves per SIMD.  Measured
-// against one thread per column looping over its fields with every work array
-// in HBM (at C96 144 waves on 1024 SIMDs): C384 L127 9 tracers + pt FP64 18.7
-// -> 4.9 ms plus 0.76 ms of tables, C96 L64 4 tracers + pt 1.79 -> 0.19 + 0.06
-// ms; the FP32 full remap of C192 L127 (13 fields) 12.4 -> 1.9 + 1.0 ms.
+// The columns of a wave go through the target layers in lockstep: a cell's
+// three coefficients go to a ring of FD_RING cells in LDS, and once the cell is
+// done in which the target's bottom lies in every column, each column takes its
+// pieces from the ring.  Records are loaded and results stored a whole level at
+// a time.  A block where one target takes in more cells than the ring holds
+// (tab.win) runs column by column instead, each with a target of its own: its
+// scattered records and stores, and loops of several turns per level, were most
+// of the time (C384 L127, 9 tracers + pt in FP64: 4.86 ms in that form, 3.75 in
+// lockstep, 3.53 with the levels walked by adding to scalar bases and the waves
+// dealt to (column block, field) pairs without gaps; the full remap of C192
+// L127 in FP32, 13 fields: 1.85, 1.65, 1.44 ms).
+// Only the block ends, one block and the ring are kept (20 KB of LDS per wave
+// in FP64 at 127 levels: two waves per SIMD); the field's second and third
+// reads come from cache.  The divisions by the field-independent pivots use
+// their stored reciprocals (quot).  Bound by dependent FP64 operations at two
+// waves per SIMD (VALU a third busy).  One thread per column looping over its
+// fields with every work array in HBM (at C96 144 waves on 1024 SIMDs) took
+// 18.7 ms for the C384 case, tables included (now 3.53 + 0.45), 1.79 ms for C96
+// L64 4 tracers + pt (0.125 + 0.027), 12.4 ms for the FP32 remap (1.44 + 0.44).
 template <typename T>
 __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields(const FieldsArgs<T> a) {
   using R = typename RealOf<T>::type;
   extern __shared__ __align__(16) char fd_lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // blocks are dealt round-robin to the 8 XCDs: renumber so that the field
-  // groups of one column block run on one XCD, one after another
+  // blocks are dealt round-robin to the 8 XCDs: renumber so that the fields
+  // of one column block run on one XCD, one after another
   const unsigned bid = blockIdx.x, nx = 8, q8 = a.nwg / nx, r8 = a.nwg % nx;
   const unsigned xcd = bid % nx, idx = bid / nx;
   const unsigned logical = xcd < r8 ? xcd * (q8 + 1) + idx : r8 * (q8 + 1) + (xcd - r8) * q8 + idx;
-  const int cblk = (int)(logical / a.nfg), fg = (int)(logical % a.nfg);
-  const int f = fg * FD_WAVES + wave;
-  if (f >= a.nf) return;  // whole wave; no barriers below
+  const unsigned job = logical * FD_WAVES + wave;
+  const int cblk = (int)(job / (unsigned)a.nf), f = (int)(job % (unsigned)a.nf);
+  if (cblk >= a.ncb * a.ntiles) return;  // whole wave; no barriers below
   int si = 0, fi = f;
   while (si + 1 < a.nset && fi >= a.set[si].count) fi -= a.set[si++].count;
   const FieldSet<T> &S = a.set[si];
@@ -266,22 +300,27 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
   if constexpr (sizeof(T) != sizeof(R)) src_t = S.src_t + sbase;
   const long long lev = S.lev;
   const unsigned cbyte = cell * (unsigned)sizeof(R);
-  auto ld = [&](int k) -> T {  // scalar level base, lane byte offset
-    const R v = *reinterpret_cast<const R *>(reinterpret_cast<const char *>(src + (k - 1) * lev) + cbyte);
+  // scalar level bases, lane byte offsets; levels are walked by adding to the
+  // bases (a 64-bit product per load was half of the scalar work)
+  const long long levb = lev * (long long)sizeof(R), elb = nc * (long long)sizeof(Elim<R>);
+  auto ldat = [&](long long o) -> T {  // o: (k - 1) levb
+    const R v = *reinterpret_cast<const R *>(reinterpret_cast<const char *>(src) + o + cbyte);
     if constexpr (sizeof(T) == sizeof(R)) {
       return v;
     } else {
       T r(v);
-      r.d[0] = *reinterpret_cast<const R *>(reinterpret_cast<const char *>(src_t + (k - 1) * lev) + cbyte);
+      r.d[0] = *reinterpret_cast<const R *>(reinterpret_cast<const char *>(src_t) + o + cbyte);
       return r;
     }
   };
-  const Elim<R> *el = a.tab.el + col;
-  auto lde = [&](int k) -> Elim<R> { return el[(long long)(k - 1) * nc]; };
-  T *lds = reinterpret_cast<T *>(fd_lds) + (size_t)wave * (nb + 2 * FD_B + 4) * 64 + lane;
+  auto ld = [&](int k) -> T { return ldat((k - 1) * levb); };
+  const long long colu = tile * a.ncol + (long long)cb * 64;  // the block's first column
+  const unsigned cl = (unsigned)(lc - (long long)cb * 64), ebyte = cl * (unsigned)sizeof(Elim<R>);
+  T *lds = reinterpret_cast<T *>(fd_lds) + (size_t)wave * fd_rows<T>(nb) * 64 + lane;
   auto CP = [&](int b) -> T & { return lds[b * 64]; };
   auto BQ = [&](int j) -> T & { return lds[(nb + j) * 64]; };
-  auto BA = [&](int j) -> T & { return lds[(nb + FD_B + 2 + j) * 64]; };
+  constexpr int NR = FD_RING<T>;
+  T *ring = lds + (nb + FD_B) * 64;  // [NR][3][64]
   const bool iv2 = iv == -2;
   const T qs = iv2 ? T(S.qs[tile * a.ncol + lc]) : T(R(0));
   const R bot0 = a.tab.bot[col], bot1 = a.tab.bot[nc + col], bot2 = a.tab.bot[2 * nc + col];
@@ -292,14 +331,38 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
   };
   auto fetch = [&](int b, Blk &x) {
     const int k0 = b * FD_B + 1;
+    const char *e = reinterpret_cast<const char *>(a.tab.el + colu) + (k0 - 1) * elb;
+    long long o = (k0 - 1) * levb;
+    x.av[0] = ldat(b > 0 ? o - levb : o);
+    if (k0 + FD_B - 1 <= km) {
 #pragma unroll
-    for (int j = 0; j <= FD_B; j++) x.av[j] = ld(min(max(k0 - 1 + j, 1), km));
+      for (int j = 0; j < FD_B; j++) {
+        x.av[j + 1] = ldat(o);
+        x.e[j] = *reinterpret_cast<const Elim<R> *>(e + ebyte);
+        o += levb;
+        e += elb;
+      }
+    } else {
 #pragma unroll
-    for (int j = 0; j < FD_B; j++) x.e[j] = lde(min(k0 + j, km));
+      for (int j = 0; j < FD_B; j++) {
+        x.av[j + 1] = ldat(o);
+        x.e[j] = *reinterpret_cast<const Elim<R> *>(e + ebyte);
+        if (k0 + j < km) {
+          o += levb;
+          e += elb;
+        }
+      }
+    }
   };
   // the eliminated values of block b from the one above it
   auto eliminate = [&](int b, const Blk &x, T q, T (&qv)[FD_B], const T &a2nd) {
     const int k0 = b * FD_B + 1;
+    if (b > 0 && k0 + FD_B - 1 < km) {
+#pragma unroll
+      for (int j = 0; j < FD_B; j++)
+        qv[j] = q = quot(R(3) * (x.av[j] + x.e[j].d4 * x.av[j + 1]) - q, x.e[j].bt, x.e[j].y);
+      return q;
+    }
 #pragma unroll
     for (int j = 0; j < FD_B; j++) {
       const int k = k0 + j;
@@ -313,6 +376,19 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
         }
       }
       qv[j] = q;
+    }
+    return q;
+  };
+  // block b's interface values from the one below it: put(j, value)
+  auto substitute = [&](int b, const Blk &x, T q, const T (&qv)[FD_B], auto put) {
+    const int k0 = b * FD_B + 1;
+    if (k0 + FD_B - 1 <= km) {
+#pragma unroll
+      for (int j = FD_B - 1; j >= 0; j--) put(j, q = qv[j] - x.e[j].g * q);
+    } else {
+#pragma unroll
+      for (int j = FD_B - 1; j >= 0; j--)
+        if (k0 + j <= km) put(j, q = qv[j] - x.e[j].g * q);
     }
     return q;
   };
@@ -345,9 +421,7 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
       if (b > 0) {
         T qv[FD_B];
         eliminate(b, cur, entry, qv, a2nd);
-#pragma unroll
-        for (int j = FD_B - 1; j >= 0; j--)
-          if (b * FD_B + 1 + j <= km) q = qv[j] - cur.e[j].g * q;
+        q = substitute(b, cur, q, qv, [](int, const T &) {});
       }
       cur = nxt;
     }
@@ -356,48 +430,77 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
   // ---- down: limits, cells, layer integrals
   const bool lim = akord <= 16;
   const T zero = T(R(0));
-  T A_4 = zero, A_3 = zero, A_2 = zero, A_1 = zero, A_0 = zero, A_p = ld(1);  // a(p-4 .. p+1)
+  T A_4 = zero, A_3 = zero, A_2 = zero, A_1 = zero, A_0 = zero, A_p = ld(1), A_n = a2nd;  // a(p-4 .. p+2)
   T L_2 = zero, L_1 = zero, L_0 = zero;                                      // limited Q(p-2 .. p)
   int E_3 = 0, E_2 = 0, E_1 = 0;                                             // flags of cells p-3 .. p-1
-  // the open target: its records (and the next target's, in flight), partial sum
-  int kt = 1;
-  bool open = false;
-  const double2 *p0 = a.tab.r0 + col, *p1 = a.tab.r1 + col, *p2 = a.tab.r2 + col;
-  const int *pc = a.tab.rc + col;
-  auto rec = [&](int k) -> TargetRec {
-    const long long o = (long long)(min(k, km) - 1) * nc;
-    return TargetRec{p0[o], p1[o], p2[o], pc[o]};
+  auto recat = [&](long long o) -> TargetRec {  // o: 4 (k - 1) nc
+    auto r = [&](const double2 *p) {
+      return *reinterpret_cast<const double2 *>(reinterpret_cast<const char *>(p + colu) + 4 * o + cl * 16);
+    };
+    return TargetRec{r(a.tab.r0), r(a.tab.r1), r(a.tab.r2),
+                     *reinterpret_cast<const int *>(reinterpret_cast<const char *>(a.tab.rc + colu) + o + cl * 4)};
   };
-  TargetRec tr = rec(1), tn = rec(2);
-  char *dlane = reinterpret_cast<char *>(S.dst + fbase) + cbyte;
-  char *dlane_t = nullptr;
-  if constexpr (sizeof(T) != sizeof(R)) dlane_t = reinterpret_cast<char *>(S.dst_t + fbase) + cbyte;
-  const long long levb = lev * (long long)sizeof(R);
+  const long long nc4 = 4 * nc;
+  auto rec = [&](int k) -> TargetRec { return recat((min(k, km) - 1) * nc4); };
+  TargetRec tr = rec(1), tn = rec(2);  // the next two targets'
   using SumT = typename std::conditional<sizeof(T) == sizeof(R), double, D1>::type;  // sums in FP64
-  SumT acc(0.0);
   auto wide = [](const T &v) -> SumT { return (SumT)v; };
-  auto emit = [&](const T &v) {
-    if (act) {
-      if constexpr (sizeof(T) == sizeof(R)) {
-        *reinterpret_cast<R *>(dlane) = v;
-      } else {
-        *reinterpret_cast<R *>(dlane) = v.v;
-        *reinterpret_cast<R *>(dlane_t) = v.d[0];
-      }
-    }
-    dlane += levb;
-    if constexpr (sizeof(T) != sizeof(R)) dlane_t += levb;
-    kt++;
-    tr = tn;
-    tn = rec(kt + 1);
-  };
   auto narrow = [](const SumT &v) -> T {
     if constexpr (sizeof(T) == sizeof(R)) return T(v);
     else return v;
   };
-  const double *d1p = a.tab.d1 + col;
-  double d1n = d1p[0];  // thickness of the next cell
+  auto ldd = [&](long long o) -> double {  // o: 8 (k - 1) nc
+    return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(a.tab.d1 + colu) + o + cl * 8);
+  };
+  double d1n = ldd(0);  // thickness of the next cell
+  const double r3 = 1.0 / 3.0, r23 = 2.0 / 3.0;
+  // pieces of a target in a cell's parabola: within one cell, from pl to the
+  // cell's bottom, from its top to esl
+  auto within = [&](const T &a2, const T &a3, const T &a4, double pl, double pr) -> T {
+    const double z = pr * (pr + pl) + pl * pl;
+    const T tail = mapn ? T(a4 * R(r3 * z)) : T(a4 * R(r3) * R(z));
+    return a2 + (a4 + a3 - a2) * R(0.5 * (pr + pl)) - tail;
+  };
+  auto top_piece = [&](const T &a2, const T &a3, const T &a4, double pl, double dp) -> SumT {
+    return dp * wide(a2 + (a4 + a3 - a2) * R(0.5 * (1.0 + pl)) - a4 * R(r3 * (1.0 + pl * (1.0 + pl))));
+  };
+  auto bottom_piece = [&](const T &a2, const T &a3, const T &a4, double esl, double dp) -> SumT {
+    return dp * wide(a2 + R(0.5 * esl) * (a3 - a2 + a4 * R(1.0 - r23 * esl)));
+  };
+  char *dst = reinterpret_cast<char *>(S.dst + fbase), *dst_t = nullptr;
+  if constexpr (sizeof(T) != sizeof(R)) dst_t = reinterpret_cast<char *>(S.dst_t + fbase);
+  auto store = [&](char *at, char *at_t, const T &v) {
+    if constexpr (sizeof(T) == sizeof(R)) {
+      *reinterpret_cast<R *>(at) = v;
+    } else {
+      *reinterpret_cast<R *>(at) = v.v;
+      *reinterpret_cast<R *>(at_t) = v.d[0];
+    }
+  };
 
+  auto sweep = [&](auto lockstep) {
+  int kt = 1;  // the target in hand: the wave's in lockstep, else the lane's
+  // in lockstep: slot of cell c; thickness times mean of cells c-1 ..
+  int cs = NR - 1;
+  long long ro = (min(3, km) - 1) * nc4;  // of the record to be loaded next
+  char *du = dst, *du_t = dst_t;          // of the target in hand
+  SumT M[NR - 1];
+#pragma unroll
+  for (int m = 0; m < NR - 1; m++) M[m] = SumT(0.0);
+  // lane by lane: the open target's sum
+  bool open = false;
+  SumT acc(0.0);
+  char *dl = dst + cbyte, *dl_t = dst_t + cbyte;
+  auto emit = [&](const T &v) {
+    if (act) store(dl, dl_t, v);
+    dl += levb;
+    dl_t += levb;
+    kt++;
+    tr = tn;
+    tn = rec(kt + 1);
+  };
+
+  long long ao = (min(3, km) - 1) * levb, dof = 0;  // of the next mean, of the next cell's thickness
   T chain = zero;  // the eliminated value above the block
   Blk cur, nxt;
   fetch(0, cur);
@@ -406,35 +509,29 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
     {
       T qv[FD_B];
       chain = eliminate(b, cur, chain, qv, a2nd);
-      q = CP(b);
-#pragma unroll
-      for (int j = FD_B - 1; j >= 0; j--)
-        if (k0 + j <= km) {
-          q = qv[j] - cur.e[j].g * q;
-          BQ(j) = q;
-        }
+      substitute(b, cur, CP(b), qv, [&](int j, const T &v) { BQ(j) = v; });
     }
     const bool last = b + 1 == nb;
     if (!last) fetch(b + 1, nxt);
-#pragma unroll
-    for (int j = 0; j + 1 < FD_B; j++) BA(j) = cur.av[j + 2];  // a(k0+1 ..)
-    if (!last) BA(FD_B - 1) = nxt.av[1];
-    if (last) BQ(km + 1 - k0) = qbot;
     const int pend = last ? km + 2 : k0 + FD_B - 1;
-    for (int p = k0; p <= pend; p++) {
+    auto step = [&](int p, auto inner) {  // inner: 5 <= p < km, no special cells
+      constexpr bool IN = decltype(inner)::value;
       A_4 = A_3;
       A_3 = A_2;
       A_2 = A_1;
       A_1 = A_0;
       A_0 = A_p;
-      if (p < km) A_p = BA(p - k0);
+      A_p = A_n;
+      A_n = ldat(ao);
+      if (p + 2 < km) ao += levb;
       L_2 = L_1;
       L_1 = L_0;
-      if (p <= km + 1) L_0 = BQ(p - k0);
+      if (IN || p <= km) L_0 = BQ(p - k0);
+      else if (p == km + 1) L_0 = qbot;
       // interface p lies between cells p-1 (A_1) and p (A_0)
-      if (lim && p >= 2 && p <= km) {
+      if (lim && (IN || (p >= 2 && p <= km))) {
         const T lo = mn2(A_1, A_0), hi = mx2(A_1, A_0);
-        if (p == 2 || p == km) {
+        if (!IN && (p == 2 || p == km)) {
           L_0 = mx2(mn2(L_0, hi), lo);
         } else {
           const T glo = A_1 - A_2, ghi = A_p - A_0;
@@ -453,9 +550,9 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
       E_3 = E_2;
       E_2 = E_1;
       // flags of cell p-1: 1 extm, 2 ext5, 4 ext6
-      if (lim && p >= 2 && p <= km + 1) {
+      if (lim && (IN || (p >= 2 && p <= km + 1))) {
         const int e = p - 1;
-        const bool em = e == 1 || e == km ? (L_1 - A_1) * (L_0 - A_1) > zero
+        const bool em = !IN && (e == 1 || e == km) ? (L_1 - A_1) * (L_0 - A_1) > zero
                                           : (A_1 - A_2) * (A_0 - A_1) < zero;
         E_1 = em ? 1 : 0;
         if (akord > 9) {
@@ -464,12 +561,12 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
         }
       }
       const int c = p - 2;
-      if (c < 1) continue;
+      if (!IN && c < 1) return;
       // ---- cell c = p-2: a(c) is A_2, its interface values L_2, L_1
       T a1 = A_2, a2 = L_2, a3 = L_1, a4;
       if (!lim) {
         a4 = R(3) * (R(2) * a1 - (a2 + a3));
-      } else if (c == 1 || c == 2 || c >= km - 1) {
+      } else if (!IN && (c == 1 || c == 2 || c >= km - 1)) {
         if (c == 1) {
           if (iv == 0) {
             a2 = mx2(zero, a2);
@@ -518,52 +615,100 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
         }
         if (iv == 0) cs_lim1(a1, a2, a3, a4, (E_2 & 1) != 0, 0);
       }
-      // ---- the target layers that end, lie or begin in source layer c
       const double d1c = d1n;
-      d1n = d1p[(long long)(min(c + 1, km) - 1) * nc];
-      const double r3 = 1.0 / 3.0, r23 = 2.0 / 3.0;
-      while (kt <= km) {
-        const int lt = tr.rc & 0xfff, lb = (tr.rc >> 12) & 0xfff;
-        if (open) {
-          if (lb != c) {
-            acc = acc + d1c * wide(A_2);
-            break;
-          }
-          const double esl = tr.r0.y;
-          acc = acc + tr.r1.y * wide(a2 + R(0.5 * esl) * (a3 - a2 + a4 * R(1.0 - r23 * esl)));
-          emit(narrow(quot(acc, tr.r2.x, tr.r2.y)));
-          open = false;
-        } else if (lt == 0) {
-          emit(narrow(SumT(0.0 / tr.r2.x)));
-        } else if (lt > c) {
-          break;
-        } else {
-          const double pl = tr.r0.x;
-          if (tr.rc >> 24) {
-            const double pr = tr.r0.y, z = pr * (pr + pl) + pl * pl;
-            const T tail = mapn ? T(a4 * R(r3 * z)) : T(a4 * R(r3) * R(z));
-            emit(a2 + (a4 + a3 - a2) * R(0.5 * (pr + pl)) - tail);
+      if (IN || c < km) dof += 2 * nc4;
+      d1n = ldd(dof);
+      if constexpr (decltype(lockstep)::value) {
+        // ---- the targets whose last cell, over the wave's columns, is c
+        cs = cs + 1 == NR ? 0 : cs + 1;
+        T *slot = ring + cs * 192;
+        slot[0] = a2;
+        slot[64] = a3;
+        slot[128] = a4;
+#pragma unroll
+        for (int m = NR - 2; m > 0; m--) M[m] = M[m - 1];
+        M[0] = d1c * wide(A_2);  // c's own; M[m]: cell c-m's
+        while (kt <= km && __ballot(((tr.rc >> 12) & 0xfff) > c) == 0) {
+          const TargetRec t = tr;
+          tr = tn;
+          tn = recat(ro);
+          if (kt + 2 < km) ro += nc4;
+          const int lt = t.rc & 0xfff, lb = (t.rc >> 12) & 0xfff;
+          auto at = [&](int l) -> const T * {
+            const int s = cs - (c - l);
+            return ring + (s < 0 ? s + NR : s) * 192;
+          };
+          const T *x = at(lt);
+          const T x2 = x[0], x3 = x[64], x4 = x[128];
+          T v;
+          if (t.rc >> 24) {
+            v = within(x2, x3, x4, t.r0.x, t.r0.y);
           } else {
-            acc = tr.r1.x * wide(a2 + (a4 + a3 - a2) * R(0.5 * (1.0 + pl)) - a4 * R(r3 * (1.0 + pl * (1.0 + pl))));
+            const T *y = at(lb);
+            const T y2 = y[0], y3 = y[64], y4 = y[128];
+            SumT sum = top_piece(x2, x3, x4, t.r0.x, t.r1.x);
+#pragma unroll
+            for (int m = NR - 2; m > 0; m--)
+              if (lt < c - m && c - m < lb) sum = sum + M[m];
+            sum = sum + bottom_piece(y2, y3, y4, t.r0.y, t.r1.y);
+            v = narrow(quot(sum, t.r2.x, t.r2.y));
+          }
+          if (act) store(du + cbyte, du_t + cbyte, v);
+          du += levb;
+          du_t += levb;
+          kt++;
+        }
+      } else {
+        // ---- the target layers that end, lie or begin in source layer c
+        while (kt <= km) {
+          const int lt = tr.rc & 0xfff, lb = (tr.rc >> 12) & 0xfff;
+          if (open) {
+            if (lb != c) {
+              acc = acc + d1c * wide(A_2);
+              break;
+            }
+            acc = acc + bottom_piece(a2, a3, a4, tr.r0.y, tr.r1.y);
+            emit(narrow(quot(acc, tr.r2.x, tr.r2.y)));
+            open = false;
+          } else if (lt == 0) {
+            emit(narrow(SumT(0.0 / tr.r2.x)));
+          } else if (lt > c) {
+            break;
+          } else if (tr.rc >> 24) {
+            emit(within(a2, a3, a4, tr.r0.x, tr.r0.y));
+          } else {
+            acc = top_piece(a2, a3, a4, tr.r0.x, tr.r1.x);
             open = true;
             break;
           }
         }
       }
+    };
+    for (int p = k0; p <= pend; p++) {
+      if (decltype(lockstep)::value && p >= 5 && p < km)
+        step(p, std::true_type{});
+      else
+        step(p, std::false_type{});
     }
     cur = nxt;
   }
-  // a target that ends below the source, and those no layer holds
-  while (kt <= km) {
-    emit(narrow(open ? quot(acc, tr.r2.x, tr.r2.y) : SumT(0.0 / tr.r2.x)));
-    open = false;
-  }
+  if constexpr (!decltype(lockstep)::value)
+    // a target that ends below the source, and those no layer holds
+    while (kt <= km) {
+      emit(narrow(open ? quot(acc, tr.r2.x, tr.r2.y) : SumT(0.0 / tr.r2.x)));
+      open = false;
+    }
+  };
+  if (__builtin_amdgcn_readfirstlane(a.tab.win[col]) <= NR)
+    sweep(std::true_type{});
+  else
+    sweep(std::false_type{});
 }
 
 template <typename T>
 size_t fields_lds(int km) {
   const int nb = (km + FD_B - 1) / FD_B;
-  return sizeof(T) * FD_WAVES * (size_t)(nb + 2 * FD_B + 4) * 64;
+  return sizeof(T) * FD_WAVES * (size_t)fd_rows<T>(nb) * 64;
 }
 
 }  // namespace
@@ -573,7 +718,7 @@ size_t coltab_bytes(int km, long long ncols) {
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t n = (size_t)km * ncols;
   return al(sizeof(Elim<R>) * n) + al(sizeof(double) * n) + 3 * al(sizeof(double2) * n) + al(sizeof(int) * n) +
-         al(sizeof(R) * 3 * (size_t)ncols);
+         al(sizeof(R) * 3 * (size_t)ncols) + al(sizeof(int) * (size_t)ncols);
 }
 
 template <typename R>
@@ -593,6 +738,7 @@ ColTab<R> coltab_carve(void *base, int km, long long ncols) {
   t.r2 = (double2 *)take(sizeof(double2) * n);
   t.rc = (int *)take(sizeof(int) * n);
   t.bot = (R *)take(sizeof(R) * 3 * (size_t)ncols);
+  t.win = (int *)take(sizeof(int) * (size_t)ncols);
   return t;
 }
 
@@ -645,9 +791,9 @@ int fields_run(Ctx &c, FieldsArgs<T> &a, int ni, int nj) {
   for (int s = 0; s < a.nset; s++) a.nf += a.set[s].count;
   if (a.nf == 0) return 0;
   if (fields_lds<T>(a.km) > 160 * 1024) return set_error("remap of %d levels does not fit in LDS", a.km);
-  a.nfg = (a.nf + FD_WAVES - 1) / FD_WAVES;
-  const long long nwg = (long long)a.ncb * c.ntiles * a.nfg;
-  if (nwg > 0x7fffffffLL) return set_error("remap grid too large");
+  a.ntiles = c.ntiles;
+  const long long nwg = ((long long)a.ncb * c.ntiles * a.nf + FD_WAVES - 1) / FD_WAVES;
+  if (nwg > 0x7fffffffLL / FD_WAVES) return set_error("remap grid too large");
   a.nwg = (unsigned)nwg;
   hipLaunchKernelGGL(k_fields<T>, dim3(a.nwg), dim3(64 * FD_WAVES), fields_lds<T>(a.km), c.stream, a);
   FV3_HIP(hipGetLastError());
