@@ -13,13 +13,14 @@
 // FV3_FORM_PLAIN64 runs every (tile, level) slab of a sub-step in one launch
 // per stage (the staged transport's stage kernels, in the FP64 oracle's
 // operation order); FV3_FORM_FUSED64 / FUSED32 run a whole sub-step in one
-// launch of blocks that keep every intermediate in LDS, with the same
-// expressions, so both FP64 forms match the oracle bit for bit.
+// launch that streams rows and keeps every intermediate in registers, with the
+// same expressions, so both FP64 forms match the oracle bit for bit.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 
 #include "../../include/fv3atm_amd.h"
+#include "fused_tp.h"
 #include "fv3_internal.h"
 
 namespace fv3 {
@@ -59,204 +60,358 @@ struct ColQ {
 
 
 // ---- one acoustic sub-step in one launch ---------------------------------------
-// A workgroup owns a TX x TY block of one (tile, level) slab and computes every
-// stage of the sub-step for it in LDS, reading delp (with its 3-cell halo),
-// the sub-step's winds and the metrics once: the Courant numbers and area
-// fluxes, the inner y-sweep of delp and q_i, the outer x-sweep, the inner
-// x-sweep and q_j, the outer y-sweep, the flux averages, the accumulations
-// and the delp update.  Each quantity is the same expression as in the stage
-// kernels above, so the FP64 form rounds as they do.  delp is read from one
-// buffer and written to another (a neighbouring block still reads the old
-// values as its halo); the halo cells are carried over, and the corner-block
-// cells get their x-sweep (dir 1) copy_corners sources, as the stages leave
-// them in place.
+// A wave owns a strip of DYN_W columns and a block of rows of one (tile, level)
+// slab, one lane per column (three more on each side), and streams over the
+// rows: a row's x-side (Courant numbers and area fluxes, the inner x-sweep,
+// q_j) when it is loaded, the y-faces two rows behind it (Courant numbers,
+// inner and outer y-sweep, the y-fluxes), and three rows behind it q_i, the
+// outer x-sweep, the x-fluxes and the delp update.  Neighbours in x come from
+// the neighbouring lanes (DPP), neighbours in y from rows kept in registers, so
+// that each slope, face value and cell limiter is computed once per cell and
+// sweep, and nothing goes through LDS.  Each quantity is the same expression as
+// in the stage kernels, so the FP64 form rounds as they do.  The next row's
+// loads are issued before a row is worked on; the four waves of a workgroup
+// take four levels, whose metric loads hit the same lines.  Cube edges: rows at
+// the y-edges by uniform branches, columns at the x-edges in a second form of
+// the row loop for the strips that hold some.  Bound by VALU issue (85% busy in
+// FP32).  C384 L127, per sub-step: 335 us in FP32, 640 in FP64; 32 x 16 (FP64
+// 32 x 8) blocks in LDS, each face recomputing its cell's slopes and limiter
+// from there, took 940 and 1500 us.  delp is read from one buffer and written to another (a
+// neighbouring wave still reads the old values as its halo); the halo cells are
+// carried over, and the corner-block cells get their x-sweep (dir 1)
+// copy_corners sources, as the stages leave them in place.
 struct DynSubArgs {
   Dims d;
-  int npz, ord_in, ord_ou, first;
+  int npz, nz, ord_in, ord_ou, first, rows;  // rows: per block
   long long gs2, gdx, gdy;
 };
 
-template <typename T, int TX, int TY>
-struct DynTile {
-  static constexpr int C = TX + 6, R = TY + 6;  // delp block with its halo: columns i0-3 .. i1+3
-  static constexpr int FX = TX + 1;             // x-faces i0 .. i1+1
-  static constexpr int FY = TY + 1;             // y-faces j0 .. j1+1
-  T py[R * C], px[R * C];                       // delp with the y- (dir 2) and x-sweep (dir 1) corners
-  T crx[R * FX], xfx[R * FX], fx2[R * FX];      // x-faces of rows j0-3 .. j1+3
-  T cry[FY * C], yfx[FY * C];                   // y-faces of columns i0-3 .. i1+3
-  T fy2[FY * C];                                // y-faces of columns i0-3 .. i1+3
-  T qi[TY * C];                                 // rows j0 .. j1, columns i0-3 .. i1+3
-  T fx[TY * FX];                                // x-faces of rows j0 .. j1
-  T qj[R * TX];                                 // rows j0-3 .. j1+3, columns i0 .. i1
-  T fy[FY * TX];                                // y-faces of columns i0 .. i1
+constexpr int DYN_W = 58;
+
+// cells m-2 .. m+2 of a sweep line, cell m at index 2
+template <typename T>
+struct Win5 {
+  T v[5];
+  __device__ __forceinline__ T operator()(int k) const { return v[k]; }
+};
+
+// place of cell m on a sweep line: 0 inner, 1 .. 3 cells 0, 1, 2 of an edge,
+// 4 .. 6 cells npx-2, npx-1, npx
+__device__ __forceinline__ int edge_place(const LineGeom &g, int m) {
+  if (!g.edge) return 0;
+  if (g.is == 1 && m <= 2) return m == 0 ? 1 : (m == 1 ? 2 : 3);
+  if (g.ie + 1 == g.npx && m >= g.npx - 2) return m == g.npx - 2 ? 4 : (m == g.npx - 1 ? 5 : 6);
+  return 0;
+}
+
+// The expressions of ppm_dm, ppm_al, ppm_edge_face and ppm_cell, with minima
+// and maxima as instructions: two thirds of a sweep's compares and selects.
+template <typename T>
+__device__ __forceinline__ T slope(T qm, T q, T qp) {
+  const T xt = T(0.25) * (qp - qm);
+  return fsign(fmn3(fabs(xt), fmx3(qm, q, qp) - q, q - fmn3(qm, q, qp)), xt);
+}
+template <typename T>
+__device__ __forceinline__ T face(T ql, T q, T dml, T dm) {
+  return T(0.5) * (ql + q) + K<T>::r3 * (dml - dm);
+}
+// the cube-edge face between cells 1 and 2 of four (their spacings: d)
+template <typename T>
+__device__ __forceinline__ T edge_face(T q0, T q1, T q2, T q3, T d0, T d1, T d2, T d3) {
+  const T xt = T(0.5) * (((T(2) * d1 + d0) * q1 - d1 * q0) / (d0 + d1) + ((T(2) * d2 + d3) * q2 - d2 * q3) / (d2 + d3));
+  return fmn(fmx(xt, fmn(fmn3(q0, q1, q2), q3)), fmx(fmx3(q0, q1, q2), q3));
+}
+
+// (bl, br) of an inner cell: orders 8 and 11 from its slope and its two face
+// values, the others from the window
+template <bool O8, typename T>
+__device__ __forceinline__ void inner_cell(const Win5<T> &q, T dm, T al, T ar, int iord, T &bl, T &br) {
+  if (O8 || iord == 8 || iord == 11) {
+    const T xt = iord == 8 ? T(2) * dm : K<T>::ppm_fac * dm;
+    bl = -fsign(fmn(fabs(xt), fabs(al - q(2))), xt);
+    br = fsign(fmn(fabs(xt), fabs(ar - q(2))), xt);
+  } else {
+    ppm_cell<T>(q, q, 2, LineGeom{0, 0, 0, false}, iord, bl, br);
+  }
+}
+
+// (bl, br) of an edge cell from its face values, the slopes beside it and the
+// cells beside it
+template <typename T>
+__device__ __forceinline__ void edge_cell(int place, T qm, T q, T qp, T al, T ar, T dml, T dmr, T &bl, T &br) {
+  bl = place == 1 ? K<T>::s14 * dml + K<T>::s11 * (qm - q) : al - q;
+  br = place == 6 ? K<T>::s11 * (qp - q) - K<T>::s14 * dmr : ar - q;
+  pert_ppm1(q, bl, br, 1);
+}
+
+// flux through a face between cells l and r for Courant number c
+template <typename T>
+__device__ __forceinline__ T upwind(T c, T ql, T bll, T brl, T qr, T blr, T brr) {
+  const bool pos = c > T(0);
+  const T b = pos ? bll + brl : blr + brr, a = pos ? brl : blr, q = pos ? ql : qr, s = pos ? c : -c;
+  return q + (T(1) - s) * (a - s * b);
+}
+
+// One y-line per lane, a row at a time: after add(r) the window holds rows
+// r-4 .. r and (bl, br) belong to row r-2, (blp, brp) to row r-3.  The face
+// values next to a cube edge replace the inner ones.
+template <typename T, bool O8>
+struct YLine {
+  Win5<T> q;
+  T dm0, dm1, al, bl, br, blp, brp;  // slopes of rows r-3, r-2; face value of row r-2
+  template <typename D>
+  __device__ __forceinline__ void add(T v, const LineGeom &g, int r, const D &spacing, int iord) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) q.v[k] = q.v[k + 1];
+    q.v[4] = v;
+    const T dm2 = slope<T>(q(2), q(3), q(4));  // of row r-1
+    T ar = face<T>(q(2), q(3), dm1, dm2);      // of face r-1
+    const int f = r - 1;
+    int place = 0;
+    if (g.edge && ((g.is == 1 && f <= 3) || (g.ie + 1 == g.npx && f >= g.npx - 1))) {
+      place = edge_place(g, r - 2);
+      const bool lo = g.is == 1 && f <= 3;
+      if (f == (lo ? 1 : g.npx)) {
+        const Win5<T> d = spacing();  // of rows r-3 .. r
+        ar = edge_face<T>(q(1), q(2), q(3), q(4), d(0), d(1), d(2), d(3));
+      } else if (lo && f == 2) {
+        ar = K<T>::s15 * q(2) + K<T>::s11 * q(3) - K<T>::s14 * dm2;
+      } else if (!lo && f == g.npx - 1) {
+        ar = K<T>::s15 * q(3) + K<T>::s11 * q(2) + K<T>::s14 * dm1;
+      }
+    }
+    blp = bl;
+    brp = br;
+    if (place)
+      edge_cell<T>(place, q(1), q(2), q(3), al, ar, dm0, dm2, bl, br);
+    else
+      inner_cell<O8, T>(q, dm1, al, ar, iord, bl, br);
+    dm0 = dm1;
+    dm1 = dm2;
+    al = ar;
+  }
+  __device__ __forceinline__ T flux(T c) const { return upwind<T>(c, q(1), blp, brp, q(2), bl, br); }
 };
 
 template <typename T>
-struct LdsLine {  // cells of one LDS line indexed by their global index
-  const T *p;
-  int lo, stride;
-  __device__ __forceinline__ T operator()(int m) const { return p[(m - lo) * stride]; }
+struct DynRow {
+  T p, u, dxa, sg0, sg2, dy, area, cx;  // row r
+  T v, dx, dya, sg1, sg3, cy, mfy;      // y-faces (and cells) r-2
+  T mfx, areaj, rarea;                  // row r-3
+  __device__ __forceinline__ void arrived() {
+    asm volatile("" : "+v"(p), "+v"(u), "+v"(dxa), "+v"(sg0), "+v"(sg2), "+v"(dy), "+v"(area), "+v"(cx));
+    asm volatile("" : "+v"(v), "+v"(dx), "+v"(dya), "+v"(sg1), "+v"(sg3), "+v"(cy), "+v"(mfy));
+    asm volatile("" : "+v"(mfx), "+v"(areaj), "+v"(rarea));
+  }
 };
 
-template <typename T, int TX, int TY>
-__global__ void __launch_bounds__(256) k_dyn_sub(const DynSubArgs a, const GridDev<T> g, T bdt, const T *u,
-                                                 const T *v, const T *din, T *dout, T *cx, T *cy, T *mfx, T *mfy) {
-  using TL = DynTile<T, TX, TY>;
-  constexpr int C = TL::C, R = TL::R, FX = TL::FX, FY = TL::FY;
-  extern __shared__ __align__(16) unsigned char dyn_lds[];
-  TL &L = *reinterpret_cast<TL *>(dyn_lds);
+template <typename T, bool O8>  // O8: both orders are 8 or 11
+__global__ void __launch_bounds__(256) k_dyn_sub(const DynSubArgs a, const GridDev<T> g, T bdt,
+                                                 const T *__restrict__ u, const T *__restrict__ v,
+                                                 const T *__restrict__ din, T *__restrict__ dout, T *cx, T *cy, T *mfx,
+                                                 T *mfy) {
   const Dims &d = a.d;
-  const int tid = threadIdx.x, z = blockIdx.z, tile = z / a.npz;
-  const int i0 = d.is + (int)blockIdx.x * TX, j0 = d.js + (int)blockIdx.y * TY;
-  const int i1 = min(i0 + TX - 1, d.ie), j1 = min(j0 + TY - 1, d.je);
-  const T *dl = din + (long long)z * d.s2;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int z = (int)blockIdx.x * 4 + wave;
+  if (z >= a.nz) return;  // whole wave; no barriers below
+  const int tile = z / a.npz;
+  const int i0 = d.is + (int)blockIdx.y * DYN_W, i1 = min(i0 + DYN_W - 1, d.ie);
+  const int j0 = d.js + (int)blockIdx.z * a.rows, j1 = min(j0 + a.rows - 1, d.je);
+  const int i = i0 - 3 + lane;
   const LineGeom gx{d.is, d.ie, d.npx, d.edge}, gy{d.js, d.je, d.npy, d.edge};
+  // lanes past the slab repeat its last column and store nothing
+  const int oc = min(i, d.ied) - d.isd, of = min(max(i, d.is), d.ie + 1) - d.is, om = min(max(i, d.is), d.ie) - d.is;
+  const T *dl = din + (long long)z * d.s2;
+  T *dw = dout + (long long)z * d.s2;
   const long long gt = tile * a.gs2;
-  auto cell = [&](int i, int j) { return (long long)(j - d.jsd) * d.nid + (i - d.isd); };
-  auto in_dom = [&](int i, int j) { return i >= d.isd && i <= d.ied && j >= d.jsd && j <= d.jed; };
-  // only blocks whose halo reaches a cube corner have copy_corners cells
-  const bool corner_blk = !d.bounded && (i0 - 3 <= 0 || i1 + 3 >= d.npx) && (j0 - 3 <= 0 || j1 + 3 >= d.npy);
+  const T *dxa = g.dxa + gt, *dya = g.dya + gt, *area = g.area + gt, *rarea = g.rarea + gt;
+  const T *sg = g.sin_sg + tile * 9 * a.gs2, *dx = g.dx + tile * a.gdx, *dy = g.dy + tile * a.gdy;
+  const T *sg1 = sg + a.gs2, *sg2 = sg + 2 * a.gs2, *sg3 = sg + 3 * a.gs2;
+  u += (long long)z * d.sx;
+  v += (long long)z * d.sy;
+  cx += (long long)z * d.sx;
+  cy += (long long)z * d.sy;
+  mfx += (long long)z * d.smx;
+  mfy += (long long)z * d.smy;
+  const bool first = a.first != 0;
+  const bool x_edge = d.edge && ((d.is == 1 && i0 - 3 <= 2) || (d.ie + 1 == d.npx && i1 + 3 >= d.npx - 2));
+  const bool corner_strip = !d.bounded && (i0 - 3 <= 0 || i1 + 3 >= d.npx);
+  const int x_place = edge_place(gx, i);
+  // faces next to an edge: 1 the edge's own, 2 and 3 the ones one cell inside
+  const bool x_lo = d.is == 1, x_hi = d.ie + 1 == d.npx;
+  const int x_face = (x_lo && i == 1) || (x_hi && i == d.npx) ? 1 : x_lo && i == 2 ? 2 : x_hi && i == d.npx - 1 ? 3 : 0;
+  const bool own_x = i >= i0 && i <= i1;                                      // cells
+  const bool own_xf = own_x || (i == d.ie + 1 && i1 == d.ie);                 // x-faces
+  const bool own_xh = own_x || (i < d.is && i0 == d.is) || (i > d.ie && i <= d.ied && i1 == d.ie);  // with the halo
+  auto left = [](T x) { return from_left(x); };
+  auto right = [](T x) { return from_right(x); };
 
-  // ---- delp block (both corner versions)
-  for (int e = tid; e < R * C; e += 256) {
-    const int r = e / C, c = e % C, i = i0 - 3 + c, j = j0 - 3 + r;
-    T vy = T(0), vx = T(0);
-    if (in_dom(i, j)) {
-      vy = vx = dl[cell(i, j)];
-      int si, sj;
-      if (corner_blk) {
-        if (corner_src(i, j, d.npx, d.npy, 2, d.corners, si, sj)) vy = dl[cell(si, sj)];
-        if (corner_src(i, j, d.npx, d.npy, 1, d.corners, si, sj)) vx = dl[cell(si, sj)];
+  // scalar bases and 32-bit lane offsets in bytes
+  constexpr unsigned B = sizeof(T);
+  const unsigned lc = (unsigned)oc * B, lf = (unsigned)of * B, lm = (unsigned)om * B;
+  const unsigned rc = (unsigned)d.nid * B, rf = (unsigned)d.nix * B, rm = (unsigned)d.niy * B;
+  auto at = [](const T *p, unsigned o) -> T { return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + o); };
+  auto put = [](T *p, unsigned o, T x) { *reinterpret_cast<T *>(reinterpret_cast<char *>(p) + o) = x; };
+  auto load = [&](int r, DynRow<T> &w) {
+    const unsigned rr = (unsigned)(min(r, d.jed) - d.jsd);
+    const unsigned o = rr * rc + lc, ou = rr * rf + lf;
+    w.p = at(dl, o);
+    w.u = at(u, ou);
+    w.dxa = at(dxa, o);
+    w.sg0 = at(sg, o);
+    w.sg2 = at(sg2, o);
+    w.area = at(area, o);
+    w.dy = at(dy, o + rr * B);
+    const unsigned of2 = (unsigned)(max(r - 2, d.jsd) - d.jsd) * rc + lc;  // r-2 <= je+1
+    const unsigned f = (unsigned)(min(max(r - 2, d.js), d.je + 1) - d.js), ov = f * rc + lc;
+    w.v = at(v, ov);
+    w.dx = at(dx, of2);
+    w.dya = at(dya, of2);
+    w.sg1 = at(sg1, of2);
+    w.sg3 = at(sg3, of2);
+    const unsigned j = (unsigned)(min(max(r - 3, d.js), d.je) - d.js), oj = (j + (unsigned)(d.js - d.jsd)) * rc + lc;
+    w.areaj = at(area, oj);
+    w.rarea = at(rarea, oj);
+    if (!first) {
+      w.cx = at(cx, ou);
+      w.cy = at(cy, ov);
+      w.mfy = at(mfy, f * rm + lm);
+      w.mfx = at(mfx, j * rf + lf);
+    }
+  };
+  // flux through x-face i of the row whose cells (and spacings dr) the lanes hold
+  auto x_flux = [&](auto edge, T q, T c, T dr, int iord) -> T {
+    constexpr bool XE = decltype(edge)::value;
+    const T qm = left(q), qp = right(q), qmm = left(qm);
+    const T dm = slope<T>(qm, q, qp), dml = left(dm);
+    T al = face<T>(qm, q, dml, dm), bl, br;
+    if constexpr (XE) {
+      const T d1 = left(dr), e = edge_face<T>(qmm, qm, q, qp, left(d1), d1, dr, right(dr));
+      al = x_face == 1 ? e
+           : x_face == 2 ? K<T>::s15 * qm + K<T>::s11 * q - K<T>::s14 * dm
+           : x_face == 3 ? K<T>::s15 * q + K<T>::s11 * qm + K<T>::s14 * dml : al;
+    }
+    const T ar = right(al);
+    inner_cell<O8, T>(Win5<T>{{qmm, qm, q, qp, right(qp)}}, dm, al, ar, iord, bl, br);
+    if constexpr (XE) {
+      const T dmr = right(dm);
+      if (x_place) edge_cell<T>(x_place, qm, q, qp, al, ar, dml, dmr, bl, br);
+    }
+    return upwind<T>(c, qm, left(bl), left(br), q, bl, br);
+  };
+
+  auto rows = [&](auto edge) {  // edge: the strip holds columns of a cube edge
+    DynRow<T> w, nx;
+    w.cx = w.cy = w.mfx = w.mfy = T(0);
+    nx = w;
+    YLine<T, O8> yp{}, yq{};                         // delp, q_j
+    T c1 = T(0), c2 = T(0), c3 = T(0);               // x-Courant numbers of rows r-1, r-2, r-3
+    T x1 = T(0), x2 = T(0), x3 = T(0);               // their area fluxes
+    T e1 = T(0), e2 = T(0), e3 = T(0);               // their inner x-fluxes
+    T d1 = T(1), d2 = T(1), d3 = T(1);               // their spacings
+    T dya_m = T(0), sg3_m = T(0);                    // of cell row f-1
+    T yf_m = T(0), fyi_m = T(0), fy_m = T(0);        // area flux, inner and total flux of face f-1
+    load(j0 - 3, nx);
+    for (int r = j0 - 3; r <= j1 + 3; r++) {
+      w = nx;
+      if (r < j1 + 3) load(r + 1, nx);
+      // ---- row r
+      T py = w.p, px = w.p;
+      if (corner_strip && (r <= 0 || r >= d.npy)) {
+        int si, sj;
+        if (corner_src(i, r, d.npx, d.npy, 2, d.corners, si, sj)) py = dl[(sj - d.jsd) * d.nid + (si - d.isd)];
+        if (corner_src(i, r, d.npx, d.npy, 1, d.corners, si, sj)) px = dl[(sj - d.jsd) * d.nid + (si - d.isd)];
+      }
+      const bool own_y = r >= j0 && r <= j1;
+      const bool own_yh = own_y || (r < d.js && j0 == d.js) || (r > d.je && j1 == d.je);
+      const bool upl = w.u > T(0);
+      const T da_l = left(w.dxa), sg_l = left(w.sg2);
+      const T dax = upl ? da_l : w.dxa;
+      const T c0 = bdt * w.u / dax;
+      const T x0 = c0 * dax * w.dy * (upl ? sg_l : w.sg0);
+      const T e0 = x_flux(edge, px, c0, w.dxa, a.ord_in);
+      const T fa = x0 * e0, xr = right(x0), fb = right(fa);
+      const T qj = (px * w.area + fa - fb) / (w.area + x0 - xr);
+      // ---- cell row r-2 of the y-lines, y-face f = r-2
+      auto spacing = [&]() {
+        Win5<T> s;
+#pragma unroll
+        for (int k = 0; k < 4; k++) s.v[k] = dya[(r - 3 + k - d.jsd) * d.nid + oc];
+        s.v[4] = s.v[3];
+        return s;
+      };
+      yp.add(py, gy, r, spacing, a.ord_in);
+      yq.add(qj, gy, r, spacing, a.ord_ou);
+      const int f = r - 2, j = r - 3;
+      T cr = T(0), fy = T(0), fx = T(0), dp = T(0);
+      if (f >= j0) {
+        const bool up = w.v > T(0);
+        const T day = up ? dya_m : w.dya;
+        cr = bdt * w.v / day;
+        const T yf = cr * day * w.dx * (up ? sg3_m : w.sg1);
+        const T fyi = yp.flux(cr);
+        fy = T(0.5) * (yq.flux(cr) + fyi) * yf;
+        // ---- row j = r-3: q_i, the outer x-sweep, delp
+        const T qi = (yp.q(1) * w.areaj + yf_m * fyi_m - yf * fyi) / (w.areaj + yf_m - yf);
+        fx = T(0.5) * (x_flux(edge, qi, c3, d3, a.ord_ou) + e3) * x3;
+        dp = yp.q(1) + ((fx - right(fx)) + (fy_m - fy)) * w.rarea;
+        yf_m = yf;
+        fyi_m = fyi;
+        fy_m = fy;
+      }
+      dya_m = w.dya;
+      sg3_m = w.sg3;
+      c3 = c2;
+      c2 = c1;
+      c1 = c0;
+      x3 = x2;
+      x2 = x1;
+      x1 = x0;
+      e3 = e2;
+      e2 = e1;
+      e1 = e0;
+      d3 = d2;
+      d2 = d1;
+      d1 = w.dxa;
+      // ---- results.  The wait for the next row's loads is put here: after the
+      // stores it would include them, since both are counted in order
+      const T cxv = w.cx + c0, cyv = w.cy + cr, mxv = w.mfx + fx, myv = w.mfy + fy;
+      nx.arrived();
+      const bool own_f = f >= j0 && (f <= j1 || (f == d.je + 1 && j1 == d.je));
+      if (own_yh && own_xf) put(cx, (unsigned)(r - d.jsd) * rf + lf, cxv);
+      if (own_yh && own_xh && !(own_y && i >= d.is && i <= d.ie)) put(dw, (unsigned)(r - d.jsd) * rc + lc, px);
+      if (own_f) {
+        if (own_xh) put(cy, (unsigned)(f - d.js) * rc + lc, cyv);
+        if (own_x) put(mfy, (unsigned)(f - d.js) * rm + lm, myv);
+      }
+      if (j >= j0) {
+        if (own_xf) put(mfx, (unsigned)(j - d.js) * rf + lf, mxv);
+        if (own_x) put(dw, (unsigned)(j - d.jsd) * rc + lc, dp);
       }
     }
-    L.py[e] = vy;
-    L.px[e] = vx;
-  }
-  // ---- Courant numbers and area fluxes with the upwind metric; cx, cy accumulate
-  for (int e = tid; e < R * FX; e += 256) {
-    const int r = e / FX, f = e % FX, i = i0 + f, j = j0 - 3 + r;
-    if (i > d.ie + 1 || j < d.jsd || j > d.jed) continue;
-    const long long lv = (long long)z * d.sx + (long long)(j - d.jsd) * d.nix + (i - d.is);
-    // both upwind candidates, so that no address depends on the loaded wind
-    const T w = u[lv];
-    const T da_l = g.dxa[gt + cell(i - 1, j)], da_r = g.dxa[gt + cell(i, j)];
-    const T sg_l = g.sin_sg[tile * 9 * a.gs2 + 2 * a.gs2 + cell(i - 1, j)];
-    const T sg_r = g.sin_sg[tile * 9 * a.gs2 + cell(i, j)];
-    const T dyf = g.dy[tile * a.gdy + (long long)(j - d.jsd) * (d.nid + 1) + (i - d.isd)];
-    const bool pos = w > T(0);
-    const T dau = pos ? da_l : da_r;
-    const T cr = bdt * w / dau;
-    L.crx[e] = cr;
-    L.xfx[e] = cr * dau * dyf * (pos ? sg_l : sg_r);
-    // rows and faces this block owns: its own, the halo rows at the domain edges, face ie+1
-    const bool own_j = (j >= j0 && j <= j1) || (j < d.js && j0 == d.js) || (j > d.je && j1 == d.je);
-    const bool own_i = i <= i1 || (i == d.ie + 1 && i1 == d.ie);
-    if (own_j && own_i) cx[lv] = a.first ? T(0) + cr : cx[lv] + cr;
-  }
-  for (int e = tid; e < FY * C; e += 256) {
-    const int f = e / C, c = e % C, i = i0 - 3 + c, j = j0 + f;
-    if (j > d.je + 1 || i < d.isd || i > d.ied) continue;
-    const long long lv = (long long)z * d.sy + (long long)(j - d.js) * d.nid + (i - d.isd);
-    const T w = v[lv];
-    const T da_l = g.dya[gt + cell(i, j - 1)], da_r = g.dya[gt + cell(i, j)];
-    const T sg_l = g.sin_sg[tile * 9 * a.gs2 + 3 * a.gs2 + cell(i, j - 1)];
-    const T sg_r = g.sin_sg[tile * 9 * a.gs2 + 1 * a.gs2 + cell(i, j)];
-    const T dxf = g.dx[tile * a.gdx + (long long)(j - d.jsd) * d.nid + (i - d.isd)];
-    const bool pos = w > T(0);
-    const T dau = pos ? da_l : da_r;
-    const T cr = bdt * w / dau;
-    L.cry[e] = cr;
-    L.yfx[e] = cr * dau * dxf * (pos ? sg_l : sg_r);
-    const bool own_i = (i >= i0 && i <= i1) || (i < d.is && i0 == d.is) || (i > d.ie && i1 == d.ie);
-    const bool own_j = j <= j1 || (j == d.je + 1 && j1 == d.je);
-    if (own_i && own_j) cy[lv] = a.first ? T(0) + cr : cy[lv] + cr;
-  }
-  __syncthreads();
-  // ---- inner sweeps: y over delp (dir 2 corners) at faces j0 .. j1+1 of
-  // columns i0-3 .. i1+3, x over delp (dir 1) at faces i0 .. i1+1 of rows j0-3 .. j1+3
-  for (int e = tid; e < FY * C; e += 256) {
-    const int f = e / C, c = e % C, i = i0 - 3 + c, j = j0 + f;
-    if (j > j1 + 1 || i < d.isd || i > d.ied) continue;
-    const LdsLine<T> qa{L.py + c, j0 - 3, C};
-    const ColQ<T> da{g.dya + gt + (i - d.isd), d.jsd, d.nid};
-    L.fy2[e] = ppm_flux<T>(qa, da, j, L.cry[e], gy, a.ord_in);
-  }
-  for (int e = tid; e < R * FX; e += 256) {
-    const int r = e / FX, f = e % FX, i = i0 + f, j = j0 - 3 + r;
-    if (i > i1 + 1 || j < d.jsd || j > d.jed) continue;
-    const LdsLine<T> qa{L.px + r * C, i0 - 3, 1};
-    const RowQ<T> da{g.dxa + gt + (long long)(j - d.jsd) * d.nid, d.isd};
-    L.fx2[e] = ppm_flux<T>(qa, da, i, L.crx[e], gx, a.ord_in);
-  }
-  __syncthreads();
-  // ---- q_i at rows j0 .. j1, columns i0-3 .. i1+3; q_j at rows j0-3 .. j1+3, columns i0 .. i1
-  for (int e = tid; e < TY * C; e += 256) {
-    const int r = e / C, c = e % C, i = i0 - 3 + c, j = j0 + r;
-    if (j > j1 || i < d.isd || i > d.ied) continue;
-    const T ya = L.yfx[r * C + c], yb = L.yfx[(r + 1) * C + c];
-    const T fa = ya * L.fy2[r * C + c], fb = yb * L.fy2[(r + 1) * C + c];
-    const T ar = g.area[gt + cell(i, j)];
-    L.qi[e] = (L.py[(r + 3) * C + c] * ar + fa - fb) / (ar + ya - yb);
-  }
-  for (int e = tid; e < R * TX; e += 256) {
-    const int r = e / TX, c = e % TX, i = i0 + c, j = j0 - 3 + r;
-    if (i > i1 || j < d.jsd || j > d.jed) continue;
-    const T xa = L.xfx[r * FX + c], xb = L.xfx[r * FX + c + 1];
-    const T fa = xa * L.fx2[r * FX + c], fb = xb * L.fx2[r * FX + c + 1];
-    const T ar = g.area[gt + cell(i, j)];
-    L.qj[e] = (L.px[r * C + c + 3] * ar + fa - fb) / (ar + xa - xb);
-  }
-  __syncthreads();
-  // ---- outer sweeps (x over q_i, y over q_j), averaged with the inner ones
-  // and the area fluxes; mfx, mfy accumulate
-  for (int e = tid; e < TY * FX; e += 256) {
-    const int r = e / FX, f = e % FX, i = i0 + f, j = j0 + r;
-    if (i > i1 + 1 || j > j1) continue;
-    const LdsLine<T> qa{L.qi + r * C, i0 - 3, 1};
-    const RowQ<T> da{g.dxa + gt + (long long)(j - d.jsd) * d.nid, d.isd};
-    const T fo = ppm_flux<T>(qa, da, i, L.crx[(r + 3) * FX + f], gx, a.ord_ou);
-    const T fl = T(0.5) * (fo + L.fx2[(r + 3) * FX + f]) * L.xfx[(r + 3) * FX + f];
-    L.fx[e] = fl;
-    if (i <= i1 || i == d.ie + 1) {
-      const long long o = (long long)z * d.smx + (long long)(j - d.js) * d.nix + (i - d.is);
-      mfx[o] = a.first ? T(0) + fl : mfx[o] + fl;
+  };
+  if (x_edge)
+    rows(std::true_type{});
+  else
+    rows(std::false_type{});
+}
+
+// Rows per block: longer blocks repeat fewer of the six rows that a block
+// shares with its neighbours, shorter ones give more waves.  Waves that all fit
+// at once take the time of one; beyond that the last ones to start add half a
+// block's time on average.
+int dyn_rows(int nj, long long lines, long long slots) {
+  int best = 48;
+  double least = 0.0;
+  for (int rows = 48; rows >= 4; rows -= 4) {
+    const double x = (double)(lines * ((nj + rows - 1) / rows)) / (double)slots;
+    const double t = (rows + 6) * (x <= 1.0 ? 1.0 : x + 0.5);
+    if (rows == 48 || t < least) {
+      least = t;
+      best = rows;
     }
   }
-  for (int e = tid; e < FY * TX; e += 256) {
-    const int f = e / TX, c = e % TX, i = i0 + c, j = j0 + f;
-    if (i > i1 || j > j1 + 1) continue;
-    const LdsLine<T> qa{L.qj + c, j0 - 3, TX};
-    const ColQ<T> da{g.dya + gt + (i - d.isd), d.jsd, d.nid};
-    const T fo = ppm_flux<T>(qa, da, j, L.cry[f * C + c + 3], gy, a.ord_ou);
-    const T fl = T(0.5) * (fo + L.fy2[f * C + c + 3]) * L.yfx[f * C + c + 3];
-    L.fy[e] = fl;
-    if (j <= j1 || j == d.je + 1) {
-      const long long o = (long long)z * d.smy + (long long)(j - d.js) * d.niy + (i - d.is);
-      mfy[o] = a.first ? T(0) + fl : mfy[o] + fl;
-    }
-  }
-  __syncthreads();
-  // ---- delp: the block's cells by the flux divergence; its share of the halo
-  // carried over (corner blocks with their dir 1 sources)
-  T *dw = dout + (long long)z * d.s2;
-  for (int e = tid; e < R * C; e += 256) {
-    const int r = e / C, c = e % C, i = i0 - 3 + c, j = j0 - 3 + r;
-    if (!in_dom(i, j)) continue;
-    const bool inner = i >= i0 && i <= i1 && j >= j0 && j <= j1;
-    if (inner) {
-      const int ri = j - j0, ci = i - i0;
-      dw[cell(i, j)] = L.py[e] + ((L.fx[ri * FX + ci] - L.fx[ri * FX + ci + 1]) +
-                                  (L.fy[ri * TX + ci] - L.fy[(ri + 1) * TX + ci])) *
-                                     g.rarea[gt + cell(i, j)];
-    } else {
-      // halo cells of the slab, each written by the one block whose range
-      // (extended to the slab edge on the sides where it touches it) holds it
-      const bool hi_ok = (i >= i0 && i <= i1) || (i < d.is && i0 == d.is) || (i > d.ie && i1 == d.ie);
-      const bool hj_ok = (j >= j0 && j <= j1) || (j < d.js && j0 == d.js) || (j > d.je && j1 == d.je);
-      const bool halo = i < d.is || i > d.ie || j < d.js || j > d.je;
-      if (halo && hi_ok && hj_ok) dw[cell(i, j)] = L.px[e];
-    }
-  }
+  return best;
 }
 
 }  // namespace
@@ -448,8 +603,6 @@ static int dyn_core_fluxes(Ctx &c, int n_split, T bdt, int hord, const T *uc, co
 template <typename T>
 static int dyn_core_fluxes_fused(Ctx &c, int n_split, T bdt, int hord, const T *uc, const T *vc, T *delp, T *dp1,
                                  T *cx, T *cy, T *mfx, T *mfy, hipStream_t s) {
-  constexpr int TX = 32, TY = sizeof(T) == 8 ? 8 : 16;
-  using TL = DynTile<T, TX, TY>;
   const Dims d = c.d;
   const int npz = c.npz, nt = c.ntiles, nz = npz * nt;
   const GridDev<T> g = grid_of<T>(c);
@@ -460,20 +613,26 @@ static int dyn_core_fluxes_fused(Ctx &c, int n_split, T bdt, int hord, const T *
   DynSubArgs a{};
   a.d = d;
   a.npz = npz;
+  a.nz = nz;
   a.ord_in = hord == 10 ? 8 : hord;
   a.ord_ou = hord;
   a.gs2 = g.s2;
   a.gdx = g.sdx;
   a.gdy = g.sdy;
   const int ni = d.ie - d.is + 1, nj = d.je - d.js + 1;
-  const dim3 grid((unsigned)((ni + TX - 1) / TX), (unsigned)((nj + TY - 1) / TY), (unsigned)nz);
+  const int strips = (ni + DYN_W - 1) / DYN_W;
+  // waves on the chip at once: two per SIMD by registers in FP64, four in FP32
+  a.rows = dyn_rows(nj, (long long)strips * nz, 1024 * (sizeof(T) == 8 ? 2 : 4));
+  const dim3 grid((unsigned)((nz + 3) / 4), (unsigned)strips, (unsigned)((nj + a.rows - 1) / a.rows));
   T *buf[2] = {delp, alt};
   for (int it = 0; it < n_split; it++) {
     a.first = it == 0;
     const T *u = uc + (long long)it * nz * d.sx, *v = vc + (long long)it * nz * d.sy;
     T *din = buf[it & 1], *dout = buf[(it + 1) & 1];
-    hipLaunchKernelGGL((k_dyn_sub<T, TX, TY>), grid, dim3(256), sizeof(TL), s, a, g, bdt, u, v, din, dout, cx, cy,
-                       mfx, mfy);
+    if (hord == 8 || hord == 11)
+      hipLaunchKernelGGL((k_dyn_sub<T, true>), grid, dim3(256), 0, s, a, g, bdt, u, v, din, dout, cx, cy, mfx, mfy);
+    else
+      hipLaunchKernelGGL((k_dyn_sub<T, false>), grid, dim3(256), 0, s, a, g, bdt, u, v, din, dout, cx, cy, mfx, mfy);
     FV3_HIP(hipGetLastError());
     if (nt > 1 && it + 1 < n_split)
       if (halo_fill<T>(c, dout, (long long)npz * d.s2, nullptr, 0, npz)) return 1;
