@@ -181,17 +181,6 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     sc64 += b_xf + b_yf;
     q_tmp64 = (T *)sc64;
   }
-  if (device_nsplit<T>(c, cx, cy, c.step_per_level, c.step_per_level ? 0 : c.step_q_split, cmax, nspl, frac, xfx, yfx))
-    return 1;
-  int cap = nsplit_cap;
-  if (cap <= 0) {
-    std::vector<int> h(npz);
-    FV3_HIP(hipMemcpyAsync(h.data(), nspl, sizeof(int) * npz, hipMemcpyDeviceToHost, s));
-    FV3_HIP(hipStreamSynchronize(s));
-    cap = *std::max_element(h.begin(), h.end());
-    if (cap < 1) return set_error("nsplit < 1 from a non-finite Courant number");
-    c.last_nsplit = h;
-  }
   // The remap runs out of place: the last transport pass of every
   // level lands in q_tmp (the caller's q_out serves as the alternate pass
   // buffer), and the remap writes q_out.
@@ -209,7 +198,50 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     q_tmp = q_tmp64;
     pt_src = pt ? (T *)(sc64 + b_q) : nullptr;
     tab = sc64 + b_q + b_pt;
-  } else if (cap > 1) {
+  }
+  // The remap's column tables (thicknesses only) and the copies it needs run
+  // on their own stream beside the sub-cycle counts, the host's wait for them
+  // and the transport; the field kernel joins them below.  In order on one
+  // stream where the caller has the target thickness overwrite the source's.
+  const size_t b_dp = sizeof(double) * d.s2 * npz * nt;
+  const bool same_dp = reinterpret_cast<uintptr_t>(delp_out) < reinterpret_cast<uintptr_t>(dp1) + b_dp &&
+                       reinterpret_cast<uintptr_t>(dp1) < reinterpret_cast<uintptr_t>(delp_out) + b_dp;
+  const bool early = (fast_remap || (fields && !same_dp)) && c.concurrent_kinds && c.aux[3];
+  hipStream_t sp = early ? c.aux[3] : s;
+  FieldsArgs<T> fa{};
+  auto remap_prep = [&]() -> int {
+    FV3_HIP(hipMemcpyAsync(delp_out, dp1, b_dp, hipMemcpyDeviceToDevice, sp));
+    if (pt) FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(T) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, sp));
+    if (fast_remap) return remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1, delp_out, cols, b_col, sp);
+    fa.tab = coltab_carve<T>(tab, npz, (long long)ni * nj * nt);
+    ColSource cs{};
+    cs.ptop = ptop;
+    cs.ak = ak;
+    cs.bk = bk;
+    cs.delp = cs.delp_out = delp_out;
+    return fields_prep<T>(c, fa.tab, cs, ni, nj, false, sp);
+  };
+  if (early) FV3_HIP(hipEventRecord(c.fork_ev, s));
+  if (device_nsplit<T>(c, cx, cy, c.step_per_level, c.step_per_level ? 0 : c.step_q_split, cmax, nspl, frac, xfx, yfx))
+    return 1;
+  if (early) {
+    FV3_HIP(hipStreamWaitEvent(sp, c.fork_ev, 0));
+    if (remap_prep()) return 1;
+    FV3_HIP(hipEventRecord(c.prep_ev, sp));
+  }
+  int cap = nsplit_cap;
+  if (cap <= 0) {
+    std::vector<int> h(npz);
+    FV3_HIP(hipMemcpyAsync(h.data(), nspl, sizeof(int) * npz, hipMemcpyDeviceToHost, s));
+    FV3_HIP(hipStreamSynchronize(s));
+    cap = *std::max_element(h.begin(), h.end());
+    if (cap < 1) {
+      if (early) FV3_HIP(hipStreamSynchronize(sp));  // the next call reuses the scratch
+      return set_error("nsplit < 1 from a non-finite Courant number");
+    }
+    c.last_nsplit = h;
+  }
+  if (!q_tmp && cap > 1) {
     q_tmp = (T *)ctx_scratch(c, sizeof(T) * qsize);
     if (!q_tmp) return 1;
   }
@@ -223,21 +255,6 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   a.cx = cx; a.cy = cy; a.mfx = mfx; a.mfy = mfy; a.dp1 = dp1;
   const bool timing = c.timing && !c.graph_safe;
   if (timing) FV3_HIP(hipEventRecord(c.ev[0], s));
-  // the remap's column prep (thicknesses only) and the copies it needs run on
-  // their own stream beside the transport; the field kernel joins it below
-  const bool early = fast_remap && c.concurrent_kinds && c.aux[3];
-  hipStream_t sp = early ? c.aux[3] : s;
-  auto remap_prep = [&]() -> int {
-    FV3_HIP(hipMemcpyAsync(delp_out, dp1, sizeof(double) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, sp));
-    if (pt) FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(T) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, sp));
-    return remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1, delp_out, cols, b_col, sp);
-  };
-  if (early) {
-    FV3_HIP(hipEventRecord(c.fork_ev, s));
-    FV3_HIP(hipStreamWaitEvent(sp, c.fork_ev, 0));
-    if (remap_prep()) return 1;
-    FV3_HIP(hipEventRecord(c.prep_ev, sp));
-  }
   // FP32 pipelining: the tracers go through the passes in chunks of cq, and
   // each chunk's remap runs on aux[3] (behind the column prep) while the
   // next chunk is transported; pt is remapped with the last chunk
@@ -308,7 +325,7 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     if (timing) FV3_HIP(hipEventRecord(c.ev[2], s));
     FV3_HIP(hipEventRecord(c.prep_ev, sp));
     FV3_HIP(hipStreamWaitEvent(s, c.prep_ev, 0));
-  } else if (fast_remap) {
+  } else if (oop) {
     if (early)
       FV3_HIP(hipStreamWaitEvent(s, c.prep_ev, 0));
     else if (remap_prep())
@@ -324,18 +341,9 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     }
   }
   if (fields) {
-    FieldsArgs<T> fa{};
-    fa.tab = coltab_carve<T>(tab, npz, (long long)ni * nj * nt);
-    ColSource cs{};
-    cs.ptop = ptop;
-    cs.ak = ak;
-    cs.bk = bk;
-    cs.delp = cs.delp_out = delp_out;
-    if (fields_prep<T>(c, fa.tab, cs, ni, nj, false)) return 1;
     fa.set[fa.nset++] = tracer_set<T>(c, q_tmp, q_out, nq);
     for (int iq = 0; iq <= nq; iq++) fa.kord[iq] = (signed char)std::min(iq < nq ? kord_tr : kord_tm, 17);
     if (pt) {
-      FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(T) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, s));
       FieldSet<T> &x = fa.set[fa.nset++] = cell_set<T>(c, pt_src, pt, 1);
       x.use_qmin = true;
       x.qmin = (T)t_min;

@@ -407,7 +407,7 @@ int l2e_full(Ctx &c, const fv3_l2e_args &a) {
       cs.delp = a.delp;
       cs.pe = a.pe;
       cs.ps = a.ps;
-      if (fields_prep<T>(c, f.tab, cs, ni, nj, x.iv == -2)) return 1;
+      if (fields_prep<T>(c, f.tab, cs, ni, nj, x.iv == -2, c.stream)) return 1;
       x.src = copy + (x.src - field);
       f.nset = 1;
       f.set[0] = x;

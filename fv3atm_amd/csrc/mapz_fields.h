@@ -114,7 +114,7 @@ int fields_setup();
 // tables of the columns (ni x nj per tile, every tile of c); iv2: factors of
 // the iv = -2 solve (bottom value given)
 template <typename R>
-int fields_prep(Ctx &c, const ColTab<R> &tab, const ColSource &src, int ni, int nj, bool iv2);
+int fields_prep(Ctx &c, const ColTab<R> &tab, const ColSource &src, int ni, int nj, bool iv2, hipStream_t s);
 // remap every field of the sets; sources and destinations must not overlap
 template <typename T>
 int fields_run(Ctx &c, FieldsArgs<T> &a, int ni, int nj);

@@ -761,7 +761,7 @@ int fields_setup() {
 }
 
 template <typename R>
-int fields_prep(Ctx &c, const ColTab<R> &tab, const ColSource &src, int ni, int nj, bool iv2) {
+int fields_prep(Ctx &c, const ColTab<R> &tab, const ColSource &src, int ni, int nj, bool iv2, hipStream_t s) {
   const Dims &d = c.d;
   if (c.npz > FIELDS_MAX_KM) return set_error("column tables support km <= %d (got %d)", FIELDS_MAX_KM, c.npz);
   if (fields_setup()) return 1;
@@ -774,8 +774,7 @@ int fields_prep(Ctx &c, const ColTab<R> &tab, const ColSource &src, int ni, int 
   g.spe = (long long)(g.cni + 2) * (g.km + 1) * (d.je - d.js + 3);
   g.ncb = (int)((g.ncol + 63) / 64);
   hipLaunchKernelGGL(k_fields_prep<R>, dim3((unsigned)g.ncb * (unsigned)c.ntiles), dim3(64 * PREP_WAVES), prep_lds(g.km),
-                     c.stream,
-                     g, src, tab, iv2);
+                     s, g, src, tab, iv2);
   FV3_HIP(hipGetLastError());
   return 0;
 }
@@ -828,7 +827,7 @@ FieldSet<T> tracer_set(const Ctx &c, const T *src, T *dst, int nq) {
 #define FV3_FIELDS(T)                                                                                            \
   template size_t coltab_bytes<T>(int, long long);                                                               \
   template ColTab<T> coltab_carve<T>(void *, int, long long);                                                    \
-  template int fields_prep<T>(Ctx &, const ColTab<T> &, const ColSource &, int, int, bool);                      \
+  template int fields_prep<T>(Ctx &, const ColTab<T> &, const ColSource &, int, int, bool, hipStream_t);         \
   template int fields_run<T>(Ctx &, FieldsArgs<T> &, int, int);                                                  \
   template FieldSet<T> cell_set<T>(const Ctx &, const T *, T *, int);                                            \
   template FieldSet<T> tracer_set<T>(const Ctx &, const T *, T *, int);

@@ -104,7 +104,7 @@ int remap_cells_inplace(Ctx &c, int km, int nq, const double *ak, const double *
   src.ak = ak;
   src.bk = bk;
   src.delp = src.delp_out = delp;
-  if (fields_prep<T>(c, tab, src, ni, nj, false)) return 1;
+  if (fields_prep<T>(c, tab, src, ni, nj, false, c.stream)) return 1;
   if (pt) FV3_HIP(hipMemcpyAsync(cpt, pt, b_field, hipMemcpyDeviceToDevice, s));
   if (dz) FV3_HIP(hipMemcpyAsync(cdz, dz, b_dz, hipMemcpyDeviceToDevice, s));
   for (int q0 = 0; q0 == 0 || q0 < nq; q0 += part) {

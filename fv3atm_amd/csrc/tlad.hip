@@ -1297,7 +1297,7 @@ int step_tl(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
     cs.bk = bk;
     cs.delp = dp1;
     cs.delp_out = delp_out;
-    if (fields_prep<double>(c, f.tab, cs, ni, nj, false)) return 1;
+    if (fields_prep<double>(c, f.tab, cs, ni, nj, false, c.stream)) return 1;
     for (int q1st = 0; q1st < nq; q1st += REMAP_MAX_NQ) {  // the sub-cycled tracers, REMAP_MAX_NQ at a time
       const long long oq = (long long)q1st * npz * d.s2 + o0;
       f.nset = 1;
