@@ -210,6 +210,10 @@ int fv3_ctx_create(const fv3_bounds *bd, int npx, int npy, int npz, int ntiles, 
     fv3_ctx_destroy(h);
     return set_error("hipEventCreateWithFlags failed");
   }
+  if (hipHostMalloc((void **)&c.ns_host, sizeof(int) * npz, hipHostMallocDefault) != hipSuccess) {
+    fv3_ctx_destroy(h);
+    return set_error("pinned allocation failed");
+  }
   const long long s2 = c.d.s2, sdx = (long long)c.d.nid * (c.d.njd + 1), sdy = (long long)(c.d.nid + 1) * c.d.njd;
   const long long per_tile = s2 * 4 + sdx * 2 + sdy * 2 + s2 * 9;
   if (hipMalloc(&c.g64, sizeof(double) * per_tile * ntiles) != hipSuccess ||
@@ -272,6 +276,7 @@ int fv3_ctx_destroy(fv3_ctx *h) {
   (void)hipFree(c.scratch);
   (void)hipFree(c.stage);
   (void)hipFree(c.step_flag);
+  if (c.ns_host) (void)hipHostFree(c.ns_host);
   for (auto *t : c.halo_tab) (void)hipFree(t);
   (void)hipFree(c.l2e_buf);
   for (auto &e : c.ev)

@@ -17,10 +17,11 @@ int launch_fused_f32(const FusedArgs<float> &a, int cfg, const KindStreams &s);
 int fused32_round(int cfg);
 
 // per-level sub-cycle counts on the device (cmax, nsplit; no scaling); with
-// xfx, yfx (layouts of cx, cy) the same pass writes the area fluxes
+// xfx, yfx (layouts of cx, cy) the same pass writes the area fluxes; host:
+// pinned memory for a copy of the counts
 template <typename T>
 int device_nsplit(Ctx &c, const T *cx, const T *cy, bool per_level, int q_split, double *cmax,
-                  int *nsplit, T *frac, T *xfx = nullptr, T *yfx = nullptr);
+                  int *nsplit, T *frac, T *xfx = nullptr, T *yfx = nullptr, int *host = nullptr);
 
 // the area fluxes alone, FP64 (unscaled, every tile)
 int area_fluxes(Ctx &c, const double *cx, const double *cy, double *xfx, double *yfx);

@@ -222,7 +222,8 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     return fields_prep<T>(c, fa.tab, cs, ni, nj, false, sp);
   };
   if (early) FV3_HIP(hipEventRecord(c.fork_ev, s));
-  if (device_nsplit<T>(c, cx, cy, c.step_per_level, c.step_per_level ? 0 : c.step_q_split, cmax, nspl, frac, xfx, yfx))
+  if (device_nsplit<T>(c, cx, cy, c.step_per_level, c.step_per_level ? 0 : c.step_q_split, cmax, nspl, frac, xfx, yfx,
+                       nsplit_cap > 0 ? nullptr : c.ns_host))
     return 1;
   if (early) {
     FV3_HIP(hipStreamWaitEvent(sp, c.fork_ev, 0));
@@ -231,9 +232,8 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   }
   int cap = nsplit_cap;
   if (cap <= 0) {
-    std::vector<int> h(npz);
-    FV3_HIP(hipMemcpyAsync(h.data(), nspl, sizeof(int) * npz, hipMemcpyDeviceToHost, s));
-    FV3_HIP(hipStreamSynchronize(s));
+    FV3_HIP(hipStreamSynchronize(s));  // the counts are in ns_host
+    const std::vector<int> h(c.ns_host, c.ns_host + npz);
     cap = *std::max_element(h.begin(), h.end());
     if (cap < 1) {
       if (early) FV3_HIP(hipStreamSynchronize(sp));  // the next call reuses the scratch

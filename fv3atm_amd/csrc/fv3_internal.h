@@ -92,6 +92,7 @@ struct Ctx {
   // nsplit_cap check lands in step_flag for fv3_step_status
   bool graph_safe = false;
   int *step_flag = nullptr;
+  int *ns_host = nullptr;  // pinned: a step's sub-cycle counts, written by the kernel that makes them
   hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
   // the fused transport's edge kinds run beside the lean kind on three
   // auxiliary streams (default priority), forked from and joined to the
