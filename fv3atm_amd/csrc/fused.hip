@@ -86,10 +86,13 @@ static FusedArgs<T> fused_geometry(const Ctx &c, int nq, int hord) {
       if (strip_ok(st)) { if (s0 < 0) s0 = st; s1 = st; }
     const bool inner = s0 >= 0 && a.lb >= a.lt;
     const int rows = inner ? a.lb - a.lt + 1 : nj;
-    // (resident workgroups of four waves: three per CU in FP32, two in FP64)
+    // (resident workgroups of four waves: three per CU in FP32, two in FP64.  A
+    // lean block's six first rows cost about four: with 2.5, two tracers on a
+    // C420 L63 tile 953 us a step and on C260 L127 827, with 4 913 and 800, with
+    // 12 930 and 804; ten or more tracers the same within 0.5 %)
     const long long units = (long long)a.nstrip * npz * nt * ((nq + 3) / 4);
     a.H = c.fused_h > 0 ? c.fused_h
-                        : fused_block_rows(rows, units, sizeof(T) == 4 ? 768 : 512, inner ? 2.5 : 2.0 * NG);
+                        : fused_block_rows(rows, units, sizeof(T) == 4 ? 768 : 512, inner ? 4.0 : 2.0 * NG);
     a.H = std::min(nj, a.H);
     a.nvblk = (nj + a.H - 1) / a.H;
     if (inner) {
