@@ -176,7 +176,7 @@ __global__ void k_te(Geo g, int t, double cp, const T *u, const T *v, const T *p
 // Eulerian pe (compute domain), peln, pk, pkz: one thread per column and
 // PR_LEV levels, each with its layers' upper interfaces (and the next one's,
 // recomputed, for the hydrostatic layer means).  One thread per column was one
-// log and exp after another: C192 L127 150 us.
+// log and exp after another: C192 L127 150 us, now 59.
 constexpr int PR_LEV = 4;
 template <typename T>
 __global__ void k_pressures(Geo g, int t, double ptop, const double *__restrict__ ak, const double *__restrict__ bk,
