@@ -636,8 +636,7 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
   sc.edge_strip = EK >= 2 && a.edge && (i0 - NG <= 2 || i0 - NG + FT_LANES - 1 >= a.npx - 2);
   if constexpr (sizeof(T) == 4) sc.ec = edge_coef_of(sc.edge_strip ? edge_role(sc.i, a.is, a.ie, a.npx, a.edge) : 0);
   sc.edge_rows = EK != 0 && EK <= 4;
-  sc.corner_wg = a.corners != 0u && (strip == 0 || strip == a.nstrip - 1) &&
-                 (EK == 2 ? (vb == 0 || vb == a.nvblk - 1) : (EK == 3 || EK == 4));
+  sc.corner_wg = EK >= 2 && EK <= 4 && a.corners != 0u && fused_reads_corners(i0, j0, h, a.is, a.ie, a.js, a.je);
   sc.scale = nspl > 1;
   sc.frac = T(1) / T(nspl);
   sc.nix = a.ie - a.is + 2;

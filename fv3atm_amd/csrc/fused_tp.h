@@ -137,6 +137,14 @@ __host__ __device__ __forceinline__ void fused_block_round(int x, int nb, int ro
   }
 }
 
+// Whether a strip's lanes (from column i0 - NG) and a block's input rows (j0 - NG
+// .. j0 + h - 1 + NG) reach halo columns and halo rows together: the blocks that
+// may read corner cells.  Not only the outermost strips and blocks do: one before
+// a last strip or block of one or two columns or rows reads corner cells too.
+__host__ __device__ __forceinline__ bool fused_reads_corners(int i0, int j0, int h, int is, int ie, int js, int je) {
+  return (i0 - NG < is || i0 - NG + FT_LANES - 1 > ie) && (j0 - NG < js || j0 + h - 1 + NG > je);
+}
+
 // ---- cross-lane shifts: value of lane l-1 / l+1 (DPP wave_shr:1 / wave_shl:1)
 // (bound_ctrl: the lane past the wave edge reads 0, so no destination
 // initialisation is needed; that lane is a halo lane whose result is unused)

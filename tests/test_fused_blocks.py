@@ -45,3 +45,52 @@ def test_blocks_and_rows(tmp_path):
                     os.path.join(ROOT, "fv3atm_amd", "csrc"), "-o", str(exe)], check=True, capture_output=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0 and "ok" in r.stdout, r.returncode
+
+
+# Every strip and row block of a tile with three halo cells: one that holds a
+# corner cell (corner_src, the exact rule) has to be marked as reading corners.
+# Rows per block as the transport derives them and every other value up to 60.
+CORNERS = r"""
+#include "fused_tp.h"
+#include <algorithm>
+#include <cstdio>
+using namespace fv3;
+int main() {
+  for (int n = 8; n <= 260; n++)
+    for (int H0 = -5; H0 <= 60; H0++) {
+      if (H0 == 0) continue;
+      // H0 < 0: the rule, at -H0 levels, FP32 or FP64, one or a few tracers
+      const int ns = (n + FT_BX - 1) / FT_BX;
+      const int H = std::min(n, H0 > 0 ? H0 : fused_block_rows(n, (long long)ns * -H0 * 16, H0 & 1 ? 768 : 512, 2.0 * NG));
+      for (int s = 0; s < ns; s++)
+        for (int b = 0; b * H < n; b++) {
+          const int i0 = 1 + s * FT_BX, j0 = 1 + b * H, h = std::min(H, n + 1 - j0);
+          bool holds = false;
+          for (int l = 0; l < FT_LANES && !holds; l++)
+            for (int j = j0 - NG; j <= j0 + h - 1 + NG && !holds; j++) {
+              int si, sj;
+              const int i = std::min(i0 - NG + l, n + NG);
+              holds = corner_src(i, j, n + 1, n + 1, 1, 15u, si, sj);
+            }
+          if (holds && !fused_reads_corners(i0, j0, h, 1, n, 1, n)) {
+            std::printf("n %d rows %d strip %d block %d\n", n, H, s, b);
+            return 1;
+          }
+        }
+    }
+  std::puts("ok");
+  return 0;
+}
+"""
+
+
+def test_corner_blocks(tmp_path):
+    if not os.path.exists(HIPCC):
+        pytest.skip("hipcc not found")
+    src = tmp_path / "corners.cpp"
+    src.write_text(CORNERS)
+    exe = tmp_path / "corners"
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O1", "-std=c++17", "-w", "-x", "hip", str(src), "-I",
+                    os.path.join(ROOT, "fv3atm_amd", "csrc"), "-o", str(exe)], check=True, capture_output=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0 and "ok" in r.stdout, r.stdout
