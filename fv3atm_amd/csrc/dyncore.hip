@@ -657,7 +657,10 @@ extern "C" int fv3_dyn_core_fluxes(fv3_ctx *h, int form, int n_split, double bdt
   Ctx &c = h->c;
   std::lock_guard<std::mutex> lk(c.mu);
   if (!c.grid_set) return set_error("grid metrics not set (fv3_ctx_set_grid)");
-  hipStream_t s = stream ? (hipStream_t)stream : c.stream;
+  // the context's stream for the call: halo_fill launches there
+  hipStream_t saved = c.stream;
+  if (stream) c.stream = (hipStream_t)stream;
+  hipStream_t s = c.stream;
   int rc;
   if (form == FV3_FORM_PLAIN64)
     rc = dyn_core_fluxes<double>(c, n_split, bdt, hord_dp, (const double *)uc, (const double *)vc, (double *)delp,
@@ -673,6 +676,7 @@ extern "C" int fv3_dyn_core_fluxes(fv3_ctx *h, int form, int n_split, double bdt
   else
     rc = set_error("form %d: the dyn_core fluxes run FV3_FORM_PLAIN64 or FV3_FORM_FUSED64 (double), "
                    "FV3_FORM_FUSED32 (float)", form);
+  c.stream = saved;
   if (rc) return 1;
   FV3_HIP(hipStreamSynchronize(s));
   return 0;
