@@ -209,11 +209,11 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   const size_t b_dp = sizeof(double) * d.s2 * npz * nt;
   const bool same_dp = reinterpret_cast<uintptr_t>(delp_out) < reinterpret_cast<uintptr_t>(dp1) + b_dp &&
                        reinterpret_cast<uintptr_t>(dp1) < reinterpret_cast<uintptr_t>(delp_out) + b_dp;
-  const bool early = (fast_remap || (fields && !same_dp)) && c.concurrent_kinds && c.aux[3];
+  const bool early = oop && !same_dp && c.concurrent_kinds && c.aux[3];
   hipStream_t sp = early ? c.aux[3] : s;
   FieldsArgs<T> fa{};
   auto remap_prep = [&]() -> int {
-    FV3_HIP(hipMemcpyAsync(delp_out, dp1, b_dp, hipMemcpyDeviceToDevice, sp));
+    if (delp_out != dp1) FV3_HIP(hipMemcpyAsync(delp_out, dp1, b_dp, hipMemcpyDeviceToDevice, sp));
     if (pt) FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(T) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, sp));
     if (fast_remap) return remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1, delp_out, cols, b_col, sp);
     fa.tab = coltab_carve<T>(tab, npz, (long long)ni * nj * nt);
@@ -333,8 +333,8 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
       FV3_HIP(hipStreamWaitEvent(s, c.prep_ev, 0));
     else if (remap_prep())
       return 1;
-  } else if (remap_phase) {
-    FV3_HIP(hipMemcpyAsync(delp_out, dp1, sizeof(double) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, s));
+  } else if (remap_phase && delp_out != dp1) {
+    FV3_HIP(hipMemcpyAsync(delp_out, dp1, b_dp, hipMemcpyDeviceToDevice, s));
   }
   if (timing && !pipe) FV3_HIP(hipEventRecord(c.ev[2], s));
   if constexpr (std::is_same<T, float>::value) {

@@ -149,7 +149,7 @@ int fv3_lagrangian_to_eulerian_tracers_r4(fv3_ctx *ctx, int km, int nq, const do
  * applied in flight.  Element types: form PLAIN64/FUSED64 -> q, pt, cx, cy,
  * mfx, mfy double; FUSED32 -> float.  dp1 (the Lagrangian thickness) and
  * delp_out are always double.  pt (may be NULL) is remapped in place; delp_out
- * receives the target thicknesses.  stream is a hipStream_t (NULL: the
+ * receives the target thicknesses and may be dp1 itself (then not read-only).  stream is a hipStream_t (NULL: the
  * context's stream).  nsplit_cap bounds the per-level sub-cycle count the
  * fused forms schedule (0 = derive it, with one device-to-host read). */
 int fv3_step_dev(fv3_ctx *ctx, int form, int nq, const void *q_in, void *q_out, void *pt,
