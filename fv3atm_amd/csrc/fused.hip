@@ -8,6 +8,7 @@
 #include "fused_kernel.h"
 #include "mapz_fast.h"
 #include "mapz_fields.h"
+#include "mapz_prep.h"
 
 namespace fv3 {
 
@@ -41,6 +42,25 @@ __global__ void k_nsplit_check(const int *nsplit, int npz, int cap, int *flag) {
     for (int k = 0; k < npz; k++) bad |= nsplit[k] > cap || nsplit[k] < 1;
     *flag = bad;
   }
+}
+
+// The halo cells of the target thickness, which keep the source's (blockIdx.y:
+// level, of every tile), unless the host will refuse the step.
+__global__ void __launch_bounds__(256) k_halo_dp(const double *dp1, double *delp_out, Dims d, StepCounts counts) {
+  if (!__syncthreads_or(counts.any(threadIdx.x, 256))) return;
+  const int e = blockIdx.x * 256 + threadIdx.x, nj = d.je - d.js + 1, rows = NG * d.nid;
+  if (e >= 2 * (rows + NG * nj)) return;
+  int i, j;
+  if (e < 2 * rows) {
+    i = e % d.nid;
+    j = e < rows ? e / d.nid : NG + nj + (e - rows) / d.nid;
+  } else {
+    const int m = (e - 2 * rows) % (2 * NG);
+    i = m < NG ? m : d.nid - 2 * NG + m;
+    j = NG + (e - 2 * rows) / (2 * NG);
+  }
+  const long long o = blockIdx.y * d.s2 + (long long)j * d.nid + i;
+  delp_out[o] = dp1[o];
 }
 
 // The geometry, metrics and strides of a pass over nq tracers of every tile.
@@ -202,35 +222,54 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     pt_src = pt ? (T *)(sc64 + b_q) : nullptr;
     tab = sc64 + b_q + b_pt;
   }
-  // The remap's column tables (thicknesses only) and the copies it needs run
-  // on their own stream beside the sub-cycle counts, the host's wait for them
-  // and the transport; the field kernel joins them below.  In order on one
-  // stream where the caller has the target thickness overwrite the source's.
+  // The remap's column tables (thicknesses only) and the copy of pt that it needs
+  // run on their own stream beside the host's wait for the sub-cycle counts and the
+  // transport, the FP64 form's also beside the counts; the field kernel joins them
+  // below.  What writes the target thickness comes after the counts and looks at
+  // them (StepCounts).  In order on one stream where the caller has the target
+  // thickness overwrite the source's.
   const size_t b_dp = sizeof(double) * d.s2 * npz * nt;
   const bool same_dp = reinterpret_cast<uintptr_t>(delp_out) < reinterpret_cast<uintptr_t>(dp1) + b_dp &&
                        reinterpret_cast<uintptr_t>(dp1) < reinterpret_cast<uintptr_t>(delp_out) + b_dp;
   const bool early = oop && !same_dp && c.concurrent_kinds && c.aux[3];
   hipStream_t sp = early ? c.aux[3] : s;
+  const int *counts = nsplit_cap > 0 ? nullptr : nspl;
   FieldsArgs<T> fa{};
-  auto remap_prep = [&]() -> int {
-    if (delp_out != dp1) FV3_HIP(hipMemcpyAsync(delp_out, dp1, b_dp, hipMemcpyDeviceToDevice, sp));
+  auto remap_tables = [&]() -> int {  // FP64
     if (pt) FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(T) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, sp));
-    if (fast_remap) return remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1, delp_out, cols, b_col, sp);
     fa.tab = coltab_carve<T>(tab, npz, (long long)ni * nj * nt);
     ColSource cs{};
     cs.ptop = ptop;
     cs.ak = ak;
     cs.bk = bk;
-    cs.delp = cs.delp_out = delp_out;
+    cs.delp = dp1;
     return fields_prep<T>(c, fa.tab, cs, ni, nj, false, sp);
   };
-  if (early) FV3_HIP(hipEventRecord(c.fork_ev, s));
+  auto remap_target = [&]() -> int {  // FP32: with the tables
+    if constexpr (std::is_same<T, double>::value) {
+      return fields_target(c, fa.tab, dp1, delp_out, counts, sp);
+    } else {
+      if (delp_out != dp1) {
+        hipLaunchKernelGGL(k_halo_dp, dim3((unsigned)((2 * NG * (d.nid + nj) + 255) / 256), (unsigned)(npz * nt)),
+                           dim3(256), 0, sp, dp1, delp_out, d, StepCounts{counts, npz});
+        FV3_HIP(hipGetLastError());
+      }
+      if (pt) FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(T) * d.s2 * npz * nt, hipMemcpyDeviceToDevice, sp));
+      return remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1, delp_out, counts, cols, b_col, sp);
+    }
+  };
+  if (early && fields) FV3_HIP(hipEventRecord(c.fork_ev, s));
   if (device_nsplit<T>(c, cx, cy, c.step_per_level, c.step_per_level ? 0 : c.step_q_split, cmax, nspl, frac, xfx, yfx,
                        nsplit_cap > 0 ? nullptr : c.ns_host))
     return 1;
   if (early) {
-    FV3_HIP(hipStreamWaitEvent(sp, c.fork_ev, 0));
-    if (remap_prep()) return 1;
+    if (fields) {
+      FV3_HIP(hipStreamWaitEvent(sp, c.fork_ev, 0));
+      if (remap_tables()) return 1;
+    }
+    FV3_HIP(hipEventRecord(c.chunk_ev, s));
+    FV3_HIP(hipStreamWaitEvent(sp, c.chunk_ev, 0));
+    if (remap_target()) return 1;
     FV3_HIP(hipEventRecord(c.prep_ev, sp));
   }
   int cap = nsplit_cap;
@@ -331,7 +370,7 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   } else if (oop) {
     if (early)
       FV3_HIP(hipStreamWaitEvent(s, c.prep_ev, 0));
-    else if (remap_prep())
+    else if ((fields && remap_tables()) || remap_target())
       return 1;
   } else if (remap_phase && delp_out != dp1) {
     FV3_HIP(hipMemcpyAsync(delp_out, dp1, b_dp, hipMemcpyDeviceToDevice, s));
@@ -416,7 +455,7 @@ int remap_only_f32(Ctx &c, int nq, const float *q_src, float *q_dst, float *pt, 
   FV3_HIP(hipMemcpyAsync(delp_out, dp1, sizeof(double) * tl * nt, hipMemcpyDeviceToDevice, s));
   if (pt) FV3_HIP(hipMemcpyAsync(pt_src, pt, sizeof(float) * tl * nt, hipMemcpyDeviceToDevice, s));
   const RemapCols cols = remap_cols_carve(sc + b_pt, npz, (long long)ni * nj);
-  if (remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1, delp_out, cols, b_col, s)) return 1;
+  if (remap_fast_prep_f32(c, npz, ak, bk, ptop, dp1, delp_out, nullptr, cols, b_col, s)) return 1;
   return remap_fast_fields_f32(c, npz, nq, q_src, q_dst, pt_src, pt, kord_tr, kord_tm, t_min, cols, b_col, tq, s);
 }
 

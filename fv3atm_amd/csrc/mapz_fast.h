@@ -30,8 +30,8 @@ RemapCols remap_cols_carve(void *base, int km, long long ncol);
 
 // Remap of every tile's interior columns in two launches.  The prep (column
 // pressures, Thomas factors, target cut list; dp2 into delp_out) depends on
-// the thicknesses only, so it may run before or beside the transport; the
-// field kernel then remaps nq tracers (iv=0, kord_tr) from q_src into q_dst
+// the thicknesses only, so it may run before or beside the transport (counts:
+// StepCounts, or NULL); the field kernel then remaps nq tracers (iv=0, kord_tr) from q_src into q_dst
 // and, when pt_src is given, pt (iv=1, kord_tm, t_min) into pt_dst.  Sources
 // and destinations must not overlap.  cols: the first tile's column data, the
 // next tile's cols_stride bytes on; tq: elements between tiles of q.
@@ -39,7 +39,8 @@ int remap_fast_check(int km, long long ncol, long long s2, int kord_tr, int kord
 // once per process, before the first remap launch: the lane remap kernel's LDS limit
 int remap_rows_setup();
 int remap_fast_prep_f32(Ctx &c, int km, const double *ak, const double *bk, double ptop,
-                        const double *dp1, double *delp_out, const RemapCols &cols, size_t cols_stride, hipStream_t s);
+                        const double *dp1, double *delp_out, const int *counts, const RemapCols &cols,
+                        size_t cols_stride, hipStream_t s);
 int remap_fast_fields_f32(Ctx &c, int km, int nq, const float *q_src, float *q_dst, const float *pt_src,
                           float *pt_dst, int kord_tr, int kord_tm, double t_min, const RemapCols &cols,
                           size_t cols_stride, long long tq, hipStream_t s);

@@ -44,6 +44,7 @@ struct PrepArgs {
   double ptop;
   const double *dp1, *ak, *bk;
   double *delp_out;
+  StepCounts counts;
   RemapCols cols;      // of the first tile
   long long tdp, tcol; // tile strides: levels (elements), column data (bytes)
 };
@@ -62,7 +63,7 @@ __device__ __forceinline__ RemapCols tile_cols(RemapCols c, long long bytes) {
 // transport, one launch per tile; six tiles in one launch take 1.2 ms there.
 __global__ void __launch_bounds__(64 * PREP_WAVES) k_remap_prep(const PrepArgs a) {
   extern __shared__ double pe1_lds[];  // [km + 1][columns]
-  __shared__ int bad[64];
+  __shared__ int bad[64], go;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const long long tile = blockIdx.y;
   const int pc = prep_cols(a.km);
@@ -75,7 +76,11 @@ __global__ void __launch_bounds__(64 * PREP_WAVES) k_remap_prep(const PrepArgs a
   const int km = a.km;
   const RemapCols o = tile_cols(a.cols, tile * a.tcol);
   const ColPe P{pe1_lds + (lane & (pc - 1)), pc};
-  if (wave == 0) bad[lane] = 0;
+  const bool counted = a.counts.any(threadIdx.x, 64 * PREP_WAVES);
+  if (wave == 0) {
+    bad[lane] = 0;
+    go = 0;
+  }
   // Lagrangian interfaces by running sums from ptop, thicknesses as their
   // differences (the Lagrangian_to_Eulerian pe1 / dp1 of the upstream)
   stage_interfaces(P, km, a.ptop, a.dp1 + tile * a.tdp + cell, s2, wave);
@@ -90,6 +95,7 @@ __global__ void __launch_bounds__(64 * PREP_WAVES) k_remap_prep(const PrepArgs a
     bool b = false;
     for (int k = 1 + wave; k <= km; k += PREP_WAVES) b = b || !(P(k + 1) > P(k)) || !(pe2_of(k + 1) >= pe2_of(k));
     if (b) bad[lane] = 1;
+    if (counted) go = 1;
   }
   __syncthreads();
   if (wave == 0) {
@@ -141,14 +147,14 @@ __global__ void __launch_bounds__(64 * PREP_WAVES) k_remap_prep(const PrepArgs a
   // of every target interface (the first layer l with pe2 <= PE1(l+1), the
   // choice the upstream search makes when an interface falls on a source
   // interface)
-  double *dout = a.delp_out + tile * a.tdp + cell;
+  double *dout = go ? a.delp_out + tile * a.tdp + cell : nullptr;
   auto put = [&](int k, double p, double p_next, int l, int lb) {
     const double dp2 = p_next - p, lo = P(l), hi = P(l + 1);
     if (!act) return;
     const long long o_t = (long long)(k - 1) * nc + col;
     o.cut[o_t] = make_float4((float)((p - lo) / (hi - lo)), (float)(hi - p), (float)(p_next - P(lb)), (float)(1.0 / dp2));
     o.lk[o_t] = l;
-    dout[(long long)(k - 1) * s2] = dp2;
+    if (dout) dout[(long long)(k - 1) * s2] = dp2;
   };
   if (!bad[lane]) {
     for (int k = wave; k <= km; k += PREP_WAVES - 1) {
@@ -1061,7 +1067,8 @@ static int check_orders(int km, int kord_tr, int kord_tm, bool with_pt) {
 }
 
 int remap_fast_prep_f32(Ctx &c, int km, const double *ak, const double *bk, double ptop,
-                        const double *dp1, double *delp_out, const RemapCols &cols, size_t cols_stride, hipStream_t s) {
+                        const double *dp1, double *delp_out, const int *counts, const RemapCols &cols,
+                        size_t cols_stride, hipStream_t s) {
   const Dims &d = c.d;
   if (km < 8) return set_error("fast remap needs km >= 8 (got %d)", km);
   const int ni = d.ie - d.is + 1, nj = d.je - d.js + 1;
@@ -1069,7 +1076,7 @@ int remap_fast_prep_f32(Ctx &c, int km, const double *ak, const double *bk, doub
   PrepArgs pa{};
   pa.km = km; pa.ni = ni; pa.is = d.is; pa.js = d.js; pa.isd = d.isd; pa.jsd = d.jsd; pa.nid = d.nid;
   pa.ncol = ncol; pa.s2 = d.s2; pa.ptop = ptop; pa.dp1 = dp1; pa.ak = ak; pa.bk = bk;
-  pa.delp_out = delp_out; pa.cols = cols; pa.tdp = d.s2 * km; pa.tcol = (long long)cols_stride;
+  pa.delp_out = delp_out; pa.counts = {counts, km}; pa.cols = cols; pa.tdp = d.s2 * km; pa.tcol = (long long)cols_stride;
   if (remap_rows_setup()) return 1;
   hipLaunchKernelGGL(k_remap_prep, dim3((unsigned)((ncol + prep_cols(km) - 1) / prep_cols(km)), (unsigned)c.ntiles),
                      dim3(64 * PREP_WAVES), prep_lds(km), s, pa);

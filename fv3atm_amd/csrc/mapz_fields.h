@@ -115,6 +115,9 @@ int fields_setup();
 // the iv = -2 solve (bottom value given)
 template <typename R>
 int fields_prep(Ctx &c, const ColTab<R> &tab, const ColSource &src, int ni, int nj, bool iv2, hipStream_t s);
+// the target thickness of the cell columns from their tables (halo cells as dp1's;
+// out may be dp1; counts: StepCounts, or NULL)
+int fields_target(Ctx &c, const ColTab<double> &tab, const double *dp1, double *out, const int *counts, hipStream_t s);
 // remap every field of the sets; sources and destinations must not overlap
 template <typename T>
 int fields_run(Ctx &c, FieldsArgs<T> &a, int ni, int nj);

@@ -5,6 +5,21 @@
 
 namespace fv3 {
 
+// The sub-cycle counts (n of them) of a step whose remap launches are submitted
+// before the host knows them: where none is at least 1 the host refuses the step,
+// and a kernel may not write the target thickness.  No counts (NULL): it may.
+struct StepCounts {
+  const int *ns;
+  int n;
+  // whether the calling thread's share of the counts lets the step go on
+  __device__ __forceinline__ bool any(int tid, int threads) const {
+    bool a = ns == nullptr;
+    if (ns)
+      for (int k = tid; k < n; k += threads) a = a || ns[k] >= 1;
+    return a;
+  }
+};
+
 constexpr int PREP_WAVES = 8;
 
 // Columns per workgroup: one per lane, or per two lanes (which then do the

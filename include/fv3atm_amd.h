@@ -151,7 +151,9 @@ int fv3_lagrangian_to_eulerian_tracers_r4(fv3_ctx *ctx, int km, int nq, const do
  * delp_out are always double.  pt (may be NULL) is remapped in place; delp_out
  * receives the target thicknesses and may be dp1 itself (then not read-only).  stream is a hipStream_t (NULL: the
  * context's stream).  nsplit_cap bounds the per-level sub-cycle count the
- * fused forms schedule (0 = derive it, with one device-to-host read). */
+ * fused forms schedule (0 = derive it, with one device-to-host read; a call
+ * whose Courant numbers give no level a sub-cycle is refused then, its outputs
+ * as they were). */
 int fv3_step_dev(fv3_ctx *ctx, int form, int nq, const void *q_in, void *q_out, void *pt,
                  const double *dp1, double *delp_out, const void *cx, const void *cy,
                  const void *mfx, const void *mfy, const double *ak, const double *bk,
