@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(256) k_area_flux(const T *cx, const T *cy, con
   const double *s5 = sin_sg64 + (long long)tile * 9 * g.s2 + 4 * g.s2;
   const bool top = (k + 1) < npz / 6;
   const int i = d.isd + (int)(blockIdx.x * 64 + (threadIdx.x & 63));
-  double m = 0.0;
+  double m = -1.0;  // none: a thread without cells takes no part in the maxima (a 0 would hide a NaN)
   for (int r = threadIdx.x >> 6; r < AF_ROWS; r += 4) {
     const int j = d.jsd + (int)blockIdx.y * AF_ROWS + r;
     if (j > d.jed || i > d.ied) continue;
@@ -143,10 +143,11 @@ __global__ void __launch_bounds__(256) k_area_flux(const T *cx, const T *cy, con
   red[threadIdx.x] = m;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) red[threadIdx.x] = mx2(red[threadIdx.x], red[threadIdx.x + s]);
+    if ((int)threadIdx.x < s && red[threadIdx.x + s] != -1.0)
+      red[threadIdx.x] = mx2(red[threadIdx.x], red[threadIdx.x + s]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) atomic_max_nonneg(&cmax[k], red[0]);
+  if (threadIdx.x == 0 && red[0] != -1.0) atomic_max_nonneg(&cmax[k], red[0]);
 }
 
 // nsplit(k) and 1/nsplit from cmax (tracer_2d_1L per level, tracer_2d global),

@@ -48,3 +48,22 @@ def test_outputs_untouched(gpu_ready, form, nt, n):
     new.close()
     for a, b, k in zip(out, keep, ("q", "pt", "delp")):
         assert torch.equal(a, b), k
+
+
+@pytest.mark.parametrize("form", [fa.FORM_FUSED32, fa.FORM_FUSED64])
+@pytest.mark.parametrize("n", [20, 48, 62])
+def test_refused_at_small_tiles(gpu_ready, form, n):
+    """Tiles whose columns leave lanes of a wave without a cell."""
+    npz = 9
+    case = cases.make_case(f"C{n}L9Q1", n=n, npz=npz, nq=1, delp_kind=1, delp_amp=(0.05, 0.1), seed=n)
+    w = np.float64 if form == fa.FORM_FUSED64 else np.float32
+    print(f"[refused] form {form} C{n}", flush=True)
+    q, dp1 = _dev(case.q, w), _dev(case.dp1, np.float64)
+    wind = [_dev(getattr(case, k), w) for k in ("cx", "cy", "mfx", "mfy")]
+    for a in wind[:2]:
+        a.fill_(float("nan"))
+    ctx = fa.Context(case.grids, npz)
+    with pytest.raises(RuntimeError, match="nsplit < 1"):
+        fa.step_dev(ctx, form, 1, q, torch.zeros_like(q), None, dp1, torch.zeros_like(dp1), *wind,
+                    _dev(case.ak, np.float64), _dev(case.bk, np.float64), case.ptop, 8, 9, 10)
+    ctx.close()
