@@ -23,10 +23,10 @@ struct StepCounts {
 constexpr int PREP_WAVES = 8;
 
 // Columns per workgroup: one per lane, or per two lanes (which then do the
-// same) where 64 columns of interfaces do not fit in LDS; at most 128 KB up to
-// 511 levels.
+// same) where 64 columns of interfaces do not fit in LDS; at most 129 KB up to
+// 512 levels.
 __host__ __device__ constexpr int prep_cols(int km) { return km <= 255 ? 64 : 32; }
-constexpr int PREP_MAX_KM = 511;
+constexpr int PREP_MAX_KM = 512;  // what the one-thread-per-column field kernel takes (64 KB of LDS)
 __host__ __device__ constexpr size_t prep_lds(int km) { return sizeof(double) * (size_t)(km + 1) * prep_cols(km); }
 
 // interface k (1-based) of the lane's column: [km + 1][columns] doubles
