@@ -191,18 +191,20 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
   T *frac = (T *)(base + o_frac);
   int *nspl = (int *)(base + o_ns), *flag = c.graph_safe ? c.step_flag : (int *)(base + o_flag);
   // FP64: the scratch (area fluxes first, which the sub-cycle counts' pass over
-  // the Courant numbers also computes) is sized before the counts are known
+  // the Courant numbers also computes) is sized before the counts are known; a
+  // step without the tables' remap gets its second q after them, if it has
+  // sub-cycles
   T *xfx = nullptr, *yfx = nullptr, *q_tmp64 = nullptr;
   const size_t b_xf = (sizeof(T) * d.sx * npz * nt + 255) & ~(size_t)255;
   const size_t b_yf = (sizeof(T) * d.sy * npz * nt + 255) & ~(size_t)255;
   char *sc64 = nullptr;
   if constexpr (std::is_same<T, double>::value) {
-    sc64 = (char *)ctx_scratch(c, b_xf + b_yf + b_q + (fields ? b_pt + coltab_bytes<T>(npz, (long long)ni * nj * nt) : 0));
+    sc64 = (char *)ctx_scratch(c, b_xf + b_yf + (fields ? b_q + b_pt + coltab_bytes<T>(npz, (long long)ni * nj * nt) : 0));
     if (!sc64) return 1;
     xfx = (T *)sc64;
     yfx = (T *)(sc64 + b_xf);
     sc64 += b_xf + b_yf;
-    q_tmp64 = (T *)sc64;
+    if (fields) q_tmp64 = (T *)sc64;
   }
   // The remap runs out of place: the last transport pass of every
   // level lands in q_tmp (the caller's q_out serves as the alternate pass
@@ -217,7 +219,7 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     q_tmp = (T *)sc;
     pt_src = pt ? (T *)(sc + b_q) : nullptr;
     cols = remap_cols_carve(sc + b_q + b_pt, npz, (long long)ni * nj);
-  } else if (sc64) {
+  } else if (fields) {
     q_tmp = q_tmp64;
     pt_src = pt ? (T *)(sc64 + b_q) : nullptr;
     tab = sc64 + b_q + b_pt;
@@ -284,8 +286,17 @@ static int fused_step_t(Ctx &c, int nq, const T *q_in, T *q_out, T *pt, const do
     c.last_nsplit = h;
   }
   if (!q_tmp && cap > 1) {
-    q_tmp = (T *)ctx_scratch(c, sizeof(T) * qsize);
-    if (!q_tmp) return 1;
+    const size_t b_flux = xfx ? b_xf + b_yf : 0;
+    char *sc = (char *)ctx_scratch(c, b_flux + b_q);
+    if (!sc) return 1;
+    q_tmp = (T *)(sc + b_flux);
+    if constexpr (std::is_same<T, double>::value) {
+      if (sc != (char *)xfx) {  // the scratch has grown: the fluxes once more
+        xfx = (T *)sc;
+        yfx = (T *)(sc + b_xf);
+        if (area_fluxes(c, cx, cy, xfx, yfx)) return 1;
+      }
+    }
   }
   FusedArgs<T> a = fused_geometry<T>(c, nq, hord);
   a.cap = cap;
