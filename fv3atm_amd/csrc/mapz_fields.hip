@@ -18,26 +18,11 @@
 #include "fv3_internal.h"
 #include "mapz_fields.h"
 #include "mapz_prep.h"
+#include "quot.h"
 
 namespace fv3 {
 
 namespace {
-
-// ---- a / b from y = 1/b (rounded): two residual corrections of a*y.  The
-// first leaves q within one unit in the last place, so that the second is
-// a/b correctly rounded (Markstein, IBM J. Res. Dev. 34, 1990): the value of
-// the division it replaces, in five instructions.
-template <typename R>
-__device__ __forceinline__ R quot(R a, R b, R y) {
-  R q = a * y;
-  q = fma(fma(-b, q, a), y, q);
-  return fma(fma(-b, q, a), y, q);
-}
-__device__ __forceinline__ D1 quot(const D1 &a, double b, double y) {
-  D1 r(quot(a.v, b, y));
-  r.d[0] = a.d[0] * y;
-  return r;
-}
 
 struct PrepGeo {
   int km, ni, nj, ncb, is, js, isd, jsd, nid, cni;  // cni: cells along i (the pe array's rows are cni + 2)
