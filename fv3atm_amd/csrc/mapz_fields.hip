@@ -652,7 +652,7 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
             for (int m = NR - 2; m > 0; m--)
               if (lt < c - m && c - m < lb) sum = sum + M[m];
             sum = sum + bottom_piece(y2, y3, y4, t.r0.y, t.r1.y);
-            v = narrow(quot(sum, t.r2.x, t.r2.y));
+            v = narrow(quot_any(sum, t.r2.x, t.r2.y));
           }
           if (act) store(du + cbyte, du_t + cbyte, v);
           du += levb;
@@ -669,7 +669,7 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
               break;
             }
             acc = acc + bottom_piece(a2, a3, a4, tr.r0.y, tr.r1.y);
-            emit(narrow(quot(acc, tr.r2.x, tr.r2.y)));
+            emit(narrow(quot_any(acc, tr.r2.x, tr.r2.y)));
             open = false;
           } else if (lt == 0) {
             emit(narrow(SumT(0.0 / tr.r2.x)));
@@ -696,7 +696,7 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
   if constexpr (!decltype(lockstep)::value)
     // a target that ends below the source, and those no layer holds
     while (kt <= km) {
-      emit(narrow(open ? quot(acc, tr.r2.x, tr.r2.y) : SumT(0.0 / tr.r2.x)));
+      emit(narrow(open ? quot_any(acc, tr.r2.x, tr.r2.y) : SumT(0.0 / tr.r2.x)));
       open = false;
     }
   };

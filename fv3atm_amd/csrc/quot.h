@@ -24,4 +24,20 @@ __host__ __device__ __forceinline__ Dual<1> quot(const Dual<1> &a, double b, dou
   return r;
 }
 
+// the same for any operands: infinities, NaNs and zero divisors as the division
+// has them (one instruction more)
+__host__ __device__ __forceinline__ double quot_any(double a, double b, double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_div_fixup(quot(a, b, y), b, a);
+#else
+  (void)y;
+  return a / b;
+#endif
+}
+__host__ __device__ __forceinline__ Dual<1> quot_any(const Dual<1> &a, double b, double y) {
+  Dual<1> r(quot_any(a.v, b, y));
+  r.d[0] = quot_any(a.d[0], b, y);
+  return r;
+}
+
 }  // namespace fv3
