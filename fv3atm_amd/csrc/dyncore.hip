@@ -74,7 +74,7 @@ struct ColQ {
 // take four levels, whose metric loads hit the same lines.  Cube edges: rows at
 // the y-edges by uniform branches, columns at the x-edges in a second form of
 // the row loop for the strips that hold some.  Bound by VALU issue (85% busy in
-// FP32).  C384 L127, per sub-step: 335 us in FP32, 640 in FP64; 32 x 16 (FP64
+// FP32).  C384 L127, per sub-step: 345 us in FP32, 640 in FP64; 32 x 16 (FP64
 // 32 x 8) blocks in LDS, each face recomputing its cell's slopes and limiter
 // from there, took 940 and 1500 us.  delp is read from one buffer and written to another (a
 // neighbouring wave still reads the old values as its halo); the halo cells are
@@ -104,12 +104,14 @@ __device__ __forceinline__ int edge_place(const LineGeom &g, int m) {
   return 0;
 }
 
-// The expressions of ppm_dm, ppm_al, ppm_edge_face and ppm_cell, with minima
-// and maxima as instructions: two thirds of a sweep's compares and selects.
+// The expressions of ppm_dm, ppm_al, ppm_edge_face and ppm_cell.  Minima and
+// maxima are the same compares and selects: as instructions (2.11 against 2.16 ms
+// at C384 L127) they pass over a NaN, and a thickness that has gone bad spread to
+// fewer cells than in the stages.
 template <typename T>
 __device__ __forceinline__ T slope(T qm, T q, T qp) {
   const T xt = T(0.25) * (qp - qm);
-  return fsign(fmn3(fabs(xt), fmx3(qm, q, qp) - q, q - fmn3(qm, q, qp)), xt);
+  return fsign(mn3(fabs(xt), mx3(qm, q, qp) - q, q - mn3(qm, q, qp)), xt);
 }
 template <typename T>
 __device__ __forceinline__ T face(T ql, T q, T dml, T dm) {
@@ -119,7 +121,7 @@ __device__ __forceinline__ T face(T ql, T q, T dml, T dm) {
 template <typename T>
 __device__ __forceinline__ T edge_face(T q0, T q1, T q2, T q3, T d0, T d1, T d2, T d3) {
   const T xt = T(0.5) * (((T(2) * d1 + d0) * q1 - d1 * q0) / (d0 + d1) + ((T(2) * d2 + d3) * q2 - d2 * q3) / (d2 + d3));
-  return fmn(fmx(xt, fmn(fmn3(q0, q1, q2), q3)), fmx(fmx3(q0, q1, q2), q3));
+  return mn2(mx2(xt, mn2(mn3(q0, q1, q2), q3)), mx2(mx3(q0, q1, q2), q3));
 }
 
 // (bl, br) of an inner cell: orders 8 and 11 from its slope and its two face
@@ -128,8 +130,8 @@ template <bool O8, typename T>
 __device__ __forceinline__ void inner_cell(const Win5<T> &q, T dm, T al, T ar, int iord, T &bl, T &br) {
   if (O8 || iord == 8 || iord == 11) {
     const T xt = iord == 8 ? T(2) * dm : K<T>::ppm_fac * dm;
-    bl = -fsign(fmn(fabs(xt), fabs(al - q(2))), xt);
-    br = fsign(fmn(fabs(xt), fabs(ar - q(2))), xt);
+    bl = -fsign(mn2(fabs(xt), fabs(al - q(2))), xt);
+    br = fsign(mn2(fabs(xt), fabs(ar - q(2))), xt);
   } else {
     ppm_cell<T>(q, q, 2, LineGeom{0, 0, 0, false}, iord, bl, br);
   }
