@@ -372,8 +372,11 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
           q = iv2 ? R(1.5) * x.av[1] : quot(x.e[0].d4 * x.av[1] + a2nd, x.e[0].bt, x.e[0].y);
         } else {
           T n = R(3) * (x.av[j] + x.e[j].d4 * x.av[j + 1]);
-          if (iv2 && k == km) n = n - bot0 * qs;
-          q = quot(n - q, x.e[j].bt, x.e[j].y);
+          if (iv2 && k == km) {
+            q = (n - bot0 * qs - q) / x.e[j].bt;  // the division: an infinite value reaches the rows above
+          } else {
+            q = quot(n - q, x.e[j].bt, x.e[j].y);
+          }
         }
       }
       qv[j] = q;
@@ -414,7 +417,7 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
   {
     Blk cur, nxt;
     fetch(nb - 1, cur);
-    q = qbot;
+    q = iv2 ? T(R(0)) : qbot;  // iv = -2: the last row has no value below it (its factor is 0)
     for (int b = nb - 1; b >= 0; b--) {
       if (b > 0) fetch(b - 1, nxt);
       const T entry = CP(b);
