@@ -675,7 +675,7 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
             emit(narrow(quot_any(acc, tr.r2.x, tr.r2.y)));
             open = false;
           } else if (lt == 0) {
-            emit(narrow(SumT(0.0 / tr.r2.x)));
+            emit(narrow(SumT(0.0) / tr.r2.x));
           } else if (lt > c) {
             break;
           } else if (tr.rc >> 24) {
@@ -699,7 +699,7 @@ __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields
   if constexpr (!decltype(lockstep)::value)
     // a target that ends below the source, and those no layer holds
     while (kt <= km) {
-      emit(narrow(open ? quot_any(acc, tr.r2.x, tr.r2.y) : SumT(0.0 / tr.r2.x)));
+      emit(narrow(open ? quot_any(acc, tr.r2.x, tr.r2.y) : SumT(0.0) / tr.r2.x));
       open = false;
     }
   };

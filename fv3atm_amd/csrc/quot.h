@@ -17,10 +17,11 @@ __host__ __device__ __forceinline__ R quot(R a, R b, R y) {
   q = fma(fma(-b, q, a), y, q);
   return fma(fma(-b, q, a), y, q);
 }
-// of a (value, tangent) pair: each component's quotient, as Dual's division
+// of a (value, tangent) pair: each component's quotient, as Dual's division (whose
+// tangent is a NaN where the value is not finite: the divisor's is 0, times it)
 __host__ __device__ __forceinline__ Dual<1> quot(const Dual<1> &a, double b, double y) {
   Dual<1> r(quot(a.v, b, y));
-  r.d[0] = quot(a.d[0], b, y);
+  r.d[0] = quot(a.d[0] - r.v * 0.0, b, y);
   return r;
 }
 
@@ -36,7 +37,7 @@ __host__ __device__ __forceinline__ double quot_any(double a, double b, double y
 }
 __host__ __device__ __forceinline__ Dual<1> quot_any(const Dual<1> &a, double b, double y) {
   Dual<1> r(quot_any(a.v, b, y));
-  r.d[0] = quot_any(a.d[0], b, y);
+  r.d[0] = quot_any(a.d[0] - r.v * 0.0, b, y);
   return r;
 }
 

@@ -1,6 +1,7 @@
 """The remap's division by tabulated divisors (quot.h), compiled for the host: bit
 for bit the division, for float, double and both components of (value, tangent)
-pairs, over random operands of the elimination's and the layer sums' ranges."""
+pairs, over random operands of the elimination's and the layer sums' ranges; the
+tangent beside a value that is not finite is a NaN, as the division's."""
 import os
 import subprocess
 
@@ -39,6 +40,16 @@ int main() {
     const Dual<1> q = quot(a, b, y), r = a / Dual<1>(b);
     if (!same(q.v, r.v) || !same(q.d[0], r.d[0])) return 3;
   }
+  // a tangent beside a value that is not finite, or over a divisor that is not one
+  const double inf = INFINITY, odd[] = {inf, -inf, NAN};
+  for (double v : odd) {
+    Dual<1> a(v);
+    a.d[0] = 0.5;
+    if (!std::isnan(quot(a, 3.0, 1.0 / 3.0).d[0]) || !std::isnan((a / Dual<1>(3.0)).d[0])) return 4;
+  }
+  Dual<1> a(1.0);
+  a.d[0] = 0.5;
+  if (!std::isnan(quot(a, NAN, NAN).d[0]) || !std::isnan((a / Dual<1>(NAN)).d[0])) return 5;
   std::puts("ok");
   return 0;
 }
