@@ -1342,6 +1342,18 @@ int step_tl(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
   return 0;
 }
 
+// *flag = 1 if a cell of slabs (blockIdx.z: of a or b) that a transport may read is
+// not finite; the corner blocks that copy_corners fills are not read
+__global__ void __launch_bounds__(256) k_not_finite(const double *a, const double *b, Dims d, long long nslab, int *flag) {
+  const int c = (int)(blockIdx.x * 256 + threadIdx.x), i = c % d.nid + d.isd, j = c / d.nid + d.jsd;
+  int si, sj;
+  if (j > d.jed || (!d.bounded && corner_src(i, j, d.npx, d.npy, 1, d.corners, si, sj))) return;
+  const double *q = blockIdx.z ? b : a;
+  bool bad = false;
+  for (long long z = blockIdx.y; z < nslab; z += gridDim.y) bad = bad || !isfinite(q[z * d.s2 + c]);
+  if (bad) *flag = 1;
+}
+
 int step_ad(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const double *qbar1,
             double *qbar0, const double *dp1, const double *cx, const double *cy,
             const double *mfx, const double *mfy, const double *ak, const double *bk,
@@ -1430,13 +1442,44 @@ int step_ad(Ctx &c, bool per_level, int q_split, int nq, const double *q0, const
   }
   if (area_fluxes(c, cx, cy, xfx, yfx)) return 1;
   const long long tdp = nt > 1 ? P[1].dp_hist - P[0].dp_hist : 0;
-  for (int it = 1; it <= nb; it++) {
-    double *prev = ck + (long long)(it - 1) * qsize, *next = ck + (long long)it * qsize;
-    if (faces && halo_fill<double>(c, prev, qt, nullptr, 0, nslab)) return 1;
-    FV3_HIP(hipMemcpyAsync(next, prev, sizeof(double) * qsize, hipMemcpyDeviceToDevice, s));
-    if (fused_pass64(c, nq, hord, prev, next, P[0].dp_hist + (long long)(it - 1) * npz * d.s2, tdp, cx, cy, mfx, mfy,
-                     xfx, yfx, ns_it + (size_t)(it - 1) * npz))
-      return 1;
+  auto stages = [&](int it, double *next) -> int {
+    const std::vector<int> &act = acts[it];
+    FV3_HIP(hipMemcpyAsync(zs, act.data(), sizeof(int) * act.size(), hipMemcpyHostToDevice, s));
+    for (int t = 0; t < nt; t++) {
+      const double *dpa = P[t].dp_hist + (long long)(it - 1) * npz * d.s2, *dpb = P[t].dp_hist + (long long)it * npz * d.s2;
+      for (size_t p0 = 0; p0 < act.size(); p0 += chunk)
+        if (subcycle_forward<double>(s, geo_of(c, t), P[t].L, zs + p0, (int)std::min<size_t>(chunk, act.size() - p0),
+                                     next + t * qt, nullptr, T, dpa, dpb, ord_in, ord_ou, true))
+          return 1;
+    }
+    FV3_HIP(hipStreamSynchronize(s));
+    return 0;
+  };
+  // A state with NaNs or infinities goes through the stages: the fused transport's
+  // minima and maxima pass over a NaN, theirs do not.  Seen at the end of the sweep
+  // (a bad cell, face or thickness leaves its own cells bad) and in the given state,
+  // whose halo cells reach others through their slopes alone.
+  for (bool fused = true;; fused = false) {
+    for (int it = 1; it <= nb; it++) {
+      double *prev = ck + (long long)(it - 1) * qsize, *next = ck + (long long)it * qsize;
+      if (faces && halo_fill<double>(c, prev, qt, nullptr, 0, nslab)) return 1;
+      FV3_HIP(hipMemcpyAsync(next, prev, sizeof(double) * qsize, hipMemcpyDeviceToDevice, s));
+      if (!fused) {
+        if (stages(it, next)) return 1;
+      } else if (fused_pass64(c, nq, hord, prev, next, P[0].dp_hist + (long long)(it - 1) * npz * d.s2, tdp, cx, cy, mfx,
+                              mfy, xfx, yfx, ns_it + (size_t)(it - 1) * npz)) {
+        return 1;
+      }
+    }
+    if (!fused) break;
+    int bad = 0;
+    FV3_HIP(hipMemcpyAsync(zs, &bad, sizeof(int), hipMemcpyHostToDevice, s));
+    const dim3 g((unsigned)((d.s2 + 255) / 256), (unsigned)std::min<long long>((long long)nslab * nt, 65535), 2);
+    hipLaunchKernelGGL(k_not_finite, g, dim3(256), 0, s, ck, ck + (long long)nb * qsize, d, (long long)nslab * nt, zs);
+    FV3_HIP(hipGetLastError());
+    FV3_HIP(hipMemcpyAsync(&bad, zs, sizeof(int), hipMemcpyDeviceToHost, s));
+    FV3_HIP(hipStreamSynchronize(s));
+    if (!bad) break;
   }
   const double *qT = ck + (long long)nb * qsize;
   // ---- remap adjoint: qbar = (d remap / d qT)^T qbar1 on the interior

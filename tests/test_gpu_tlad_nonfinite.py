@@ -28,3 +28,30 @@ def test_tangent_of_a_bad_thickness(gpu_ready, value):
     bad = ~np.isfinite(interior(q1))
     assert bad.any()
     assert np.isnan(interior(dq1)[bad]).all()
+
+
+@pytest.mark.parametrize("value,halo,nt", [(np.nan, False, 1), (np.inf, False, 1), (np.nan, True, 1),
+                                           (np.nan, False, 6), (np.inf, False, 6)])
+def test_adjoint_of_a_bad_state(gpu_ready, value, halo, nt):
+    """The adjoint's forward sweep has its NaNs where the tangent linear's values,
+    from the stages, have theirs (also those of halo cells, which reach the interior
+    through slopes alone): in the remap's adjoint such a cell takes its column, in
+    the transport's a cell the three either side of it along i."""
+    case = cases.make_case("C40L8Q2", n=40, npz=8, nq=2, ntiles=nt, courant=0.9, q_split=1, delp_kind=1,
+                           delp_amp=(0.05, 0.2), seed=4)
+    rng = np.random.default_rng(4)
+    for i, j, k in rng.integers((0 if halo else 3, 3, 0), (3 if halo else 43, 43, 8), (9, 3)):
+        case.q[i, j, k] = value
+    print(f"[tlad nonfinite] q {value} halo {halo} tiles {nt}", flush=True)
+    fwd, r = Runner(case, False, 1, 0), Runner(case, False, 1, 9)
+    q1, _, _ = fwd.tl(case.q, np.zeros_like(case.q))
+    qb = r.ad(case.q, grf(case.q.shape, 2))
+    fwd.ctx.close()
+    r.ctx.close()
+    bad = ~np.isfinite(interior(q1)).all(axis=2, keepdims=True)
+    assert bad.any()
+    reach = bad.copy()
+    for m in range(1, 4):
+        reach[m:] |= bad[:-m]
+        reach[:-m] |= bad[m:]
+    assert np.isnan(interior(qb)[np.broadcast_to(reach, interior(qb).shape)]).all()
