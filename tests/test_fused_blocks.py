@@ -25,10 +25,12 @@ int main() {
       }
     }
   for (int rows = 1; rows < 1600; rows = rows < 40 ? rows + 1 : rows * 5 / 4)
-    for (long long units = 1; units < 40000; units *= 3) {
-      const int h = fv3::fused_block_rows(rows, units, 768, 2.5);
-      if (h < 12 || h > 60 || h % 6) return 3;
-    }
+    for (long long units = 1; units < 40000; units *= 3)
+      for (int slots : {512, 768})        // FP64, FP32
+        for (double warm : {4.0, 6.0}) {  // with interior strips, without
+          const int h = fv3::fused_block_rows(rows, units, slots, warm);
+          if (h < 12 || h > 60 || h % 6) return 3;
+        }
   std::puts("ok");
   return 0;
 }
