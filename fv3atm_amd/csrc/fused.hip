@@ -106,10 +106,12 @@ static FusedArgs<T> fused_geometry(const Ctx &c, int nq, int hord) {
       if (strip_ok(st)) { if (s0 < 0) s0 = st; s1 = st; }
     const bool inner = s0 >= 0 && a.lb >= a.lt;
     const int rows = inner ? a.lb - a.lt + 1 : nj;
-    // (resident workgroups of four waves: three per CU in FP32, two in FP64.  A
-    // lean block's six first rows cost about four: with 2.5, two tracers on a
-    // C420 L63 tile 953 us a step and on C260 L127 827, with 4 913 and 800, with
-    // 12 930 and 804; ten or more tracers the same within 0.5 %)
+    // The units are the edge kinds' and FP64's workgroups of four tracers, three
+    // resident per CU in FP32 and two in FP64; the FP32 lean kind, whose workgroups
+    // hold 4 to 32 tracers by configuration, takes the same height, since all kinds of
+    // a pass share it.  A lean block's six first rows cost about four: with 2.5, two
+    // tracers on a C420 L63 tile 953 us a step and on C260 L127 827, with 4 913 and
+    // 800, with 12 930 and 804; ten or more tracers the same within 0.5 %.
     const long long units = (long long)a.nstrip * npz * nt * ((nq + 3) / 4);
     a.H = c.fused_h > 0 ? c.fused_h
                         : fused_block_rows(rows, units, sizeof(T) == 4 ? 768 : 512, inner ? 4.0 : 2.0 * NG);
@@ -122,11 +124,8 @@ static FusedArgs<T> fused_geometry(const Ctx &c, int nq, int hord) {
     }
   }
   const GridDev<T> &g = grid_of<T>(c);
-  a.area = g.area; a.rarea = g.rarea; a.dxa = g.dxa; a.dya = g.dya; a.dx = g.dx; a.dy = g.dy;
-  a.sin_sg = g.sin_sg; a.ms2 = g.s2;
+  a.area = g.area; a.rarea = g.rarea; a.dxa = g.dxa; a.dya = g.dya;
   a.tgs2 = g.s2;
-  a.tgdx = g.sdx;
-  a.tgdy = g.sdy;
   if (sizeof(T) == 4) {
     a.gxp = (const T *)c.gfac32;
     a.gxm = a.gxp + (long long)(d.nid + 1) * d.njd;

@@ -18,12 +18,12 @@ __device__ __forceinline__ void pass_buffers(const FusedArgs<T> &a, int nspl, co
 template <typename T>
 struct StripCtx {
   int i, ic, j0, h, nix, niy, lo_q, lo_fx, lo_mx;  // lane column; block rows; lane offsets in the row layouts
-  bool col_out, lane_in, edge_strip, edge_rows, corner_wg, scale;
+  bool col_out, lane_in, edge_strip, edge_rows, corner_wg;
   T frac;
   const T *cxk, *cyk, *mfxk, *mfyk, *xfxk, *yfxk;
   const double *dp1k;
-  long long tg, tdx, tdy, tgf;  // this tile's offsets in the metric arrays (s2, dx, dy, gfac)
-  EdgeCoef ec;                  // FP32 edge strips: the lane's cube-edge coefficients
+  long long tg, tgf;  // this tile's offsets in the metric arrays (s2, gfac)
+  EdgeCoef ec;        // FP32 edge strips: the lane's cube-edge coefficients
 };
 
 // per tracer streaming state
@@ -309,13 +309,13 @@ __device__ __forceinline__ void row_step(const FusedArgs<T> &a, const StripCtx<T
 // x-fluxes there for the three rows until they are averaged: fewer VGPRs,
 // more waves per CU.
 //
-// FP64 (W = 4, one tracer per wave): 61 KB of LDS, two workgroups per CU.  (A
-// shorter ring for the level arrays, three workgroups, ran the same: 5.2
-// against 5.0 ms; 5 to 8 waves per workgroup 3.3-3.6 against 3.5 ms at 7
-// tracers, 2.2-2.4 against 1.9 at 4: the vector pipe is the bound.)  The form it replaced held its windows in
-// registers (326 of them: one wave per SIMD) and fetched one row ahead into
-// registers, so that every row waited for HBM: C384 L127 9 tracers, two
-// passes: 10.0 -> 5.0 ms.
+// FP64 (W = 4, one tracer per wave): 61 KB of LDS, two workgroups per CU.  The
+// form before held its windows in registers (326 of them: one wave per SIMD) and
+// fetched one row ahead into registers, so that every row waited for HBM: C384
+// L127 9 tracers, two passes: 10.0 -> 5.0 ms.  The vector pipe is the bound now:
+// a shorter ring for the level arrays (three workgroups per CU) took 5.2 ms, and
+// 5 to 8 waves per workgroup 3.3-3.6 against 3.5 ms at 7 tracers, 2.2-2.4 against
+// 1.9 at 4.
 constexpr int LR_DEPTH = 8;  // slots: rows t-4 .. t+3 at row t
 constexpr int LR_AHEAD = 3;  // rows issued ahead of the row computed
 
@@ -637,7 +637,6 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
   if constexpr (sizeof(T) == 4) sc.ec = edge_coef_of(sc.edge_strip ? edge_role(sc.i, a.is, a.ie, a.npx, a.edge) : 0);
   sc.edge_rows = EK != 0 && EK <= 4;
   sc.corner_wg = EK >= 2 && EK <= 4 && a.corners != 0u && fused_reads_corners(i0, j0, h, a.is, a.ie, a.js, a.je);
-  sc.scale = nspl > 1;
   sc.frac = T(1) / T(nspl);
   sc.nix = a.ie - a.is + 2;
   sc.niy = a.ie - a.is + 1;
@@ -645,8 +644,6 @@ __global__ void __launch_bounds__(FT_LANES *W, OCC) k_fused_tp(const FusedArgs<T
   // argument written to is copied to the private stack)
   const long long tile = blockIdx.z;
   sc.tg = tile * a.tgs2;
-  sc.tdx = tile * a.tgdx;
-  sc.tdy = tile * a.tgdy;
   sc.tgf = tile * a.tgf;
   sc.cxk = a.cx + tile * a.tcx + (long long)k * a.sx;
   sc.cyk = a.cy + tile * a.tcy + (long long)k * a.sy;

@@ -53,7 +53,7 @@ struct FusedArgs {
   // metrics and the FP32 factors; halo cells are read from the neighbour
   // tile's interior in the pass input buffer
   int ntiles;
-  long long tq, tcx, tcy, tmx, tmy, tdp, tgs2, tgdx, tgdy, tgf;
+  long long tq, tcx, tcy, tmx, tmy, tdp, tgs2, tgf;
   const int *nsplit;  // per level
   // fields (device)
   const T *q_in;  // step input (also the frozen halo source)
@@ -62,10 +62,9 @@ struct FusedArgs {
   const double *dp1;
   const T *xfx, *yfx;  // FP64 form: area fluxes in the layouts of cx, cy (unscaled)
   // metrics (one tile)
-  const T *area, *rarea, *dxa, *dya, *dx, *dy, *sin_sg;
+  const T *area, *rarea, *dxa, *dya;
   const T *gxp, *gxm, *gyp, *gym;  // FP32 form: combined upwind area-flux factors
   const T *gex;  // FP32 form: per-cell weights of the cube-edge face value (tile stride tgf)
-  long long ms2;                   // metric slab (isd:ied, jsd:jed)
 };
 
 // Block counts of the kernel kinds over (strip, row block): n[0] lean

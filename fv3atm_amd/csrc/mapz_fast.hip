@@ -1147,23 +1147,20 @@ int remap_fast_fields_f32(Ctx &c, int km, int nq, const float *q_src, float *q_d
     fa.ncol = ncol; fa.s2 = d.s2; fa.t_min = (float)t_min;
     fa.q_src = q_src + t * tq; fa.pt_src = pt_src ? pt_src + t * tl : nullptr;
     fa.q_dst = q_dst + t * tq; fa.pt_dst = pt_dst ? pt_dst + t * tl : nullptr; fa.cols = cols;
-    {
-      const char *b = (const char *)cols.d4;
-      const long long cut = (long long)sizeof(float4) * km * ncol, span = (const char *)cols.lk - b + 4LL * km * ncol;
-      fa.o_rbt = (unsigned)((const char *)cols.rbt - b);
-      fa.o_gg = (unsigned)((const char *)cols.gg - b);
-      fa.o_dp1 = (unsigned)((const char *)cols.dp1 - b);
-      fa.o_bot = (unsigned)((const char *)cols.bot - b);
-      fa.o_lk = (unsigned)((const char *)cols.lk - b);
-      fa.b_cols = (unsigned)span;
-      fa.b_cut = (unsigned)cut;
-    }
+    const char *b = (const char *)cols.d4;
+    fa.o_rbt = (unsigned)((const char *)cols.rbt - b);
+    fa.o_gg = (unsigned)((const char *)cols.gg - b);
+    fa.o_dp1 = (unsigned)((const char *)cols.dp1 - b);
+    fa.o_bot = (unsigned)((const char *)cols.bot - b);
+    fa.o_lk = (unsigned)((const char *)cols.lk - b);
+    fa.b_cols = (unsigned)((const char *)cols.lk - b + 4LL * km * ncol);
+    fa.b_cut = (unsigned)((long long)sizeof(float4) * km * ncol);
     const long long ncb = (ncol + RF_COLS - 1) / RF_COLS;
     const long long nwg = ncb * fa.nfg;
     if (nwg > 0x7fffffffLL) return set_error("remap grid too large");
     fa.nwg = (unsigned)nwg;
     const size_t lds = sizeof(float) * fa.nb * RF_COLS * RF_WAVES;
-      hipLaunchKernelGGL((k_remap_fields<RF_B>), dim3((unsigned)nwg), dim3(RF_COLS * RF_WAVES), lds, s, fa);
+    hipLaunchKernelGGL((k_remap_fields<RF_B>), dim3((unsigned)nwg), dim3(RF_COLS * RF_WAVES), lds, s, fa);
     FV3_HIP(hipGetLastError());
   }
   return 0;
