@@ -262,15 +262,15 @@ struct TargetRec {
 // scattered records and stores, and loops of several turns per level, were most
 // of the time (C384 L127, 9 tracers + pt in FP64: 4.86 ms in that form, 3.75 in
 // lockstep, 3.53 with the levels walked by adding to scalar bases and the waves
-// dealt to (column block, field) pairs without gaps; the full remap of C192
-// L127 in FP32, 13 fields: 1.85, 1.65, 1.44 ms).
+// dealt to (column block, field) pairs without gaps, 3.58 with sums divided for any
+// operands; the full remap of C192 L127 in FP32, 13 fields: 1.85, 1.65, 1.44 ms).
 // Only the block ends, one block and the ring are kept (20 KB of LDS per wave
 // in FP64 at 127 levels: two waves per SIMD); the field's second and third
 // reads come from cache.  The divisions by the field-independent pivots use
 // their stored reciprocals (quot).  Bound by dependent FP64 operations at two
 // waves per SIMD (VALU a third busy).  One thread per column looping over its
 // fields with every work array in HBM (at C96 144 waves on 1024 SIMDs) took
-// 18.7 ms for the C384 case, tables included (now 3.53 + 0.45), 1.79 ms for C96
+// 18.7 ms for the C384 case, tables included (now 3.58 + 0.45), 1.79 ms for C96
 // L64 4 tracers + pt (0.125 + 0.027), 12.4 ms for the FP32 remap (1.44 + 0.44).
 template <typename T>
 __global__ void __launch_bounds__(64 * FD_WAVES, sizeof(T) > 8 ? 1 : 2) k_fields(const FieldsArgs<T> a) {

@@ -1,9 +1,8 @@
 """dyn_core's accumulation of the tracer inputs (fv3_dyn_core_fluxes) on the
 GPU against the FP64 oracle (fv3o_dyn_core_fluxes): bit for bit in FP64 on
 one tile and on six faces (delp halos refreshed between sub-steps), in the
-staged form and in the one-launch-per-sub-step form (blocks of 32 x 8 cells:
-sizes 16 and 40 give one block, and full and partial blocks), which also
-equal each other element for element, halos included; within FP32 rounding in
+staged form and in the one-launch-per-sub-step form (strips of 58 columns, rows
+streamed in blocks), which also equal each other element for element, halos included; within FP32 rounding in
 FP32; then end to end, the outputs drive tracer_2d_1L and a constant tracer
 stays constant."""
 import numpy as np
