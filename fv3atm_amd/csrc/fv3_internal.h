@@ -134,6 +134,24 @@ int set_error(const char *fmt, ...);
       return ::fv3::set_error("%s:%d %s: %s", __FILE__, __LINE__, #call, hipGetErrorString(e_)); \
   } while (0)
 
+// A setup that a device needs once before its first launch of some kernels (function
+// attributes belong to the device that is current when they are set).
+struct DeviceOnce {
+  std::mutex mu;
+  std::vector<int> done;
+  template <typename F>
+  hipError_t operator()(F setup) {
+    int dev = 0;
+    if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
+    std::lock_guard<std::mutex> lk(mu);
+    for (const int d : done)
+      if (d == dev) return hipSuccess;
+    const hipError_t e = setup();
+    if (e == hipSuccess) done.push_back(dev);
+    return e;
+  }
+};
+
 void *ctx_scratch(Ctx &c, size_t bytes);
 void *ctx_stage(Ctx &c, size_t bytes);
 

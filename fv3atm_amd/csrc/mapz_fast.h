@@ -36,7 +36,7 @@ RemapCols remap_cols_carve(void *base, int km, long long ncol);
 // and destinations must not overlap.  cols: the first tile's column data, the
 // next tile's cols_stride bytes on; tq: elements between tiles of q.
 int remap_fast_check(int km, long long ncol, long long s2, int kord_tr, int kord_tm, bool with_pt);
-// once per process, before the first remap launch: the lane remap kernel's LDS limit
+// once per device, before the first remap launch: the kernels' LDS limits
 int remap_rows_setup();
 int remap_fast_prep_f32(Ctx &c, int km, const double *ak, const double *bk, double ptop,
                         const double *dp1, double *delp_out, const int *counts, const RemapCols &cols,

@@ -22,7 +22,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <mutex>
 #include <type_traits>
 
 #include "fv3_internal.h"
@@ -1085,22 +1084,20 @@ int remap_fast_prep_f32(Ctx &c, int km, const double *ak, const double *bk, doub
 }
 
 // More than 64 KB of dynamic LDS per workgroup must be allowed per kernel:
-// done once per process, at context creation (before any stream capture).
+// done once per device, at context creation (before any stream capture).
 int remap_rows_setup() {
-  static std::once_flag once;
-  static hipError_t err = hipSuccess;
-  std::call_once(once, [] {
-    const void *fn[3] = {reinterpret_cast<const void *>(&k_remap_rows<2, 16>),
+  static DeviceOnce once;
+  FV3_HIP(once([] {
+    const void *fn[4] = {reinterpret_cast<const void *>(&k_remap_rows<2, 16>),
                          reinterpret_cast<const void *>(&k_remap_rows<4, 16>),
-                         reinterpret_cast<const void *>(&k_remap_rows<4, 32>)};
-    const size_t lds[3] = {rows_lds_bytes<2, 16>(), rows_lds_bytes<4, 16>(), rows_lds_bytes<4, 32>()};
-    for (int v = 0; v < 3 && err == hipSuccess; v++)
+                         reinterpret_cast<const void *>(&k_remap_rows<4, 32>),
+                         reinterpret_cast<const void *>(&k_remap_prep)};
+    const size_t lds[4] = {rows_lds_bytes<2, 16>(), rows_lds_bytes<4, 16>(), rows_lds_bytes<4, 32>(), prep_lds(PREP_MAX_KM)};
+    hipError_t err = hipSuccess;
+    for (int v = 0; v < 4 && err == hipSuccess; v++)
       err = hipFuncSetAttribute(fn[v], hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds[v]);
-    if (err == hipSuccess)
-      err = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_remap_prep),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)prep_lds(PREP_MAX_KM));
-  });
-  FV3_HIP(err);
+    return err;
+  }));
   return 0;
 }
 

@@ -109,7 +109,7 @@ struct FieldsArgs {
   signed char kord[REMAP_MAX_NQ + FIELDS_MAX_SETS];  // by field
 };
 
-// once per process, before any capture: the kernels' LDS limits
+// once per device, before any capture: the kernels' LDS limits
 int fields_setup();
 // tables of the columns (ni x nj per tile, every tile of c); iv2: factors of
 // the iv = -2 solve (bottom value given)

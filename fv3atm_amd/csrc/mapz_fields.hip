@@ -13,7 +13,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <mutex>
 
 #include "fv3_internal.h"
 #include "mapz_fields.h"
@@ -751,10 +750,10 @@ ColTab<R> coltab_carve(void *base, int km, long long ncols) {
 
 // More than 64 KB of dynamic LDS per workgroup must be allowed per kernel.
 int fields_setup() {
-  static std::once_flag once;
-  static hipError_t err = hipSuccess;
-  std::call_once(once, [] {
-    auto allow = [](const void *fn, size_t b) {
+  static DeviceOnce once;
+  FV3_HIP(once([] {
+    hipError_t err = hipSuccess;
+    auto allow = [&](const void *fn, size_t b) {
       if (err == hipSuccess) err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)b);
     };
     allow(reinterpret_cast<const void *>(&k_fields_prep<float>), prep_lds(FIELDS_MAX_KM));
@@ -762,8 +761,8 @@ int fields_setup() {
     allow(reinterpret_cast<const void *>(&k_fields<float>), fields_lds<float>(FIELDS_MAX_KM));
     allow(reinterpret_cast<const void *>(&k_fields<double>), fields_lds<double>(FIELDS_MAX_KM));
     allow(reinterpret_cast<const void *>(&k_fields<D1>), std::min<size_t>(fields_lds<D1>(FIELDS_MAX_KM), 160 * 1024));
-  });
-  FV3_HIP(err);
+    return err;
+  }));
   return 0;
 }
 
