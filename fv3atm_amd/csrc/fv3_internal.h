@@ -82,7 +82,7 @@ struct Ctx {
   bool timing = false;
   // fused-kernel launch shape: configuration id and interior rows per block
   int fused_cfg = FUSED32_DEFAULT_CFG, fused_h = 0;
-  // FP32 step remap: 0 column-shared fast kernel, 1 one thread per column
+  // FP32 step remap: 0 column-shared fast kernel, 1 in upstream's evaluation order
   int remap_mode = 0;
   // fused step's sub-cycling: per-level nsplit(k) (tracer_2d_1L) or one
   // nsplit for every level (tracer_2d), forced to q_split when > 0

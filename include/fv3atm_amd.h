@@ -173,8 +173,9 @@ int fv3_ctx_set_timing(fv3_ctx *ctx, int on);
  * block (0 = chosen by the tile's size, at most 60);
  * remap the vertical remap kernel: 0 (default) = column-shared, a column's
  * levels spread over 16 or 32 lanes of a wave (npz <= 127; larger npz take
- * kernel 2), 1 = one thread per column, 2 = column-shared, one thread per
- * (column, field).  Transport results do not depend on cfg/rows; the remap
+ * kernel 2), 1 = upstream's evaluation order (one thread per (column, field);
+ * above 255 levels one per column), 2 = column-shared, one thread per (column,
+ * field; npz <= 512).  Transport results do not depend on cfg/rows; the remap
  * kernels agree to FP32 rounding. */
 int fv3_ctx_set_launch(fv3_ctx *ctx, int cfg, int rows, int remap);
 /* No counterpart upstream: run the fused transport's two edge kernels (the

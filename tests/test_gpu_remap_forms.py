@@ -8,13 +8,14 @@ of a call whose columns are all displaced the same way (in step); the tangent li
 by its values (1e-12) and the dot product with the adjoint (1e-12)."""
 import numpy as np
 import pytest
+import torch
 
 import fv3atm_amd as fa
 from fv3atm_amd import cases
 from oracle import oracle
 from tests._util import assert_close, interior
 from tests.test_gpu_l2e import _interior, _run_gpu, _run_ref
-from tests.test_gpu_tlad import Runner, dot, grf
+from tests.test_gpu_tlad import Runner, _dev, dot, grf
 
 pytestmark = pytest.mark.gpu
 
@@ -109,3 +110,66 @@ def test_full_remap_long(gpu_ready, hydrostatic, nt):
     for k in ("u", "v", "pt", "q", "delp", "pkz") + (() if hydrostatic else ("w", "delz")):
         a, b = _interior(k, got[k], case.n), _interior(k, ref[k], case.n)
         assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max(), k
+
+
+@pytest.mark.parametrize("nt,n", [(1, 200), (6, 82)])
+def test_tracers_in_parts(gpu_ready, nt, n):
+    """More tracers than the in-place remap copies at a time (512 MB): each as in a
+    call with fewer (six or more: the same integral form)."""
+    km, nq, half = 127, 13, 7
+    case = cases.make_case(f"{nt}xC{n}L{km}Q1", n=n, npz=km, nq=1, ntiles=nt, delp_kind=1, delp_amp=(0.05, 0.1), seed=n,
+                           with_pt=True)
+    print(f"[remap forms] {nt} x C{n} L{km}, {nq} tracers", flush=True)
+    k = np.arange(km) / km
+    q = np.stack([1.0 + 0.5 * np.sin((3.0 + m) * k) for m in range(nq)], axis=-1)  # (level, tracer)
+    shape = case.dp1.shape[:3] + (nq,) + case.dp1.shape[3:]
+    full = np.empty(shape, order="F")
+    full[...] = q.reshape((1, 1, km, nq) + (1,) * (full.ndim - 4))
+    assert full.nbytes > 512 << 20
+    ctx = fa.Context(case.grids, km)
+
+    def remap(part):
+        a = [np.array(x, order="F") for x in (full[:, :, :, part], case.dp1, case.pt)]
+        fa.lagrangian_to_eulerian_tracers(ctx, km, a[0].shape[3], case.ak, case.bk, case.ptop, a[1], a[0], a[2], 9, 10)
+        return a
+
+    whole, first, rest = remap(slice(0, nq)), remap(slice(0, half)), remap(slice(half - 1, nq))
+    ctx.close()
+    np.testing.assert_array_equal(whole[0][:, :, :, :half], first[0])
+    np.testing.assert_array_equal(whole[0][:, :, :, half - 1:], rest[0])
+    for a, b in zip(whole[1:], first[1:]):
+        np.testing.assert_array_equal(a, b)
+    assert not np.array_equal(whole[0][5, 5], full[5, 5])
+
+
+def test_derivative_tracers_in_parts(gpu_ready):
+    """More tracers than the tangent linear's field launch takes (64) and than the
+    adjoint's remap holds scratch for (2 GB): each as in calls with fewer."""
+    n, npz, nq = 150, 16, 72
+    case = cases.make_case("C150L16Q1", n=n, npz=npz, nq=1, courant=0.4, q_split=1, delp_kind=1, delp_amp=(0.05, 0.1),
+                           seed=2)
+    assert 8 * n * n * (npz + 2) * 16 * nq > 2 << 30
+    print(f"[remap forms] C{n} L{npz}, {nq} tracers, tangent linear and adjoint", flush=True)
+    d = {k: _dev(getattr(case, k)) for k in ("dp1", "cx", "cy", "mfx", "mfy", "ak", "bk")}
+    g = torch.Generator(device="cuda").manual_seed(1)
+    shape = (nq, npz, n + 6, n + 6)
+    q0 = 1.0 + torch.rand(shape, generator=g, device="cuda", dtype=torch.float64)
+    dq = torch.zeros_like(q0)
+    dq[..., 3:-3, 3:-3] = torch.rand((nq, npz, n, n), generator=g, device="cuda", dtype=torch.float64)
+    ctx = fa.Context(case.grids, npz)
+
+    def pair(a, b):
+        q, dd = q0[a:b].contiguous(), dq[a:b].contiguous()
+        q1, dq1, qb = (torch.zeros_like(q) for _ in range(3))
+        delp = torch.zeros_like(d["dp1"])
+        tail = (d["cx"], d["cy"], d["mfx"], d["mfy"], d["ak"], d["bk"], case.ptop, 8, 9)
+        fa.step_tl_dev(ctx, False, 1, b - a, q, dd, q1, dq1, d["dp1"], delp, *tail)
+        fa.step_ad_dev(ctx, False, 1, b - a, q, dd, qb, d["dp1"], *tail)
+        torch.cuda.synchronize()
+        return q1, dq1, qb
+
+    whole = pair(0, nq)
+    for a, b in ((0, 10), (58, 70), (62, 72)):
+        for x, y in zip(whole, pair(a, b)):
+            assert torch.equal(x[a:b], y), (a, b)
+    ctx.close()
